@@ -72,26 +72,30 @@ def algorithmic_bytes(plan):
     coordinates, window tables and weights are shared by all slices and left out."""
     M, n0, n1, N0, N1 = plan.M, plan.n0, plan.n1, plan.N0, plan.N1
     grid = 8 * n0 * n1
+    # width a power of two: the iteration's images are real, its grid rows hold
+    # the columns 0..n1/2 (in n1/2 + 8), and half of the nodes give all values
+    half = N0 & (N0 - 1) == 0
+    rows = 8 * N0 * (n1 // 2 + 8 if half else n1)
+    nodes, img = (M // 2 if half else M), (4 if half else 8)
     return {
-        # interpolation: the full oversampled grid once + the node values once
+        # the update: image and Re(rhat) in, image out (f32), the reference iterate in; + the grid rows out
+        "row_fwd": 16 * N0 * N1 + rows,
+        # A^H W A along x: the grid rows in and out + the node values of the residual out
+        "col_normal": 2 * rows + 8 * nodes,
+        # grid rows in + A^H W b in + Re(rhat) out (f32, all the update reads) + the grid rows of rhat out
+        "row_adj": 2 * rows + (img + 4) * N0 * N1,
+        # the grid rows of rhat in
+        "col_energy": rows,
+        # the residual (node partials, <= 3 per node, and data in) and the step size (row and tile sums)
+        "combine": 24 * nodes + 8 * M + 8 * N0 + n1,
+        # transforms: node values and the full oversampled grid once
         "col_fwd": grid + 8 * M,
-        # spread: the node values once + the full oversampled grid once
         "col_adj": 8 * M + grid,
-        # the update: image and Re(rhat) in, image out (f32); + the N0 non-zero grid rows out
-        "row_fwd": 12 * N0 * N1 + 8 * N0 * n1,
-        # N0 grid rows in + A^H W b in (c64) + Re(rhat) out (f32, all the update reads) + the N0 grid
-        # rows of A rhat out
-        "row_adj": 8 * N0 * n1 + 12 * N0 * N1 + 8 * N0 * n1,
-        # interpolation partials in (<= 2 per node) + data + weighted values out
-        "combine": 16 * M + 8 * M + 8 * M,
-        # the step size: interpolation partials of A rhat in + the row sums of |rhat|^2 (f64)
-        "combine_alpha": 16 * M + 8 * N0,
     }
 
 
-# row_adj also does the row pass of A rhat (fused), so row_fwd runs once; the
-# second combine is the step size's
-LAUNCHES_PER_ITER = {"row_fwd": 1, "col_fwd": 2, "combine": 1, "col_adj": 1, "row_adj": 1, "combine_alpha": 1}
+LAUNCHES_PER_ITER = {"row_fwd": 1, "col_normal": 1, "row_adj": 1, "col_energy": 1, "combine": 1}
+TRANSFORM_KERNELS = ("col_fwd", "col_adj")
 
 
 def cpu_model():
@@ -135,7 +139,7 @@ COPY_BYTES = 1 << 30
 
 
 def iteration_roofline(plan, S, per_iter_ms):
-    """One ICON iteration (7 launches) against HBM with this build's own
+    """One ICON iteration (5 launches) against HBM with this build's own
     algorithmic bytes per slice: the per-kernel bytes of algorithmic_bytes()
     times the launches per iteration.  The reference's dataflow (17 G + 6 S +
     8 I_c + 3 I_r per slice: three FFTs, pads, spread, two interpolations,
@@ -236,7 +240,7 @@ def measure_traffic(kernel, S):
     plain read request, is calibrated on a 1 GiB copy (its reads then equal
     1 GiB; on gfx950 u = 128, a full L2 line) and the copy's write bytes are
     checked against 1 GiB the same way."""
-    name = {"col_fwd": "k_col_fwd", "col_adj": "k_col_adj", "row_fwd": "k_row_fwd", "row_adj": "k_row_adj"}[kernel]
+    name = "k_" + kernel
     rk = counter_pass(READ_COUNTERS, kernel, S, name)
     wk = counter_pass(WRITE_COUNTERS, kernel, S, name)
     rc = counter_pass(READ_COUNTERS, "copy", S, "k_copy_f4")
@@ -500,7 +504,7 @@ def config3_bench(args):
                value=round(total / dt_packed, 2), per_series_slices_per_s=round(total / dt_series, 2),
                speedup=round(dt_series / dt_packed, 3), same_result=bool(same), series=len(specs), slices=total,
                iterations=iters, schedule=[pre, icon_it, post], launches_per_iteration=batch.launches_per_iteration(),
-               launches_per_iteration_one_at_a_time=7 * len(specs), grid_and_tile_classes=classes,
+               launches_per_iteration_one_at_a_time=5 * len(specs), grid_and_tile_classes=classes,
                device_gb=round(dev_bytes / 1e9, 1), slice_scale=args.c3_scale, steps=args.steps, warmup=args.warmup,
                resid_final_mean=float(np.mean([r[:, -1].mean() for r in r_packed])))
     print(json.dumps(out), flush=True)
@@ -623,8 +627,11 @@ def main():
         gbs = kb[k] * S / (kt[k] * 1e-3) / 1e9
         kernels[k] = dict(ms=round(kt[k], 4), algo_bytes_per_slice=kb[k], GBs=round(gbs, 1),
                           share=round(share[k] / per_iter_ms, 3))
+    for k in TRANSFORM_KERNELS:
+        ms = plan.time_kernel(k, S, args.kernel_reps)
+        kernels[k] = dict(ms=round(ms, 4), algo_bytes_per_slice=kb[k], GBs=round(kb[k] * S / (ms * 1e-3) / 1e9, 1))
     log("kernels:", json.dumps(kernels))
-    dom = max(("col_fwd", "col_adj"), key=lambda k: share[k])
+    dom = max(share, key=share.get)
     ach = kb[dom] * S / (kt[dom] * 1e-3) / 1e9
     roofline = dict(bound="hbm", achieved=round(ach, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                     frac=round(ach / HBM_PEAK_GBS, 4), traffic=None, kernel=dom,
@@ -644,7 +651,7 @@ def main():
         log("Kaiser-Bessel (width 6) plan: kernel timing and a plain solve")
         pk = feilab_amd.Plan(cfg["N"], cfg["tilt"], max_slices=S, device=0, window="kb6")
         kk = {}
-        for k in ("col_fwd", "col_adj"):
+        for k in TRANSFORM_KERNELS:
             ms = pk.time_kernel(k, S, args.kernel_reps)
             gbs = kb[k] * S / (ms * 1e-3) / 1e9
             kk[k] = dict(ms=round(ms, 4), GBs=round(gbs, 1), frac=round(gbs / HBM_PEAK_GBS, 4))

@@ -70,7 +70,7 @@ struct icon_batch {
   int device = 0;
   std::vector<icon_plan*> plans;
   std::vector<int> S;
-  std::vector<int> C_built;   // column tile of each plan when the items were built
+  std::vector<int> C_built;   // column tile of each plan's spread when the items were built
   hipStream_t stream = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
   // item tables per size class
@@ -78,6 +78,8 @@ struct icon_batch {
   // the spread's items: those of col, by their tile's entry count, largest
   // first across the class's series (each tile's blocks stay together)
   std::vector<Items> col_adj;
+  std::vector<Items> normal;   // the normal operator's column kernels, by n0
+  std::vector<Items> row_grad, row64;   // the iteration's gradient; rows (or pairs) of the FP64 one
   Items combine;
   // argument blocks, one per series (device copies written before each solve)
   std::vector<RowFwdArgs> h_rf;
@@ -86,12 +88,24 @@ struct icon_batch {
   std::vector<CombineArgs> h_cm;
   std::vector<SinoArgs> h_sa;
   std::vector<ReprojArgs> h_rp;
+  std::vector<RowAdjArgs> h_rg, h_rg2;     // gradient; ... against the reference iterate
+  std::vector<RowFwdArgs> h_rf2, h_rr;     // row pass against the reference iterate; of rhat
+  std::vector<RefArgs> h_re;
+  std::vector<ColArgs> h_c64;
+  std::vector<ColArgs> h_cn, h_ce, h_cl;   // normal operator; energy; last forward pass
+  std::vector<FinishArgs> h_fa;
   RowFwdArgs* d_rf = nullptr;
   RowAdjArgs* d_ra = nullptr;
   ColArgs* d_ca = nullptr;
   CombineArgs* d_cm = nullptr;
   SinoArgs* d_sa = nullptr;
   ReprojArgs* d_rp = nullptr;
+  RowAdjArgs *d_rg = nullptr, *d_rg2 = nullptr;
+  RowFwdArgs *d_rf2 = nullptr, *d_rr = nullptr;
+  RefArgs* d_re = nullptr;
+  ColArgs* d_c64 = nullptr;
+  ColArgs *d_cn = nullptr, *d_ce = nullptr, *d_cl = nullptr;
+  FinishArgs* d_fa = nullptr;
   hipGraphExec_t graph = nullptr;
   SolveKey graph_key;
 };
@@ -120,13 +134,16 @@ int build_items(icon_batch* b) {
   free_items(b->row_adj);
   free_items(b->col);
   free_items(b->col_adj);
+  free_items(b->normal);
+  free_items(b->row_grad);
+  free_items(b->row64);
   free_items(b->sino);
   free_items(b->reproj);
   if (b->combine.d) (void)hipFree(b->combine.d);
   b->combine = Items{};
   const int ns = (int)b->plans.size();
   b->C_built.assign(ns, 0);
-  for (int i = 0; i < ns; i++) b->C_built[i] = b->plans[i]->bins.C;
+  for (int i = 0; i < ns; i++) b->C_built[i] = b->plans[i]->spread().h.C;
   auto group = [](std::vector<Items>& v, int k0, int k1, int k2) -> Items& {
     for (auto& it : v)
       if (it.key0 == k0 && it.key1 == k1 && it.key2 == k2) return it;
@@ -135,20 +152,36 @@ int build_items(icon_batch* b) {
     return v.back();
   };
   for (int i = 0; i < ns; i++) {
-    const icon_plan* p = b->plans[i];
+    icon_plan* p = b->plans[i];
     const Geometry& g = p->g;
+    const Bins& sb = p->spread().h;
     const int S = b->S[i];
     const int rows = S * g.N0;
-    Items& rf = group(b->row_fwd, g.n1, 0, 0);
-    const int rpf = row_fwd_rows_per_block(g.n1);
+    // the iteration's row kernels: key1 1 for real rows, two per transform
+    const int half = p->half ? 1 : 0;
+    // (key2 1: series that take FP64 gradients)
+    const int r64ok = p->refreshes() ? 1 : 0;
+    Items& rf = group(b->row_fwd, g.n1, half, r64ok);
+    const int rpf = half ? 2 * half_row_pairs_per_block(g.n1) : row_fwd_rows_per_block(g.n1);
     for (int k = 0; k < (rows + rpf - 1) / rpf; k++) rf.h.push_back(make_int2(i, k));
-    Items& ra = group(b->row_adj, g.n1, 0, 0);
-    const int rpa = row_adj_rows_per_block(g.n1);
-    for (int k = 0; k < (rows + rpa - 1) / rpa; k++) ra.h.push_back(make_int2(i, k));
-    if (!col_tile_ok(g.n0, g.n1, p->bins.C, g.K))
-      return bfail(ICON_ERR_ARG, "series %d: column tile %d unsupported for grid %d x %d", i, p->bins.C, g.n0, g.n1);
-    Items& cl = group(b->col, g.n0, p->bins.C, g.K);
-    for (int k = 0; k < S * (g.n1 / p->bins.C); k++) cl.h.push_back(make_int2(i, k));
+    // the data adjoint's rows: key1 1 in FP64 (one row per block)
+    const int a64 = adj64_ok(g.n0, sb.C, sb.K) ? 1 : 0;
+    Items& ra = group(b->row_adj, g.n1, a64, 0);
+    const int rpa = row_adj_rows_per_block(g.n1), rpd = a64 ? 1 : rpa;
+    for (int k = 0; k < (rows + rpd - 1) / rpd; k++) ra.h.push_back(make_int2(i, k));
+    if (r64ok) {
+      Items& r64 = group(b->row64, g.n1, half, 0);
+      for (int k = 0; k < (half ? rows / 2 : rows); k++) r64.h.push_back(make_int2(i, k));
+    }
+    Items& rg = group(b->row_grad, g.n1, half, r64ok);
+    const int rpg = half ? 2 * half_row_pairs_per_block(g.n1) : rpa;
+    for (int k = 0; k < (rows + rpg - 1) / rpg; k++) rg.h.push_back(make_int2(i, k));
+    if (!col_tile_ok(g.n0, g.n1, sb.C, sb.K))
+      return bfail(ICON_ERR_ARG, "series %d: column tile %d unsupported for grid %d x %d", i, sb.C, g.n0, g.n1);
+    Items& cl = group(b->col, g.n0, sb.C, sb.K);
+    for (int k = 0; k < S * (g.n1 / sb.C); k++) cl.h.push_back(make_int2(i, k));
+    Items& nm = group(b->normal, g.n0, 0, 0);
+    for (int k = 0; k < S * (p->ncol / kNormalC); k++) nm.h.push_back(make_int2(i, k));
     Items& sn = group(b->sino, g.n0, 0, 0);
     const int rps = sino_rows_per_block(g.n0);
     for (int k = 0; k < (S * g.nz + rps - 1) / rps; k++) sn.h.push_back(make_int2(i, k));
@@ -163,15 +196,15 @@ int build_items(icon_batch* b) {
     Items a = c;
     a.d = nullptr;
     auto cnt = [&](const int2& q) {
-      const icon_plan* p = b->plans[q.x];
-      const int t = p->bins.order[q.y / b->S[q.x]];
-      return p->bins.off[t + 1] - p->bins.off[t];
+      const Bins& sb = b->plans[q.x]->spread().h;
+      const int t = sb.order[q.y / b->S[q.x]];
+      return sb.off[t + 1] - sb.off[t];
     };
     std::stable_sort(a.h.begin(), a.h.end(), [&](const int2& u, const int2& v) { return cnt(u) > cnt(v); });
     b->col_adj.push_back(std::move(a));
   }
   int rc;
-  for (auto* v : {&b->row_fwd, &b->row_adj, &b->col, &b->col_adj, &b->sino, &b->reproj})
+  for (auto* v : {&b->row_fwd, &b->row_adj, &b->col, &b->col_adj, &b->normal, &b->row_grad, &b->row64, &b->sino, &b->reproj})
     for (auto& it : *v)
       if ((rc = upload_items(it))) return rc;
   if ((rc = upload_items(b->combine))) return rc;
@@ -190,7 +223,7 @@ void drop_batch_graph(icon_batch* b) {
 
 // Argument blocks of every series for a solve on the given buffers.
 void fill_args(icon_batch* b, const float* const* sino, float* const* m, float* const* reproj, double* const* resid,
-               double* const* alpha, int iters) {
+               double* const* alpha, int iters, bool any_resid) {
   const int ns = (int)b->plans.size();
   b->h_rf.assign(ns, RowFwdArgs{});
   b->h_ra.assign(ns, RowAdjArgs{});
@@ -198,32 +231,44 @@ void fill_args(icon_batch* b, const float* const* sino, float* const* m, float* 
   b->h_cm.assign(ns, CombineArgs{});
   b->h_sa.assign(ns, SinoArgs{});
   b->h_rp.assign(ns, ReprojArgs{});
+  for (auto* v : {&b->h_rg, &b->h_rg2}) v->assign(ns, RowAdjArgs{});
+  for (auto* v : {&b->h_rf2, &b->h_rr}) v->assign(ns, RowFwdArgs{});
+  b->h_re.assign(ns, RefArgs{});
+  for (auto* v : {&b->h_cn, &b->h_ce, &b->h_cl, &b->h_c64}) v->assign(ns, ColArgs{});
+  b->h_fa.assign(ns, FinishArgs{});
   for (int i = 0; i < ns; i++) {
     icon_plan* p = b->plans[i];
     const Geometry& g = p->g;
     const int S = b->S[i];
-    const int E = (int)p->bins.ent.size();
     RowFwdArgs& rf = b->h_rf[i];
     rf.rows = S * g.N0; rf.N0 = g.N0; rf.N1 = g.N1; rf.m = m[i]; rf.grad = p->d_grad; rf.alpha = p->d_alpha;
-    rf.ck = p->d_ck; rf.tw = p->d_tw1; rf.out = p->d_tmp;
+    rf.tw = p->d_tw1; rf.out = p->d_tmp;
+    // the adjoint of the data set-up, then the gradient
     RowAdjArgs& ra = b->h_ra[i];
-    ra.rows = S * g.N0; ra.N0 = g.N0; ra.N1 = g.N1; ra.in = p->d_tmp; ra.ck = p->d_ck; ra.tw = p->d_tw1;
-    ra.img = p->d_ahwb; ra.ahwb = p->d_ahwb; ra.grad = p->d_grad; ra.rowpart = p->d_rowpart; ra.fwd_out = p->d_tmp;
-    ColArgs& ca = b->h_ca[i];
-    ca.S = S; ca.N0 = g.N0; ca.N1 = g.N1; ca.M = g.M; ca.n1 = g.n1; ca.E = E; ca.K = g.K;
-    ca.in = p->d_tmp; ca.out = p->d_tmp; ca.tw = p->d_tw0; ca.ent_off = p->d_ent_off; ca.tile_order = p->d_tile_order; ca.split_min = split_min_entries(p->bins); ca.ent = p->d_ent;
-    ca.xoff = p->d_xoff; ca.phix = p->d_phix; ca.phiy = p->d_phiy; ca.ix0 = p->d_ix0; ca.ent_px = p->d_ent_px;
-    ca.ent_py = p->d_ent_py; ca.fent = p->d_fent; ca.fent_px = p->d_fent_px; ca.fent_py = p->d_fent_py;
-    ca.part = p->d_part; ca.fw = p->d_fw;
-    zero_band(p->bins, &rf.zlo, &rf.zhi);
-    zero_band(p->bins, &ra.zlo, &ra.zhi);
-    zero_band(p->bins, &ca.zlo, &ca.zhi);
+    ra = data_row_args(p, S);
+    b->h_rg[i] = grad_args(p, S);
+    b->h_rg2[i] = b->h_rg[i];
+    b->h_rf2[i] = rf;
+    if (p->refreshes()) {
+      b->h_rg2[i].ahwb = p->d_base;
+      b->h_rg2[i].ahwb_re = reinterpret_cast<const float*>(p->d_base);
+      b->h_rf2[i].mref = p->d_mref;
+    }
+    b->h_rr[i] = rhat_row_args(p, S);
+    b->h_re[i] = ref_args(p, S, m[i]);
+    b->h_c64[i] = normal64_args(p, S, any_resid);
+    b->h_ca[i] = spread_args(p, S);
     CombineArgs& cm = b->h_cm[i];
-    cm.S = S; cm.M = g.M; cm.N0 = g.N0; cm.nz = g.nz; cm.E = E; cm.part = p->d_part; cm.nslot = p->d_nslot;
-    cm.w = p->d_w; cm.b = p->d_b; cm.fw = p->d_fw; cm.ent_of_node = p->d_ent_of_node; cm.bnorm = p->d_bnorm;
-    cm.resid = resid ? resid[i] : nullptr; cm.resid_stride = iters + 1; cm.rowpart = p->d_rowpart;
-    cm.alpha = p->d_alpha; cm.alpha_trace = alpha ? alpha[i] : nullptr; cm.alpha_stride = iters;
-    cm.frep = p->d_frep; cm.iomit = g.iomit;
+    cm.S = S; cm.M = g.M; cm.N0 = g.N0; cm.nz = g.nz; cm.mode = 2; cm.E = b->h_ca[i].E;
+    cm.w = p->d_w; cm.b = p->d_b; cm.fw = p->d_fw; cm.ent_of_node = p->spread().of_node; cm.bnorm = p->d_bnorm;
+    b->h_cn[i] = normal_args(p, S, any_resid);
+    b->h_ce[i] = energy_args(p, S);
+    b->h_cl[i] = normal_args(p, S, true);
+    FinishArgs& fa = b->h_fa[i];
+    fa = finish_args(p, S);
+    fa.beff = p->refreshes() ? p->d_beff : nullptr;
+    fa.resid = resid ? resid[i] : nullptr; fa.resid_stride = iters + 1; fa.frep = p->d_frep;
+    fa.alpha = p->d_alpha; fa.alpha_trace = alpha ? alpha[i] : nullptr; fa.alpha_stride = iters;
     SinoArgs& sa = b->h_sa[i];
     sa.rows = S * g.nz; sa.N0 = g.N0; sa.K = g.K; sa.nz = g.nz; sa.skip = g.cv_skip; sa.sino = sino[i];
     sa.ck1 = p->d_ck1; sa.phi1 = p->d_phi1; sa.i10 = p->d_i10; sa.tw = p->d_tw0; sa.b = p->d_b;
@@ -251,34 +296,63 @@ int enqueue_batch(icon_batch* b, float* const* m, const float* const* m_init, bo
   const int ns = (int)b->plans.size();
   const int iters = o.pre + o.icon + o.post;
   int rc;
-  auto col_all = [&](bool adj) -> int {
-    for (auto& it : adj ? b->col_adj : b->col)
-      if ((rc = ck(launch_col_multi(it.key0, it.key1, it.key2, adj, b->d_ca, it.d, it.n(), st),
-                   adj ? "col_adj" : "col_fwd")))
+  // which: series with (1) or without (0) FP64 gradients, -1: all
+  auto row_fwd_all = [&](const RowFwdArgs* d, int update, int which) -> int {
+    for (auto& it : b->row_fwd) {
+      if (which >= 0 && it.key2 != which) continue;
+      // rhat's row pass: complex images on full grids
+      RowFwdLaunch L{d == b->d_rr && !it.key1 ? 1 : 0, update, o.data_type, o.threshold};
+      if ((rc = ck(it.key1 ? launch_row_fwd_half_multi(it.key0, d, it.d, it.n(), L, st)
+                           : launch_row_fwd_multi(it.key0, d, it.d, it.n(), L, st), "row_fwd")))
         return rc;
+    }
     return ICON_OK;
   };
-  auto row_fwd_all = [&](int update) -> int {
+  auto gradient = [&](bool against_ref, int update, int which) -> int {
+    if ((rc = row_fwd_all(against_ref ? b->d_rf2 : b->d_rf, update, which))) return rc;
+    for (auto& nm : b->normal)
+      if (which < 0 || (nm.key0 <= 1024) == (which == 1))
+        if ((rc = ck(launch_col_normal_multi(nm.key0, b->d_cn, nm.d, nm.n(), st), "col_normal"))) return rc;
+    for (auto& it : b->row_grad) {
+      if (which >= 0 && it.key2 != which) continue;
+      const RowAdjArgs* d = against_ref ? b->d_rg2 : b->d_rg;
+      if ((rc = ck(it.key1 ? launch_row_grad_half_multi(it.key0, d, it.d, it.n(), st)
+                           : launch_row_adj_multi(it.key0, d, it.d, it.n(), true, st), "row_grad")))
+        return rc;
+    }
+    return ICON_OK;
+  };
+  // the gradient in FP64 from the whole images (as in enqueue_solve), where a
+  // series takes it
+  auto reference = [&](int update) -> int {
     RowFwdLaunch L{0, update, o.data_type, o.threshold};
-    for (auto& it : b->row_fwd)
-      if ((rc = ck(launch_row_fwd_multi(it.key0, b->d_rf, it.d, it.n(), L, st), "row_fwd"))) return rc;
-    return ICON_OK;
+    for (auto& it : b->row64)
+      if ((rc = ck(launch_row_fwd64_multi(it.key0, it.key1, b->d_re, it.d, it.n(), L, st), "row_fwd64"))) return rc;
+    for (auto& nm : b->normal)
+      if (nm.key0 <= 1024)
+        if ((rc = ck(launch_col_normal64_multi(nm.key0, b->d_c64, nm.d, nm.n(), st), "col_normal64"))) return rc;
+    for (auto& it : b->row64)
+      if ((rc = ck(launch_row_grad64_multi(it.key0, it.key1, b->d_re, it.d, it.n(), st), "row_grad64"))) return rc;
+    if ((rc = row_fwd_all(b->d_rr, 0, 1))) return rc;
+    return gradient(false, update, 0);
   };
-  auto row_adj_all = [&](int mode, bool fwd) -> int {
-    for (auto& it : b->row_adj)
-      if ((rc = ck(launch_row_adj_multi(it.key0, b->d_ra, it.d, it.n(), mode, fwd, st), "row_adj"))) return rc;
-    return ICON_OK;
-  };
-  auto combine = [&](int mode, int ri, int ai, int with_frep) -> int {
-    CombineLaunch L{mode, ri, ai, 1, with_frep};
-    return ck(launch_combine_multi(b->d_cm, b->combine.d, b->combine.n(), L, st), "combine");
+  auto finish = [&](int ri, int ai, bool with_frep, int beff) -> int {
+    FinishLaunch L{any_resid ? ri : -1, ai, with_frep ? 1 : 0, beff};
+    return ck(launch_finish_multi(b->d_fa, b->combine.d, b->combine.n(), L, st), "finish");
   };
   // data set-up: b, w b, bnorm, A^H W b
   for (auto& it : b->sino)
     if ((rc = ck(launch_sino_multi(it.key0, b->d_sa, it.d, it.n(), st), "sino"))) return rc;
-  if ((rc = combine(2, 0, 0, 0))) return rc;
-  if ((rc = col_all(true))) return rc;
-  if ((rc = row_adj_all(0, false))) return rc;
+  if ((rc = ck(launch_combine_multi(b->d_cm, b->combine.d, b->combine.n(), st), "combine"))) return rc;
+  for (auto& it : b->col_adj)
+    if ((rc = ck(adj64_ok(it.key0, it.key1, it.key2)
+                     ? launch_col_adj64_multi(it.key0, it.key1, b->d_ca, it.d, it.n(), st)
+                     : launch_col_multi(it.key0, it.key1, it.key2, true, b->d_ca, it.d, it.n(), st), "col_adj")))
+      return rc;
+  for (auto& it : b->row_adj)
+    if ((rc = ck(it.key1 ? launch_row_adj64_multi(it.key0, b->d_ra, it.d, it.n(), st)
+                         : launch_row_adj_multi(it.key0, b->d_ra, it.d, it.n(), false, st), "row_adj")))
+      return rc;
   // m = 0 or the warm start
   for (int i = 0; i < ns; i++) {
     const size_t n = (size_t)b->S[i] * b->plans[i]->g.N0 * b->plans[i]->g.N1;
@@ -286,20 +360,23 @@ int enqueue_batch(icon_batch* b, float* const* m, const float* const* m_init, bo
     if ((rc = ck(e, "init"))) return rc;
   }
   auto phase = [&](int it) { return (o.pre <= it && it < iters - o.post) ? 2 : 1; };
+  bool referred = false;
   for (int it = 0; it < iters; it++) {
-    if ((rc = row_fwd_all(it == 0 ? 0 : phase(it - 1)))) return rc;
-    if ((rc = col_all(false))) return rc;
-    if ((rc = combine(0, it, 0, 0))) return rc;
-    if ((rc = col_all(true))) return rc;
-    if ((rc = row_adj_all(1, true))) return rc;
-    if ((rc = col_all(false))) return rc;
-    if ((rc = combine(1, 0, it, 0))) return rc;
+    const int update = it == 0 ? 0 : phase(it - 1);
+    bool ref = false;
+    for (const icon_plan* p : b->plans) ref |= refresh(p, o, it);
+    if ((rc = ref ? reference(update) : gradient(referred, update, -1))) return rc;
+    for (auto& nm : b->normal)
+      if ((rc = ck(launch_col_energy_multi(nm.key0, b->d_ce, nm.d, nm.n(), st), "col_energy"))) return rc;
+    if ((rc = finish(it, it, false, ref ? 1 : referred ? 2 : 0))) return rc;
+    referred |= ref;
   }
   if (iters > 0 || any_resid || any_reproj)
-    if ((rc = row_fwd_all(iters > 0 ? phase(iters - 1) : 0))) return rc;
+    if ((rc = row_fwd_all(b->d_rf, iters > 0 ? phase(iters - 1) : 0, -1))) return rc;
   if (any_resid || any_reproj) {
-    if ((rc = col_all(false))) return rc;
-    if ((rc = combine(0, iters, 0, any_reproj ? 1 : 0))) return rc;
+    for (auto& nm : b->normal)
+      if ((rc = ck(launch_col_fwd_nodes_multi(nm.key0, b->d_cl, nm.d, nm.n(), st), "col_fwd"))) return rc;
+    if ((rc = finish(iters, -1, any_reproj, 0))) return rc;
     if (any_reproj)
       for (auto& it : b->reproj)
         if ((rc = ck(launch_reproj_multi(it.key0, b->d_rp, it.d, it.n(), st), "reproj"))) return rc;
@@ -322,10 +399,15 @@ int icon_batch_destroy(icon_batch* b) {
   free_items(b->row_adj);
   free_items(b->col);
   free_items(b->col_adj);
+  free_items(b->normal);
+  free_items(b->row_grad);
+  free_items(b->row64);
   free_items(b->sino);
   free_items(b->reproj);
   if (b->combine.d) (void)hipFree(b->combine.d);
-  for (void* q : {(void*)b->d_rf, (void*)b->d_ra, (void*)b->d_ca, (void*)b->d_cm, (void*)b->d_sa, (void*)b->d_rp})
+  for (void* q : {(void*)b->d_rf, (void*)b->d_ra, (void*)b->d_ca, (void*)b->d_cm, (void*)b->d_sa, (void*)b->d_rp,
+                  (void*)b->d_cn, (void*)b->d_ce, (void*)b->d_cl, (void*)b->d_rg, (void*)b->d_fa,
+                  (void*)b->d_rg2, (void*)b->d_rf2, (void*)b->d_rr, (void*)b->d_re, (void*)b->d_c64})
     if (q) (void)hipFree(q);
   if (b->ev_in) (void)hipEventDestroy(b->ev_in);
   if (b->ev_out) (void)hipEventDestroy(b->ev_out);
@@ -371,6 +453,14 @@ int icon_batch_create(icon_batch** out, int nseries, icon_plan* const* plans, co
   if (e == hipSuccess) e = hipMalloc(&b->d_cm, sizeof(CombineArgs) * nseries);
   if (e == hipSuccess) e = hipMalloc(&b->d_sa, sizeof(SinoArgs) * nseries);
   if (e == hipSuccess) e = hipMalloc(&b->d_rp, sizeof(ReprojArgs) * nseries);
+  if (e == hipSuccess) e = hipMalloc(&b->d_rg, sizeof(RowAdjArgs) * nseries);
+  if (e == hipSuccess) e = hipMalloc(&b->d_rg2, sizeof(RowAdjArgs) * nseries);
+  if (e == hipSuccess) e = hipMalloc(&b->d_rf2, sizeof(RowFwdArgs) * nseries);
+  if (e == hipSuccess) e = hipMalloc(&b->d_rr, sizeof(RowFwdArgs) * nseries);
+  if (e == hipSuccess) e = hipMalloc(&b->d_re, sizeof(RefArgs) * nseries);
+  for (ColArgs** q : {&b->d_cn, &b->d_ce, &b->d_cl, &b->d_c64})
+    if (e == hipSuccess) e = hipMalloc(q, sizeof(ColArgs) * nseries);
+  if (e == hipSuccess) e = hipMalloc(&b->d_fa, sizeof(FinishArgs) * nseries);
   if (e != hipSuccess) return done(bfail(ICON_ERR_DEVICE, "icon_batch_create: %s", hipGetErrorString(e)));
   return done(build_items(b));
 }
@@ -425,7 +515,7 @@ int icon_batch_reconstruct(icon_batch* b, const void* const* d_sino, void* const
   // a plan whose column tile changed since the items were built (its bins
   // have another tile count): rebuild the items before any launch
   for (int i = 0; i < ns && rc == ICON_OK; i++)
-    if (b->plans[i]->bins.C != b->C_built[i]) {
+    if (b->plans[i]->spread().h.C != b->C_built[i]) {
       drop_batch_graph(b);
       rc = build_items(b);
     }
@@ -436,10 +526,15 @@ int icon_batch_reconstruct(icon_batch* b, const void* const* d_sino, void* const
     if (e != hipSuccess) { rc = bfail(ICON_ERR_DEVICE, "icon_batch_reconstruct: %s", hipGetErrorString(e)); break; }
     if (!(b->graph && b->graph_key == key)) {
       drop_batch_graph(b);
-      fill_args(b, sino.data(), m.data(), rp.data(), rs.data(), al.data(), iters);
+      fill_args(b, sino.data(), m.data(), rp.data(), rs.data(), al.data(), iters, any_resid);
       if ((rc = upload_args(b->d_rf, b->h_rf, b->stream)) || (rc = upload_args(b->d_ra, b->h_ra, b->stream)) ||
           (rc = upload_args(b->d_ca, b->h_ca, b->stream)) || (rc = upload_args(b->d_cm, b->h_cm, b->stream)) ||
-          (rc = upload_args(b->d_sa, b->h_sa, b->stream)) || (rc = upload_args(b->d_rp, b->h_rp, b->stream)))
+          (rc = upload_args(b->d_sa, b->h_sa, b->stream)) || (rc = upload_args(b->d_rp, b->h_rp, b->stream)) ||
+          (rc = upload_args(b->d_rg, b->h_rg, b->stream)) || (rc = upload_args(b->d_rg2, b->h_rg2, b->stream)) ||
+          (rc = upload_args(b->d_rf2, b->h_rf2, b->stream)) || (rc = upload_args(b->d_rr, b->h_rr, b->stream)) ||
+          (rc = upload_args(b->d_re, b->h_re, b->stream)) || (rc = upload_args(b->d_c64, b->h_c64, b->stream)) ||
+          (rc = upload_args(b->d_cn, b->h_cn, b->stream)) ||
+          (rc = upload_args(b->d_ce, b->h_ce, b->stream)) || (rc = upload_args(b->d_cl, b->h_cl, b->stream)) || (rc = upload_args(b->d_fa, b->h_fa, b->stream)))
         break;
       e = hipStreamSynchronize(b->stream);
       if (e == hipSuccess) e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
@@ -471,7 +566,7 @@ int icon_batch_reconstruct(icon_batch* b, const void* const* d_sino, void* const
 
 int icon_batch_launches_per_iteration(const icon_batch* b, int* launches) {
   if (!b || !launches) return bfail(ICON_ERR_ARG, "icon_batch_launches_per_iteration: null pointer");
-  *launches = (int)b->row_fwd.size() + (int)b->row_adj.size() + 3 * (int)b->col.size() + 2;
+  *launches = (int)b->row_fwd.size() + (int)b->row_grad.size() + 2 * (int)b->normal.size() + 1;
   return ICON_OK;
 }
 
@@ -488,7 +583,7 @@ int icon_batch_autotune(icon_batch* b, int* col_blocks) {
   const int ns = (int)b->plans.size();
   // classes by (n0, K)
   std::map<std::pair<int, int>, std::vector<int>> cls;
-  for (int i = 0; i < ns; i++) cls[{b->plans[i]->g.n0, b->plans[i]->g.K}].push_back(i);
+  for (int i = 0; i < ns; i++) cls[{b->plans[i]->g.n0, b->plans[i]->op.h.K}].push_back(i);
   int rc = ICON_OK;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   (void)hipEventCreate(&e0);
@@ -505,10 +600,10 @@ int icon_batch_autotune(icon_batch* b, int* col_blocks) {
       for (int i : kv.second) ok = ok && col_tile_ok(n0, b->plans[i]->g.n1, C, K);
       if (!ok) continue;
       for (int i : kv.second)
-        if (b->plans[i]->bins.C != C && (rc = icon_plan_set_col_block(b->plans[i], C)))
+        if (b->plans[i]->op.h.C != C && (rc = icon_plan_set_col_block(b->plans[i], C)))
           return bfail(rc, "icon_batch_autotune: %s", icon_last_error());
       if ((rc = build_items(b))) return rc;
-      fill_args(b, sino.data(), m.data(), rp.data(), rs.data(), al.data(), 0);
+      fill_args(b, sino.data(), m.data(), rp.data(), rs.data(), al.data(), 0, false);
       if ((rc = upload_args(b->d_ca, b->h_ca, b->stream))) return rc;
       const Items *it = nullptr, *ia = nullptr;
       for (auto& c : b->col)
@@ -534,14 +629,14 @@ int icon_batch_autotune(icon_batch* b, int* col_blocks) {
     }
     if (rc) break;
     for (int i : kv.second)
-      if (best_c && b->plans[i]->bins.C != best_c && (rc = icon_plan_set_col_block(b->plans[i], best_c)))
+      if (best_c && b->plans[i]->op.h.C != best_c && (rc = icon_plan_set_col_block(b->plans[i], best_c)))
         return bfail(rc, "icon_batch_autotune: %s", icon_last_error());
   }
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   if (!rc) rc = build_items(b);
   if (!rc && col_blocks)
-    for (int i = 0; i < ns; i++) col_blocks[i] = b->plans[i]->bins.C;
+    for (int i = 0; i < ns; i++) col_blocks[i] = b->plans[i]->op.h.C;
   if (prev >= 0 && prev != b->device) (void)hipSetDevice(prev);
   return rc;
 }

@@ -49,6 +49,29 @@ int fail(int code, const char* fmt, ...) {
 std::mutex g_tw_mu;
 std::map<std::pair<int, int>, float2*> g_tw;
 
+// exp(-2 pi i q / n), q < n, in double, per (device, n).
+std::map<std::pair<int, int>, double2*> g_w64;
+
+int twiddles64(int n, const double2** out) {
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lk(g_tw_mu);
+  auto key = std::make_pair(dev, n);
+  auto it = g_w64.find(key);
+  if (it != g_w64.end()) { *out = it->second; return ICON_OK; }
+  std::vector<double2> w(n);
+  for (int q = 0; q < n; q++) {
+    const double a = -2.0 * M_PI * (double)q / (double)n;
+    w[q] = make_double2(std::cos(a), std::sin(a));
+  }
+  double2* d = nullptr;
+  HIPCHK(hipMalloc(&d, sizeof(double2) * n));
+  HIPCHK(hipMemcpy(d, w.data(), sizeof(double2) * n, hipMemcpyHostToDevice));
+  g_w64[key] = d;
+  *out = d;
+  return ICON_OK;
+}
+
 int twiddles(int n, const float2** out) {
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
@@ -110,41 +133,69 @@ int upload(icon_plan* p, T** ptr, const std::vector<T>& h) {
   return ICON_OK;
 }
 
-void free_bins(icon_plan* p) {
-  if (p->d_ent_off) (void)hipFree(p->d_ent_off);
-  if (p->d_tile_order) (void)hipFree(p->d_tile_order);
-  p->d_tile_order = nullptr;
-  if (p->d_ent) (void)hipFree(p->d_ent);
-  if (p->d_nslot) (void)hipFree(p->d_nslot);
-  if (p->d_xoff) (void)hipFree(p->d_xoff);
-  if (p->d_ent_px) (void)hipFree(p->d_ent_px);
-  if (p->d_ent_py) (void)hipFree(p->d_ent_py);
-  if (p->d_ent_of_node) (void)hipFree(p->d_ent_of_node);
-  if (p->d_fw) (void)hipFree(p->d_fw);
-  if (p->d_fent) (void)hipFree(p->d_fent);
-  if (p->d_fent_px) (void)hipFree(p->d_fent_px);
-  if (p->d_fent_py) (void)hipFree(p->d_fent_py);
-  p->d_ent_off = nullptr; p->d_ent = nullptr; p->d_nslot = nullptr; p->d_xoff = nullptr;
-  p->d_ent_px = nullptr; p->d_ent_py = nullptr; p->d_ent_of_node = nullptr; p->d_fw = nullptr;
-  p->d_fent = nullptr; p->d_fent_px = nullptr; p->d_fent_py = nullptr;
+void free_bins(DevBins& b) {
+  for (void* q : {(void*)b.ck, (void*)b.off, (void*)b.order, (void*)b.xoff, (void*)b.of_node, (void*)b.ent,
+                  (void*)b.fent, (void*)b.px, (void*)b.py, (void*)b.fpx, (void*)b.fpy, (void*)b.nslot})
+    if (q) (void)hipFree(q);
+  b = DevBins{};
 }
 
-int upload_bins(icon_plan* p) {
+// Bins of a Kaiser-Bessel window of K taps in tiles of C columns; records and
+// deapodisation are computed on the device.
+int make_bins(icon_plan* p, DevBins& b, int C, int K) {
+  const Geometry& g = p->g;
+  build_bins(g, C, K, b.h);
+  b.beta0 = kb_beta(g.sig0, K);
+  b.beta1 = kb_beta(g.sig1, K);
+  const size_t E = b.h.ent.size();
+  std::vector<float> c(g.N0 + g.N1);
+  kb_deapod(g.N0, g.sig0, b.beta0, K, c.data());
+  kb_deapod(g.N1, g.sig1, b.beta1, K, c.data() + g.N0);
   int rc;
-  if ((rc = upload(p, &p->d_ent_off, p->bins.off))) return rc;
-  if ((rc = upload(p, &p->d_tile_order, p->bins.order))) return rc;
-  if ((rc = upload(p, &p->d_ent, p->bins.ent))) return rc;
-  if ((rc = upload(p, &p->d_nslot, p->bins.nslot))) return rc;
-  if ((rc = upload(p, &p->d_xoff, p->bins.xoff))) return rc;
-  if ((rc = upload(p, &p->d_ent_px, p->bins.px))) return rc;
-  if ((rc = upload(p, &p->d_ent_py, p->bins.py))) return rc;
-  if ((rc = upload(p, &p->d_ent_of_node, p->bins.of_node))) return rc;
-  if ((rc = upload(p, &p->d_fent, p->bins.fent))) return rc;
-  if ((rc = upload(p, &p->d_fent_px, p->bins.fpx))) return rc;
-  if ((rc = upload(p, &p->d_fent_py, p->bins.fpy))) return rc;
-  // weighted node value per bin entry, per slice
-  if ((rc = dalloc(p, &p->d_fw, (size_t)p->S_max * p->bins.ent.size()))) return rc;
+  if ((rc = upload(p, &b.off, b.h.off)) || (rc = upload(p, &b.order, b.h.order)) || (rc = upload(p, &b.ent, b.h.ent)) ||
+      (rc = upload(p, &b.fent, b.h.fent)) || (rc = upload(p, &b.nslot, b.h.nslot)) ||
+      (rc = upload(p, &b.xoff, b.h.xoff)) || (rc = upload(p, &b.of_node, b.h.of_node)) ||
+      (rc = dalloc(p, &b.px, E * K)) || (rc = dalloc(p, &b.py, E * C)) || (rc = dalloc(p, &b.fpx, E * K)) ||
+      (rc = dalloc(p, &b.fpy, E * C)) || (rc = dalloc(p, &b.ck, (size_t)g.N0 * g.N1)))
+    return rc;
+  float* dc = nullptr;
+  HIPCHK(hipMalloc(&dc, sizeof(float) * c.size()));
+  hipError_t e = hipMemcpy(dc, c.data(), sizeof(float) * c.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = launch_outer(dc, dc + g.N0, g.N0, g.N1, b.ck, p->stream);
+  if (e == hipSuccess)
+    e = launch_window_records(b.ent, b.off, p->d_nodes, (int)E, g.n0, g.n1, K, C, b.beta0, b.beta1, b.px, b.py, p->stream);
+  if (e == hipSuccess)
+    e = launch_window_records(b.fent, b.off, p->d_nodes, (int)E, g.n0, g.n1, K, C, b.beta0, b.beta1, b.fpx, b.fpy,
+                              p->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(p->stream);
+  (void)hipFree(dc);
+  if (e != hipSuccess) return fail(ICON_ERR_DEVICE, "window tables: %s", hipGetErrorString(e));
   return ICON_OK;
+}
+
+int op_taps(const Geometry& g) { return g.window == ICON_WINDOW_KB6 ? kTapsKB : kTapsWide; }
+
+// The transforms' bins at tile width C, and the weighted values' buffer.
+int make_op_bins(icon_plan* p, int C) {
+  if (p->d_fw) (void)hipFree(p->d_fw);
+  p->d_fw = nullptr;
+  free_bins(p->op);
+  int rc = make_bins(p, p->op, C, op_taps(p->g));
+  if (rc) return rc;
+  const size_t E = std::max(p->op.h.ent.size(), p->data.h.ent.size());
+  return dalloc(p, &p->d_fw, (size_t)p->S_max * E);
+}
+
+// Column-kernel arguments of a window's bins over S slices.
+ColArgs window_args(icon_plan* p, const DevBins& b, int S) {
+  const Geometry& g = p->g;
+  ColArgs a{};
+  a.K = b.h.K; a.S = S; a.N0 = g.N0; a.N1 = g.N1; a.M = g.M; a.n1 = g.n1; a.E = (int)b.h.ent.size();
+  a.in = p->d_tmp; a.out = p->d_tmp; a.tw = p->d_tw0; a.ent_off = b.off; a.tile_order = b.order;
+  a.split_min = split_min_entries(b.h); a.ent = b.ent; a.xoff = b.xoff; a.ent_px = b.px; a.ent_py = b.py;
+  a.fent = b.fent; a.fent_px = b.fpx; a.fent_py = b.fpy; a.part = p->d_part; a.slots = kMaxSlot; a.fw = p->d_fw;
+  zero_band(b.h, &a.zlo, &a.zhi);
+  return a;
 }
 
 void drop_graph(icon_plan* p) {
@@ -182,53 +233,40 @@ int check_launch(hipError_t e, const char* what) {
 
 int op_forward(icon_plan* p, int S, const void* img, int cplx, float2* out, hipStream_t st) {
   const Geometry& g = p->g;
+  const ColArgs ca = window_args(p, p->op, S);
   RowFwdArgs ra{};
   ra.rows = S * g.N0; ra.N0 = g.N0; ra.N1 = g.N1; ra.cplx = cplx; ra.update = 0;
   ra.m = cplx ? nullptr : (float*)img;
   ra.rhat = cplx ? (const float2*)img : nullptr;
-  ra.ck = p->d_ck; ra.tw = p->d_tw1; ra.out = p->d_tmp;
-  zero_band(p->bins, &ra.zlo, &ra.zhi);
+  ra.ck = p->op.ck; ra.tw = p->d_tw1; ra.out = p->d_tmp; ra.zlo = ca.zlo; ra.zhi = ca.zhi;
   int rc = check_launch(launch_row_fwd(g.n1, ra, st), "row_fwd");
   if (rc) return rc;
-  ColArgs ca{};
-  ca.K = p->g.K;
-  ca.S = S; ca.N0 = g.N0; ca.N1 = g.N1; ca.M = g.M; ca.n1 = g.n1;
-  ca.in = p->d_tmp; ca.tw = p->d_tw0; ca.ent_off = p->d_ent_off; ca.tile_order = p->d_tile_order; ca.split_min = split_min_entries(p->bins); ca.ent = p->d_ent; ca.xoff = p->d_xoff; ca.E = (int)p->bins.ent.size(); ca.ent_px = p->d_ent_px; ca.ent_py = p->d_ent_py;
-  ca.fent = p->d_fent; ca.fent_px = p->d_fent_px; ca.fent_py = p->d_fent_py;
-  ca.phix = p->d_phix; ca.phiy = p->d_phiy; ca.ix0 = p->d_ix0; ca.part = p->d_part;
-  if ((rc = check_launch(launch_col(g.n0, p->bins.C, false, ca, st), "col_fwd"))) return rc;
+  if ((rc = check_launch(launch_col(g.n0, p->op.h.C, false, ca, st), "col_fwd"))) return rc;
   CombineArgs cb{};
   cb.S = S; cb.M = g.M; cb.N0 = g.N0; cb.nz = g.nz; cb.mode = 3; cb.part = p->d_part;
-  cb.nslot = p->d_nslot; cb.w = p->d_w; cb.fw = out;
+  cb.nslot = p->op.nslot; cb.w = p->d_w; cb.fw = out;
   return check_launch(launch_combine(cb, st), "combine");
 }
 
-// A^H of the per-entry weighted values already in p->d_fw.
-int op_adjoint_ent(icon_plan* p, int S, float2* img, hipStream_t st) {
+// A^H of the per-entry weighted values already in p->d_fw (entries of b): the
+// image, or its real part to img_re.
+int op_adjoint_ent(icon_plan* p, const DevBins& b, int S, float2* img, hipStream_t st, float* img_re = nullptr) {
   const Geometry& g = p->g;
-  const float2* f = p->d_fw;
-  ColArgs ca{};
-  ca.K = p->g.K;
-  ca.S = S; ca.N0 = g.N0; ca.N1 = g.N1; ca.M = g.M; ca.n1 = g.n1;
-  ca.out = p->d_tmp; ca.tw = p->d_tw0; ca.ent_off = p->d_ent_off; ca.tile_order = p->d_tile_order; ca.split_min = split_min_entries(p->bins); ca.ent = p->d_ent; ca.xoff = p->d_xoff; ca.E = (int)p->bins.ent.size(); ca.ent_px = p->d_ent_px; ca.ent_py = p->d_ent_py;
-  ca.fent = p->d_fent; ca.fent_px = p->d_fent_px; ca.fent_py = p->d_fent_py;
-  ca.phix = p->d_phix; ca.phiy = p->d_phiy; ca.ix0 = p->d_ix0; ca.fw = f;
-  zero_band(p->bins, &ca.zlo, &ca.zhi);
-  int rc = check_launch(launch_col(g.n0, p->bins.C, true, ca, st), "col_adj");
+  const ColArgs ca = window_args(p, b, S);
+  int rc = check_launch(launch_col(g.n0, b.h.C, true, ca, st), "col_adj");
   if (rc) return rc;
   RowAdjArgs ra{};
-  ra.rows = S * g.N0; ra.N0 = g.N0; ra.N1 = g.N1; ra.mode = 0; ra.in = p->d_tmp;
-  ra.ck = p->d_ck; ra.tw = p->d_tw1; ra.img = img;
-  zero_band(p->bins, &ra.zlo, &ra.zhi);
+  ra.rows = S * g.N0; ra.N0 = g.N0; ra.N1 = g.N1; ra.in = p->d_tmp;
+  ra.ck = b.ck; ra.tw = p->d_tw1; ra.img = img; ra.img_re = img_re; ra.zlo = ca.zlo; ra.zhi = ca.zhi;
   return check_launch(launch_row_adj(g.n1, ra, st), "row_adj");
 }
 
 // A^H of node vectors f [S][M].
 int op_adjoint(icon_plan* p, int S, const float2* f, float2* img, hipStream_t st) {
-  int rc = check_launch(launch_node_to_ent(f, p->d_fw, p->d_ent, S, p->g.M, (int)p->bins.ent.size(), st),
+  int rc = check_launch(launch_node_to_ent(f, p->d_fw, p->op.ent, S, p->g.M, (int)p->op.h.ent.size(), st),
                         "node_to_ent");
   if (rc) return rc;
-  return op_adjoint_ent(p, S, img, st);
+  return op_adjoint_ent(p, p->op, S, img, st);
 }
 
 int op_sino(icon_plan* p, int S, const float* sino, float2* b, hipStream_t st) {
@@ -239,6 +277,26 @@ int op_sino(icon_plan* p, int S, const float* sino, float2* b, hipStream_t st) {
   sa.phi1 = p->d_phi1;
   sa.i10 = p->d_i10; sa.tw = p->d_tw0; sa.b = b;
   return check_launch(launch_sino(g.n0, sa, st), "sino");
+}
+
+// A^H of the data's weighted values in p->d_fw, as the gradient subtracts it
+// (with paired nodes its real part), in FP64 where the plan takes FP64 gradients.
+int op_adjoint_data(icon_plan* p, int S, hipStream_t st) {
+  const DevBins& b = p->spread();
+  float* re = p->half ? reinterpret_cast<float*>(p->d_ahwb) : nullptr;
+  if (!adj64_ok(p->g.n0, b.h.C, b.h.K)) return op_adjoint_ent(p, b, S, re ? nullptr : p->d_ahwb, st, re);
+  int rc = check_launch(launch_col_adj64(p->g.n0, b.h.C, spread_args(p, S), st), "col_adj64");
+  if (rc) return rc;
+  return check_launch(launch_row_adj64(p->g.n1, data_row_args(p, S), st), "row_adj64");
+}
+
+// An iteration's launches over S slices: with paired nodes the real-row
+// kernels on half grids, otherwise the full ones.
+hipError_t iter_row_fwd(icon_plan* p, const RowFwdArgs& a, hipStream_t st) {
+  return p->half ? launch_row_fwd_half(p->g.n1, a, st) : launch_row_fwd(p->g.n1, a, st);
+}
+hipError_t iter_row_grad(icon_plan* p, const RowAdjArgs& a, hipStream_t st) {
+  return p->half ? launch_row_grad_half(p->g.n1, a, st) : launch_row_adj(p->g.n1, a, st);
 }
 
 // The whole solve of S slices, enqueued on st (captured into a graph by the caller
@@ -253,11 +311,11 @@ int enqueue_solve(icon_plan* p, int S, const float* sino, float* m, const float*
     if ((rc = op_sino(p, S, sino, p->d_b, st))) return rc;
     CombineArgs c0{};
     c0.S = S; c0.M = g.M; c0.N0 = g.N0; c0.nz = g.nz; c0.mode = 2; c0.b = p->d_b; c0.w = p->d_w;
-    c0.fw = p->d_fw; c0.bnorm = p->d_bnorm; c0.nslot = p->d_nslot; c0.part = p->d_part;
-    c0.E = (int)p->bins.ent.size(); c0.ent_of_node = p->d_ent_of_node;
+    c0.fw = p->d_fw; c0.bnorm = p->d_bnorm;
+    c0.E = (int)p->spread().h.ent.size(); c0.ent_of_node = p->spread().of_node;
     if ((rc = check_launch(launch_combine(c0, st), "combine_b"))) return rc;
     // A^H W b
-    if ((rc = op_adjoint_ent(p, S, p->d_ahwb, st))) return rc;
+    if ((rc = op_adjoint_data(p, S, st))) return rc;
   }
   // m = 0 (Iteration2.cu:33) or the warm start
   const size_t NN = (size_t)g.N0 * g.N1;
@@ -267,59 +325,66 @@ int enqueue_solve(icon_plan* p, int S, const float* sino, float* m, const float*
 
   RowFwdArgs rf{};
   rf.rows = S * g.N0; rf.N0 = g.N0; rf.N1 = g.N1; rf.data_type = o.data_type; rf.thr = o.threshold;
-  rf.m = m; rf.grad = p->d_grad; rf.alpha = p->d_alpha; rf.ck = p->d_ck; rf.tw = p->d_tw1; rf.out = p->d_tmp;
-  ColArgs ca{};
-  ca.K = p->g.K;
-  ca.S = S; ca.N0 = g.N0; ca.N1 = g.N1; ca.M = g.M; ca.n1 = g.n1; ca.in = p->d_tmp; ca.out = p->d_tmp;
-  ca.tw = p->d_tw0; ca.ent_off = p->d_ent_off; ca.tile_order = p->d_tile_order; ca.split_min = split_min_entries(p->bins); ca.ent = p->d_ent; ca.xoff = p->d_xoff; ca.E = (int)p->bins.ent.size(); ca.ent_px = p->d_ent_px; ca.ent_py = p->d_ent_py;
-  ca.fent = p->d_fent; ca.fent_px = p->d_fent_px; ca.fent_py = p->d_fent_py; ca.phix = p->d_phix; ca.phiy = p->d_phiy;
-  ca.ix0 = p->d_ix0; ca.part = p->d_part; ca.fw = p->d_fw;
-  CombineArgs cm{};
-  cm.S = S; cm.M = g.M; cm.N0 = g.N0; cm.nz = g.nz; cm.mode = 0; cm.part = p->d_part; cm.nslot = p->d_nslot;
-  cm.w = p->d_w; cm.b = p->d_b; cm.fw = p->d_fw; cm.bnorm = p->d_bnorm; cm.resid = resid;
-  cm.resid_stride = iters + 1; cm.iomit = g.iomit;
-  cm.E = (int)p->bins.ent.size(); cm.ent_of_node = p->d_ent_of_node;
-  CombineArgs cr = cm;
-  cr.mode = 1; cr.resid = nullptr; cr.rowpart = p->d_rowpart; cr.alpha = p->d_alpha; cr.alpha_trace = alpha_tr;
-  cr.alpha_stride = iters;
-  RowAdjArgs ra{};
-  ra.rows = S * g.N0; ra.N0 = g.N0; ra.N1 = g.N1; ra.mode = 1; ra.in = p->d_tmp; ra.ck = p->d_ck;
-  ra.tw = p->d_tw1; ra.ahwb = p->d_ahwb; ra.grad = p->d_grad; ra.rowpart = p->d_rowpart;
-  ra.fwd_out = p->d_tmp;   // the row pass of A rhat fused in
-  zero_band(p->bins, &rf.zlo, &rf.zhi);
-  zero_band(p->bins, &ca.zlo, &ca.zhi);
-  zero_band(p->bins, &ra.zlo, &ra.zhi);
+  rf.m = m; rf.grad = p->d_grad; rf.alpha = p->d_alpha; rf.tw = p->d_tw1; rf.out = p->d_tmp;
+  ColArgs ca = normal_args(p, S, resid != nullptr);
+  const ColArgs ce = energy_args(p, S), c64 = normal64_args(p, S, resid != nullptr);
+  RowAdjArgs ra = grad_args(p, S);
+  RefArgs rr = ref_args(p, S, m);
+  rr.data_type = o.data_type; rr.thr = o.threshold;
+  FinishArgs fa = finish_args(p, S);
+  fa.resid = resid; fa.resid_stride = iters + 1; fa.alpha = p->d_alpha; fa.alpha_trace = alpha_tr;
+  fa.alpha_stride = iters;
   auto phase = [&](int it) { return (o.pre <= it && it < iters - o.post) ? 2 : 1; };
 
   for (int it = 0; it < iters; it++) {
-    // f = A m (with the previous iteration's update fused in front)
-    rf.cplx = 0;
-    rf.update = it == 0 ? 0 : phase(it - 1);
-    if ((rc = check_launch(launch_row_fwd(g.n1, rf, st), "row_fwd"))) return rc;
-    if ((rc = check_launch(launch_col(g.n0, p->bins.C, false, ca, st), "col_fwd"))) return rc;
-    // R(m_it), fw = w f
-    cm.resid_index = it;
-    cm.frep = nullptr;
-    if ((rc = check_launch(launch_combine(cm, st), "combine_m"))) return rc;
-    // rhat = A^H fw - A^H W b, row sums of |rhat|^2, and the row pass of A rhat
-    if ((rc = check_launch(launch_col(g.n0, p->bins.C, true, ca, st), "col_adj"))) return rc;
-    if ((rc = check_launch(launch_row_adj(g.n1, ra, st), "row_adj"))) return rc;
-    // alpha = |rhat|^2 / sum w |A rhat|^2
-    if ((rc = check_launch(launch_col(g.n0, p->bins.C, false, ca, st), "col_fwd_c"))) return rc;
-    cr.alpha_index = it;
-    if ((rc = check_launch(launch_combine(cr, st), "combine_r"))) return rc;
+    const int update = it == 0 ? 0 : phase(it - 1);
+    const bool ref = refresh(p, o, it);
+    if (ref) {
+      // the iterate's gradient in FP64, from the whole image; from here on the
+      // transforms take the difference from it
+      rr.update = update;
+      if ((rc = check_launch(launch_row_fwd64(g.n1, p->half, rr, st), "row_fwd64"))) return rc;
+      if ((rc = check_launch(launch_col_normal64(g.n0, c64, st), "col_normal64"))) return rc;
+      if ((rc = check_launch(launch_row_grad64(g.n1, p->half, rr, st), "row_grad64"))) return rc;
+      if ((rc = check_launch(iter_row_fwd(p, rhat_row_args(p, S), st), "row_fwd_rhat"))) return rc;
+      rf.mref = p->d_mref;
+      ra.ahwb = p->d_base;
+      ra.ahwb_re = reinterpret_cast<const float*>(p->d_base);
+      fa.b = p->d_b;
+      fa.beff = p->d_beff;
+    } else {
+      // y FFT of m (with the previous iteration's update fused in front)
+      rf.update = update;
+      if ((rc = check_launch(iter_row_fwd(p, rf, st), "row_fwd"))) return rc;
+      // A^H W A m up to its inverse y FFT, and A m at the nodes for R(m_it)
+      if ((rc = check_launch(launch_col_normal(g.n0, ca, st), "col_normal"))) return rc;
+      // rhat = A^H W A m - A^H W b, row sums of |rhat|^2, y FFT of rhat
+      if ((rc = check_launch(iter_row_grad(p, ra, st), "row_adj"))) return rc;
+    }
+    // <rhat, A^H W A rhat> by column tile
+    if ((rc = check_launch(launch_col_energy(g.n0, ce, st), "col_energy"))) return rc;
+    // alpha = |rhat|^2 / <rhat, A^H W A rhat>, R(m_it)
+    fa.resid_index = fa.alpha_index = it;
+    if ((rc = check_launch(launch_finish(fa, st), "finish"))) return rc;
+    if (ref) {
+      fa.beff = nullptr;
+      fa.b = p->d_beff;
+    }
   }
+  rf.mref = nullptr;
+  fa.b = p->d_b;
   // last update, then A m_final for the final residual and the reprojection
   if (iters > 0 || resid || reproj) {
-    rf.cplx = 0;
     rf.update = iters > 0 ? phase(iters - 1) : 0;
-    if ((rc = check_launch(launch_row_fwd(g.n1, rf, st), "row_fwd_final"))) return rc;
+    if ((rc = check_launch(iter_row_fwd(p, rf, st), "row_fwd_final"))) return rc;
   }
   if (resid || reproj) {
-    if ((rc = check_launch(launch_col(g.n0, p->bins.C, false, ca, st), "col_fwd_final"))) return rc;
-    cm.resid_index = iters;
-    cm.frep = reproj ? p->d_frep : nullptr;
-    if ((rc = check_launch(launch_combine(cm, st), "combine_final"))) return rc;
+    ca = normal_args(p, S, true);
+    if ((rc = check_launch(launch_col_fwd_nodes(g.n0, ca, st), "col_fwd_final"))) return rc;
+    fa.resid_index = iters;
+    fa.alpha = nullptr;
+    fa.frep = reproj ? p->d_frep : nullptr;
+    if ((rc = check_launch(launch_finish(fa, st), "finish_final"))) return rc;
     if (reproj) {
       ReprojArgs rp{};
       rp.K = p->g.K;
@@ -328,6 +393,82 @@ int enqueue_solve(icon_plan* p, int S, const float* sino, float* m, const float*
       if ((rc = check_launch(launch_reproj(g.n0, rp, st), "reproj"))) return rc;
     }
   }
+  return ICON_OK;
+}
+
+// The normal operator's tables: interpolation entries and records, spectrum
+// and, with paired nodes, the unpaired nodes' waves.  The spectrum takes
+// 2 M n0 n1 FP64 operations on the matrix cores, in chunks of nodes whose
+// factors fit the scratch.
+int build_normal(icon_plan* p) {
+  const Geometry& g = p->g;
+  p->half = g.nz <= kMaxUnpaired && paired_nodes(g);
+  p->nq = p->half ? g.nz : 0;
+  p->rows = p->half ? g.nz * (g.N0 / 2 + 1) : g.M;
+  p->ncol = p->half ? g.n1 / 2 + kNormalC : g.n1;
+  NodeBins nb, ub;
+  build_node_bins(g, p->half, nb);
+  if (p->half) {
+    unpaired_bins(g, nb, ub);
+  } else {
+    ub.off.assign(nb.off.size(), 0);   // no entries
+  }
+  std::vector<int4> entr = ub.ent;
+  for (int4& e : entr) e.x /= g.N0 / 2 + 1;   // rows of d_rpart: the tilt line
+  const size_t E = nb.ent.size(), U = ub.ent.size(), cells = (size_t)g.n0 * g.n1;
+  const size_t S = (size_t)p->S_max;
+  double chol[kInterpTaps * kInterpTaps];
+  interp_factor(chol);
+  int rc;
+  if ((rc = upload(p, &p->d_nd_off, nb.off)) || (rc = upload(p, &p->d_nd_ent, nb.ent)) ||
+      (rc = upload(p, &p->d_nd_nslot, nb.nslot)) || (rc = dalloc(p, &p->d_nd_px, E * kInterpTaps)) ||
+      (rc = dalloc(p, &p->d_nd_py, E * kNormalC)) || (rc = dalloc(p, &p->d_spec, (size_t)g.n0 * p->ncol)) ||
+      (rc = dalloc(p, &p->d_epart, S * (p->ncol / kNormalC))) || (rc = upload(p, &p->d_nq_off, ub.off)))
+    return rc;
+  if (p->half &&
+      ((rc = upload(p, &p->d_nq_ent, ub.ent)) || (rc = upload(p, &p->d_nq_entr, entr)) ||
+       (rc = upload(p, &p->d_nq_nslot, ub.nslot)) || (rc = dalloc(p, &p->d_nq_px, U * kInterpTaps)) ||
+       (rc = dalloc(p, &p->d_nq_py, U * kNormalC)) || (rc = dalloc(p, &p->d_rpart, S * p->nq * kNodeSlots)) ||
+       (rc = dalloc(p, &p->d_gram, (size_t)8 * p->nq * p->nq))))
+    return rc;
+  constexpr int kChunk = 1024;
+  const int ld = (2 * p->nq + 63) / 64 * 64;
+  const size_t head = (sizeof(chol) + 255) / 256 * 256;
+  const size_t acc_n = std::max(cells * spectrum_splits(g.n0, g.n1),
+                                ld ? (size_t)ld * ld * spectrum_splits(ld, ld) : (size_t)0);
+  const size_t fac_n = std::max((size_t)kChunk * (g.n0 + g.n1), (size_t)4 * kChunk * ld);
+  char* scratch = nullptr;
+  HIPCHK(hipMalloc(&scratch, head + sizeof(double) * (acc_n + fac_n)));
+  const float2* nodes = p->d_nodes;
+  auto* d_chol = reinterpret_cast<double*>(scratch);
+  auto* acc = reinterpret_cast<double*>(scratch + head);
+  double* fac = acc + acc_n;
+  hipStream_t st = p->stream;
+  const int half = p->half ? g.N0 / 2 : 0;
+  hipError_t e = hipMemcpy(d_chol, chol, sizeof(chol), hipMemcpyHostToDevice);
+  if (e == hipSuccess)
+    e = launch_interp_records(p->d_nd_ent, p->d_nd_off, nodes, (int)E, g.n0, g.n1, half, d_chol, p->d_nd_px,
+                              p->d_nd_py, st);
+  if (e == hipSuccess && p->half)
+    e = launch_interp_records(p->d_nq_ent, p->d_nq_off, nodes, (int)U, g.n0, g.n1, half, d_chol, p->d_nq_px,
+                              p->d_nq_py, st);
+  if (e == hipSuccess) e = launch_zero(reinterpret_cast<float*>(acc), 2 * acc_n, st);
+  for (int j = 0; j < g.M && e == hipSuccess; j += kChunk)
+    e = launch_spectrum_chunk(nodes, p->d_w, j, std::min(kChunk, g.M - j), g.N0, g.N1, g.n0, g.n1, fac,
+                              fac + (size_t)kChunk * g.n0, acc, st);
+  if (e == hipSuccess) e = launch_spectrum_store(acc, g.n0, g.n1, p->half, p->d_spec, st);
+  if (e == hipSuccess && p->half) {
+    e = launch_wave_gram(nodes, p->nq, g.N0, g.N1, p->d_gram, st);
+    if (e == hipSuccess) e = launch_zero(reinterpret_cast<float*>(acc), 2 * acc_n, st);
+    for (int j = 0; j < g.M && e == hipSuccess; j += kChunk)
+      e = launch_wave_chunk(nodes, p->d_w, j, std::min(kChunk, g.M - j), p->nq, ld, g.N0, g.N1, fac,
+                            fac + (size_t)2 * kChunk * ld, acc, st);
+    if (e == hipSuccess) e = launch_wave_store(acc, p->nq, ld, p->d_gram + (size_t)4 * p->nq * p->nq, st);
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  (void)hipFree(scratch);
+  if (e == hipSuccess) e = set_normal_attrs(g.n0);
+  if (e != hipSuccess) return fail(ICON_ERR_DEVICE, "normal operator: %s", hipGetErrorString(e));
   return ICON_OK;
 }
 
@@ -343,6 +484,108 @@ int prepare_col(int n0, int n1, int C, int K) {
 }  // namespace
 
 void icon::set_last_error(const char* msg) { g_err = msg; }
+
+// Arguments of the iteration's kernels over S slices of a plan.
+ColArgs icon::normal_args(const icon_plan* p, int S, bool with_nodes) {
+  const Geometry& g = p->g;
+  ColArgs a{};
+  a.S = S; a.N0 = g.N0; a.N1 = g.N1; a.M = p->rows; a.n1 = p->ncol; a.K = kInterpTaps; a.slots = kNodeSlots;
+  a.in = p->d_tmp; a.out = p->d_tmp; a.tw = p->d_tw0; a.part = p->d_part; a.spec = p->d_spec;
+  // all nodes for the residual; otherwise the unpaired ones (none on a full grid)
+  a.ent_off = with_nodes ? p->d_nd_off : p->d_nq_off;
+  a.fent = with_nodes ? p->d_nd_ent : p->d_nq_ent;
+  a.fent_px = with_nodes ? p->d_nd_px : p->d_nq_px;
+  a.fent_py = with_nodes ? p->d_nd_py : p->d_nq_py;
+  return a;
+}
+
+ColArgs icon::energy_args(const icon_plan* p, int S) {
+  ColArgs a = normal_args(p, S, false);
+  a.M = p->nq; a.part = p->d_rpart; a.fent = p->d_nq_entr; a.epart = p->d_epart;
+  a.nyq = p->half ? p->g.n1 / 2 : 0;
+  return a;
+}
+
+ColArgs icon::normal64_args(const icon_plan* p, int S, bool with_nodes) {
+  ColArgs a = normal_args(p, S, with_nodes);
+  a.io64 = reinterpret_cast<double2*>(p->d_tmp);
+  a.w64 = p->d_w640;
+  return a;
+}
+
+RefArgs icon::ref_args(const icon_plan* p, int S, float* m) {
+  const Geometry& g = p->g;
+  RefArgs a{};
+  a.rows = S * g.N0; a.N0 = g.N0; a.N1 = g.N1; a.ncol = p->ncol; a.m = m; a.mref = p->d_mref; a.alpha = p->d_alpha;
+  a.w64 = p->d_w641; a.io = reinterpret_cast<double2*>(p->d_tmp); a.ahwb = p->d_ahwb;
+  a.ahwb_re = reinterpret_cast<const float*>(p->d_ahwb); a.grad = p->d_grad; a.base = p->d_base;
+  a.base_re = reinterpret_cast<float*>(p->d_base); a.rowpart = p->d_rowpart;
+  return a;
+}
+
+// Phase of iteration it: 0 before, 1 in and 2 after the ICON iterations.
+static int phase_of(const icon_solve_opts& o, int it) { return it < o.pre ? 0 : it < o.pre + o.icon ? 1 : 2; }
+
+// Iterations whose gradient is computed in FP64: the iterates after 2, 8, 32,
+// ... updates of each phase (the bound moves the image at once where it sets
+// in or ends), where at least 6 more follow in the phase.
+bool icon::refresh(const icon_plan* p, const icon_solve_opts& o, int it) {
+  if (!p->refreshes() || it == 0) return false;
+  const int ph = phase_of(o, it - 1);
+  const int begin = ph == 0 ? 0 : ph == 1 ? o.pre : o.pre + o.icon;
+  const int len = ph == 0 ? o.pre : ph == 1 ? o.icon : o.post;
+  const int j = it - begin;   // updates of this phase so far
+  for (int k = 2; k <= j; k *= 4)
+    if (k == j) return j + 6 <= len;
+  return false;
+}
+
+RowFwdArgs icon::rhat_row_args(const icon_plan* p, int S) {
+  RowFwdArgs a{};
+  a.rows = S * p->g.N0; a.N0 = p->g.N0; a.N1 = p->g.N1; a.tw = p->d_tw1; a.out = p->d_tmp;
+  a.cplx = p->half ? 0 : 1;
+  a.m = p->d_grad;
+  a.rhat = p->d_base;   // -rhat: its energy is rhat's
+  return a;
+}
+
+ColArgs icon::spread_args(icon_plan* p, int S) {
+  ColArgs a = window_args(p, p->spread(), S);
+  a.io64 = reinterpret_cast<double2*>(p->d_tmp);
+  a.w64 = p->d_w640;
+  return a;
+}
+
+RowAdjArgs icon::data_row_args(icon_plan* p, int S) {
+  const Geometry& g = p->g;
+  RowAdjArgs a{};
+  a.rows = S * g.N0; a.N0 = g.N0; a.N1 = g.N1; a.in = p->d_tmp; a.ck = p->spread().ck; a.tw = p->d_tw1;
+  a.in64 = reinterpret_cast<const double2*>(p->d_tmp); a.w64 = p->d_w641;
+  if (p->half) a.img_re = reinterpret_cast<float*>(p->d_ahwb);
+  else a.img = p->d_ahwb;
+  zero_band(p->spread().h, &a.zlo, &a.zhi);
+  return a;
+}
+
+RowAdjArgs icon::grad_args(const icon_plan* p, int S) {
+  const Geometry& g = p->g;
+  RowAdjArgs a{};
+  a.rows = S * g.N0; a.N0 = g.N0; a.N1 = g.N1; a.in = p->d_tmp; a.tw = p->d_tw1; a.ahwb = p->d_ahwb;
+  a.ahwb_re = reinterpret_cast<const float*>(p->d_ahwb); a.grad = p->d_grad; a.rowpart = p->d_rowpart;
+  a.fwd_out = p->d_tmp;
+  return a;
+}
+
+FinishArgs icon::finish_args(const icon_plan* p, int S) {
+  const Geometry& g = p->g;
+  FinishArgs a{};
+  a.S = S; a.M = p->rows; a.Mb = g.M; a.N0 = g.N0; a.nblk = p->ncol / kNormalC; a.nrow = p->half ? g.N0 / 2 : g.N0;
+  a.slots = kNodeSlots; a.part = p->d_part; a.nslot = p->d_nd_nslot;
+  a.w = p->d_w; a.b = p->d_b; a.bnorm = p->d_bnorm; a.iomit = g.iomit;
+  a.rowpart = p->d_rowpart; a.epart = p->d_epart;
+  a.nq = p->nq; a.rpart = p->d_rpart; a.rslot = p->d_nq_nslot; a.gram = p->d_gram;
+  return a;
+}
 
 // ====================================================================== ABI
 extern "C" {
@@ -515,35 +758,47 @@ int plan_create(icon_plan** out, int device, int nx, int thickness, int nz, cons
   auto* p = new icon_plan();
   p->device = device;
   std::string err;
-  if (!build_geometry(p->g, nx, thickness > 0 ? thickness : nx, nz, tilt_deg, &err, cv, window)) {
+  if (!build_geometry(p->g, nx, thickness > 0 ? thickness : nx, nz, tilt_deg, &err, cv, window, false)) {
     delete p;
     return fail(ICON_ERR_ARG, "%s", err.c_str());
   }
   p->S_max = max_slices;
-  build_bins(p->g, default_col_block(p->g.n0), p->bins);
   const Geometry& g = p->g;
   int rc = ICON_OK;
   auto bail = [&](int code) {
     icon_plan_destroy(p);
     return code;
   };
-  if ((rc = upload(p, &p->d_ck, g.ck))) return bail(rc);
+  {
+    hipError_t e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&p->ev_in, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&p->ev_out, hipEventDisableTiming);
+    if (e != hipSuccess) return bail(fail(ICON_ERR_DEVICE, "stream/event create: %s", hipGetErrorString(e)));
+  }
+  if ((rc = dalloc(p, &p->d_nodes, (size_t)g.M))) return bail(rc);
+  {
+    hipError_t e = hipMemcpy(p->d_nodes, g.nodes.data(), sizeof(float2) * g.M, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return bail(fail(ICON_ERR_DEVICE, "node upload: %s", hipGetErrorString(e)));
+  }
   if ((rc = upload(p, &p->d_ck1, g.ck1))) return bail(rc);
   if ((rc = upload(p, &p->d_w, g.w))) return bail(rc);
-  if ((rc = upload(p, &p->d_phix, g.phix))) return bail(rc);
-  if ((rc = upload(p, &p->d_phiy, g.phiy))) return bail(rc);
-  if ((rc = upload(p, &p->d_ix0, g.ix0))) return bail(rc);
   if ((rc = upload(p, &p->d_phi1, g.phi1))) return bail(rc);
   if ((rc = upload(p, &p->d_i10, g.i10))) return bail(rc);
-  if ((rc = upload_bins(p))) return bail(rc);
+  // The solve subtracts A^H W b from the exact A^H W A m in every iteration, so
+  // that an error of it in the directions that no tilt covers adds up over the
+  // iterations: it needs the accurate window also where the transforms use the
+  // 6-tap one (with it, and with the 14-tap Gaussian, a 100-iteration solve was
+  // 4 to 5 times as far from the exact one as now).
+  p->own_data = op_taps(g) != kTapsWide;
+  if (p->own_data && (rc = make_bins(p, p->data, 8, kTapsWide))) return bail(rc);
+  if ((rc = make_op_bins(p, default_col_block(g.n0)))) return bail(rc);
   if ((rc = twiddles(g.n0, &p->d_tw0))) return bail(rc);
   if ((rc = twiddles(g.n1, &p->d_tw1))) return bail(rc);
+  if ((rc = twiddles64(g.n0, &p->d_w640))) return bail(rc);
+  if ((rc = twiddles64(g.n1, &p->d_w641))) return bail(rc);
   const size_t S = (size_t)max_slices, M = (size_t)g.M, NN = (size_t)g.N0 * g.N1;
   if ((rc = dalloc(p, &p->d_b, S * M))) return bail(rc);
-  if ((rc = dalloc(p, &p->d_part, S * M * kMaxSlot))) return bail(rc);
-  if ((rc = dalloc(p, &p->d_ahwb, S * NN))) return bail(rc);
   if ((rc = dalloc(p, &p->d_grad, S * NN))) return bail(rc);
-  if ((rc = dalloc(p, &p->d_tmp, S * g.N0 * (size_t)g.n1))) return bail(rc);
   if ((rc = dalloc(p, &p->d_frep, S * g.N0))) return bail(rc);
   if ((rc = dalloc(p, &p->d_rowpart, S * g.N0))) return bail(rc);
   if ((rc = dalloc(p, &p->d_bnorm, S))) return bail(rc);
@@ -553,13 +808,20 @@ int plan_create(icon_plan** out, int device, int nx, int thickness, int nz, cons
     hipError_t e = hipMemset(p->d_alpha, 0, sizeof(double) * S);
     if (e != hipSuccess) return bail(fail(ICON_ERR_DEVICE, "hipMemset: %s", hipGetErrorString(e)));
   }
+  if ((rc = prepare_col(g.n0, g.n1, p->op.h.C, p->op.h.K))) return bail(rc);
+  if (p->own_data && (rc = prepare_col(g.n0, g.n1, p->data.h.C, p->data.h.K))) return bail(rc);
+  if ((rc = build_normal(p))) return bail(rc);
+  if ((rc = dalloc(p, &p->d_part, S * std::max(M * kMaxSlot, (size_t)p->rows * kNodeSlots)))) return bail(rc);
+  if ((rc = dalloc(p, &p->d_ahwb, p->half ? (S * NN + 1) / 2 : S * NN))) return bail(rc);
+  if ((rc = dalloc(p, &p->d_base, p->half ? (S * NN + 1) / 2 : S * NN))) return bail(rc);
+  if ((rc = dalloc(p, &p->d_mref, S * NN))) return bail(rc);
+  if ((rc = dalloc(p, &p->d_beff, S * M))) return bail(rc);
+  // the grid rows, in single precision or (the FP64 gradients) in double
+  if ((rc = dalloc(p, &p->d_tmp, S * g.N0 * (size_t)g.n1 * (p->refreshes() ? 2 : 1)))) return bail(rc);
   {
-    hipError_t e = hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&p->ev_in, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&p->ev_out, hipEventDisableTiming);
-    if (e != hipSuccess) return bail(fail(ICON_ERR_DEVICE, "stream/event create: %s", hipGetErrorString(e)));
+    const hipError_t e = set_adj64_attrs();
+    if (e != hipSuccess) return bail(fail(ICON_ERR_DEVICE, "hipFuncSetAttribute: %s", hipGetErrorString(e)));
   }
-  if ((rc = prepare_col(g.n0, g.n1, p->bins.C, g.K))) return bail(rc);
   *out = p;
   return ICON_OK;
 }
@@ -572,12 +834,15 @@ int icon_plan_destroy(icon_plan* p) {
   DevGuard dg(p->device);
   if (p->stream) (void)hipStreamSynchronize(p->stream);
   drop_graph(p);
-  void* ptrs[] = {p->d_ck, p->d_ck1, p->d_w, p->d_phix, p->d_phiy, p->d_ix0, p->d_phi1, p->d_i10,
+  void* ptrs[] = {p->d_nodes, p->d_ck1, p->d_w, p->d_phi1, p->d_i10, p->d_fw,
                   p->d_b, p->d_part, p->d_ahwb, p->d_grad, p->d_tmp, p->d_frep, p->d_rowpart,
-                  p->d_bnorm, p->d_alpha};
+                  p->d_bnorm, p->d_alpha, p->d_spec, p->d_nd_off, p->d_nd_ent, p->d_nd_nslot, p->d_nd_px, p->d_nd_py,
+                  p->d_epart, p->d_nq_off, p->d_nq_ent, p->d_nq_entr, p->d_nq_px, p->d_nq_py, p->d_nq_nslot,
+                  p->d_rpart, p->d_gram, p->d_base, p->d_mref, p->d_beff};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
-  free_bins(p);
+  free_bins(p->op);
+  free_bins(p->data);
   if (p->ev_in) (void)hipEventDestroy(p->ev_in);
   if (p->ev_out) (void)hipEventDestroy(p->ev_out);
   if (p->stream) (void)hipStreamDestroy(p->stream);
@@ -590,23 +855,21 @@ int icon_plan_get_info(const icon_plan* p, icon_plan_info* info) {
   const Geometry& g = p->g;
   info->N0 = g.N0; info->N1 = g.N1; info->nz = g.nz; info->M = g.M; info->n0 = g.n0; info->n1 = g.n1;
   info->m = g.K == kTaps ? kWindowM : g.K / 2; info->window = g.window; info->iomit = g.iomit; info->sigma0 = g.sig0; info->sigma1 = g.sig1;
-  info->b0 = g.b0; info->b1 = g.b1; info->max_slices = p->S_max; info->col_block = p->bins.C;
+  info->b0 = g.b0; info->b1 = g.b1; info->max_slices = p->S_max; info->col_block = p->op.h.C;
   info->device_bytes = p->device_bytes;
   return ICON_OK;
 }
 
 int icon_plan_set_col_block(icon_plan* p, int C) {
   if (!p) return fail(ICON_ERR_ARG, "icon_plan_set_col_block: null plan");
-  if (!col_tile_ok(p->g.n0, p->g.n1, C, p->g.K))
+  if (!col_tile_ok(p->g.n0, p->g.n1, C, op_taps(p->g)))
     return fail(ICON_ERR_ARG, "column tile %d unsupported for grid %d x %d", C, p->g.n0, p->g.n1);
   DevGuard dg(p->device);
   HIPCHK(hipStreamSynchronize(p->stream));
   drop_graph(p);
-  free_bins(p);
-  build_bins(p->g, C, p->bins);
-  int rc = upload_bins(p);
+  int rc = make_op_bins(p, C);
   if (rc) return rc;
-  return prepare_col(p->g.n0, p->g.n1, C, p->g.K);
+  return prepare_col(p->g.n0, p->g.n1, C, op_taps(p->g));
 }
 
 int icon_nufft_forward_real(icon_plan* p, int S, const void* d_img, void* d_f, void* stream) {
@@ -771,6 +1034,8 @@ int icon_reconstruct_host(icon_plan* p, int S, const float* sino, float* m, cons
 int icon_time_kernel(icon_plan* p, int kernel, int S, int reps, double* avg_ms) {
   if (!p || !avg_ms || reps < 1) return fail(ICON_ERR_ARG, "icon_time_kernel: bad argument");
   if (S < 1 || S > p->S_max) return fail(ICON_ERR_CAPACITY, "batch %d outside 1..%d", S, p->S_max);
+  if (kernel < ICON_K_ROW_FWD || kernel > ICON_K_COL_ENERGY)
+    return fail(ICON_ERR_ARG, "icon_time_kernel: unknown kernel %d", kernel);
   DevGuard dg(p->device);
   const Geometry& g = p->g;
   hipStream_t st = p->stream;
@@ -780,55 +1045,50 @@ int icon_time_kernel(icon_plan* p, int kernel, int S, int reps, double* avg_ms) 
   // first; the image it updates lives in the (then stale) A^H W b buffer
   rf.rows = S * g.N0; rf.N0 = g.N0; rf.N1 = g.N1; rf.cplx = 0; rf.update = 2; rf.data_type = 1;
   rf.m = reinterpret_cast<float*>(p->d_ahwb); rf.grad = p->d_grad; rf.alpha = p->d_alpha;
-  rf.ck = p->d_ck; rf.tw = p->d_tw1; rf.out = p->d_tmp;
-  ColArgs ca{};
-  ca.K = p->g.K;
-  ca.S = S; ca.N0 = g.N0; ca.N1 = g.N1; ca.M = g.M; ca.n1 = g.n1; ca.in = p->d_tmp; ca.out = p->d_tmp;
-  ca.tw = p->d_tw0; ca.ent_off = p->d_ent_off; ca.tile_order = p->d_tile_order; ca.split_min = split_min_entries(p->bins); ca.ent = p->d_ent; ca.xoff = p->d_xoff; ca.E = (int)p->bins.ent.size(); ca.ent_px = p->d_ent_px; ca.ent_py = p->d_ent_py;
-  ca.fent = p->d_fent; ca.fent_px = p->d_fent_px; ca.fent_py = p->d_fent_py; ca.phix = p->d_phix; ca.phiy = p->d_phiy;
-  ca.ix0 = p->d_ix0; ca.part = p->d_part; ca.fw = p->d_fw;
-  CombineArgs cm{};
-  cm.S = S; cm.M = g.M; cm.N0 = g.N0; cm.nz = g.nz; cm.mode = 0; cm.part = p->d_part; cm.nslot = p->d_nslot;
-  cm.w = p->d_w; cm.b = p->d_b; cm.fw = p->d_fw; cm.bnorm = p->d_bnorm;
-  cm.E = (int)p->bins.ent.size(); cm.ent_of_node = p->d_ent_of_node;
-  RowAdjArgs ra{};
-  ra.rows = S * g.N0; ra.N0 = g.N0; ra.N1 = g.N1; ra.mode = 1; ra.in = p->d_tmp; ra.ck = p->d_ck;
-  ra.tw = p->d_tw1; ra.ahwb = p->d_ahwb; ra.grad = p->d_grad; ra.rowpart = p->d_rowpart;
-  ra.fwd_out = p->d_tmp;
-  zero_band(p->bins, &rf.zlo, &rf.zhi);
-  zero_band(p->bins, &ca.zlo, &ca.zhi);
-  zero_band(p->bins, &ra.zlo, &ra.zhi);
-  // the step-size combine (mode 1) after the combine of A m, as in a solve
-  CombineArgs cr = cm;
-  cr.mode = 1; cr.rowpart = p->d_rowpart; cr.alpha = p->d_alpha;
+  rf.tw = p->d_tw1; rf.out = p->d_tmp;
+  const ColArgs cn = normal_args(p, S, true), ce = energy_args(p, S);
+  const RowAdjArgs ra = grad_args(p, S);
+  // (the residuals of these stale values go to the bnorm buffer, rewritten by the next solve's set-up)
+  FinishArgs fr = finish_args(p, S);
+  fr.resid = p->d_bnorm; fr.resid_stride = 1; fr.alpha = p->d_alpha;
+  FinishArgs fs = fr;
+  fs.resid = nullptr;
+  // the transforms' column kernels: interpolation and spread of the plan's window
+  const ColArgs ca = window_args(p, p->op, S);
   SinoArgs sa{};
   sa.K = p->g.K;
   sa.rows = S * g.nz; sa.N0 = g.N0; sa.sino = reinterpret_cast<const float*>(p->d_b); sa.ck1 = p->d_ck1;
   sa.phi1 = p->d_phi1; sa.i10 = p->d_i10; sa.tw = p->d_tw0; sa.b = p->d_fw;
   auto launch = [&](int k) -> hipError_t {
     switch (k) {
-      case ICON_K_ROW_FWD: return launch_row_fwd(g.n1, rf, st);
-      case ICON_K_COL_FWD: return launch_col(g.n0, p->bins.C, false, ca, st);
-      case ICON_K_COMBINE: return launch_combine(cm, st);
-      case ICON_K_COL_ADJ: return launch_col(g.n0, p->bins.C, true, ca, st);
-      case ICON_K_ROW_ADJ: return launch_row_adj(g.n1, ra, st);
+      case ICON_K_ROW_FWD: return iter_row_fwd(p, rf, st);
+      case ICON_K_COL_FWD: return launch_col(g.n0, p->op.h.C, false, ca, st);
+      case ICON_K_COMBINE: return launch_finish(fr, st);
+      case ICON_K_COL_ADJ: return launch_col(g.n0, p->op.h.C, true, ca, st);
+      case ICON_K_ROW_ADJ: return iter_row_grad(p, ra, st);
       case ICON_K_SINO: return launch_sino(g.n0, sa, st);
-      case ICON_K_COMBINE_ALPHA: return launch_combine(cr, st);
+      case ICON_K_COMBINE_ALPHA: return launch_finish(fs, st);
+      case ICON_K_COL_NORMAL: return launch_col_normal(g.n0, cn, st);
+      case ICON_K_COL_ENERGY: return launch_col_energy(g.n0, ce, st);
       default: return hipErrorInvalidValue;
     }
   };
-  if (kernel < ICON_K_ROW_FWD || kernel > ICON_K_COMBINE_ALPHA)
-    return fail(ICON_ERR_ARG, "icon_time_kernel: unknown kernel %d", kernel);
-  // The launch sequence of one iteration, as the solve enqueues it; the
-  // timed kernel runs inside it, so that each timed launch finds its input as
-  // in a solve (just written by its predecessor, partly in the caches) and the
-  // device busy (an idle gap before a launch lowers the clock it starts at).
-  // The sinogram transform runs once per solve and is timed back to back.
-  const int iter_seq[7] = {ICON_K_ROW_FWD, ICON_K_COL_FWD, ICON_K_COMBINE, ICON_K_COL_ADJ,
-                           ICON_K_ROW_ADJ, ICON_K_COL_FWD, ICON_K_COMBINE_ALPHA};
-  const int sino_seq[1] = {ICON_K_SINO};
-  const int* seq = kernel == ICON_K_SINO ? sino_seq : iter_seq;
-  const int nseq = kernel == ICON_K_SINO ? 1 : 7;
+  // The launch sequence of one iteration (with a residual), as the solve
+  // enqueues it; the timed kernel runs inside it, so that each timed launch
+  // finds its input as in a solve (just written by its predecessor, partly in
+  // the caches) and the device busy (an idle gap before a launch lowers the
+  // clock it starts at).  The transforms' column kernels are timed between the
+  // row passes that precede them; the sinogram transform, which runs once per
+  // solve, back to back.
+  const int iter_seq[] = {ICON_K_ROW_FWD, ICON_K_COL_NORMAL, ICON_K_ROW_ADJ, ICON_K_COL_ENERGY, ICON_K_COMBINE};
+  const int alpha_seq[] = {ICON_K_ROW_FWD, ICON_K_COL_NORMAL, ICON_K_ROW_ADJ, ICON_K_COL_ENERGY, ICON_K_COMBINE_ALPHA};
+  const int op_seq[] = {ICON_K_ROW_FWD, ICON_K_COL_FWD, ICON_K_COL_ADJ, ICON_K_ROW_ADJ};
+  const int sino_seq[] = {ICON_K_SINO};
+  const int* seq = iter_seq;
+  int nseq = 5;
+  if (kernel == ICON_K_COMBINE_ALPHA) seq = alpha_seq;
+  if (kernel == ICON_K_COL_FWD || kernel == ICON_K_COL_ADJ) seq = op_seq, nseq = 4;
+  if (kernel == ICON_K_SINO) seq = sino_seq, nseq = 1;
   // Each timed launch carries events that take the kernel's own start and end
   // (hipExtLaunchKernel), not those of extra marker packets around it; all
   // launches are enqueued before one synchronisation.
@@ -867,7 +1127,7 @@ int icon_plan_autotune(icon_plan* p, int S, int* col_block, double* ms_per_width
   for (int i = 0; i < 2; i++) {
     const int C = widths[i];
     if (ms_per_width) ms_per_width[i] = 0.0;
-    if (!col_tile_ok(p->g.n0, p->g.n1, C, p->g.K)) continue;
+    if (!col_tile_ok(p->g.n0, p->g.n1, C, op_taps(p->g))) continue;
     int rc = icon_plan_set_col_block(p, C);
     double tf = 0.0, ta = 0.0;
     if (!rc) rc = icon_time_kernel(p, ICON_K_COL_FWD, S, 3, &tf);
@@ -878,7 +1138,7 @@ int icon_plan_autotune(icon_plan* p, int S, int* col_block, double* ms_per_width
     if (best_c == 0 || t < best) { best = t; best_c = C; }
   }
   if (best_c == 0) return fail(ICON_ERR_ARG, "icon_plan_autotune: no supported column tile");
-  if (p->bins.C != best_c) {
+  if (p->op.h.C != best_c) {
     const int rc = icon_plan_set_col_block(p, best_c);
     if (rc) return rc;
   }

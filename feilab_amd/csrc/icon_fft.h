@@ -18,31 +18,36 @@
 
 namespace icon {
 
-__device__ __forceinline__ float2 c_add(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 c_sub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ float2 c_mul(float2 a, float2 b) {
-  return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+// Values are float2, or double2 in the few FP64 passes (V below).
+__device__ __forceinline__ float2 c_make(float x, float y) { return make_float2(x, y); }
+__device__ __forceinline__ double2 c_make(double x, double y) { return make_double2(x, y); }
+template <typename V>
+__device__ __forceinline__ V c_add(V a, V b) { return c_make(a.x + b.x, a.y + b.y); }
+template <typename V>
+__device__ __forceinline__ V c_sub(V a, V b) { return c_make(a.x - b.x, a.y - b.y); }
+template <typename V>
+__device__ __forceinline__ V c_mul(V a, V b) {
+  return c_make(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
 // cos / sin of 2 pi q / 16, q = 0..7.
-constexpr float kCos16[8] = {1.0f, 0.923879532511286756f, 0.707106781186547524f,
-                                        0.382683432365089772f, 0.0f, -0.382683432365089772f,
-                                        -0.707106781186547524f, -0.923879532511286756f};
-constexpr float kSin16[8] = {0.0f, 0.382683432365089772f, 0.707106781186547524f,
-                                        0.923879532511286756f, 1.0f, 0.923879532511286756f,
-                                        0.707106781186547524f, 0.382683432365089772f};
+constexpr double kCos16[8] = {1.0, 0.923879532511286756, 0.707106781186547524, 0.382683432365089772, 0.0,
+                              -0.382683432365089772, -0.707106781186547524, -0.923879532511286756};
+constexpr double kSin16[8] = {0.0, 0.382683432365089772, 0.707106781186547524, 0.923879532511286756, 1.0,
+                              0.923879532511286756, 0.707106781186547524, 0.382683432365089772};
 
 // a * exp(DIR * 2 pi i * Q / 16), Q in [0, 8), with the trivial cases exact.
-template <int Q, int DIR>
-__device__ __forceinline__ float2 rot16(float2 a) {
+template <int Q, int DIR, typename V>
+__device__ __forceinline__ V rot16(V a) {
   if constexpr (Q == 0) {
     return a;
   } else if constexpr (Q == 4) {
-    return DIR > 0 ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
+    return DIR > 0 ? c_make(-a.y, a.x) : c_make(a.y, -a.x);
   } else {
-    constexpr float c = kCos16[Q];
-    constexpr float s = DIR > 0 ? kSin16[Q] : -kSin16[Q];
-    return make_float2(a.x * c - a.y * s, a.x * s + a.y * c);
+    using T = decltype(a.x + a.x);
+    constexpr T c = (T)kCos16[Q];
+    constexpr T s = (T)(DIR > 0 ? kSin16[Q] : -kSin16[Q]);
+    return c_make(a.x * c - a.y * s, a.x * s + a.y * c);
   }
 }
 
@@ -56,13 +61,13 @@ __host__ __device__ constexpr int bitrev(int i) {
 template <int R> struct Log2 { static constexpr int v = R == 2 ? 1 : R == 4 ? 2 : R == 8 ? 3 : 4; };
 
 // Stage of the radix-2 decimation-in-time network: butterflies of span LEN.
-template <int R, int DIR, int LEN, int K>
-__device__ __forceinline__ void dit_stage_k(float2* v) {
+template <int R, int DIR, int LEN, int K, typename V>
+__device__ __forceinline__ void dit_stage_k(V* v) {
   if constexpr (K < LEN / 2) {
 #pragma unroll
     for (int i = K; i < R; i += LEN) {
-      float2 u = v[i];
-      float2 t = rot16<(16 / LEN) * K, DIR>(v[i + LEN / 2]);
+      V u = v[i];
+      V t = rot16<(16 / LEN) * K, DIR>(v[i + LEN / 2]);
       v[i] = c_add(u, t);
       v[i + LEN / 2] = c_sub(u, t);
     }
@@ -70,8 +75,8 @@ __device__ __forceinline__ void dit_stage_k(float2* v) {
   }
 }
 
-template <int R, int DIR, int LEN>
-__device__ __forceinline__ void dit_stages(float2* v) {
+template <int R, int DIR, int LEN, typename V>
+__device__ __forceinline__ void dit_stages(V* v) {
   if constexpr (LEN <= R) {
     dit_stage_k<R, DIR, LEN, 0>(v);
     dit_stages<R, DIR, LEN * 2>(v);
@@ -79,14 +84,14 @@ __device__ __forceinline__ void dit_stages(float2* v) {
 }
 
 // In-register DFT of size R (2, 4, 8, 16), natural order in and out.
-template <int R, int DIR>
-__device__ __forceinline__ void dft(float2* v) {
+template <int R, int DIR, typename V>
+__device__ __forceinline__ void dft(V* v) {
   constexpr int L = Log2<R>::v;
 #pragma unroll
   for (int i = 0; i < R; i++) {
     const int j = bitrev<L>(i);
     if (i < j) {
-      float2 t = v[i];
+      V t = v[i];
       v[i] = v[j];
       v[j] = t;
     }
@@ -367,6 +372,57 @@ __device__ __forceinline__ void fft_lds(float2* lds, int t, const float2* __rest
   // line can be overwritten now
 #pragma unroll
   for (int i = 0; i < 16; i++) lds[L::at(out_index<N>(t, i))] = v[i];
+}
+
+// FP64 transform of a line, registers (input order) -> registers (output
+// order), as fft_regs.  w: exp(-2 pi i q / N), q < N.  The exchanges go through
+// LDS one component at a time (lds: L::size(N) doubles, layout L).  Ends past
+// the last exchange's barrier.
+template <int N, typename L, int DIR, int NS = 1>
+__device__ __forceinline__ void fft64(double2 (&v)[16], double* lds, int t, const double2* __restrict__ w) {
+  constexpr int T = N / 16, RP = pass_radix<N, NS>(), B = 16 / RP;
+#pragma unroll
+  for (int q = 0; q < B; q++) {
+    if constexpr (NS > 1) {
+      const int k = (t + q * T) & (NS - 1);
+      constexpr int step = N / (NS * RP);
+#pragma unroll
+      for (int r = 1; r < RP; r++) {
+        double2 f = w[r * k * step];
+        if (DIR > 0) f.y = -f.y;
+        v[q * RP + r] = c_mul(v[q * RP + r], f);
+      }
+    }
+    dft<RP, DIR>(&v[q * RP]);
+  }
+  if constexpr (NS * RP < N) {
+    constexpr int RN = pass_radix<N, NS * RP>(), BN = 16 / RN;
+    double im[16];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+#pragma unroll
+      for (int q = 0; q < B; q++) {
+        const int j = t + q * T, k = j & (NS - 1), base = (j - k) * RP + k;
+#pragma unroll
+        for (int r = 0; r < RP; r++) lds[L::at(base + r * NS)] = c ? im[q * RP + r] : v[q * RP + r].x;
+      }
+      if (c == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) im[i] = v[i].y;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < BN; q++)
+#pragma unroll
+        for (int r = 0; r < RN; r++) {
+          const double x = lds[L::at(t + q * T + r * (N / RN))];
+          if (c) v[q * RN + r].y = x;
+          else v[q * RN + r].x = x;
+        }
+      __syncthreads();
+    }
+    fft64<N, L, DIR, NS * RP>(v, lds, t, w);
+  }
 }
 
 }  // namespace icon

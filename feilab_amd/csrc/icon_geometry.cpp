@@ -75,23 +75,18 @@ double bessel_i0(double x) {
   return sum;
 }
 
-float kb_beta(float sigma) {
-  const double W = kTapsKB, s = sigma;
-  return (float)(kPI * std::sqrt((W / s) * (W / s) * (s - 0.5) * (s - 0.5) - 0.8));
-}
+double kb_norm(double beta, int W) { return W * std::sinh(beta) / beta; }
 
-double kb_norm(double beta) { return kTapsKB * std::sinh(beta) / beta; }
-
-float deapod_kb(int k, int N, float sigma, float beta) {
+float deapod_kb(int k, int N, float sigma, float beta, int taps) {
   const double n = std::ceil((float)N * sigma);
-  const double W = kTapsKB, bt = beta;
+  const double W = taps, bt = beta;
   const double u = kPI * W * (double)k / n;
   const double a2 = bt * bt - u * u;
   double v;
   if (a2 > 0) v = W * std::sinh(std::sqrt(a2)) / std::sqrt(a2);
   else if (a2 < 0) v = W * std::sin(std::sqrt(-a2)) / std::sqrt(-a2);
   else v = W;
-  return (float)(v / kb_norm(bt));
+  return (float)(v / kb_norm(bt, taps));
 }
 
 // Kaiser-Bessel taps of one coordinate: grid points floor(n c) - 2 .. + 3.
@@ -99,7 +94,7 @@ void taps_kb(float c, int N, float sigma, float beta, float* phi, int* first) {
   const int n = (int)std::ceil((float)N * sigma);
   const double u = (double)n * (double)c;
   const int l0 = (int)std::floor(u) - (kTapsKB / 2 - 1);
-  const double Z = kb_norm(beta);
+  const double Z = kb_norm(beta, kTapsKB);
   for (int t = 0; t < kTapsKB; t++) {
     const double d = u - (double)(l0 + t);
     const double r = 1.0 - (2.0 * d / kTapsKB) * (2.0 * d / kTapsKB);
@@ -109,6 +104,15 @@ void taps_kb(float c, int N, float sigma, float beta, float* phi, int* first) {
 }
 }  // namespace
 
+float kb_beta(float sigma, int taps) {
+  const double W = taps, s = sigma;
+  return (float)(kPI * std::sqrt((W / s) * (W / s) * (s - 0.5) * (s - 0.5) - 0.8));
+}
+
+void kb_deapod(int N, float sigma, float beta, int W, float* out) {
+  for (int k = 0; k < N; k++) out[k] = deapod_kb(k - N / 2, N, sigma, beta, W);
+}
+
 void grid_size(int N, float* sigma, int* n) {
   const float uptop = (float)std::pow(2.0, std::ceil(std::log10((double)N) / std::log10(2.0)));
   const float s = (float)(2.0 * uptop / (double)N);
@@ -117,7 +121,7 @@ void grid_size(int N, float* sigma, int* n) {
 }
 
 bool build_geometry(Geometry& g, int N0, int N1, int nz, const float* tilt_deg, std::string* err, bool cv,
-                    int window) {
+                    int window, bool tables) {
   if (window != ICON_WINDOW_GAUSS && window != ICON_WINDOW_KB6) {
     if (err) *err = "icon_plan_create: unknown window";
     return false;
@@ -150,8 +154,8 @@ bool build_geometry(Geometry& g, int N0, int N1, int nz, const float* tilt_deg, 
   const bool kb = window == ICON_WINDOW_KB6;
   g.K = kb ? kTapsKB : kTaps;
   if (kb) {
-    g.b0 = kb_beta(g.sig0);
-    g.b1 = kb_beta(g.sig1);
+    g.b0 = kb_beta(g.sig0, kTapsKB);
+    g.b1 = kb_beta(g.sig1, kTapsKB);
     g.bf0 = g.bf1 = 0.f;
   } else {
     window_shape(g.sig0, kWindowM, &g.b0, &g.bf0);
@@ -227,25 +231,27 @@ bool build_geometry(Geometry& g, int N0, int N1, int nz, const float* tilt_deg, 
     else taps(c, N, sigma, b, bf, kWindowM, phi, first);
   };
   auto deapod_of = [&](int k, int N, float sigma, float b) {
-    return kb ? deapod_kb(k, N, sigma, b) : deapod(k, N, sigma, kWindowM);
+    return kb ? deapod_kb(k, N, sigma, b, kTapsKB) : deapod(k, N, sigma, kWindowM);
   };
-  g.phix.resize((size_t)M * K);
-  g.phiy.resize((size_t)M * K);
-  g.ix0.resize(M);
-  g.iy0.resize(M);
-  for (int j = 0; j < M; j++) {
-    node_taps(g.nodes[2 * (size_t)j], N0, g.sig0, g.b0, g.bf0, &g.phix[(size_t)j * K], &g.ix0[j]);
-    node_taps(g.nodes[2 * (size_t)j + 1], N1, g.sig1, g.b1, g.bf1, &g.phiy[(size_t)j * K], &g.iy0[j]);
-  }
+  if (tables) {
+    g.phix.resize((size_t)M * K);
+    g.phiy.resize((size_t)M * K);
+    g.ix0.resize(M);
+    g.iy0.resize(M);
+    for (int j = 0; j < M; j++) {
+      node_taps(g.nodes[2 * (size_t)j], N0, g.sig0, g.b0, g.bf0, &g.phix[(size_t)j * K], &g.ix0[j]);
+      node_taps(g.nodes[2 * (size_t)j + 1], N1, g.sig1, g.b1, g.bf1, &g.phiy[(size_t)j * K], &g.iy0[j]);
+    }
 
-  // deapodisation
-  g.ck.resize((size_t)N0 * N1);
-  {
-    std::vector<float> cy(N1);
-    for (int Y = 0; Y < N1; Y++) cy[Y] = deapod_of(Y - N1 / 2, N1, g.sig1, g.b1);
-    for (int X = 0; X < N0; X++) {
-      const float cx = deapod_of(X - N0 / 2, N0, g.sig0, g.b0);
-      for (int Y = 0; Y < N1; Y++) g.ck[(size_t)X * N1 + Y] = cx * cy[Y];
+    // deapodisation
+    g.ck.resize((size_t)N0 * N1);
+    {
+      std::vector<float> cy(N1);
+      for (int Y = 0; Y < N1; Y++) cy[Y] = deapod_of(Y - N1 / 2, N1, g.sig1, g.b1);
+      for (int X = 0; X < N0; X++) {
+        const float cx = deapod_of(X - N0 / 2, N0, g.sig0, g.b0);
+        for (int Y = 0; Y < N1; Y++) g.ck[(size_t)X * N1 + Y] = cx * cy[Y];
+      }
     }
   }
 
@@ -261,6 +267,21 @@ bool build_geometry(Geometry& g, int N0, int N1, int nz, const float* tilt_deg, 
   return true;
 }
 
+// The entries of each tile in groups of 16, one of every residue of the first
+// x-tap mod 16 in turn (in the order given within a residue).
+static void interp_order(const std::vector<int>& off, const std::vector<int4>& in, std::vector<int4>& out) {
+  out.resize(in.size());
+  std::vector<int> bucket[16];
+  for (size_t blk = 0; blk + 1 < off.size(); blk++) {
+    for (auto& v : bucket) v.clear();
+    for (int e = off[blk]; e < off[blk + 1]; e++) bucket[in[e].z & 15].push_back(e);
+    size_t pos[16] = {};
+    for (int f = off[blk]; f < off[blk + 1];)
+      for (int r = 0; r < 16; r++)
+        if (pos[r] < bucket[r].size()) out[f++] = in[bucket[r][pos[r]++]];
+  }
+}
+
 // Bins every node's run of y-taps by grid-column tile.  A node's K taps are
 // consecutive columns (mod n1), so they fall into at most ceil((K-1)/C)+1 tiles;
 // each (tile, node) pair is one entry recording the tap range, the node's
@@ -268,20 +289,27 @@ bool build_geometry(Geometry& g, int N0, int N1, int nz, const float* tilt_deg, 
 // x-tap.  A tile's entries are sorted by first x-tap (then node), and xoff
 // gives, per tile and grid row x, the first entry whose first x-tap is >= x,
 // so the entries covering row x are those with first x-tap in [x-K+1, x].
-void build_bins(const Geometry& g, int C, Bins& b) {
-  const int K = g.K;
+void build_bins(const Geometry& g, int C, int K, Bins& b) {
+  const int n0 = g.n0, n1 = g.n1, M = g.M;
   b.C = C;
-  b.nblk = g.n1 / C;
+  b.K = K;
+  b.nblk = n1 / C;
+  b.nslot.resize(M);
   b.off.assign(b.nblk + 1, 0);
-  b.nslot.assign(g.M, 0);
-  const int mask = g.n1 - 1;
-  for (int j = 0; j < g.M; j++) {
-    int prev = -1;
-    for (int t = 0; t < K; t++) {
-      const int blk = ((g.iy0[j] + t) & mask) / C;
-      if (blk != prev) { b.off[blk + 1]++; prev = blk; }
-    }
+  // first taps floor(n v) - (K/2 - 1); the run of K columns from iy touches
+  // the tiles iy/C .. (iy + K - 1)/C (mod n1)
+  auto first = [&](float v, int n) { return ((int)std::floor((double)n * (double)v) - (K / 2 - 1)) & (n - 1); };
+  std::vector<int> ix(M), iy(M), xs(n0 + 1, 0), byx(M);
+  for (int j = 0; j < M; j++) {
+    ix[j] = first(g.nodes[2 * (size_t)j], n0);
+    iy[j] = first(g.nodes[2 * (size_t)j + 1], n1);
+    xs[ix[j] + 1]++;
+    const int k0 = iy[j] / C, ns = (iy[j] + K - 1) / C - k0 + 1;
+    b.nslot[j] = (int8_t)ns;
+    for (int q = 0; q < ns; q++) b.off[(k0 + q) % b.nblk + 1]++;
   }
+  for (int x = 0; x < n0; x++) xs[x + 1] += xs[x];
+  for (int j = 0; j < M; j++) byx[xs[ix[j]]++] = j;   // nodes by first x-tap (stable)
   for (int i = 0; i < b.nblk; i++) b.off[i + 1] += b.off[i];
   b.order.resize(b.nblk);
   for (int i = 0; i < b.nblk; i++) b.order[i] = i;
@@ -289,54 +317,25 @@ void build_bins(const Geometry& g, int C, Bins& b) {
     return b.off[u + 1] - b.off[u] > b.off[v + 1] - b.off[v];
   });
   b.ent.resize(b.off[b.nblk]);
+  b.of_node.assign((size_t)M * kMaxSlot, -1);
   std::vector<int> fill(b.off.begin(), b.off.end() - 1);
-  for (int j = 0; j < g.M; j++) {
-    int t = 0, slot = 0;
-    while (t < K) {
-      const int col = (g.iy0[j] + t) & mask;
-      const int blk = col / C;
-      int t1 = t;
-      while (t1 + 1 < K && (((g.iy0[j] + t1 + 1) & mask) / C) == blk) t1++;
-      const int col0 = col - blk * C;
-      b.ent[fill[blk]++] = make_int4(j, t | (t1 << 8) | (slot << 16) | (col0 << 24), g.ix0[j], 0);
-      slot++;
-      t = t1 + 1;
+  for (int i = 0; i < M; i++) {
+    const int j = byx[i], k0 = iy[j] / C;
+    for (int q = 0; q < b.nslot[j]; q++) {
+      const int col = (k0 + q) * C;                       // first column of the tile, unwrapped
+      const int t0 = std::max(0, col - iy[j]), t1 = std::min(K - 1, col + C - 1 - iy[j]);
+      const int blk = (k0 + q) % b.nblk, e = fill[blk]++;
+      b.ent[e] = make_int4(j, t0 | (t1 << 8) | (q << 16) | ((iy[j] + t0 - col) << 24), ix[j], blk);
+      b.of_node[(size_t)j * kMaxSlot + q] = e;
     }
-    b.nslot[j] = (int8_t)slot;
   }
-  const int n0 = g.n0;
   b.xoff.assign((size_t)b.nblk * (n0 + 1), 0);
   for (int blk = 0; blk < b.nblk; blk++) {
-    std::stable_sort(b.ent.begin() + b.off[blk], b.ent.begin() + b.off[blk + 1],
-                     [](const int4& u, const int4& v) { return u.z < v.z; });
     int* xo = &b.xoff[(size_t)blk * (n0 + 1)];
     int e = b.off[blk];
     for (int x = 0; x <= n0; x++) {
       while (e < b.off[blk + 1] && b.ent[e].z < x) e++;
       xo[x] = e;
-    }
-  }
-  // self-contained records: the node's x-taps, the y-tap under every column
-  // of the tile (zero outside the run) and the node -> entries map.  Within a
-  // tile the records are interleaved by field (x-tap pairs, y-tap quads) so
-  // that consecutive entries of one field are contiguous.
-  const size_t E = b.ent.size();
-  b.px.assign(E * K, 0.f);
-  b.py.assign(E * (size_t)C, 0.f);
-  b.of_node.assign((size_t)g.M * kMaxSlot, -1);
-  for (int blk = 0; blk < b.nblk; blk++) {
-    const size_t e0 = b.off[blk], ne = b.off[blk + 1] - e0;
-    for (size_t e = e0; e < e0 + ne; e++) {
-      const int4 r = b.ent[e];
-      const int j = r.x, t0 = r.y & 0xff, t1 = (r.y >> 8) & 0xff, slot = (r.y >> 16) & 0xff;
-      const int col0 = (r.y >> 24) & 0xff;
-      for (int t = 0; t < K; t++)
-        b.px[e0 * K + ((t / 2) * ne + (e - e0)) * 2 + (t & 1)] = g.phix[(size_t)j * K + t];
-      for (int t = t0; t <= t1; t++) {
-        const int c = col0 + t - t0;
-        b.py[e0 * C + ((c / 4) * ne + (e - e0)) * 4 + (c & 3)] = g.phiy[(size_t)j * K + t];
-      }
-      b.of_node[(size_t)j * kMaxSlot + slot] = (int)e;
     }
   }
   // Interpolation order.  The interpolation reads rows of 80 bytes from the
@@ -345,27 +344,97 @@ void build_bins(const Geometry& g, int C, Bins& b) {
   // banks.  Each group of 16 takes the next entry (by x0) of every residue
   // x0 mod 16 in turn, so its first taps differ mod 16 while entries remain
   // in 16 residues, and stay close to each other.
-  b.fent.resize(E);
-  b.fpx.assign(E * K, 0.f);
-  b.fpy.assign(E * (size_t)C, 0.f);
-  for (int blk = 0; blk < b.nblk; blk++) {
-    const size_t e0 = b.off[blk], ne = b.off[blk + 1] - e0;
-    std::vector<size_t> bucket[16];
-    for (size_t e = e0; e < e0 + ne; e++) bucket[b.ent[e].z & 15].push_back(e);
-    size_t pos[16] = {}, f = e0;
-    while (f < e0 + ne) {
-      for (int r = 0; r < 16; r++) {
-        if (pos[r] == bucket[r].size()) continue;
-        const size_t e = bucket[r][pos[r]++];
-        b.fent[f] = b.ent[e];
-        for (int t = 0; t < K; t++)
-          b.fpx[e0 * K + ((t / 2) * ne + (f - e0)) * 2 + (t & 1)] = b.px[e0 * K + ((t / 2) * ne + (e - e0)) * 2 + (t & 1)];
-        for (int c = 0; c < C; c++)
-          b.fpy[e0 * C + ((c / 4) * ne + (f - e0)) * 4 + (c & 3)] = b.py[e0 * C + ((c / 4) * ne + (e - e0)) * 4 + (c & 3)];
-        f++;
-      }
+  interp_order(b.off, b.ent, b.fent);
+}
+
+bool paired_nodes(const Geometry& g) {
+  if (g.N0 % 2) return false;
+  for (int i = 0; i < g.nz; i++)
+    for (int k = 1; k < g.N0 / 2; k++) {
+      const size_t p = (size_t)i * g.N0 + k, q = (size_t)i * g.N0 + g.N0 - k;
+      if (g.nodes[2 * p] != -g.nodes[2 * q] || g.nodes[2 * p + 1] != -g.nodes[2 * q + 1] || g.w[p] != g.w[q])
+        return false;
+    }
+  return true;
+}
+
+// Per column tile of 8, the node rows whose 16 taps (grid points floor(n v) - 7
+// .. + 8 in each dimension) reach it.
+void build_node_bins(const Geometry& g, bool half, NodeBins& b) {
+  constexpr int K = 16, C = 8;
+  const int n0 = g.n0, n1 = g.n1, nblk = (half ? n1 / 2 + C : n1) / C;
+  const int per = half ? g.N0 / 2 + 1 : g.N0, rows = per * g.nz;
+  std::vector<int4> all;
+  all.reserve((size_t)rows * 3);
+  b.nslot.assign(rows, 0);
+  auto add = [&](int r, int t0, int t1, int col0, int x, int blk, unsigned flags) {
+    all.push_back(make_int4(r, t0 | (t1 << 8) | (b.nslot[r] << 16) | (col0 << 24), x & (n0 - 1), (int)(blk | flags)));
+    b.nslot[r]++;
+  };
+  for (int r = 0; r < rows; r++) {
+    const int line = r / per, k = r % per;
+    const size_t j = (size_t)line * g.N0 + (!half ? k : k < per - 1 ? g.N0 / 2 + k : 0);
+    double vx = g.nodes[2 * j], vy = g.nodes[2 * j + 1];
+    const bool mirror = half && vy < 0;
+    if (mirror) vx = -vx, vy = -vy;
+    const int x0 = (int)std::floor((double)n0 * vx) - (K / 2 - 1);
+    const int y0 = (int)std::floor((double)n1 * vy) - (K / 2 - 1);
+    // runs of taps [t0, t1] on consecutive stored columns of one tile: ascending
+    // (column y), or, on the half grid, descending (column -y or n1 - y)
+    for (int t = 0; t < K;) {
+      const int y = y0 + t;
+      const bool rev = half && (y < 0 || y > n1 / 2);
+      const int col = rev ? (y < 0 ? -y : n1 - y) : y & (n1 - 1);
+      int len = rev ? col % C + 1 : C - col % C;   // taps left in the tile
+      if (half && !rev) len = std::min(len, n1 / 2 - y + 1);
+      if (rev && y < 0) len = std::min(len, -y);
+      const int t1 = std::min(K - 1, t + len - 1);
+      const unsigned flags = (mirror ? 1u << 16 : 0u) | (rev ? 1u << 17 : 0u) | (mirror != rev ? 1u << 31 : 0u);
+      add(r, t, t1, col % C, rev ? -x0 - (K - 1) : x0, col / C, flags);
+      t = t1 + 1;
     }
   }
+  // by first x-tap (a counting sort), then by tile
+  std::vector<int> xs(n0 + 1, 0);
+  for (const int4& e : all) xs[e.z + 1]++;
+  for (int x = 0; x < n0; x++) xs[x + 1] += xs[x];
+  std::vector<int> byx(all.size());
+  for (size_t e = 0; e < all.size(); e++) byx[xs[all[e].z]++] = (int)e;
+  b.off.assign(nblk + 1, 0);
+  for (const int4& e : all) b.off[(e.w & 0xffff) + 1]++;
+  for (int k = 0; k < nblk; k++) b.off[k + 1] += b.off[k];
+  std::vector<int4> sorted(all.size());
+  std::vector<int> fill(b.off.begin(), b.off.end() - 1);
+  for (int e : byx) sorted[fill[all[e].w & 0xffff]++] = all[e];
+  interp_order(b.off, sorted, b.ent);
+}
+
+void unpaired_bins(const Geometry& g, const NodeBins& b, NodeBins& u) {
+  const int per = g.N0 / 2 + 1, nblk = (int)b.off.size() - 1;
+  u.off.assign(nblk + 1, 0);
+  u.ent.clear();
+  u.nslot.resize(g.nz);
+  for (int t = 0; t < g.nz; t++) u.nslot[t] = b.nslot[(size_t)t * per + per - 1];
+  for (int blk = 0; blk < nblk; blk++) {
+    for (int e = b.off[blk]; e < b.off[blk + 1]; e++)
+      if (b.ent[e].x % per == per - 1) u.ent.push_back(b.ent[e]);
+    u.off[blk + 1] = (int)u.ent.size();
+  }
+}
+
+void interp_factor(double* l) {
+  constexpr int K = 16;
+  for (int p = 0; p < K; p++)
+    for (int q = 0; q < K; q++) {
+      if (q > p) {
+        l[p * K + q] = 0.0;
+        continue;
+      }
+      double v = p == q ? 0.5 : std::sin(M_PI * 0.5 * (p - q)) / (M_PI * (p - q));
+      for (int k = 0; k < q; k++) v -= l[p * K + k] * l[q * K + k];
+      l[p * K + q] = p == q ? std::sqrt(v) : v / l[q * K + q];
+    }
+  for (int p = 0; p < K; p++) l[p * K + p] = 1.0 / l[p * K + p];
 }
 
 }  // namespace icon

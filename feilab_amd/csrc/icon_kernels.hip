@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "icon_col.h"
 #include "icon_fft.h"
 #include "icon_kernels.h"
 
@@ -40,10 +41,6 @@ namespace icon {
 
 // ------------------------------------------------------------------ row pass
 // One grid row of length NR per team of NR/16 threads; RPB rows per block.
-// LDS rows carry one float2 of padding after every 32 elements: the first
-// pass stores 16 consecutive elements per thread, which without it would put
-// every second thread of a wavefront on the same banks.
-using RowLay = Lay<1, 5, 1>;
 template <int NR>
 constexpr int kRowLds = RowLay::size(NR);
 
@@ -51,14 +48,16 @@ constexpr int kRowLds = RowLay::size(NR);
 // Inputs 0..3 and 12..15 of thread t's first pass over image row X of slice
 // s (the others are padding): CPLX, the complex image rhat; otherwise the
 // real image m, with the ICON update m <- (float)(m - alpha Re(rhat)) and its
-// threshold applied and stored first (UPD; Re(rhat) from a.grad).  All loads are issued before any
+// threshold applied and stored first (UPD; Re(rhat) from a.grad); divided by
+// the deapodisation where DEAP (the transforms; the solve's normal operator
+// takes the plain image).  All loads are issued before any
 // value is used (clamped to column 0 where the input is padding, the value
 // then dropped): a load under a per-lane condition would be compiled into a
 // branch whose merge waits for it before the next load is issued.
-template <int NR, bool CPLX, bool UPD>
+template <int NR, bool CPLX, bool UPD, bool DEAP>
 __device__ __forceinline__ void row_fwd_inputs(float2 (&v)[16], const RowFwdArgs& a, int t, int s, int X,
                                                bool valid, int h1) {
-  float cj[8], mj[8], gj[8];
+  float cj[8], mj[8], gj[8], zj[8];
   float2 rj[8];
   bool ok[8];
   int Yj[8];
@@ -68,15 +67,22 @@ __device__ __forceinline__ void row_fwd_inputs(float2 (&v)[16], const RowFwdArgs
     const int Y = (in_index<NR>(t, j < 4 ? j : j + 8) + h1) & (NR - 1);
     ok[j] = valid && Y < a.N1;
     Yj[j] = ok[j] ? Y : 0;
-    cj[j] = a.ck[(size_t)X * a.N1 + Yj[j]];
+    if constexpr (DEAP) cj[j] = a.ck[(size_t)X * a.N1 + Yj[j]];
     if constexpr (!CPLX) mj[j] = a.m[row0 + Yj[j]];
     if constexpr (CPLX) rj[j] = a.rhat[row0 + Yj[j]];
     if constexpr (UPD) gj[j] = a.grad[row0 + Yj[j]];
+    zj[j] = 0.f;
+  }
+  if constexpr (!CPLX && !DEAP) {
+    if (a.mref) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) zj[j] = a.mref[row0 + Yj[j]];
+    }
   }
   const double al = UPD ? a.alpha[s] : 0.0;
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    asm volatile("" : "+v"(cj[j]));
+    if constexpr (DEAP) asm volatile("" : "+v"(cj[j]));
     if constexpr (!CPLX) asm volatile("" : "+v"(mj[j]));
     if constexpr (CPLX) asm volatile("" : "+v"(rj[j].x), "+v"(rj[j].y));
     if constexpr (UPD) asm volatile("" : "+v"(gj[j]));
@@ -99,10 +105,13 @@ __device__ __forceinline__ void row_fwd_inputs(float2 (&v)[16], const RowFwdArgs
         a.m[row0 + Yj[j]] = nv;
         mv = nv;
       }
-      v[r].x = mv / cj[j];
-    } else {
+      if constexpr (DEAP) v[r].x = mv / cj[j];
+      else v[r].x = mv - zj[j];
+    } else if constexpr (DEAP) {
       v[r].x = rj[j].x / cj[j];
       v[r].y = rj[j].y / cj[j];
+    } else {
+      v[r] = rj[j];
     }
   }
 }
@@ -122,10 +131,13 @@ __device__ __forceinline__ void row_fwd_body(const RowFwdArgs& a, int bid) {
   // with N1 <= NR/2 the inputs 4..11 of every thread are padding
   float2 v[16];
   if (!a.cplx) {
-    if (a.update) row_fwd_inputs<NR, false, true>(v, a, t, s, X, valid, h1);
-    else row_fwd_inputs<NR, false, false>(v, a, t, s, X, valid, h1);
+    if (a.update) row_fwd_inputs<NR, false, true, false>(v, a, t, s, X, valid, h1);
+    else if (a.ck) row_fwd_inputs<NR, false, false, true>(v, a, t, s, X, valid, h1);
+    else row_fwd_inputs<NR, false, false, false>(v, a, t, s, X, valid, h1);
+  } else if (a.ck) {
+    row_fwd_inputs<NR, true, false, true>(v, a, t, s, X, valid, h1);
   } else {
-    row_fwd_inputs<NR, true, false>(v, a, t, s, X, valid, h1);
+    row_fwd_inputs<NR, true, false, false>(v, a, t, s, X, valid, h1);
   }
   FftTwiddles Tw;
   load_twiddles<NR, -1>(Tw, t, a.tw);
@@ -157,18 +169,18 @@ __global__ __launch_bounds__(RPB * (NR / 16)) void k_row_fwd_multi(const RowFwdA
 }
 
 
-// FWD: also the first row pass of A rhat (what k_row_fwd does for a complex
-// image): rhat / ck padded to NR and y-transformed, written to a.fwd_out.
-// The inverse's output slot i and the forward's input slot r of a thread hold
-// the same element t + k T, so the hand-over is a fixed register permutation.
-// Output slots of the inverse row transform that the crop keeps: the image
-// (MODE 0: A^H result), or rhat = image - ahwb with its |rhat|^2 added to acc
-// and, FWD, rhat / ck placed in u as the forward transform's input.  The ck
-// and ahwb values of all slots are loaded before any is used (clamped to
-// column 0 where the slot is padding, the value then dropped): a load under
-// a per-lane condition would be compiled into a branch whose merge waits for
-// it before the next load is issued.
-template <int NR, bool MODE1, bool FWD>
+// Output slots of the inverse row transform that the crop keeps.  MODE 0 (the
+// adjoint transform): the image, deapodised.  MODE 1 (the solve's gradient):
+// rhat = A^H W A m - A^H W b, its real part stored (all that the update
+// takes), its |rhat|^2 added to acc and rhat itself placed in u as the input
+// of the forward row transform that follows.  The inverse's output slot i and
+// the forward's input slot r of a thread hold the same element t + k T, so the
+// hand-over is a fixed register permutation.  The ck or ahwb values of all
+// slots are loaded before any is used (clamped to column 0 where the slot is
+// padding, the value then dropped): a load under a per-lane condition would be
+// compiled into a branch whose merge waits for it before the next load is
+// issued.
+template <int NR, bool MODE1>
 __device__ __forceinline__ void row_adj_outputs(const float2 (&v)[16], float2 (&u)[16], double& acc,
                                                 const RowAdjArgs& a, int t, int s, int X, bool valid, int h1) {
   const size_t row0 = ((size_t)s * a.N0 + X) * a.N1;
@@ -182,40 +194,39 @@ __device__ __forceinline__ void row_adj_outputs(const float2 (&v)[16], float2 (&
     const int Y = (out_index<NR>(t, i) + h1) & (NR - 1);
     ok[i] = valid && Y < a.N1;
     Yj[i] = ok[i] ? Y : 0;
-    cj[i] = a.ck[(size_t)X * a.N1 + Yj[i]];
     if constexpr (MODE1) wj[i] = a.ahwb[row0 + Yj[i]];
+    else cj[i] = a.ck[(size_t)X * a.N1 + Yj[i]];
   }
 #pragma unroll
   for (int i = 0; i < 16; i++) {
     if (out_slot_cropped<NR>(i)) continue;
-    asm volatile("" : "+v"(cj[i]));
     if constexpr (MODE1) asm volatile("" : "+v"(wj[i].x), "+v"(wj[i].y));
+    else asm volatile("" : "+v"(cj[i]));
   }
 #pragma unroll
   for (int i = 0; i < 16; i++) {
     if (out_slot_cropped<NR>(i)) continue;
     if (!ok[i]) continue;
-    const float c = cj[i];
-    const float2 f = make_float2(v[i].x / c, v[i].y / c);
     if constexpr (!MODE1) {
-      a.img[row0 + Yj[i]] = f;
+      const float c = cj[i];
+      if (a.img_re) a.img_re[row0 + Yj[i]] = v[i].x / c;
+      else a.img[row0 + Yj[i]] = make_float2(v[i].x / c, v[i].y / c);
     } else {
-      const float2 r = make_float2(f.x - wj[i].x, f.y - wj[i].y);
+      const float2 r = make_float2(v[i].x - wj[i].x, v[i].y - wj[i].y);
       a.grad[row0 + Yj[i]] = r.x;   // the update reads only Re(rhat)
       acc += (double)r.x * (double)r.x + (double)r.y * (double)r.y;
-      if constexpr (FWD) {
-        constexpr int RL = last_radix<NR>();
-        u[i / RL + (i % RL) * (16 / RL)] = make_float2(r.x / c, r.y / c);
-      }
+      constexpr int RL = last_radix<NR>();
+      u[i / RL + (i % RL) * (16 / RL)] = r;
     }
   }
 }
 
-template <int NR, int RPB, bool FWD>
+// GRAD: mode 1 with the forward row transform; otherwise mode 0.
+template <int NR, int RPB, bool GRAD>
 __device__ __forceinline__ void row_adj_body(const RowAdjArgs& a, int bid) {
   constexpr int T = NR / 16;
   __shared__ float2 lds[RPB * kRowLds<NR>];
-  __shared__ double red[RPB * T];
+  __shared__ double red[RPB * (T > 64 ? T / 64 : 1)];
   const int team = threadIdx.x / T;
   const int t = threadIdx.x % T;
   const int row = bid * RPB + team;
@@ -244,29 +255,30 @@ __device__ __forceinline__ void row_adj_body(const RowAdjArgs& a, int bid) {
   fft_from_lazy<NR, RowLay, 1, 1>(v, lds + team * kRowLds<NR>, t, Tw, a.tw);
   const int h1 = a.N1 >> 1;
   double acc = 0.0;
-  float2 u[16];   // FWD: forward input, slot r holds element t + r T
+  float2 u[16];   // GRAD: forward input, slot r holds element t + r T
 #pragma unroll
   for (int r = 0; r < 16; r++) u[r] = make_float2(0.f, 0.f);
-  if (a.mode == 0) row_adj_outputs<NR, false, false>(v, u, acc, a, t, s, X, valid, h1);
-  else row_adj_outputs<NR, true, FWD>(v, u, acc, a, t, s, X, valid, h1);
-  if (a.mode == 1) {
-    red[threadIdx.x] = acc;
+  row_adj_outputs<NR, GRAD>(v, u, acc, a, t, s, X, valid, h1);
+  if constexpr (GRAD) {
+    // FP64 sum over the team: lane halves within a wavefront, then the
+    // wavefronts in order
+    constexpr int W = T > 64 ? 64 : T;
+#pragma unroll
+    for (int h = W / 2; h > 0; h >>= 1) acc += __shfl_down(acc, h, W);
+    if (t % W == 0) red[team * (T / W) + t / W] = acc;
     __syncthreads();
     if (valid && t == 0) {
       double sum = 0.0;
-      for (int i = 0; i < T; i++) sum += red[team * T + i];
+#pragma unroll
+      for (int w = 0; w < T / W; w++) sum += red[team * (T / W) + w];
       a.rowpart[row] = sum;
     }
-  }
-  if constexpr (FWD) {
     // the inverse's last LDS exchange ended with a barrier
     fft_from_lazy<NR, RowLay, -1, 1, 0, true>(u, lds + team * kRowLds<NR>, t, Tw, a.tw);
     if (valid) {
       float2* o = a.fwd_out + (size_t)row * NR;
-      const unsigned zw = (unsigned)(a.zhi - a.zlo);
 #pragma unroll
-      for (int i = 0; i < 16; i++)
-        if ((unsigned)(out_index<NR>(t, i) - a.zlo) >= zw) o[out_index<NR>(t, i)] = u[i];
+      for (int i = 0; i < 16; i++) o[out_index<NR>(t, i)] = u[i];
     }
   }
 }
@@ -274,19 +286,17 @@ __device__ __forceinline__ void row_adj_body(const RowAdjArgs& a, int bid) {
 // The launch bound asks for 2 waves per SIMD (up to 256 registers); with the
 // twiddles loaded pass by pass the kernel needs 112 and runs 4 waves per SIMD
 // (with all twiddles up front it needed 132, and capped at 128 it spilled).
-template <int NR, int RPB, bool FWD>
+template <int NR, int RPB, bool GRAD>
 __global__ __launch_bounds__(RPB * (NR / 16), 2) void k_row_adj(RowAdjArgs a) {
-  row_adj_body<NR, RPB, FWD>(a, blockIdx.x);
+  row_adj_body<NR, RPB, GRAD>(a, blockIdx.x);
 }
 
-template <int NR, int RPB, bool FWD>
+template <int NR, int RPB, bool GRAD>
 __global__ __launch_bounds__(RPB * (NR / 16), 2) void k_row_adj_multi(const RowAdjArgs* __restrict__ descs,
-                                                                     const int2* __restrict__ items, int mode) {
+                                                                     const int2* __restrict__ items) {
   const int2 it = items[blockIdx.x];
-  RowAdjArgs a = descs[it.x];
-  a.mode = mode;
-  if (!FWD) a.fwd_out = nullptr;
-  row_adj_body<NR, RPB, FWD>(a, it.y);
+  const RowAdjArgs a = descs[it.x];
+  row_adj_body<NR, RPB, GRAD>(a, it.y);
 }
 
 // --------------------------------------------------------------- column pass
@@ -311,39 +321,8 @@ __device__ __forceinline__ const float4* tile_py(const ColArgs& a, int e0) {
   return reinterpret_cast<const float4*>(a.ent_py + (size_t)e0 * C);
 }
 
-// Row stride (float2) of the LDS tile: C + 2 keeps rows 16-byte aligned for
-// vector reads while two blocks still share a CU's LDS; otherwise C + 1.
-template <int NC, int C>
-__host__ __device__ constexpr int col_stride() {
-  return NC * (C + 2) * 8 <= 81920 ? C + 2 : C + 1;
-}
-
-// Layouts of the tile during the x FFT's exchanges.  A wavefront holds 64/C
-// threads per column; at C = 8 each of its 8-byte loads and stores touches 8
-// rows of the C columns at once, and the layout puts those rows on disjoint
-// banks (2 cycles per 64-lane access, the minimum):
-// * interpolation: row stride C, 8 float2 of padding after every 16 rows;
-// * spread: row stride C, 1 float2 of padding after every 4 rows, which also
-//   keeps the spread's own stores conflict-free (each thread writes its two
-//   whole rows, 2 apart across lanes, where the padding every 16 rows would
-//   put 4 lanes on one bank).
-// The stride C + 1 used before took 3 cycles for most FFT accesses.
-template <int C>
-using ColFftLayFwd = Lay<C, 4, 8>;
-template <int C>
-using ColFftLay = Lay<C, 2, 1>;
-
-// float2 of LDS per column block: the tile, or an FFT layout if larger
-template <int NC, int C>
-__host__ __device__ constexpr int col_lds() {
-  constexpr int tile = NC * col_stride<NC, C>();
-  constexpr int fwd = ColFftLayFwd<C>::at(NC - 1) + C, adj = ColFftLay<C>::at(NC - 1) + C;
-  return tile > fwd ? (tile > adj ? tile : adj) : (fwd > adj ? fwd : adj);
-}
-
 template <int NC, int C, int K>
 __device__ __forceinline__ void col_fwd_body(const ColArgs& a, int bid) {
-  constexpr int NT = C * (NC / 16);
   constexpr int LS = col_stride<NC, C>();
   extern __shared__ __align__(16) float2 tile[];   // col_lds<NC, C>()
   // tile-major order: blocks in flight together work on the same column
@@ -357,108 +336,19 @@ __device__ __forceinline__ void col_fwd_body(const ColArgs& a, int bid) {
   const int s = bid % a.S;
   const int y0 = blk * C;
   const int tid = threadIdx.x;
-  const int h0 = a.N0 >> 1;
   // a tile no node reaches (beyond the largest |ky| of the tilt range) has
   // nothing to interpolate: its FFT is not needed
   if (a.ent_off[blk] == a.ent_off[blk + 1]) return;
-  // x FFT of column c = tid % C: the first pass takes its 16 inputs (grid
-  // rows t + r NC/16; zero padding outside the N0 non-zero rows) straight
-  // from global memory, all loads in flight together; the transform leaves
-  // its output in the LDS tile for the interpolation
   {
     const int c = tid % C, t = tid / C;
     float2 v[16];
-    // rows x in [NC/4, 3NC/4) (inputs 4..11) are padding, as N0 <= NC/2;
-    // the other inputs are loaded unconditionally (rows past N0, only when
-    // N0 < NC/2, read row 0 and are dropped afterwards).  A conditional load
-    // per input would be compiled into branches whose merges wait for each
-    // load before the next is issued; the empty asm below takes the loaded
-    // values unconditionally, so that all loads are issued first.
-    float2 g[8];
-    bool ok[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int X = (in_index<NC>(t, j < 4 ? j : j + 8) + h0) & (NC - 1);
-      ok[j] = X < a.N0;
-      g[j] = a.in[((size_t)s * a.N0 + (ok[j] ? X : 0)) * a.n1 + y0 + c];
-    }
-    // the twiddles (first used after the first pass) are requested after
-    // the grid rows, so that the first pass waits for the rows only
-    FftTwiddles T;
-    load_twiddles<NC, -1>(T, t, a.tw);
-#pragma unroll
-    for (int j = 0; j < 8; j++) asm volatile("" : "+v"(g[j].x), "+v"(g[j].y));
-#pragma unroll
-    for (int r = 0; r < 16; r++) v[r] = make_float2(0.f, 0.f);
-#pragma unroll
-    for (int j = 0; j < 8; j++)
-      if (ok[j]) v[j < 4 ? j : j + 8] = g[j];
-    fft_regs_half<NC, ColFftLayFwd<C>, -1>(v, tile + c, t, T);
+    col_fft_fwd<NC, C>(v, a, tile, s, y0);
     // the last exchange ended with a barrier: the column can be overwritten
 #pragma unroll
     for (int i = 0; i < 16; i++) tile[out_index<NC>(t, i) * LS + c] = v[i];
   }
   __syncthreads();
-  // interpolation partials of this tile's nodes: one bin entry per thread;
-  // the entry's record (first x-tap, 14 x-taps, C y-taps) comes in with
-  // vector loads and the thread sums its 14 x C cells from the LDS tile
-  const int e0 = a.ent_off[blk], e1 = a.ent_off[blk + 1], ne = e1 - e0;
-  for (int e = e0 + tid; e < e1; e += NT) {
-    const int4 en = a.fent[e];
-    float px[K];
-    const float2* pxv = reinterpret_cast<const float2*>(a.fent_px + (size_t)e0 * K) + (e - e0);
-#pragma unroll
-    for (int q = 0; q < K / 2; q++) {
-      const float2 p = pxv[q * ne];
-      px[2 * q] = p.x;
-      px[2 * q + 1] = p.y;
-    }
-    float py[C];
-    const float4* pyv = reinterpret_cast<const float4*>(a.fent_py + (size_t)e0 * C) + (e - e0);
-#pragma unroll
-    for (int c4 = 0; c4 < C / 4; c4++) {
-      const float4 v = pyv[c4 * ne];
-      py[4 * c4] = v.x; py[4 * c4 + 1] = v.y; py[4 * c4 + 2] = v.z; py[4 * c4 + 3] = v.w;
-    }
-    // separable window: each grid row is first reduced over its C y-taps,
-    // then weighted by its x-tap
-    float ax = 0.f, ay = 0.f;
-    auto add_row = [&](const float2* row, int q) {
-      float2 gv[C];
-      if constexpr (LS % 2 == 0) {
-#pragma unroll
-        for (int c2 = 0; c2 < C / 2; c2++) {
-          const float4 g4 = reinterpret_cast<const float4*>(row)[c2];
-          gv[2 * c2] = make_float2(g4.x, g4.y);
-          gv[2 * c2 + 1] = make_float2(g4.z, g4.w);
-        }
-      } else {
-#pragma unroll
-        for (int c = 0; c < C; c++) gv[c] = row[c];
-      }
-      float tx = 0.f, ty = 0.f;
-#pragma unroll
-      for (int c = 0; c < C; c++) {
-        tx = __fmaf_rn(gv[c].x, py[c], tx);
-        ty = __fmaf_rn(gv[c].y, py[c], ty);
-      }
-      ax = __fmaf_rn(tx, px[q], ax);
-      ay = __fmaf_rn(ty, px[q], ay);
-    };
-    // Entries whose taps wrap past row NC-1 have the largest first taps and
-    // come last in the tile's order: only the last wavefronts can hold them;
-    // the others take the fully unrolled loop with one base address and
-    // constant row offsets.
-    if (__builtin_amdgcn_ballot_w64(en.z > NC - K) == 0) {
-      const float2* base = tile + en.z * LS;
-#pragma unroll
-      for (int q = 0; q < K; q++) add_row(base + q * LS, q);
-    } else {
-#pragma unroll 2
-      for (int q = 0; q < K; q++) add_row(tile + ((en.z + q) & (NC - 1)) * LS, q);
-    }
-    a.part[((size_t)s * a.M + en.x) * kMaxSlotK + ((en.y >> 16) & 0xff)] = make_float2(ax, ay);
-  }
+  interp_tile<NC, C, K>(a, tile, blk, s);
 }
 
 template <int NC, int C, int K>
@@ -474,9 +364,15 @@ __global__ __launch_bounds__(C * (NC / 16), 4) void k_col_fwd_multi(const ColArg
   col_fwd_body<NC, C, K>(a, it.y);
 }
 
-template <int NC, int C, int K>
+// V: float2 (the adjoint transform), or double2, which accumulates and transforms
+// in FP64 into out64 (the solve's data set-up: its gradient subtracts A^H W b
+// in every iteration, so that an error of it in directions that no tilt covers
+// adds up over the iterations).
+template <int NC, int C, int K, typename V>
 __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
   constexpr int NT = C * (NC / 16);
+  constexpr bool DBL = sizeof(V) == 16;
+  using T = decltype(V::x);
   constexpr int RL = NC / NT;                    // adjacent grid rows per thread
   static_assert(RL >= 1 && RL <= 2 && NT * RL == NC, "one or two grid rows per thread");
   // staged record, 16-byte aligned fields: the K x-taps at [RL-1, RL-1+K)
@@ -498,8 +394,11 @@ __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
   // inside the zero band the row kernel takes the zeros without loading them
   if (a.ent_off[blk] == a.ent_off[blk + 1]) {
     if (y0 >= a.zlo && y0 < a.zhi) return;
-    for (int i = tid; i < a.N0 * C; i += NT)
-      a.out[((size_t)s * a.N0 + i / C) * a.n1 + y0 + i % C] = make_float2(0.f, 0.f);
+    for (int i = tid; i < a.N0 * C; i += NT) {
+      const size_t o = ((size_t)s * a.N0 + i / C) * a.n1 + y0 + i % C;
+      if constexpr (DBL) a.io64[o] = make_double2(0.0, 0.0);
+      else a.out[o] = make_float2(0.f, 0.f);
+    }
     return;
   }
   // Spread as a gather.  Rows [x, x+RL) of the tile are covered by the
@@ -534,7 +433,7 @@ __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
     h[1] = xo[x + RL];
   };
   // adds entry record `rec` to the rows at x (accumulators ac)
-  auto add = [&](const float* rec, int x, float2 (&ac)[RL][C]) {
+  auto add = [&](const float* rec, int x, V (&ac)[RL][C]) {
     const float4 tail = reinterpret_cast<const float4*>(rec)[XS / 4 + C / 4];
     // x-tap slot of row x: (x - z) + RL - 1, in [0, K + RL - 2] by the range
     const int q = (x - __float_as_int(tail.z) + RL - 1) & (NC - 1);
@@ -550,16 +449,21 @@ __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
 #pragma unroll
     for (int r = 0; r < RL; r++) {
       // the value weighted by this row's x-tap, then by each y-tap
-      const float fx = tail.x * px[r], fy = tail.y * px[r];
+      const T fx = (T)tail.x * (T)px[r], fy = (T)tail.y * (T)px[r];
 #pragma unroll
       for (int c = 0; c < C; c++) {
-        ac[r][c].x = __fmaf_rn(fx, py[c], ac[r][c].x);
-        ac[r][c].y = __fmaf_rn(fy, py[c], ac[r][c].y);
+        if constexpr (DBL) {
+          ac[r][c].x = __fma_rn(fx, (T)py[c], ac[r][c].x);
+          ac[r][c].y = __fma_rn(fy, (T)py[c], ac[r][c].y);
+        } else {
+          ac[r][c].x = __fmaf_rn(fx, py[c], ac[r][c].x);
+          ac[r][c].y = __fmaf_rn(fy, py[c], ac[r][c].y);
+        }
       }
     }
   };
   // adds the staged entries [lo, hi) of the chunk at cb (cn records) to the rows at x
-  auto add_range = [&](int lo, int hi, int cb, int cn, int x, float2 (&ac)[RL][C]) {
+  auto add_range = [&](int lo, int hi, int cb, int cn, int x, V (&ac)[RL][C]) {
     const int k1 = min(hi, cb + cn) - cb;
     int k = max(lo, cb) - cb;
     for (; k + 1 < k1; k += 2) {
@@ -569,6 +473,7 @@ __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
     if (k < k1) add(stage + k * REC, x, ac);
   };
   FftTwiddles Tw;   // of the inverse x FFT, loaded while the tile is written
+  double2 w[DBL ? 16 : 1];   // FP64: the column for the inverse x FFT
   auto gather = [&](auto split_tag) {
     constexpr bool SPLIT = decltype(split_tag)::value;
     int lo[2], hi[2], lp[2], hp[2];
@@ -583,17 +488,17 @@ __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
       lp[0] += min(m0, g);
       lp[1] += max(0, g - m0);
     }
-    float2 acc[RL][C], accp[SPLIT ? RL : 1][C];
+    V acc[RL][C], accp[SPLIT ? RL : 1][C];
 #pragma unroll
     for (int r = 0; r < RL; r++) {
 #pragma unroll
-      for (int c = 0; c < C; c++) acc[r][c] = make_float2(0.f, 0.f);
+      for (int c = 0; c < C; c++) acc[r][c] = c_make((T)0, (T)0);
     }
     if constexpr (SPLIT) {
 #pragma unroll
       for (int r = 0; r < RL; r++) {
 #pragma unroll
-        for (int c = 0; c < C; c++) accp[r][c] = make_float2(0.f, 0.f);
+        for (int c = 0; c < C; c++) accp[r][c] = c_make((T)0, (T)0);
       }
     }
     for (int cb = e0; cb < e1; cb += CAP) {
@@ -627,7 +532,39 @@ __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
         if constexpr (SPLIT) add_range(lp[run], hp[run], cb, cn, xp, accp);
       }
     }
-    if constexpr (SPLIT) {
+    if constexpr (DBL) {
+      // the same, one component at a time through the tile's LDS as doubles,
+      // and the rows' columns into v
+      double* lds = reinterpret_cast<double*>(tile);
+      const int c0 = tid % C, t = tid / C;
+      __syncthreads();   // the staged records are consumed
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        if constexpr (SPLIT) {
+#pragma unroll
+          for (int r = 0; r < RL; r++)
+#pragma unroll
+            for (int c = 0; c < C; c++) lds[ColFftLay<C>::at(xp + r) + c] = k ? accp[r][c].y : accp[r][c].x;
+          __syncthreads();
+        }
+#pragma unroll
+        for (int r = 0; r < RL; r++)
+#pragma unroll
+          for (int c = 0; c < C; c++) {
+            double& cell = lds[ColFftLay<C>::at(x0 + r) + c];
+            const double own = k ? acc[r][c].y : acc[r][c].x;
+            cell = SPLIT ? own + cell : own;
+          }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const double x = lds[ColFftLay<C>::at(in_index<NC>(t, r)) + c0];
+          if (k) w[r].y = x;
+          else w[r].x = x;
+        }
+        __syncthreads();
+      }
+    } else if constexpr (SPLIT) {
       __syncthreads();   // the staged records are consumed
       // the partner's second halves into the tile, then each thread adds
       // its own first halves to them
@@ -659,6 +596,17 @@ __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
   };
   if (e1 - e0 >= a.split_min) gather(std::true_type{});
   else gather(std::false_type{});
+  if constexpr (DBL) {
+    const int c = tid % C, t = tid / C, h0 = a.N0 >> 1;
+    fft64<NC, ColFftLay<C>, 1>(w, reinterpret_cast<double*>(tile) + c, t, a.w64);
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      if (out_slot_cropped<NC>(i)) continue;
+      const int X = (out_index<NC>(t, i) + h0) & (NC - 1);
+      if (X < a.N0) a.io64[((size_t)s * a.N0 + X) * a.n1 + y0 + c] = w[i];
+    }
+    return;
+  }
   __syncthreads();
   // inverse x FFT of column c = tid % C; the last pass writes the N0 rows the
   // crop keeps (grid row x -> image row X = x + N0/2 mod NC) straight to global
@@ -680,7 +628,7 @@ __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
 
 template <int NC, int C, int K>
 __global__ __launch_bounds__(C * (NC / 16), 4) void k_col_adj(ColArgs a) {
-  col_adj_body<NC, C, K>(a, blockIdx.x);
+  col_adj_body<NC, C, K, float2>(a, blockIdx.x);
 }
 
 template <int NC, int C, int K>
@@ -688,64 +636,73 @@ __global__ __launch_bounds__(C * (NC / 16), 4) void k_col_adj_multi(const ColArg
                                                                    const int2* __restrict__ items) {
   const int2 it = items[blockIdx.x];
   const ColArgs a = descs[it.x];
-  col_adj_body<NC, C, K>(a, it.y);
+  col_adj_body<NC, C, K, float2>(a, it.y);
+}
+
+template <int NC, int C, int K>
+__global__ __launch_bounds__(C * (NC / 16), 2) void k_col_adj64(ColArgs a) {
+  col_adj_body<NC, C, K, double2>(a, blockIdx.x);
+}
+
+template <int NC, int C, int K>
+__global__ __launch_bounds__(C * (NC / 16), 2) void k_col_adj64_multi(const ColArgs* __restrict__ descs,
+                                                                     const int2* __restrict__ items) {
+  const int2 it = items[blockIdx.x];
+  const ColArgs a = descs[it.x];
+  col_adj_body<NC, C, K, double2>(a, it.y);
+}
+
+// The FP64 adjoint's row pass: the image (or its real part), deapodised, one
+// grid row per block.
+template <int NR>
+__device__ __forceinline__ void row_adj64_body(const RowAdjArgs& a, int row) {
+  __shared__ double lds[RowLay::size(NR)];
+  const int t = threadIdx.x, X = row % a.N0, h1 = a.N1 >> 1;
+  double2 v[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int y = in_index<NR>(t, r);
+    const bool zero = y >= a.zlo && y < a.zhi;
+    v[r] = zero ? make_double2(0.0, 0.0) : a.in64[(size_t)row * NR + y];
+  }
+  fft64<NR, RowLay, 1>(v, lds, t, a.w64);
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    if (out_slot_cropped<NR>(i)) continue;
+    const int Y = (out_index<NR>(t, i) + h1) & (NR - 1);
+    if (Y >= a.N1) continue;
+    const double c = (double)a.ck[(size_t)X * a.N1 + Y];
+    const size_t p = (size_t)row * a.N1 + Y;
+    if (a.img_re) a.img_re[p] = (float)(v[i].x / c);
+    else a.img[p] = make_float2((float)(v[i].x / c), (float)(v[i].y / c));
+  }
+}
+
+template <int NR>
+__global__ __launch_bounds__(NR / 16) void k_row_adj64(RowAdjArgs a) { row_adj64_body<NR>(a, blockIdx.x); }
+
+template <int NR>
+__global__ __launch_bounds__(NR / 16) void k_row_adj64_multi(const RowAdjArgs* __restrict__ descs,
+                                                             const int2* __restrict__ items) {
+  const int2 it = items[blockIdx.x];
+  const RowAdjArgs a = descs[it.x];
+  row_adj64_body<NR>(a, it.y);
 }
 
 // ------------------------------------------------------------ node combine
 // One block (1024 threads) per slice.  FP64 block reductions in a fixed order.
 
-
-__device__ __forceinline__ double block_sum_1024(double v, double* red) {
-  const int tid = threadIdx.x;
-  red[tid] = v;
-  __syncthreads();
-#pragma unroll
-  for (int h = 512; h > 0; h >>= 1) {
-    if (tid < h) red[tid] += red[tid + h];
-    __syncthreads();
-  }
-  const double r = red[0];
-  __syncthreads();
-  return r;
-}
-
+// Mode 2: f = b of the projection rows, weighted into every bin entry of its
+// node, and bnorm = sum w |b|^2; mode 3: the node values of a forward
+// transform from the column tiles' partials.
 __device__ __forceinline__ void combine_body(const CombineArgs& a, int s) {
   __shared__ double red[1024];
   const int tid = threadIdx.x;
   double acc = 0.0;
-  const float2* P = a.part + (size_t)s * a.M * kMaxSlotK;
   for (int j = tid; j < a.M; j += 1024) {
-    float2 f;
     if (a.mode == 2) {
-      f = a.b[(size_t)s * a.M + j];
-    } else {
-      const int ns = a.nslot[j];
-      f = P[(size_t)j * kMaxSlotK];
-      for (int q = 1; q < ns; q++) {
-        const float2 p = P[(size_t)j * kMaxSlotK + q];
-        f.x += p.x;
-        f.y += p.y;
-      }
-    }
-    const float wj = a.w[j];
-    if (a.mode == 0) {
-      if (a.resid) {
-        const float2 bj = a.b[(size_t)s * a.M + j];
-        const double dx = (double)f.x - (double)bj.x, dy = (double)f.y - (double)bj.y;
-        acc += (double)wj * (dx * dx + dy * dy);
-      }
-      if (a.frep) {
-        const int i = j / a.N0;
-        if (i == a.iomit) a.frep[(size_t)s * a.N0 + (j - i * a.N0)] = f;
-      }
-      const float2 v = make_float2(f.x * wj, f.y * wj);
-      for (int q = 0; q < kMaxSlotK; q++) {
-        const int e = a.ent_of_node[(size_t)j * kMaxSlotK + q];
-        if (e >= 0) a.fw[(size_t)s * a.E + e] = v;
-      }
-    } else if (a.mode == 1) {
-      acc += (double)f.x * (double)f.x * (double)wj + (double)f.y * (double)f.y * (double)wj;
-    } else if (a.mode == 2) {
+      const float2 f = a.b[(size_t)s * a.M + j];
+      const float wj = a.w[j];
       acc += (double)wj * ((double)f.x * (double)f.x + (double)f.y * (double)f.y);
       const float2 v = make_float2(f.x * wj, f.y * wj);
       for (int q = 0; q < kMaxSlotK; q++) {
@@ -753,53 +710,20 @@ __device__ __forceinline__ void combine_body(const CombineArgs& a, int s) {
         if (e >= 0) a.fw[(size_t)s * a.E + e] = v;
       }
     } else {
-      a.fw[(size_t)s * a.M + j] = f;
+      a.fw[(size_t)s * a.M + j] = node_value(a.part + (size_t)s * a.M * kMaxSlotK, a.nslot, j, kMaxSlotK);
     }
   }
   if (a.mode == 3) return;
-  if (a.mode == 0 && !a.resid) return;
   const double tot = block_sum_1024(acc, red);
-  if (a.mode == 0) {
-    if (tid == 0) {
-      const double bn = a.bnorm[s];
-      a.resid[(size_t)s * a.resid_stride + a.resid_index] = bn > 0 ? sqrt(tot / bn) : 0.0;
-    }
-  } else if (a.mode == 2) {
-    if (tid == 0) a.bnorm[s] = tot;
-  } else {
-    // rtr = sum of the row partials in row order, summed from LDS (red is
-    // free after block_sum_1024's last barrier): the block loads them in one
-    // round trip, where a loop of global loads on one thread waits for each
-    double rtr = 0.0;
-    for (int X0 = 0; X0 < a.N0; X0 += 1024) {
-      if (X0 + tid < a.N0) red[tid] = a.rowpart[(size_t)s * a.N0 + X0 + tid];
-      __syncthreads();
-      if (tid == 0)
-        for (int X = 0; X < min(1024, a.N0 - X0); X++) rtr += red[X];
-      __syncthreads();
-    }
-    if (tid == 0) {
-      const double al = tot != 0.0 ? rtr / tot : 0.0;
-      a.alpha[s] = al;
-      if (a.alpha_trace) a.alpha_trace[(size_t)s * a.alpha_stride + a.alpha_index] = al;
-    }
-  }
+  if (tid == 0) a.bnorm[s] = tot;
 }
 
 __global__ __launch_bounds__(1024) void k_combine(CombineArgs a) { combine_body(a, blockIdx.x); }
 
-// Packed launch: the per-launch mode and trace indices by value; with_resid /
-// with_frep switch the series' residual trace and reprojection values on.
 __global__ __launch_bounds__(1024) void k_combine_multi(const CombineArgs* __restrict__ descs,
-                                                        const int2* __restrict__ items, CombineLaunch L) {
+                                                        const int2* __restrict__ items) {
   const int2 it = items[blockIdx.x];
-  CombineArgs a = descs[it.x];
-  a.mode = L.mode;
-  a.resid_index = L.resid_index;
-  a.alpha_index = L.alpha_index;
-  if (!L.with_resid) a.resid = nullptr;
-  if (!L.with_frep) a.frep = nullptr;
-  combine_body(a, it.y);
+  combine_body(descs[it.x], it.y);
 }
 
 // ------------------------------------------------------- projection rows (1D)
@@ -1005,8 +929,6 @@ __global__ __launch_bounds__(256) void k_copy_f4(float4* __restrict__ dst, const
 
 namespace {
 
-thread_local hipEvent_t t_ev_start = nullptr, t_ev_stop = nullptr;
-
 template <int NR>
 constexpr int rows_per_block() {
   return NR >= 2048 ? 2 : 256 / (NR / 16) > 16 ? 16 : 256 / (NR / 16);
@@ -1023,20 +945,12 @@ constexpr int row_adj_rows_per_block() {
 
 }  // namespace
 
+thread_local hipEvent_t t_ev_start = nullptr, t_ev_stop = nullptr;
+
 void set_launch_events(hipEvent_t start, hipEvent_t stop) {
   t_ev_start = start;
   t_ev_stop = stop;
 }
-
-// hipLaunchKernelGGL, or, while timing events are set, hipExtLaunchKernelGGL
-// with them (the events then bracket the kernel itself, not the enqueue)
-#define LAUNCH_TIMED(KERNEL, GRID, BLOCK, SHM, ST, ...)                                          \
-  do {                                                                                           \
-    if (t_ev_start)                                                                              \
-      hipExtLaunchKernelGGL(KERNEL, GRID, BLOCK, SHM, ST, t_ev_start, t_ev_stop, 0, __VA_ARGS__); \
-    else                                                                                         \
-      hipLaunchKernelGGL(KERNEL, GRID, BLOCK, SHM, ST, __VA_ARGS__);                             \
-  } while (0)
 
 #define ROW_CASES(X) X(128) X(256) X(512) X(1024) X(2048)
 
@@ -1063,7 +977,7 @@ hipError_t launch_row_adj(int NR, const RowAdjArgs& a, hipStream_t st) {
 #define CASE(N)                                                                                     \
   case N: {                                                                                         \
     constexpr int RPB = row_adj_rows_per_block<N>();                                                \
-    if (h.fwd_out)                                                                                  \
+    if (h.grad)                                                                                     \
       LAUNCH_TIMED((k_row_adj<N, RPB, true>), dim3((h.rows + RPB - 1) / RPB), dim3(RPB * (N / 16)), 0, \
                          st, a);                                                                    \
     else                                                                                            \
@@ -1126,11 +1040,13 @@ hipError_t launch_fft_rows(int NR, float2* data, int rows, int sign, const float
 }
 
 // Column kernels: (NC, C) with NC * C * 8 bytes of LDS.
-// (n0, C, taps) of the column kernels built: the Gaussian window at every
-// tile width, the Kaiser-Bessel window at C = 8
+// (n0, C, taps) of the column kernels built: the 10-tap window at every tile
+// width, the 6-tap one at C = 8
 #define COL_CASES(X)                                                                                 \
-  X(128, 8, 14) X(128, 16, 14) X(256, 8, 14) X(256, 16, 14) X(512, 8, 14) X(512, 16, 14) X(1024, 8, 14) \
-  X(1024, 16, 14) X(2048, 8, 14) X(128, 8, 6) X(256, 8, 6) X(512, 8, 6) X(1024, 8, 6) X(2048, 8, 6)
+  X(128, 8, 10) X(128, 16, 10) X(256, 8, 10) X(256, 16, 10) X(512, 8, 10) X(512, 16, 10) X(1024, 8, 10) \
+  X(1024, 16, 10) X(2048, 8, 10) X(128, 8, 6) X(256, 8, 6) X(512, 8, 6) X(1024, 8, 6) X(2048, 8, 6)
+// ... and the solve's 16-tap interpolation (forward only, C = 8)
+#define COL_FWD_CASES(X) X(128, 8, 16) X(256, 8, 16) X(512, 8, 16) X(1024, 8, 16) X(2048, 8, 16)
 #define FFT_COL_CASES(X) X(128, 8) X(128, 16) X(256, 8) X(256, 16) X(512, 8) X(512, 16) X(1024, 8) X(1024, 16) X(2048, 8)
 
 bool col_tile_ok(int NC, int n1, int C, int K) {
@@ -1202,6 +1118,115 @@ hipError_t launch_col(int NC, int C, bool adjoint, const ColArgs& a, hipStream_t
   return e;
 }
 
+// FP64 data adjoint (10 taps, C = 8 or 16, n0 <= 1024)
+#define COL64_CASES(X) X(128, 8) X(128, 16) X(256, 8) X(256, 16) X(512, 8) X(512, 16) X(1024, 8)
+
+hipError_t set_adj64_attrs() {
+#define CASE(N, CC)                                                                                                  \
+  for (const void* p : {(const void*)k_col_adj64<N, CC, 10>, (const void*)k_col_adj64_multi<N, CC, 10>}) {           \
+    hipError_t e = hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize,                                \
+                                       col_lds<N, CC>() * (int)sizeof(float2));                                      \
+    if (e != hipSuccess) return e;                                                                                   \
+  }
+  COL64_CASES(CASE)
+#undef CASE
+  return hipSuccess;
+}
+
+bool adj64_ok(int NC, int C, int K) {
+#define CASE(N, CC) if (NC == N && C == CC) return K == 10;
+  COL64_CASES(CASE)
+#undef CASE
+  return false;
+}
+
+hipError_t launch_col_adj64(int NC, int C, const ColArgs& a, hipStream_t st) {
+#define CASE(N, CC)                                                                                    \
+  if (NC == N && C == CC) {                                                                            \
+    hipLaunchKernelGGL((k_col_adj64<N, CC, 10>), dim3(a.S * (a.n1 / CC)), dim3(CC * (N / 16)),         \
+                       (col_lds<N, CC>()) * sizeof(float2), st, a);                                    \
+    return hipGetLastError();                                                                          \
+  }
+  COL64_CASES(CASE)
+#undef CASE
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_col_adj64_multi(int NC, int C, const ColArgs* descs, const int2* items, int n, hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+#define CASE(N, CC)                                                                                    \
+  if (NC == N && C == CC) {                                                                            \
+    hipLaunchKernelGGL((k_col_adj64_multi<N, CC, 10>), dim3(n), dim3(CC * (N / 16)),                   \
+                       (col_lds<N, CC>()) * sizeof(float2), st, descs, items);                         \
+    return hipGetLastError();                                                                          \
+  }
+  COL64_CASES(CASE)
+#undef CASE
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_row_adj64(int NR, const RowAdjArgs& a, hipStream_t st) {
+  switch (NR) {
+#define CASE(N) case N: hipLaunchKernelGGL((k_row_adj64<N>), dim3(a.rows), dim3(N / 16), 0, st, a); break;
+    ROW_CASES(CASE)
+#undef CASE
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_row_adj64_multi(int NR, const RowAdjArgs* descs, const int2* items, int n, hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+  switch (NR) {
+#define CASE(N) case N: hipLaunchKernelGGL((k_row_adj64_multi<N>), dim3(n), dim3(N / 16), 0, st, descs, items); break;
+    ROW_CASES(CASE)
+#undef CASE
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+// The forward column pass at the solve's nodes (16 taps), after the last update.
+hipError_t launch_col_fwd_nodes(int NC, const ColArgs& a, hipStream_t st) {
+#define CASE(N, CC, KK)                                                                                  \
+  if (NC == N) {                                                                                         \
+    static_assert(CC == kNormalC && KK == kInterpTaps, "the solve's interpolation");                     \
+    LAUNCH_TIMED((k_col_fwd<N, CC, KK>), dim3(a.S * (a.n1 / CC)), dim3(CC * (N / 16)),                   \
+                 (col_lds<N, CC>()) * sizeof(float2), st, a);                                            \
+    return hipGetLastError();                                                                            \
+  }
+  COL_FWD_CASES(CASE)
+#undef CASE
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_col_fwd_nodes_multi(int NC, const ColArgs* descs, const int2* items, int n, hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+#define CASE(N, CC, KK)                                                                                  \
+  if (NC == N) {                                                                                         \
+    LAUNCH_TIMED((k_col_fwd_multi<N, CC, KK>), dim3(n), dim3(CC * (N / 16)),                             \
+                 (col_lds<N, CC>()) * sizeof(float2), st, descs, items);                                 \
+    return hipGetLastError();                                                                            \
+  }
+  COL_FWD_CASES(CASE)
+#undef CASE
+  return hipErrorInvalidValue;
+}
+
+hipError_t set_col_fwd_nodes_attrs(int NC) {
+#define CASE(N, CC, KK)                                                                                            \
+  if (NC == N) {                                                                                                   \
+    hipError_t e = hipFuncSetAttribute((const void*)k_col_fwd<N, CC, KK>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                       col_lds<N, CC>() * (int)sizeof(float2));                                    \
+    if (e != hipSuccess) return e;                                                                                 \
+    return hipFuncSetAttribute((const void*)k_col_fwd_multi<N, CC, KK>, hipFuncAttributeMaxDynamicSharedMemorySize,  \
+                               col_lds<N, CC>() * (int)sizeof(float2));                                            \
+  }
+  COL_FWD_CASES(CASE)
+#undef CASE
+  return hipErrorInvalidValue;
+}
+
 hipError_t launch_fft_cols(int NC, int C, float2* data, int n1, int count, int sign, const float2* tw,
                            hipStream_t st) {
   const int nblk = n1 / C;
@@ -1257,17 +1282,17 @@ hipError_t launch_row_fwd_multi(int NR, const RowFwdArgs* descs, const int2* ite
   return hipGetLastError();
 }
 
-hipError_t launch_row_adj_multi(int NR, const RowAdjArgs* descs, const int2* items, int n, int mode, bool fwd,
+hipError_t launch_row_adj_multi(int NR, const RowAdjArgs* descs, const int2* items, int n, bool grad,
                                 hipStream_t st) {
   if (n <= 0) return hipSuccess;
   switch (NR) {
 #define CASE(N)                                                                                         \
   case N: {                                                                                             \
     constexpr int RPB = row_adj_rows_per_block<N>();                                                    \
-    if (fwd)                                                                                            \
-      LAUNCH_TIMED((k_row_adj_multi<N, RPB, true>), dim3(n), dim3(RPB * (N / 16)), 0, st, descs, items, mode); \
+    if (grad)                                                                                           \
+      LAUNCH_TIMED((k_row_adj_multi<N, RPB, true>), dim3(n), dim3(RPB * (N / 16)), 0, st, descs, items); \
     else                                                                                                \
-      LAUNCH_TIMED((k_row_adj_multi<N, RPB, false>), dim3(n), dim3(RPB * (N / 16)), 0, st, descs, items, mode); \
+      LAUNCH_TIMED((k_row_adj_multi<N, RPB, false>), dim3(n), dim3(RPB * (N / 16)), 0, st, descs, items); \
     break;                                                                                              \
   }
     ROW_CASES(CASE)
@@ -1351,10 +1376,9 @@ hipError_t launch_col_multi(int NC, int C, int K, bool adjoint, const ColArgs* d
   return e;
 }
 
-hipError_t launch_combine_multi(const CombineArgs* descs, const int2* items, int n, const CombineLaunch& L,
-                                hipStream_t st) {
+hipError_t launch_combine_multi(const CombineArgs* descs, const int2* items, int n, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  LAUNCH_TIMED(k_combine_multi, dim3(n), dim3(1024), 0, st, descs, items, L);
+  LAUNCH_TIMED(k_combine_multi, dim3(n), dim3(1024), 0, st, descs, items);
   return hipGetLastError();
 }
 

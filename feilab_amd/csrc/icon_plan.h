@@ -13,6 +13,10 @@ namespace icon {
 constexpr int kTaps = 14;      // Gaussian window: 2m+2, m = 6 (nufft_gpu_v8.cuh:5)
 constexpr int kWindowM = 6;
 constexpr int kTapsKB = 6;     // Kaiser-Bessel window of width 6
+// The device's window of the default (Gaussian) plans: Kaiser-Bessel of width
+// 10.  Its transforms are within 1e-9 of the exact ones before rounding (the
+// 14-tap Gaussian: 7e-7 rms, 3.5e-6 at most) from fewer taps and column tiles.
+constexpr int kTapsWide = 10;
 constexpr int kMaxSlot = 3;    // node y-taps split over at most 3 column tiles (tile >= 8)
 
 // Host-side geometry of one tilt series, computed exactly as the reference's
@@ -20,7 +24,8 @@ constexpr int kMaxSlot = 3;    // node y-taps split over at most 3 column tiles 
 struct Geometry {
   int N0 = 0, N1 = 0, nz = 0, M = 0, n0 = 0, n1 = 0;
   int window = ICON_WINDOW_GAUSS;  // ICON_WINDOW_GAUSS or ICON_WINDOW_KB6
-  int K = kTaps;                  // taps per dimension: 14 (Gaussian) or 6 (Kaiser-Bessel)
+  int K = kTaps;                  // taps per dimension of the window: 14 (Gaussian) or 6 (Kaiser-Bessel); the
+                                  // projection rows' 1D transform uses it
   // window shape per dimension: Gaussian b and bf, or Kaiser-Bessel beta (b)
   float sig0 = 0, sig1 = 0, b0 = 0, b1 = 0, bf0 = 0, bf1 = 0;
   int iomit = 0;                  // tilt whose nodes give the reprojection
@@ -37,24 +42,20 @@ struct Geometry {
   std::vector<int> i10;           // N0
 };
 
-// Column-tile bin lists for the spread / interpolation.
+// Column-tile bin lists for the spread / interpolation with a window of K taps.
+// An entry is (node j, t0 | t1<<8 | slot<<16 | col0<<24, first x-tap x0, tile).
 struct Bins {
   int C = 16;                     // grid columns per tile
+  int K = 0;                      // window taps per dimension
   int nblk = 0;                   // n1 / C
   std::vector<int> off;           // nblk+1
-  // (node j, t0 | t1<<8 | slot<<16 | col0<<24, first x-tap x0, 0); a tile's
-  // entries are sorted by x0 (then node)
-  std::vector<int4> ent;
+  std::vector<int4> ent;          // a tile's entries are sorted by x0 (then node)
   std::vector<int> xoff;          // nblk*(n0+1): first entry of the tile with x0 >= x
   std::vector<int8_t> nslot;      // M
-  std::vector<float> px;          // E*14: x-taps of the entry's node (interleaved per tile)
-  std::vector<float> py;          // E*C: y-tap of each tile column, 0 outside the run (interleaved per tile)
   std::vector<int> of_node;       // M*3: entries of node j by slot (-1: none)
-  // The same entries and records in the interpolation's order: within a tile,
-  // groups of 16 entries whose first x-taps differ mod 16 where possible
-  // (records interleaved by field per tile as above).
+  // The same entries in the interpolation's order: within a tile, groups of 16
+  // entries whose first x-taps differ mod 16 where possible.
   std::vector<int4> fent;
-  std::vector<float> fpx, fpy;
   // Launch order of the spread's tiles: by entry count, largest first (ties
   // by index).  A spread block costs about its tile's entries, and the few
   // dense tiles around ky = 0 (up to 10x the median block) would otherwise
@@ -62,6 +63,40 @@ struct Bins {
   // them alone on a nearly idle device.
   std::vector<int> order;
 };
+
+// Bins and their device tables.  The records (K x-taps of the entry's node, C
+// y-taps, zero outside the run) are computed on the device, interleaved by
+// field per tile.
+struct DevBins {
+  Bins h;
+  float beta0 = 0, beta1 = 0;     // Kaiser-Bessel shape per dimension
+  float* ck = nullptr;            // [N0][N1] deapodisation
+  int* off = nullptr;
+  int* order = nullptr;
+  int* xoff = nullptr;
+  int* of_node = nullptr;
+  int4* ent = nullptr;
+  int4* fent = nullptr;
+  float *px = nullptr, *py = nullptr, *fpx = nullptr, *fpy = nullptr;
+  int8_t* nslot = nullptr;
+};
+
+// Entries of the solve's interpolation (16 taps, tiles of 8 columns): per tile
+// (node row, t0 | t1<<8 | slot<<16 | col0<<24, first x-tap, tile and flags), in
+// the interpolation's order (groups of 16 whose first x-taps differ mod 16
+// where possible); the records are computed from them on the device.
+// On a full grid every node is a row.  With paired nodes (paired_nodes) the
+// grid holds columns 0..n1/2 of a real image's transform, the rows are those of
+// node_of in icon_normal.hip (per tilt line the nodes N0/2..N0-1, then node 0),
+// and an entry's w carries, beside the tile, bit 16: the node mirrored into the
+// half that is stored, bit 17: columns that stand for their mirror images
+// (descending, x-taps reversed), bit 31: the value is to be conjugated.
+struct NodeBins {
+  std::vector<int> off;           // tiles + 1
+  std::vector<int4> ent;
+  std::vector<int8_t> nslot;      // node rows
+};
+constexpr int kNodeSlots = 4;     // tiles (and mirrored runs) per node row, at most
 
 // The grid columns [zlo, zhi) (FFT order, a multiple of C at both ends) of
 // the run of column tiles without bin entries around column n1/2.  Every
@@ -97,10 +132,24 @@ inline int split_min_entries(const Bins& b) {
   return std::max(1, 2 * n[n.size() / 2]);
 }
 
-// Fills g; returns false (with a message) on an invalid geometry.
+// Fills g; returns false (with a message) on an invalid geometry.  Without
+// tables the 2D window taps and deapodisation are left out (a plan computes
+// its own on the device).
 bool build_geometry(Geometry& g, int N0, int N1, int nz, const float* tilt_deg, std::string* err, bool cv = false,
-                    int window = ICON_WINDOW_GAUSS);
-void build_bins(const Geometry& g, int C, Bins& b);
+                    int window = ICON_WINDOW_GAUSS, bool tables = true);
+void build_bins(const Geometry& g, int C, int K, Bins& b);
+// Kaiser-Bessel window of W taps: its shape for oversampling sigma, and its
+// deapodisation over N samples.
+float kb_beta(float sigma, int W);
+void kb_deapod(int N, float sigma, float beta, int W, float* out);
+// Every tilt line's nodes but the first in exact pairs (v, -v) of equal weight.
+bool paired_nodes(const Geometry& g);
+void build_node_bins(const Geometry& g, bool half, NodeBins& b);
+// The entries of the unpaired nodes alone, rows renumbered to the tilt line.
+void unpaired_bins(const Geometry& g, const NodeBins& b, NodeBins& u);
+// Cholesky factor (16 x 16 row-major, the diagonal inverted) of the matrix
+// sinc((p - q)/2)/2 of the interpolation's taps.
+void interp_factor(double* l);
 void grid_size(int N, float* sigma, int* n);
 // Sets the message icon_last_error() returns on the calling thread.
 void set_last_error(const char* msg);
@@ -132,39 +181,59 @@ constexpr int kGraphCache = 4;
 struct icon_plan {
   int device = 0;
   icon::Geometry g;
-  icon::Bins bins;
   int S_max = 0;
   hipStream_t stream = nullptr;     // plan-owned stream (capturable)
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
+  // the transforms' window: bins and tables; data: those of the solve's data
+  // set-up where the plan's own window is not accurate enough (else op's)
+  icon::DevBins op, data;
+  bool own_data = false;
+  icon::DevBins& spread() { return own_data ? data : op; }
   // shared tables
-  float* d_ck = nullptr;
+  float2* d_nodes = nullptr;        // [M]
   float* d_ck1 = nullptr;
   float* d_w = nullptr;
-  float* d_phix = nullptr;
-  float* d_phiy = nullptr;
-  int* d_ix0 = nullptr;
-  int* d_ent_off = nullptr;
-  int* d_tile_order = nullptr;      // Bins::order
-  int4* d_ent = nullptr;
-  int* d_xoff = nullptr;
-  float* d_ent_px = nullptr;
-  float* d_ent_py = nullptr;
-  int4* d_fent = nullptr;
-  float* d_fent_px = nullptr;
-  float* d_fent_py = nullptr;
-  int* d_ent_of_node = nullptr;
-  int8_t* d_nslot = nullptr;
   float* d_phi1 = nullptr;
   int* d_i10 = nullptr;
+  // the solve's normal operator (icon_normal.hip)
+  bool half = false;                // paired nodes: real images on half grids
+  int nq = 0;                       // ... and its unpaired nodes
+  int rows = 0;                     // node rows of d_part
+  int ncol = 0;                     // grid columns: n1, or n1/2 + 8
+  // FP64 gradients: not at n0 = 2048, whose column kernel (1024 threads, 128
+  // registers, 424 bytes of scratch per lane) ended in a memory aperture
+  // violation inside a packed graph; its indexes are in bounds on the CPU
+  bool refreshes() const { return g.n0 <= 1024; }
+  int* d_nq_off = nullptr;          // unpaired nodes: entries (rows of d_part / of d_rpart), records
+  int4* d_nq_ent = nullptr;
+  int4* d_nq_entr = nullptr;
+  float* d_nq_px = nullptr;
+  float* d_nq_py = nullptr;
+  int8_t* d_nq_nslot = nullptr;
+  float2* d_rpart = nullptr;        // [S][nq][kNodeSlots]
+  float* d_gram = nullptr;          // [2][2 nq][2 nq]
+  float* d_spec = nullptr;          // [ncol/8][n0][8] spectrum of A^H W A's kernel
+  int* d_nd_off = nullptr;          // NodeBins and their records
+  int4* d_nd_ent = nullptr;
+  int8_t* d_nd_nslot = nullptr;
+  float* d_nd_px = nullptr;
+  float* d_nd_py = nullptr;
+  double* d_epart = nullptr;        // [S][ncol/8] energies of the gradient by column tile
   const float2* d_tw0 = nullptr;    // twiddles for n0 (shared cache)
   const float2* d_tw1 = nullptr;    // twiddles for n1
   // per-slice work buffers (capacity S_max)
   float2* d_b = nullptr;            // [S][M] Fourier-slice data
-  float2* d_fw = nullptr;           // [S][E] weighted node value of every bin entry
+  float2* d_fw = nullptr;           // [S][E] weighted node value of every bin entry (of op or spread())
   float2* d_part = nullptr;         // [S][M][kMaxSlot] interpolation partials
   float2* d_ahwb = nullptr;         // [S][N0][N1]
   float* d_grad = nullptr;          // [S][N0][N1] Re(rhat), the gradient the update takes
-  float2* d_tmp = nullptr;          // [S][N0][n1] row-transform intermediate
+  float2* d_tmp = nullptr;          // [S][N0][n1] row-transform intermediate, in single or double precision
+  // the reference iterate of the solve's differences: image, -rhat (half: real), b - A m
+  float* d_mref = nullptr;
+  float2* d_base = nullptr;
+  float2* d_beff = nullptr;
+  const double2* d_w640 = nullptr;  // FP64 twiddles for n0, n1 (shared cache)
+  const double2* d_w641 = nullptr;
   float2* d_frep = nullptr;         // [S][N0] forward values at the omit tilt
   double* d_rowpart = nullptr;      // [S][N0] per-row partial sums
   double* d_bnorm = nullptr;        // [S]
@@ -179,3 +248,19 @@ struct icon_plan {
   const void* data_sino = nullptr;
   int data_S = 0;
 };
+
+#include "icon_kernels.h"
+
+namespace icon {
+// Arguments of the iteration's kernels over S slices of a plan (icon_capi.cpp).
+ColArgs normal_args(const icon_plan* p, int S, bool with_nodes);
+ColArgs energy_args(const icon_plan* p, int S);
+RowAdjArgs grad_args(const icon_plan* p, int S);
+ColArgs normal64_args(const icon_plan* p, int S, bool with_nodes);
+RefArgs ref_args(const icon_plan* p, int S, float* m);
+RowFwdArgs rhat_row_args(const icon_plan* p, int S);
+bool refresh(const icon_plan* p, const icon_solve_opts& o, int it);
+FinishArgs finish_args(const icon_plan* p, int S);
+ColArgs spread_args(icon_plan* p, int S);   // of the data set-up
+RowAdjArgs data_row_args(icon_plan* p, int S);
+}  // namespace icon

@@ -247,15 +247,19 @@ int icon_mrc_write_slice(const char* path, const char* template_path, const floa
 /* ---- measurement -------------------------------------------------------- */
 /* Kernels of one ICON iteration, for icon_time_kernel. */
 typedef enum {
-  ICON_K_ROW_FWD = 0,   /* deapodise + pad + y-FFT of the image (fused update) */
-  ICON_K_COL_FWD = 1,   /* x-FFT of the grid tile + interpolation to the nodes */
-  ICON_K_COMBINE = 2,   /* node sums, weights, residual (FP64)                 */
-  ICON_K_COL_ADJ = 3,   /* spread of the nodes into the grid tile + x-IFFT     */
-  ICON_K_ROW_ADJ = 4,   /* y-IFFT + crop + deapodise + gradient + |r|^2 (FP64)
-                           + deapodise, pad and y-FFT of the gradient (the row
-                           pass of A rhat, fused)                              */
+  ICON_K_ROW_FWD = 0,   /* pad + y-FFT of the image (fused update)              */
+  ICON_K_COL_FWD = 1,   /* x-FFT of the grid tile + interpolation to the nodes
+                           (transforms)                                        */
+  ICON_K_COMBINE = 2,   /* node sums, residual and step size (FP64)            */
+  ICON_K_COL_ADJ = 3,   /* spread of the nodes into the grid tile + x-IFFT
+                           (transforms, data set-up)                           */
+  ICON_K_ROW_ADJ = 4,   /* y-IFFT + crop + gradient + |r|^2 (FP64) + pad and
+                           y-FFT of the gradient (fused)                       */
   ICON_K_SINO = 5,      /* 1D transform of the projection rows                 */
-  ICON_K_COMBINE_ALPHA = 6  /* node sums of A rhat, sum w|A rhat|^2 (FP64), alpha */
+  ICON_K_COMBINE_ALPHA = 6, /* the step size alone                             */
+  ICON_K_COL_NORMAL = 7,    /* x-FFT, nodes for the residual, spectrum of
+                               A^H W A, x-IFFT                                 */
+  ICON_K_COL_ENERGY = 8     /* x-FFT of the gradient, <r, A^H W A r> (FP64)    */
 } icon_kernel_id;
 
 /* Times `reps` launches of one kernel of the iteration over S slices, each
