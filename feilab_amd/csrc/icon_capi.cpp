@@ -484,6 +484,7 @@ int prepare_col(int n0, int n1, int C, int K) {
 }  // namespace
 
 void icon::set_last_error(const char* msg) { g_err = msg; }
+int icon::fft_twiddles(int n, const float2** out) { return twiddles(n, out); }
 
 // Arguments of the iteration's kernels over S slices of a plan.
 ColArgs icon::normal_args(const icon_plan* p, int S, bool with_nodes) {

@@ -151,6 +151,8 @@ void unpaired_bins(const Geometry& g, const NodeBins& b, NodeBins& u);
 // sinc((p - q)/2)/2 of the interpolation's taps.
 void interp_factor(double* l);
 void grid_size(int N, float* sigma, int* n);
+// Twiddle table of a power-of-two length (icon_fft.h) on the current device.
+int fft_twiddles(int n, const float2** out);
 // Sets the message icon_last_error() returns on the calling thread.
 void set_last_error(const char* msg);
 

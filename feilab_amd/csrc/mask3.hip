@@ -10,15 +10,15 @@
 //
 // The masks are built on the host exactly as the reference builds them
 // (float/double placement included).  The filtering runs batched on the
-// device with this library's own 2D FFT: for a real slice f with spectrum F,
-// the reference's R2C -> (half-spectrum mask M) -> C2R / N^2 equals
+// device with this library's own transforms: for a real slice f with spectrum
+// F, the reference's R2C -> (half-spectrum mask M) -> C2R / N^2 equals
 // Re(IFFT2(F * Mfull)) / N^2 with Mfull(ky, kx) = M(ky, kx) for kx <= N/2
-// and M(-ky, N-kx) otherwise.
+// and M(-ky, N-kx) otherwise; for the columns kx = 0 and N/2, which are their
+// own mirrors, the real part leaves the even part of M.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
-#include <complex>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -27,7 +27,12 @@
 #include <vector>
 
 #include "../../include/icon_mi355x.h"
+#include "icon_col.h"
+#include "icon_fft.h"
+#include "icon_plan.h"
 #include "mrc_io.h"
+
+using namespace icon;
 
 namespace {
 
@@ -71,137 +76,264 @@ void sampling_mask(int N, const float* thita, int ang_num, std::vector<float>& o
     if (v > 1) v = 1;
 }
 
-__global__ void k_real_to_complex(const float* in, float2* out, long n) {
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    out[i] = make_float2(in[i], 0.f);
-}
-
-// F *= Mfull, the half-spectrum mask mirrored onto the other half
-__global__ void k_apply_mask(float2* f, const float* half, int N, long count) {
-  const int H = N / 2 + 1;
-  const long n = count * N * N;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int kx = (int)(i % N);
-    const int ky = (int)((i / N) % N);
-    const float m = kx <= N / 2 ? half[(long)ky * H + kx] : half[(long)((N - ky) % N) * H + (N - kx)];
-    const float2 v = f[i];
-    f[i] = make_float2(v.x * m, v.y * m);
-  }
-}
-
-// out = Re(f) / (N*N), as the reference divides after its C2R in double
-__global__ void k_real_scaled(const float2* f, float* out, long n, double factor) {
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    out[i] = (float)((double)f[i].x / factor);
-}
-
-int grid_for(long n) { return (int)std::min<long>((n + 255) / 256, 65536); }
-
-// Widths that are not powers of two: each 1D DFT of length N by Bluestein's
-// chirp-z method on this library's power-of-two row FFT of length
-// M >= 2N - 1.  With c_n = exp(sign i pi n^2 / N),
+// ------------------------------------------------------------------ filtering
+// Three passes over the stack, in place: a row pass (spectra of the real
+// rows), a column pass (forward transform, mask, inverse transform) and a row
+// pass back.  The spectrum of a real row of N samples is N floats: F_0, for even
+// N F_{N/2}, and the pairs F_k, 0 < k < N/2, so it replaces the row in the stack
+// and no other buffer is needed.  Two real rows share one complex transform.
+//
+// Lengths that are not powers of two (or below 128) use Bluestein's chirp-z
+// transform on a power-of-two transform of length M >= 2N - 1.  With
+// c_n = exp(-i pi n^2 / N),
 //   X_k = c_k sum_n (x_n c_n) conj(c_{k-n}),
-// a circular convolution of length M.  A pass transforms the rows of
-// [count][N][N] and stores the result transposed, so two passes give the 2D
-// transform in the input's orientation.
-struct Bluestein {
-  int N = 0, M = 0;
-  float2* chirp[2] = {nullptr, nullptr};   // c_n for sign -1, +1
-  float2* bhat[2] = {nullptr, nullptr};    // FFT_M of the conj(c) kernel
+// a circular convolution of length M, inside registers and LDS; the inverse is
+// the same with every factor conjugated (the kernel is even, so its spectrum's
+// conjugate is the conjugate kernel's spectrum).
+//
+// Bound by the transforms' arithmetic (two of length M per row pair and four
+// per column), not by memory (24 N^2 bytes per slice).  64 slices of 464^2 (M =
+// 1024): rows 60 us, columns 160 us, rows back 72 us, 341 us for the call with
+// the mask's upload and the device's 17 us copy of the input before it, against
+// 4440 us as separate passes over a complex stack in a chirp's buffer of its
+// own, the chirp's spectrum summed on the host and six allocations.
+
+struct FiltArgs {
+  float* data;            // [rows][N] in place
+  const float* half;      // mask [N][N/2 + 1]
+  const float2* chirp;    // c_n, n < N (chirp transforms)
+  const float2* bhat;     // spectrum of the conj(c) kernel over M
+  const float2* tw;       // twiddles of the length-M transform
+  int N;
+  long rows;              // N x slices
 };
 
-// c_n, n^2 reduced mod 2N so the phase stays exact in double
-std::vector<std::complex<double>> chirp_host(int N, int sign) {
-  std::vector<std::complex<double>> c(N);
-  for (long n = 0; n < N; n++) {
-    const double ph = sign * M_PI * (double)((n * n) % (2L * N)) / (double)N;
-    c[n] = std::complex<double>(std::cos(ph), std::sin(ph));
-  }
-  return c;
+// Spectrum entry k (0 <= k <= N/2) of a packed row.
+__device__ __forceinline__ float2 spec_get(const float* p, int k, int N) {
+  if (k == 0) return make_float2(p[0], 0.f);
+  if (2 * k == N) return make_float2(p[1], 0.f);
+  const int o = N % 2 ? 2 * k - 1 : 2 * k;
+  return make_float2(p[o], p[o + 1]);
+}
+__device__ __forceinline__ void spec_put(float* p, int k, int N, float2 v) {
+  if (k == 0) { p[0] = v.x; return; }
+  if (2 * k == N) { p[1] = v.x; return; }
+  const int o = N % 2 ? 2 * k - 1 : 2 * k;
+  p[o] = v.x;
+  p[o + 1] = v.y;
 }
 
-hipError_t bluestein_init(Bluestein& b, int N) {
-  b.N = N;
-  b.M = 128;
-  while (b.M < 2 * N - 1) b.M *= 2;
-  const int M = b.M;
-  std::vector<std::complex<double>> tw(M);
-  for (int k = 0; k < M; k++) tw[k] = std::polar(1.0, -2.0 * M_PI * k / M);
-  for (int d = 0; d < 2; d++) {
-    const auto c = chirp_host(N, d ? 1 : -1);
-    std::vector<std::complex<double>> kern(M, 0.0), hat(M);
-    kern[0] = std::conj(c[0]);
-    for (int j = 1; j < N; j++) kern[j] = kern[M - j] = std::conj(c[j]);
-    for (int k = 0; k < M; k++) {   // FP64 DFT, exponent sign -1 like the device forward FFT
-      std::complex<double> acc = 0;
-      for (int j = 0; j < M; j++)
-        if (kern[j] != 0.0) acc += kern[j] * tw[(size_t)((long)j * k % M)];
-      hat[k] = acc / (double)M;     // the 1/M of the inverse FFT folded in
+__device__ __forceinline__ float2 conj_if(bool c, float2 a) { return c ? make_float2(a.x, -a.y) : a; }
+
+// Transform of length N (direction DIR) of the line that a team of M/16 threads
+// holds in v: in, slot r element t + r M/16 (for a chirp transform already
+// times its chirp factor, and zero from N on); out, slot i element
+// out_index<M>(t, i) (without the chirp factor of the output).
+template <int M, typename L, int DIR, bool CHIRP>
+__device__ __forceinline__ void line_fft(float2 (&v)[16], float2* lds, int t, const FiltArgs& a) {
+  FftTwiddles T;
+  if constexpr (!CHIRP) {
+    fft_from_lazy<M, L, DIR, 1>(v, lds, t, T, a.tw);
+  } else {
+    fft_from_lazy<M, L, -1, 1>(v, lds, t, T, a.tw);
+    constexpr int RL = last_radix<M>();
+    float2 u[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+      u[i / RL + (i % RL) * (16 / RL)] = c_mul(v[i], conj_if(DIR > 0, a.bhat[out_index<M>(t, i)]));
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = u[i];
+    fft_from_lazy<M, L, 1, 1>(v, lds, t, T, a.tw);
+  }
+}
+
+// Row pairs: INV 0, spectra of the two real rows; INV 1, the rows back, over N^2.
+template <int M, int RPB, bool CHIRP, bool INV>
+__global__ __launch_bounds__(RPB * (M / 16)) void k_filt_rows(FiltArgs a) {
+  constexpr int T = M / 16;
+  __shared__ float2 lds[RPB * RowLay::size(M)];
+  const int team = threadIdx.x / T, t = threadIdx.x % T;
+  const long row = 2 * ((long)blockIdx.x * RPB + team);
+  const int N = a.N;
+  float2* L = lds + team * RowLay::size(M);
+  const bool v0 = row < a.rows, v1 = row + 1 < a.rows;
+  float *p0 = a.data + (v0 ? row : 0) * N, *p1 = a.data + (v1 ? row + 1 : 0) * N;
+  float2 v[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int n = in_index<M>(t, r);
+    v[r] = make_float2(0.f, 0.f);
+    if (n >= N) continue;
+    if constexpr (!INV) {
+      v[r] = make_float2(v0 ? p0[n] : 0.f, v1 ? p1[n] : 0.f);
+    } else {
+      // Z = A + iB of the rows' spectra; beyond N/2 their mirrors' conjugates
+      const bool up = 2 * n > N;
+      const int k = up ? N - n : n;
+      const float2 A = v0 ? conj_if(up, spec_get(p0, k, N)) : make_float2(0.f, 0.f);
+      const float2 B = v1 ? conj_if(up, spec_get(p1, k, N)) : make_float2(0.f, 0.f);
+      v[r] = make_float2(A.x - B.y, A.y + B.x);
     }
-    std::vector<float2> cf(N), hf(M);
-    for (int n = 0; n < N; n++) cf[n] = make_float2((float)c[n].real(), (float)c[n].imag());
-    for (int k = 0; k < M; k++) hf[k] = make_float2((float)hat[k].real(), (float)hat[k].imag());
-    hipError_t e = hipMalloc(&b.chirp[d], sizeof(float2) * N);
-    if (e == hipSuccess) e = hipMalloc(&b.bhat[d], sizeof(float2) * M);
-    if (e == hipSuccess) e = hipMemcpy(b.chirp[d], cf.data(), sizeof(float2) * N, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(b.bhat[d], hf.data(), sizeof(float2) * M, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return e;
+    if constexpr (CHIRP) v[r] = c_mul(v[r], conj_if(INV, a.chirp[n]));
   }
-  return hipSuccess;
-}
-
-void bluestein_free(Bluestein& b) {
-  for (int d = 0; d < 2; d++) {
-    if (b.chirp[d]) (void)hipFree(b.chirp[d]);
-    if (b.bhat[d]) (void)hipFree(b.bhat[d]);
+  line_fft<M, RowLay, INV ? 1 : -1, CHIRP>(v, L, t, a);
+  if constexpr (CHIRP) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int k = out_index<M>(t, i);
+      if (k < N) v[i] = c_mul(v[i], conj_if(INV, a.chirp[k]));
+    }
   }
-}
-
-__device__ inline float2 cmul(float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
-
-// work[r][m] = x[r][m] c_m for m < N, 0 up to M
-__global__ void k_bs_load(const float2* x, const float2* chirp, float2* work, int N, int M, long rows) {
-  const long n = rows * M;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int m = (int)(i % M);
-    const long r = i / M;
-    work[i] = m < N ? cmul(x[r * N + m], chirp[m]) : make_float2(0.f, 0.f);
-  }
-}
-
-__global__ void k_bs_mul(float2* work, const float2* bhat, int M, long rows) {
-  const long n = rows * M;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    work[i] = cmul(work[i], bhat[i % M]);
-}
-
-// y[s][k][r] = c_k conv[s][r][k]: the pass's result, transposed per slice
-__global__ void k_bs_store_t(const float2* work, const float2* chirp, float2* y, int N, int M, long count) {
-  const long n = count * N * N;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int r = (int)(i % N);
-    const int k = (int)((i / N) % N);
-    const long s = i / ((long)N * N);
-    y[i] = cmul(work[(s * N + r) * M + k], chirp[k]);
+  if constexpr (INV) {
+    // (the last exchange's barrier was passed after every load of the rows)
+    const double f = 1.0 / ((double)N * (double)N);
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int n = out_index<M>(t, i);
+      if (n >= N) continue;
+      if (v0) p0[n] = (float)((double)v[i].x * f);
+      if (v1) p1[n] = (float)((double)v[i].y * f);
+    }
+  } else {
+    // A_k = (Z_k + conj Z_{N-k})/2, B_k = (Z_k - conj Z_{N-k})/2i
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int k = out_index<M>(t, i);
+      if (k < N) L[RowLay::at(k)] = v[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int k = out_index<M>(t, i);
+      if (2 * k > N) continue;
+      const float2 z = v[i], y = L[RowLay::at(k ? N - k : 0)];
+      if (v0) spec_put(p0, k, N, make_float2(0.5f * (z.x + y.x), 0.5f * (z.y - y.y)));
+      if (v1) spec_put(p1, k, N, make_float2(0.5f * (z.y + y.y), 0.5f * (y.x - z.x)));
+    }
   }
 }
 
-int bluestein_2d(const Bluestein& b, float2* d_f, float2* work, int count, int sign, hipStream_t st) {
-  const int d = sign > 0 ? 1 : 0;
-  const long rows = (long)count * b.N;
-  for (int pass = 0; pass < 2; pass++) {
-    hipLaunchKernelGGL(k_bs_load, dim3(grid_for(rows * b.M)), dim3(256), 0, st, d_f, b.chirp[d], work, b.N, b.M, rows);
-    if (hipGetLastError() != hipSuccess) return ICON_ERR_DEVICE;
-    int rc = icon_fft_rows(b.M, (int)rows, -1, work, st);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_bs_mul, dim3(grid_for(rows * b.M)), dim3(256), 0, st, work, b.bhat[d], b.M, rows);
-    if (hipGetLastError() != hipSuccess) return ICON_ERR_DEVICE;
-    if ((rc = icon_fft_rows(b.M, (int)rows, 1, work, st))) return rc;
-    hipLaunchKernelGGL(k_bs_store_t, dim3(grid_for(rows * b.N)), dim3(256), 0, st, work, b.chirp[d], d_f, b.N, b.M,
-                       (long)count);
-    if (hipGetLastError() != hipSuccess) return ICON_ERR_DEVICE;
+// Tiles of C spectrum columns of one slice: column transform, mask, inverse.
+// Column 0 of an even width carries F_0 + i F_{N/2} (both columns are real
+// before the transform), separated by the mirror k -> N - k.
+template <int M, int C, bool CHIRP>
+__global__ __launch_bounds__(C * (M / 16)) void k_filt_cols(FiltArgs a, int ntiles) {
+  using Lo = ColFftLayFwd<C>;
+  extern __shared__ __align__(16) float2 tile[];   // Lo::at(M - 1) + C
+  const int N = a.N, H = N / 2 + 1, ncol = (N + 1) / 2;
+  const int c = threadIdx.x % C, t = threadIdx.x / C;
+  const int k0 = (blockIdx.x % ntiles) * C + c;      // spectrum column, 0: special
+  const bool ok = k0 < ncol;
+  float* base = a.data + (long)(blockIdx.x / ntiles) * N * N;
+  const int o = k0 == 0 ? 0 : N % 2 ? 2 * k0 - 1 : 2 * k0;
+  const bool two = k0 != 0 || N % 2 == 0;            // an odd width's column 0 is real
+  float2 v[16];
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    const int n = in_index<M>(t, r);
+    v[r] = make_float2(0.f, 0.f);
+    if (ok && n < N) v[r] = make_float2(base[(long)n * N + o], two ? base[(long)n * N + o + 1] : 0.f);
+    if constexpr (CHIRP)
+      if (n < N) v[r] = c_mul(v[r], a.chirp[n]);
   }
-  return ICON_OK;
+  line_fft<M, Lo, -1, CHIRP>(v, tile + c, t, a);
+  // the mask; the output's and the inverse's input's chirp factors cancel
+  if (blockIdx.x % ntiles == 0 && N % 2 == 0) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int k = out_index<M>(t, i);
+      if (k >= N) continue;
+      if (CHIRP && c == 0) v[i] = c_mul(v[i], a.chirp[k]);
+      tile[Lo::at(k) + c] = v[i];
+    }
+    __syncthreads();
+    if (c == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        const int k = out_index<M>(t, i), km = (N - k) % N;
+        if (k >= N) continue;
+        // the real part keeps the masks' even parts: Re over columns 0 and N/2
+        const float m0 = 0.5f * (a.half[(long)k * H] + a.half[(long)km * H]);
+        const float mn = 0.5f * (a.half[(long)k * H + N / 2] + a.half[(long)km * H + N / 2]);
+        const float s = 0.5f * (m0 + mn), d = 0.5f * (m0 - mn);
+        const float2 z = v[i], y = tile[Lo::at(km)];
+        v[i] = make_float2(s * z.x + d * y.x, s * z.y - d * y.y);
+        if (CHIRP) v[i] = c_mul(v[i], conj_if(true, a.chirp[k]));
+      }
+    }
+    __syncthreads();
+  } else if (k0 == 0) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int k = out_index<M>(t, i);
+      if (k >= N) continue;
+      const float m = 0.5f * (a.half[(long)k * H] + a.half[(long)((N - k) % N) * H]);
+      v[i] = make_float2(v[i].x * m, v[i].y * m);
+    }
+  }
+  constexpr int RL = last_radix<M>();
+  float2 u[16];
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int k = out_index<M>(t, i);
+    const float m = k0 == 0 || !ok || k >= N ? 1.f : a.half[(long)k * H + k0];
+    u[i / RL + (i % RL) * (16 / RL)] = k < N ? make_float2(v[i].x * m, v[i].y * m) : make_float2(0.f, 0.f);
+  }
+  line_fft<M, Lo, 1, CHIRP>(u, tile + c, t, a);
+  if (!ok) return;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int n = out_index<M>(t, i);
+    if (n >= N) continue;
+    float2 x = u[i];
+    if constexpr (CHIRP) x = c_mul(x, conj_if(true, a.chirp[n]));
+    base[(long)n * N + o] = x.x;
+    if (two) base[(long)n * N + o + 1] = x.y;
+  }
+}
+
+// Chirp and its kernel's spectrum, in FP64 with exact phases: block k sums
+// bhat_k = (1 + 2 sum_{0<j<N} exp(i pi j^2 / N) cos(2 pi j k / M)) / M (the 1/M
+// of the inverse transform folded in).
+__global__ __launch_bounds__(64) void k_chirp(int N, int M, float2* chirp, float2* bhat) {
+  const int k = blockIdx.x, t = threadIdx.x;
+  double x = 0.0, y = 0.0;
+  for (int j = 1 + t; j < N; j += 64) {
+    const double ph = (double)(((long)j * j) % (2L * N)) / (double)N;
+    const double f = 2.0 * cospi(2.0 * (double)(((long)j * k) % M) / (double)M);
+    x += f * cospi(ph);
+    y += f * sinpi(ph);
+  }
+#pragma unroll
+  for (int h = 32; h > 0; h >>= 1) {
+    x += __shfl_down(x, h);
+    y += __shfl_down(y, h);
+  }
+  if (t == 0) {
+    bhat[k] = make_float2((float)((1.0 + x) / M), (float)(y / M));
+    if (k < N) {
+      const double ph = (double)(((long)k * k) % (2L * N)) / (double)N;
+      chirp[k] = make_float2((float)cospi(ph), (float)-sinpi(ph));
+    }
+  }
+}
+
+template <int M, bool CHIRP>
+hipError_t launch_filter(const FiltArgs& a, int count, hipStream_t st) {
+  // columns per tile: 8 (64 bytes of each row); 4 at M = 2048, whose 8 would
+  // need 1024 threads, and so 128 registers each and scratch memory
+  constexpr int RPB = 256 / (M / 16) > 16 ? 16 : 256 / (M / 16), C = M >= 2048 ? 4 : 8;
+  constexpr int lds = (ColFftLayFwd<C>::at(M - 1) + C) * (int)sizeof(float2);
+  const hipError_t e = hipFuncSetAttribute((const void*)k_filt_cols<M, C, CHIRP>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return e;
+  const long pairs = (a.rows + 1) / 2;
+  const unsigned blocks = (unsigned)((pairs + RPB - 1) / RPB);
+  const int ntiles = ((a.N + 1) / 2 + C - 1) / C;
+  hipLaunchKernelGGL((k_filt_rows<M, RPB, CHIRP, false>), dim3(blocks), dim3(RPB * (M / 16)), 0, st, a);
+  hipLaunchKernelGGL((k_filt_cols<M, C, CHIRP>), dim3((unsigned)ntiles * count), dim3(C * (M / 16)), lds, st, a, ntiles);
+  hipLaunchKernelGGL((k_filt_rows<M, RPB, CHIRP, true>), dim3(blocks), dim3(RPB * (M / 16)), 0, st, a);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -264,42 +396,37 @@ int icon_mask3_filter(int device, float* d_slices, int N, int count, const float
     return merr(ICON_ERR_ARG, "icon_mask3_filter: widths above 1024 must be powers of two");
   if (hipSetDevice(device) != hipSuccess) return merr(ICON_ERR_ARG, "icon_mask3_filter: no such device");
   hipStream_t st = (hipStream_t)stream;
-  const long n = (long)count * N * N;
-  const size_t hb = sizeof(float) * (size_t)N * (N / 2 + 1);
-  float2 *d_f = nullptr, *d_work = nullptr;
-  float* d_m = nullptr;
-  Bluestein bs;
-  hipError_t e = hipMalloc(&d_f, sizeof(float2) * n);
-  if (e == hipSuccess) e = hipMalloc(&d_m, hb);
-  if (e == hipSuccess) e = hipMemcpy(d_m, half_mask, hb, hipMemcpyHostToDevice);
-  if (e == hipSuccess && !pow2) e = bluestein_init(bs, N);
-  if (e == hipSuccess && !pow2) e = hipMalloc(&d_work, sizeof(float2) * (size_t)count * N * bs.M);
-  int rc = ICON_OK;
-  auto fft2 = [&](int sign) {
-    return pow2 ? icon_fft_2d(N, N, count, sign, d_f, stream) : bluestein_2d(bs, d_f, d_work, count, sign, st);
-  };
+  int M = 128;
+  while (pow2 ? M < N : M < 2 * N - 1) M *= 2;
+  const float2* tw = nullptr;
+  if (int rc = fft_twiddles(M, &tw)) return merr(rc, std::string("icon_mask3_filter: ") + icon_last_error());
+  // one buffer: the mask and, for a chirp transform, its tables
+  const size_t hb = (sizeof(float) * (size_t)N * (N / 2 + 1) + 255) / 256 * 256;
+  char* buf = nullptr;
+  hipError_t e = hipMalloc(&buf, hb + (pow2 ? 0 : sizeof(float2) * (size_t)(M + N)));
+  if (e == hipSuccess)
+    e = hipMemcpy(buf, half_mask, sizeof(float) * (size_t)N * (N / 2 + 1), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_real_to_complex, dim3(grid_for(n)), dim3(256), 0, st, d_slices, d_f, n);
-    e = hipGetLastError();
+    float2 *bhat = reinterpret_cast<float2*>(buf + hb), *chirp = bhat + M;
+    FiltArgs a{d_slices, reinterpret_cast<const float*>(buf), chirp, bhat, tw, N, (long)count * N};
+    if (!pow2) {
+      hipLaunchKernelGGL(k_chirp, dim3(M), dim3(64), 0, st, N, M, chirp, bhat);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) {
+      switch (M) {
+#define CASE(MM) \
+  case MM: e = pow2 ? launch_filter<MM, false>(a, count, st) : launch_filter<MM, true>(a, count, st); break;
+        CASE(128) CASE(256) CASE(512) CASE(1024) CASE(2048)
+#undef CASE
+        default: e = hipErrorInvalidValue;
+      }
+    }
   }
-  if (e == hipSuccess) rc = fft2(-1);
-  if (e == hipSuccess && rc == ICON_OK) {
-    hipLaunchKernelGGL(k_apply_mask, dim3(grid_for(n)), dim3(256), 0, st, d_f, d_m, N, (long)count);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess && rc == ICON_OK) rc = fft2(1);
-  if (e == hipSuccess && rc == ICON_OK) {
-    hipLaunchKernelGGL(k_real_scaled, dim3(grid_for(n)), dim3(256), 0, st, d_f, d_slices, n, (double)N * (double)N);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  if (d_f) (void)hipFree(d_f);
-  if (d_m) (void)hipFree(d_m);
-  if (d_work) (void)hipFree(d_work);
-  bluestein_free(bs);
+  const hipError_t es = hipStreamSynchronize(st);
+  if (e == hipSuccess) e = es;
+  if (buf) (void)hipFree(buf);
   if (e != hipSuccess) return merr(ICON_ERR_DEVICE, std::string("icon_mask3_filter: ") + hipGetErrorString(e));
-  if (rc == ICON_ERR_DEVICE) return merr(rc, "icon_mask3_filter: kernel launch failed");
-  if (rc != ICON_OK) return merr(rc, std::string("icon_mask3_filter: ") + icon_last_error());
   return ICON_OK;
 }
 
