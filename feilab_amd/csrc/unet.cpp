@@ -82,6 +82,7 @@ struct icon_unet {
   long adam_t = 0;
   double* d_loss = nullptr;
   float* gpart = nullptr;    // training: partial sums of the weight, bias and head gradients
+  int wgrad_blocks = 0;      // blocks of the weight gradients' launch
   // activations (bf16)
   T16 x8, a1, cat1, p1, a2, cat2, p2, a3, cat3, p3, ab, bb, d3a, d3b, d2a, d2b, d1a, d1b;
   float* out = nullptr;      // [maxB][H][W] network output of the warm start
@@ -180,20 +181,15 @@ int conv(icon_unet* n, const Conv& c, const TX* x, int ldx, int cx0, TY* y, int 
   return 0;
 }
 
-// pixel splits of a weight gradient over P pixels
-int wgrad_splits(long P) { return (int)std::max<long>(1, std::min<long>(256, P / 2048)); }
-
-int wgrad(icon_unet* n, const Conv& c, const uint16_t* x, int ldx, int cx0, const float* dy, int lddy, int cdy0,
-          int B, int H, int W, hipStream_t st) {
-  WgradArgs a{};
+// a layer's weight and bias gradients, computed with those of the other layers
+// once every output gradient is there (the end of backward)
+void wgrad(icon_unet* n, WgradGroup& g, const Conv& c, const uint16_t* x, int ldx, int cx0, const float* dy, int lddy,
+           int cdy0, int B, int H, int W) {
+  WgradLayer& a = g.l[g.n++];
+  a = WgradLayer{};
   a.x = x; a.ldx = ldx; a.cx0 = cx0; a.dy = dy; a.lddy = lddy; a.cdy0 = cdy0;
-  a.dw = n->grads + c.off_w;
-  a.N = B; a.H = H; a.W = W; a.Cin = c.cin; a.Cout = c.cout; a.taps = c.taps;
-  a.part = n->gpart;
-  const long P = (long)B * H * W;
-  UCHK(launch_wgrad(a, wgrad_splits(P), st));
-  UCHK(launch_bias_grad(dy, lddy, cdy0, P, c.cout, n->grads + c.off_b, n->gpart, st));
-  return 0;
+  a.dw = n->grads + c.off_w; a.db = n->grads + c.off_b;
+  a.N = B; a.H = H; a.W = W; a.Cin = c.cin; a.Cout = c.cout;
 }
 
 int up(const T16& in, const T16& out, int co0, int B, int h, int w, hipStream_t st) {
@@ -270,39 +266,43 @@ int backward(icon_unet* n, int B, const float* d_dout, hipStream_t st) {
   int rc;
 #define R(x) do { if ((rc = (x))) return rc; } while (0)
 #define HIPR(x) do { if ((x) != hipSuccess) return ufail(2, "%s failed", #x); } while (0)
-  HIPR(launch_head_bwd(n->d1b.p, 32, n->params + n->head_w, 32, P, d_dout, n->g_d1b.p, 32, n->grads + n->head_w,
-                       n->grads + n->head_b, n->gpart, st));
+  WgradGroup wg;
+  ReduceGroup red;
+  wg.n = red.n = red.blocks = 0;
+  HIPR(launch_head_bwd(n->d1b.p, 32, n->params + n->head_w, P, d_dout, n->g_d1b.p, 32, n->gpart, st));
+  // dw and db of the head are adjacent in the parameter vector
+  add_reduce(red, n->gpart, kHeadGradParts, 33, n->grads + n->head_w, false);
   // d1b, d1a
-  R(wgrad(n, cv[D1B], n->d1a.p, 32, 0, n->g_d1b.p, 32, 0, B, H, W, st));
+  wgrad(n, wg, cv[D1B], n->d1a.p, 32, 0, n->g_d1b.p, 32, 0, B, H, W);
   R(conv(n, cv[D1B], n->g_d1b.p, 32, 0, n->g_d1a.p, 32, 0, B, H, W, false, n->d1a.p, 32, 0, true, false, st));
-  R(wgrad(n, cv[D1A], n->cat1.p, 96, 0, n->g_d1a.p, 32, 0, B, H, W, st));
+  wgrad(n, wg, cv[D1A], n->cat1.p, 96, 0, n->g_d1a.p, 32, 0, B, H, W);
   R(conv(n, cv[D1A], n->g_d1a.p, 32, 0, n->g_cat1.p, 96, 0, B, H, W, false, n->cat1.p, 96, 0, true, false, st));
   {
     PoolGradArgs u{n->g_cat1.p, 96, 0, n->g_d2b.p, 64, 0, B, H2, W2, 64, 0};
     HIPR(launch_up_bwd(u, st));
   }
   // d2b, d2a
-  R(wgrad(n, cv[D2B], n->d2a.p, 64, 0, n->g_d2b.p, 64, 0, B, H2, W2, st));
+  wgrad(n, wg, cv[D2B], n->d2a.p, 64, 0, n->g_d2b.p, 64, 0, B, H2, W2);
   R(conv(n, cv[D2B], n->g_d2b.p, 64, 0, n->g_d2a.p, 64, 0, B, H2, W2, false, n->d2a.p, 64, 0, true, false, st));
-  R(wgrad(n, cv[D2A], n->cat2.p, 192, 0, n->g_d2a.p, 64, 0, B, H2, W2, st));
+  wgrad(n, wg, cv[D2A], n->cat2.p, 192, 0, n->g_d2a.p, 64, 0, B, H2, W2);
   R(conv(n, cv[D2A], n->g_d2a.p, 64, 0, n->g_cat2.p, 192, 0, B, H2, W2, false, n->cat2.p, 192, 0, true, false, st));
   {
     PoolGradArgs u{n->g_cat2.p, 192, 0, n->g_d3b.p, 128, 0, B, H4, W4, 128, 0};
     HIPR(launch_up_bwd(u, st));
   }
   // d3b, d3a
-  R(wgrad(n, cv[D3B], n->d3a.p, 128, 0, n->g_d3b.p, 128, 0, B, H4, W4, st));
+  wgrad(n, wg, cv[D3B], n->d3a.p, 128, 0, n->g_d3b.p, 128, 0, B, H4, W4);
   R(conv(n, cv[D3B], n->g_d3b.p, 128, 0, n->g_d3a.p, 128, 0, B, H4, W4, false, n->d3a.p, 128, 0, true, false, st));
-  R(wgrad(n, cv[D3A], n->cat3.p, 384, 0, n->g_d3a.p, 128, 0, B, H4, W4, st));
+  wgrad(n, wg, cv[D3A], n->cat3.p, 384, 0, n->g_d3a.p, 128, 0, B, H4, W4);
   R(conv(n, cv[D3A], n->g_d3a.p, 128, 0, n->g_cat3.p, 384, 0, B, H4, W4, false, n->cat3.p, 384, 0, true, false, st));
   {
     PoolGradArgs u{n->g_cat3.p, 384, 0, n->g_bb.p, 256, 0, B, H8, W8, 256, 0};
     HIPR(launch_up_bwd(u, st));
   }
   // bottleneck
-  R(wgrad(n, cv[BB], n->ab.p, 256, 0, n->g_bb.p, 256, 0, B, H8, W8, st));
+  wgrad(n, wg, cv[BB], n->ab.p, 256, 0, n->g_bb.p, 256, 0, B, H8, W8);
   R(conv(n, cv[BB], n->g_bb.p, 256, 0, n->g_ab.p, 256, 0, B, H8, W8, false, n->ab.p, 256, 0, true, false, st));
-  R(wgrad(n, cv[BA], n->p3.p, 128, 0, n->g_ab.p, 256, 0, B, H8, W8, st));
+  wgrad(n, wg, cv[BA], n->p3.p, 128, 0, n->g_ab.p, 256, 0, B, H8, W8);
   R(conv(n, cv[BA], n->g_ab.p, 256, 0, n->g_p3.p, 128, 0, B, H8, W8, false, nullptr, 0, 0, true, false, st));
   {
     PoolGradArgs u{n->g_p3.p, 128, 0, n->g_cat3.p, 384, 256, B, H4, W4, 128, 1};
@@ -310,9 +310,9 @@ int backward(icon_unet* n, int B, const float* d_dout, hipStream_t st) {
     HIPR(launch_relu_mask(n->g_cat3.p, 384, 256, n->cat3.p, 384, 256, (long)B * H4 * W4, 128, st));
   }
   // e3
-  R(wgrad(n, cv[E3B], n->a3.p, 128, 0, n->g_cat3.p, 384, 256, B, H4, W4, st));
+  wgrad(n, wg, cv[E3B], n->a3.p, 128, 0, n->g_cat3.p, 384, 256, B, H4, W4);
   R(conv(n, cv[E3B], n->g_cat3.p, 384, 256, n->g_a3.p, 128, 0, B, H4, W4, false, n->a3.p, 128, 0, true, false, st));
-  R(wgrad(n, cv[E3A], n->p2.p, 64, 0, n->g_a3.p, 128, 0, B, H4, W4, st));
+  wgrad(n, wg, cv[E3A], n->p2.p, 64, 0, n->g_a3.p, 128, 0, B, H4, W4);
   R(conv(n, cv[E3A], n->g_a3.p, 128, 0, n->g_p2.p, 64, 0, B, H4, W4, false, nullptr, 0, 0, true, false, st));
   {
     PoolGradArgs u{n->g_p2.p, 64, 0, n->g_cat2.p, 192, 128, B, H2, W2, 64, 1};
@@ -320,9 +320,9 @@ int backward(icon_unet* n, int B, const float* d_dout, hipStream_t st) {
     HIPR(launch_relu_mask(n->g_cat2.p, 192, 128, n->cat2.p, 192, 128, (long)B * H2 * W2, 64, st));
   }
   // e2
-  R(wgrad(n, cv[E2B], n->a2.p, 64, 0, n->g_cat2.p, 192, 128, B, H2, W2, st));
+  wgrad(n, wg, cv[E2B], n->a2.p, 64, 0, n->g_cat2.p, 192, 128, B, H2, W2);
   R(conv(n, cv[E2B], n->g_cat2.p, 192, 128, n->g_a2.p, 64, 0, B, H2, W2, false, n->a2.p, 64, 0, true, false, st));
-  R(wgrad(n, cv[E2A], n->p1.p, 32, 0, n->g_a2.p, 64, 0, B, H2, W2, st));
+  wgrad(n, wg, cv[E2A], n->p1.p, 32, 0, n->g_a2.p, 64, 0, B, H2, W2);
   R(conv(n, cv[E2A], n->g_a2.p, 64, 0, n->g_p1.p, 32, 0, B, H2, W2, false, nullptr, 0, 0, true, false, st));
   {
     PoolGradArgs u{n->g_p1.p, 32, 0, n->g_cat1.p, 96, 64, B, H, W, 32, 1};
@@ -330,9 +330,12 @@ int backward(icon_unet* n, int B, const float* d_dout, hipStream_t st) {
     HIPR(launch_relu_mask(n->g_cat1.p, 96, 64, n->cat1.p, 96, 64, P, 32, st));
   }
   // e1
-  R(wgrad(n, cv[E1B], n->a1.p, 32, 0, n->g_cat1.p, 96, 64, B, H, W, st));
+  wgrad(n, wg, cv[E1B], n->a1.p, 32, 0, n->g_cat1.p, 96, 64, B, H, W);
   R(conv(n, cv[E1B], n->g_cat1.p, 96, 64, n->g_a1.p, 32, 0, B, H, W, false, n->a1.p, 32, 0, true, false, st));
-  R(wgrad(n, cv[E1A], n->x8.p, 8, 0, n->g_a1.p, 32, 0, B, H, W, st));
+  wgrad(n, wg, cv[E1A], n->x8.p, 8, 0, n->g_a1.p, 32, 0, B, H, W);
+  const int blocks = plan_wgrad(wg, n->wgrad_blocks);
+  HIPR(launch_wgrad(wg, blocks, n->gpart + kHeadGradParts * 33, red, st));
+  HIPR(launch_grad_reduce(red, st));
 #undef R
 #undef HIPR
   return 0;
@@ -393,16 +396,15 @@ int icon_unet_create(icon_unet** out, int device, int max_batch, int H, int W, i
       (rc = t16(n, n->d2b, P2, 64)) || (rc = t16(n, n->d1a, P, 32)) || (rc = t16(n, n->d1b, P, 32)))
     return bail(rc);
   if (n->train) {
-    // gradient partial sums: the largest of a weight gradient's splits x
-    // weights (at the level of each convolution), the bias and head blocks
-    long part = (long)kHeadGradParts * 33;
-    const long level_px[NCONV] = {P, P, P2, P2, P4, P4, P8, P8, P4, P4, P2, P2, P, P};
-    for (int i = 0; i < NCONV; i++) {
-      const Conv& c = n->convs[i];
-      part = std::max(part, (long)wgrad_splits(level_px[i]) * c.taps * c.cout * c.cin);
-      part = std::max(part, (long)kBiasGradParts * c.cout);
-    }
-    if ((rc = alloc_bytes(n, (void**)&n->gpart, sizeof(float) * part))) return bail(rc);
+    // gradient partial sums: the head's blocks and, per block of the weight
+    // gradients' launch, its channels' weights and biases.  Two blocks per CU
+    // (their LDS), or one per channel tile of every layer on a small device.
+    int cus = 256;
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+    n->wgrad_blocks = std::max(2 * cus, 64);
+    if ((rc = alloc_bytes(n, (void**)&n->gpart,
+                          sizeof(float) * (kHeadGradParts * 33 + (long)n->wgrad_blocks * (9 * 64 * 64 + 64)))))
+      return bail(rc);
     if ((rc = alloc_bytes(n, (void**)&n->grads, sizeof(float) * off)) ||
         (rc = alloc_bytes(n, (void**)&n->adam_m, sizeof(float) * off)) ||
         (rc = alloc_bytes(n, (void**)&n->adam_v, sizeof(float) * off)))
@@ -501,7 +503,6 @@ int icon_unet_gradients(icon_unet* n, int B, const float* d_in, const float* d_t
   const long P = (long)B * n->H * n->W;
   int rc = forward(n, B, d_in, n->g_out.p, st);   // prediction into g_out, then its gradient in place
   if (rc) return rc;
-  UCHK(launch_zero32(n->grads, n->nparam, st));
   UCHK(hipMemsetAsync(n->d_loss, 0, sizeof(double), st));
   // loss = sum (pred - target)^2 / P; dL/dpred = 2 (pred - target) / P
   UCHK(launch_mse(n->g_out.p, d_target, P, n->g_out.p, n->d_loss, 2.f / (float)P, st));

@@ -51,15 +51,37 @@ struct ConvArgs {
   uint16_t* a1_out;
 };
 
-// dw[tap][co][ci] += sum over pixels of dy[p][co] * x[p + offset(tap)][ci]
-struct WgradArgs {
+// dw[tap][co][ci] = sum over pixels of dy[p][co] * x[p + offset(tap)][ci] and
+// db[co] = sum of dy[p][co], 3x3 taps, of all layers of a group at once.
+// Reduced without atomics: every block writes its partial sums to a scratch
+// buffer and the reduction adds them in a fixed order, so that training is
+// reproducible run to run.
+struct WgradLayer {
   const uint16_t* x;
-  int ldx, cx0;
   const float* dy;
-  int lddy, cdy0;
-  float* dw;
-  int N, H, W, Cin, Cout, taps;
-  float* part;   // [splits][taps][Cout][Cin] scratch: each pixel split's sums, added to dw in split order
+  float *dw, *db;
+  int ldx, cx0, lddy, cdy0;
+  int N, H, W, Cin, Cout;
+  // plan_wgrad: block shape in 32-channel tiles, block tiles, pixel tiles and
+  // their cost, tiles per split, splits, first block
+  int co, ci, nco, nci, tiles_x, tiles_y, tiles, cost, per, splits, first;
+  float *part, *bpart;   // [splits][9][Cout][Cin], [splits][Cout]
+};
+constexpr int kWgradLayers = 14;
+struct WgradGroup {
+  WgradLayer l[kWgradLayers];
+  int n;
+};
+// out[i] = sum over z < nparts of part[z][i], i < n (wide: n a multiple of 4)
+struct ReduceItem {
+  const float* part;
+  float* out;
+  long n;
+  int nparts, first, wide;
+};
+struct ReduceGroup {
+  ReduceItem t[2 * kWgradLayers + 1];
+  int n, blocks;
 };
 
 // 2x2 average pool (fwd: in H x W -> out H/2 x W/2) or nearest 2x upsample
@@ -84,15 +106,15 @@ struct PoolGradArgs {
 
 template <typename TX, typename TY>
 hipError_t launch_conv(const ConvArgs<TX, TY>& a, hipStream_t st);
-hipError_t launch_wgrad(const WgradArgs& a, int splits, hipStream_t st);
-// Weight and bias gradients are reduced without atomics: every block writes
-// its partial sums to a scratch buffer and launch_sum_parts adds them to the
-// gradient in a fixed order, so that training is reproducible run to run.
-hipError_t launch_bias_grad(const float* dy, int ld, int c0, long P, int C, float* db, float* part, hipStream_t st);
-constexpr int kBiasGradParts = 256;   // partial sums per channel (launch_bias_grad's part: [256][C])
-constexpr int kHeadGradParts = 256;   // blocks of launch_head_bwd (its part: [256][C + 1])
-// out[i] += part[0][i] + part[1][i] + ... + part[nparts - 1][i] (in that order)
-hipError_t launch_sum_parts(const float* part, int nparts, long n, float* out, hipStream_t st);
+// plan_wgrad fills the layers' plan for at most `blocks` blocks (at least one per
+// channel tile of every layer) and returns their number; launch_wgrad takes
+// wgrad_part_floats floats of scratch and adds the sums to the reduction.
+int plan_wgrad(WgradGroup& g, int blocks);
+long wgrad_part_floats(const WgradGroup& g);
+hipError_t launch_wgrad(WgradGroup& g, int blocks, float* part, ReduceGroup& r, hipStream_t st);
+void add_reduce(ReduceGroup& r, const float* part, int nparts, long n, float* out, bool wide);
+hipError_t launch_grad_reduce(const ReduceGroup& r, hipStream_t st);
+constexpr int kHeadGradParts = 512;   // blocks of launch_head_bwd (its part: [512][33])
 hipError_t launch_pool_bwd(const PoolGradArgs& a, hipStream_t st);
 hipError_t launch_up_fwd(const PoolArgs& a, hipStream_t st);
 hipError_t launch_up_bwd(const PoolGradArgs& a, hipStream_t st);
@@ -100,8 +122,8 @@ hipError_t launch_relu_mask(float* g, int ldg, int cg0, const uint16_t* act, int
                             hipStream_t st);
 hipError_t launch_head_fwd(const uint16_t* x, int ldx, const float* w, const float* b, int C, long P, float* out,
                            hipStream_t st);
-hipError_t launch_head_bwd(const uint16_t* x, int ldx, const float* w, int C, long P, const float* dout, float* dx,
-                           int lddx, float* dw, float* db, float* part, hipStream_t st);
+hipError_t launch_head_bwd(const uint16_t* x, int ldx, const float* w, long P, const float* dout, float* dx, int lddx,
+                           float* part, hipStream_t st);
 hipError_t launch_flip_weights(const uint16_t* w, uint16_t* wt, int taps, int Cout, int Cin, hipStream_t st);
 hipError_t launch_adam(float* w, uint16_t* w16, const float* g, float* m, float* v, long n, float lr, float b1,
                        float b2, float eps, float c1, float c2, float gscale, hipStream_t st);
@@ -115,6 +137,5 @@ hipError_t launch_to_bf16_scaled(const float* in, const float* scale, long P, in
 // out = gain * (m + scale[b] * y) per image b (gain 1: m + scale[b] * y exactly)
 hipError_t launch_residual_add(const float* m, const float* y, const float* scale, long P, int B, float gain,
                                float* out, hipStream_t st);
-hipError_t launch_zero32(float* p, long n, hipStream_t st);
 
 }  // namespace unet
