@@ -90,8 +90,7 @@ struct icon_unet {
   float out_gain = 1.f;      // factor on the warm start's output (icon_unet_set_output_gain)
   double* rms_part = nullptr;  // [maxB][image_rms_parts()] partial sums of the scale
   // gradients (fp32)
-  T32 g_d1b, g_d1a, g_cat1, g_d2b, g_d2a, g_cat2, g_d3b, g_d3a, g_cat3, g_bb, g_ab, g_p3, g_a3, g_p2, g_a2, g_p1,
-      g_a1, g_out;
+  T32 g_d1b, g_d1a, g_cat1, g_d2b, g_d2a, g_cat2, g_d3b, g_d3a, g_cat3, g_bb, g_ab, g_a3, g_a2, g_a1, g_out;
   std::vector<void*> allocs;
 };
 
@@ -151,45 +150,29 @@ struct FirstConv {
 // up (optional): the input's first Cup channels, read from this half-size
 // tensor (nearest-neighbour 2x upsampling) instead of x; pool (optional):
 // the output's 2x2 average, written at half size
-template <typename TX, typename TY>
-int conv(icon_unet* n, const Conv& c, const TX* x, int ldx, int cx0, TY* y, int ldy, int cy0, int B, int H, int W,
-         bool relu, const uint16_t* mask, int ldm, int cm0, bool flipped, bool accumulate, hipStream_t st,
-         const T16* up = nullptr, const T16* pool = nullptr, const float* head_w = nullptr,
+int conv(icon_unet* n, const Conv& c, const uint16_t* x, int ldx, int cx0, uint16_t* y, int ldy, int cy0, int B, int H,
+         int W, hipStream_t st, const T16* up = nullptr, const T16* pool = nullptr, const float* head_w = nullptr,
          const float* head_b = nullptr, float* head_out = nullptr, const FirstConv* first = nullptr) {
-  ConvArgs<TX, TY> a{};
+  ConvArgs<uint16_t, uint16_t> a{};
   a.x = x; a.ldx = ldx; a.cx0 = cx0;
-  a.w = flipped ? c.wt16 : c.w16;
-  a.bias = flipped ? nullptr : n->params + c.off_b;
+  a.w = c.w16;
+  a.bias = n->params + c.off_b;
   a.y = y; a.ldy = ldy; a.cy0 = cy0;
-  a.mask = mask; a.ldm = ldm; a.cm0 = cm0;
   a.N = B; a.H = H; a.W = W;
-  a.Cin = flipped ? c.cout : c.cin;
-  a.Cout = flipped ? c.cin : c.cout;
+  a.Cin = c.cin;
+  a.Cout = c.cout;
   a.taps = c.taps;
-  a.relu = relu; a.accumulate = accumulate;
+  a.relu = 1;
   if (up) { a.up = up->p; a.ldu = up->C; a.cu0 = 0; a.Cup = up->C; }
   if (pool) { a.pool = pool->p; a.ldp = pool->C; a.cp0 = 0; }
   a.head_w = head_w; a.head_b = head_b; a.head_out = head_out;
-  if constexpr (sizeof(TX) == 2 && sizeof(TY) == 2) {
-    if (first) {
-      const Conv& c1 = n->convs[0];
-      a.x1 = first->img; a.x1_scale = first->scale; a.a1_out = first->a1_out;
-      a.w1 = c1.w16; a.w1_cin = c1.cin; a.b1 = n->params + c1.off_b;
-    }
+  if (first) {
+    const Conv& c1 = n->convs[0];
+    a.x1 = first->img; a.x1_scale = first->scale; a.a1_out = first->a1_out;
+    a.w1 = c1.w16; a.w1_cin = c1.cin; a.b1 = n->params + c1.off_b;
   }
   UCHK(launch_conv(a, st));
   return 0;
-}
-
-// a layer's weight and bias gradients, computed with those of the other layers
-// once every output gradient is there (the end of backward)
-void wgrad(icon_unet* n, WgradGroup& g, const Conv& c, const uint16_t* x, int ldx, int cx0, const float* dy, int lddy,
-           int cdy0, int B, int H, int W) {
-  WgradLayer& a = g.l[g.n++];
-  a = WgradLayer{};
-  a.x = x; a.ldx = ldx; a.cx0 = cx0; a.dy = dy; a.lddy = lddy; a.cdy0 = cdy0;
-  a.dw = n->grads + c.off_w; a.db = n->grads + c.off_b;
-  a.N = B; a.H = H; a.W = W; a.Cin = c.cin; a.Cout = c.cout;
 }
 
 int up(const T16& in, const T16& out, int co0, int B, int h, int w, hipStream_t st) {
@@ -224,38 +207,59 @@ int forward(icon_unet* n, int B, const float* d_in, float* d_out, hipStream_t st
   // at channel ci - u of cat, u = Cup when only the skip half is stored
   const int k1 = fuse_up ? 0 : 64, k2 = fuse_up ? 0 : 128, k3 = fuse_up ? 0 : 256;
   const int u1 = fuse_up ? 64 : 0, u2 = fuse_up ? 128 : 0, u3 = fuse_up ? 256 : 0;
-  R(conv(n, cv[E1B], n->a1.p, 32, 0, n->cat1.p, n->cat1.C, k1, B, H, W, true, nullptr, 0, 0, false, false, st, nullptr,
+  R(conv(n, cv[E1B], n->a1.p, 32, 0, n->cat1.p, n->cat1.C, k1, B, H, W, st, nullptr,
          &n->p1, nullptr, nullptr, nullptr, &first));
-  R(conv(n, cv[E2A], n->p1.p, 32, 0, n->a2.p, 64, 0, B, H2, W2, true, nullptr, 0, 0, false, false, st));
-  R(conv(n, cv[E2B], n->a2.p, 64, 0, n->cat2.p, n->cat2.C, k2, B, H2, W2, true, nullptr, 0, 0, false, false, st, nullptr,
+  R(conv(n, cv[E2A], n->p1.p, 32, 0, n->a2.p, 64, 0, B, H2, W2, st));
+  R(conv(n, cv[E2B], n->a2.p, 64, 0, n->cat2.p, n->cat2.C, k2, B, H2, W2, st, nullptr,
          &n->p2));
-  R(conv(n, cv[E3A], n->p2.p, 64, 0, n->a3.p, 128, 0, B, H4, W4, true, nullptr, 0, 0, false, false, st));
-  R(conv(n, cv[E3B], n->a3.p, 128, 0, n->cat3.p, n->cat3.C, k3, B, H4, W4, true, nullptr, 0, 0, false, false, st, nullptr,
+  R(conv(n, cv[E3A], n->p2.p, 64, 0, n->a3.p, 128, 0, B, H4, W4, st));
+  R(conv(n, cv[E3B], n->a3.p, 128, 0, n->cat3.p, n->cat3.C, k3, B, H4, W4, st, nullptr,
          &n->p3));
-  R(conv(n, cv[BA], n->p3.p, 128, 0, n->ab.p, 256, 0, B, H8, W8, true, nullptr, 0, 0, false, false, st));
-  R(conv(n, cv[BB], n->ab.p, 256, 0, n->bb.p, 256, 0, B, H8, W8, true, nullptr, 0, 0, false, false, st));
+  R(conv(n, cv[BA], n->p3.p, 128, 0, n->ab.p, 256, 0, B, H8, W8, st));
+  R(conv(n, cv[BB], n->ab.p, 256, 0, n->bb.p, 256, 0, B, H8, W8, st));
   if (!fuse_up) R(up(n->bb, n->cat3, 0, B, H8, W8, st));
-  R(conv(n, cv[D3A], n->cat3.p, n->cat3.C, -u3, n->d3a.p, 128, 0, B, H4, W4, true, nullptr, 0, 0, false, false, st,
+  R(conv(n, cv[D3A], n->cat3.p, n->cat3.C, -u3, n->d3a.p, 128, 0, B, H4, W4, st,
          fuse_up ? &n->bb : nullptr));
-  R(conv(n, cv[D3B], n->d3a.p, 128, 0, n->d3b.p, 128, 0, B, H4, W4, true, nullptr, 0, 0, false, false, st));
+  R(conv(n, cv[D3B], n->d3a.p, 128, 0, n->d3b.p, 128, 0, B, H4, W4, st));
   if (!fuse_up) R(up(n->d3b, n->cat2, 0, B, H4, W4, st));
-  R(conv(n, cv[D2A], n->cat2.p, n->cat2.C, -u2, n->d2a.p, 64, 0, B, H2, W2, true, nullptr, 0, 0, false, false, st,
+  R(conv(n, cv[D2A], n->cat2.p, n->cat2.C, -u2, n->d2a.p, 64, 0, B, H2, W2, st,
          fuse_up ? &n->d3b : nullptr));
-  R(conv(n, cv[D2B], n->d2a.p, 64, 0, n->d2b.p, 64, 0, B, H2, W2, true, nullptr, 0, 0, false, false, st));
+  R(conv(n, cv[D2B], n->d2a.p, 64, 0, n->d2b.p, 64, 0, B, H2, W2, st));
   if (!fuse_up) R(up(n->d2b, n->cat1, 0, B, H2, W2, st));
-  R(conv(n, cv[D1A], n->cat1.p, n->cat1.C, -u1, n->d1a.p, 32, 0, B, H, W, true, nullptr, 0, 0, false, false, st,
+  R(conv(n, cv[D1A], n->cat1.p, n->cat1.C, -u1, n->d1a.p, 32, 0, B, H, W, st,
          fuse_up ? &n->d2b : nullptr));
   if (n->train) {
-    R(conv(n, cv[D1B], n->d1a.p, 32, 0, n->d1b.p, 32, 0, B, H, W, true, nullptr, 0, 0, false, false, st));
+    R(conv(n, cv[D1B], n->d1a.p, 32, 0, n->d1b.p, 32, 0, B, H, W, st));
     if (launch_head_fwd(n->d1b.p, 32, n->params + n->head_w, n->params + n->head_b, 32, P, d_out, st) != hipSuccess)
       return ufail(2, "head");
   } else {
     // inference: the head in D1B's epilogue (the same sums on the same BF16
     // values), D1B's output is not stored
-    R(conv(n, cv[D1B], n->d1a.p, 32, 0, n->d1b.p, 32, 0, B, H, W, true, nullptr, 0, 0, false, false, st, nullptr,
+    R(conv(n, cv[D1B], n->d1a.p, 32, 0, n->d1b.p, 32, 0, B, H, W, st, nullptr,
            nullptr, n->params + n->head_w, n->params + n->head_b, d_out));
   }
 #undef R
+  return 0;
+}
+
+// A convolution's input gradient, from its output gradient dy.  mask: the
+// activation that is the convolution's input (its ReLU), or none.
+int dgrad(icon_unet* n, const Conv& c, const T32& dy, float* dx, int lddx, const T16* mask, int B, int H, int W,
+          hipStream_t st, const T32* usum = nullptr, const T32* pgrad = nullptr, const T16* pmask = nullptr) {
+  ConvArgs<float, float> a{};
+  a.x = dy.p; a.ldx = dy.C;
+  a.w = c.wt16;
+  a.y = dx; a.ldy = lddx;
+  if (mask) { a.mask = mask->p; a.ldm = mask->C; }
+  a.N = B; a.H = H; a.W = W;
+  a.Cin = c.cout; a.Cout = c.cin;
+  a.taps = c.taps;
+  // decoder: channels [0, Cus) are the upsampled tensor's
+  if (usum) { a.usum = usum->p; a.ldus = a.Cus = usum->C; }
+  // encoder: the pooled input's gradient, added to the full-size one; the skip
+  // half of cat holds the forward values
+  if (pgrad) { a.pgrad = pgrad->p; a.ldpg = pgrad->C; a.pmask = pmask->p; a.ldpm = pmask->C; a.cpm0 = pmask->C - pgrad->C; }
+  UCHK(launch_conv(a, st));
   return 0;
 }
 
@@ -272,67 +276,38 @@ int backward(icon_unet* n, int B, const float* d_dout, hipStream_t st) {
   HIPR(launch_head_bwd(n->d1b.p, 32, n->params + n->head_w, P, d_dout, n->g_d1b.p, 32, n->gpart, st));
   // dw and db of the head are adjacent in the parameter vector
   add_reduce(red, n->gpart, kHeadGradParts, 33, n->grads + n->head_w, false);
-  // d1b, d1a
-  wgrad(n, wg, cv[D1B], n->d1a.p, 32, 0, n->g_d1b.p, 32, 0, B, H, W);
-  R(conv(n, cv[D1B], n->g_d1b.p, 32, 0, n->g_d1a.p, 32, 0, B, H, W, false, n->d1a.p, 32, 0, true, false, st));
-  wgrad(n, wg, cv[D1A], n->cat1.p, 96, 0, n->g_d1a.p, 32, 0, B, H, W);
-  R(conv(n, cv[D1A], n->g_d1a.p, 32, 0, n->g_cat1.p, 96, 0, B, H, W, false, n->cat1.p, 96, 0, true, false, st));
-  {
-    PoolGradArgs u{n->g_cat1.p, 96, 0, n->g_d2b.p, 64, 0, B, H2, W2, 64, 0};
-    HIPR(launch_up_bwd(u, st));
-  }
-  // d2b, d2a
-  wgrad(n, wg, cv[D2B], n->d2a.p, 64, 0, n->g_d2b.p, 64, 0, B, H2, W2);
-  R(conv(n, cv[D2B], n->g_d2b.p, 64, 0, n->g_d2a.p, 64, 0, B, H2, W2, false, n->d2a.p, 64, 0, true, false, st));
-  wgrad(n, wg, cv[D2A], n->cat2.p, 192, 0, n->g_d2a.p, 64, 0, B, H2, W2);
-  R(conv(n, cv[D2A], n->g_d2a.p, 64, 0, n->g_cat2.p, 192, 0, B, H2, W2, false, n->cat2.p, 192, 0, true, false, st));
-  {
-    PoolGradArgs u{n->g_cat2.p, 192, 0, n->g_d3b.p, 128, 0, B, H4, W4, 128, 0};
-    HIPR(launch_up_bwd(u, st));
-  }
-  // d3b, d3a
-  wgrad(n, wg, cv[D3B], n->d3a.p, 128, 0, n->g_d3b.p, 128, 0, B, H4, W4);
-  R(conv(n, cv[D3B], n->g_d3b.p, 128, 0, n->g_d3a.p, 128, 0, B, H4, W4, false, n->d3a.p, 128, 0, true, false, st));
-  wgrad(n, wg, cv[D3A], n->cat3.p, 384, 0, n->g_d3a.p, 128, 0, B, H4, W4);
-  R(conv(n, cv[D3A], n->g_d3a.p, 128, 0, n->g_cat3.p, 384, 0, B, H4, W4, false, n->cat3.p, 384, 0, true, false, st));
-  {
-    PoolGradArgs u{n->g_cat3.p, 384, 0, n->g_bb.p, 256, 0, B, H8, W8, 256, 0};
-    HIPR(launch_up_bwd(u, st));
-  }
+  // decoders: g_cat1..3 hold the skip halves' gradients
+  R(dgrad(n, cv[D1B], n->g_d1b, n->g_d1a.p, 32, &n->d1a, B, H, W, st));
+  R(dgrad(n, cv[D1A], n->g_d1a, n->g_cat1.p, 32, &n->cat1, B, H, W, st, &n->g_d2b));
+  R(dgrad(n, cv[D2B], n->g_d2b, n->g_d2a.p, 64, &n->d2a, B, H2, W2, st));
+  R(dgrad(n, cv[D2A], n->g_d2a, n->g_cat2.p, 64, &n->cat2, B, H2, W2, st, &n->g_d3b));
+  R(dgrad(n, cv[D3B], n->g_d3b, n->g_d3a.p, 128, &n->d3a, B, H4, W4, st));
+  R(dgrad(n, cv[D3A], n->g_d3a, n->g_cat3.p, 128, &n->cat3, B, H4, W4, st, &n->g_bb));
   // bottleneck
-  wgrad(n, wg, cv[BB], n->ab.p, 256, 0, n->g_bb.p, 256, 0, B, H8, W8);
-  R(conv(n, cv[BB], n->g_bb.p, 256, 0, n->g_ab.p, 256, 0, B, H8, W8, false, n->ab.p, 256, 0, true, false, st));
-  wgrad(n, wg, cv[BA], n->p3.p, 128, 0, n->g_ab.p, 256, 0, B, H8, W8);
-  R(conv(n, cv[BA], n->g_ab.p, 256, 0, n->g_p3.p, 128, 0, B, H8, W8, false, nullptr, 0, 0, true, false, st));
-  {
-    PoolGradArgs u{n->g_p3.p, 128, 0, n->g_cat3.p, 384, 256, B, H4, W4, 128, 1};
-    HIPR(launch_pool_bwd(u, st));
-    HIPR(launch_relu_mask(n->g_cat3.p, 384, 256, n->cat3.p, 384, 256, (long)B * H4 * W4, 128, st));
+  R(dgrad(n, cv[BB], n->g_bb, n->g_ab.p, 256, &n->ab, B, H8, W8, st));
+  R(dgrad(n, cv[BA], n->g_ab, nullptr, 128, nullptr, B, H8, W8, st, nullptr, &n->g_cat3, &n->cat3));
+  // encoders
+  R(dgrad(n, cv[E3B], n->g_cat3, n->g_a3.p, 128, &n->a3, B, H4, W4, st));
+  R(dgrad(n, cv[E3A], n->g_a3, nullptr, 64, nullptr, B, H4, W4, st, nullptr, &n->g_cat2, &n->cat2));
+  R(dgrad(n, cv[E2B], n->g_cat2, n->g_a2.p, 64, &n->a2, B, H2, W2, st));
+  R(dgrad(n, cv[E2A], n->g_a2, nullptr, 32, nullptr, B, H2, W2, st, nullptr, &n->g_cat1, &n->cat1));
+  R(dgrad(n, cv[E1B], n->g_cat1, n->g_a1.p, 32, &n->a1, B, H, W, st));
+  // weights and biases
+  const struct { int c; const T16* x; const T32* dy; int H, W; } layers[NCONV] = {
+      {D1B, &n->d1a, &n->g_d1b, H, W},    {D1A, &n->cat1, &n->g_d1a, H, W},   {D2B, &n->d2a, &n->g_d2b, H2, W2},
+      {D2A, &n->cat2, &n->g_d2a, H2, W2}, {D3B, &n->d3a, &n->g_d3b, H4, W4},  {D3A, &n->cat3, &n->g_d3a, H4, W4},
+      {BB, &n->ab, &n->g_bb, H8, W8},     {BA, &n->p3, &n->g_ab, H8, W8},     {E3B, &n->a3, &n->g_cat3, H4, W4},
+      {E3A, &n->p2, &n->g_a3, H4, W4},    {E2B, &n->a2, &n->g_cat2, H2, W2},  {E2A, &n->p1, &n->g_a2, H2, W2},
+      {E1B, &n->a1, &n->g_cat1, H, W},    {E1A, &n->x8, &n->g_a1, H, W}};
+  for (const auto& l : layers) {
+    const Conv& c = cv[l.c];
+    WgradLayer& a = wg.l[wg.n++];
+    a = WgradLayer{};
+    a.x = l.x->p; a.ldx = l.x->C;
+    a.dy = l.dy->p; a.lddy = l.dy->C;
+    a.dw = n->grads + c.off_w; a.db = n->grads + c.off_b;
+    a.N = B; a.H = l.H; a.W = l.W; a.Cin = c.cin; a.Cout = c.cout;
   }
-  // e3
-  wgrad(n, wg, cv[E3B], n->a3.p, 128, 0, n->g_cat3.p, 384, 256, B, H4, W4);
-  R(conv(n, cv[E3B], n->g_cat3.p, 384, 256, n->g_a3.p, 128, 0, B, H4, W4, false, n->a3.p, 128, 0, true, false, st));
-  wgrad(n, wg, cv[E3A], n->p2.p, 64, 0, n->g_a3.p, 128, 0, B, H4, W4);
-  R(conv(n, cv[E3A], n->g_a3.p, 128, 0, n->g_p2.p, 64, 0, B, H4, W4, false, nullptr, 0, 0, true, false, st));
-  {
-    PoolGradArgs u{n->g_p2.p, 64, 0, n->g_cat2.p, 192, 128, B, H2, W2, 64, 1};
-    HIPR(launch_pool_bwd(u, st));
-    HIPR(launch_relu_mask(n->g_cat2.p, 192, 128, n->cat2.p, 192, 128, (long)B * H2 * W2, 64, st));
-  }
-  // e2
-  wgrad(n, wg, cv[E2B], n->a2.p, 64, 0, n->g_cat2.p, 192, 128, B, H2, W2);
-  R(conv(n, cv[E2B], n->g_cat2.p, 192, 128, n->g_a2.p, 64, 0, B, H2, W2, false, n->a2.p, 64, 0, true, false, st));
-  wgrad(n, wg, cv[E2A], n->p1.p, 32, 0, n->g_a2.p, 64, 0, B, H2, W2);
-  R(conv(n, cv[E2A], n->g_a2.p, 64, 0, n->g_p1.p, 32, 0, B, H2, W2, false, nullptr, 0, 0, true, false, st));
-  {
-    PoolGradArgs u{n->g_p1.p, 32, 0, n->g_cat1.p, 96, 64, B, H, W, 32, 1};
-    HIPR(launch_pool_bwd(u, st));
-    HIPR(launch_relu_mask(n->g_cat1.p, 96, 64, n->cat1.p, 96, 64, P, 32, st));
-  }
-  // e1
-  wgrad(n, wg, cv[E1B], n->a1.p, 32, 0, n->g_cat1.p, 96, 64, B, H, W);
-  R(conv(n, cv[E1B], n->g_cat1.p, 96, 64, n->g_a1.p, 32, 0, B, H, W, false, n->a1.p, 32, 0, true, false, st));
-  wgrad(n, wg, cv[E1A], n->x8.p, 8, 0, n->g_a1.p, 32, 0, B, H, W);
   const int blocks = plan_wgrad(wg, n->wgrad_blocks);
   HIPR(launch_wgrad(wg, blocks, n->gpart + kHeadGradParts * 33, red, st));
   HIPR(launch_grad_reduce(red, st));
@@ -409,12 +384,11 @@ int icon_unet_create(icon_unet** out, int device, int max_batch, int H, int W, i
         (rc = alloc_bytes(n, (void**)&n->adam_m, sizeof(float) * off)) ||
         (rc = alloc_bytes(n, (void**)&n->adam_v, sizeof(float) * off)))
       return bail(rc);
-    if ((rc = t32(n, n->g_d1b, P, 32)) || (rc = t32(n, n->g_d1a, P, 32)) || (rc = t32(n, n->g_cat1, P, 96)) ||
-        (rc = t32(n, n->g_d2b, P2, 64)) || (rc = t32(n, n->g_d2a, P2, 64)) || (rc = t32(n, n->g_cat2, P2, 192)) ||
-        (rc = t32(n, n->g_d3b, P4, 128)) || (rc = t32(n, n->g_d3a, P4, 128)) || (rc = t32(n, n->g_cat3, P4, 384)) ||
-        (rc = t32(n, n->g_bb, P8, 256)) || (rc = t32(n, n->g_ab, P8, 256)) || (rc = t32(n, n->g_p3, P8, 128)) ||
-        (rc = t32(n, n->g_a3, P4, 128)) || (rc = t32(n, n->g_p2, P4, 64)) || (rc = t32(n, n->g_a2, P2, 64)) ||
-        (rc = t32(n, n->g_p1, P2, 32)) || (rc = t32(n, n->g_a1, P, 32)) || (rc = t32(n, n->g_out, P, 1)))
+    if ((rc = t32(n, n->g_d1b, P, 32)) || (rc = t32(n, n->g_d1a, P, 32)) || (rc = t32(n, n->g_cat1, P, 32)) ||
+        (rc = t32(n, n->g_d2b, P2, 64)) || (rc = t32(n, n->g_d2a, P2, 64)) || (rc = t32(n, n->g_cat2, P2, 64)) ||
+        (rc = t32(n, n->g_d3b, P4, 128)) || (rc = t32(n, n->g_d3a, P4, 128)) || (rc = t32(n, n->g_cat3, P4, 128)) ||
+        (rc = t32(n, n->g_bb, P8, 256)) || (rc = t32(n, n->g_ab, P8, 256)) || (rc = t32(n, n->g_a3, P4, 128)) ||
+        (rc = t32(n, n->g_a2, P2, 64)) || (rc = t32(n, n->g_a1, P, 32)) || (rc = t32(n, n->g_out, P, 1)))
       return bail(rc);
   }
   *out = n;

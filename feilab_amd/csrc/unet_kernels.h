@@ -8,8 +8,8 @@ namespace unet {
 // Convolution y = conv(x, w) (+ bias, ReLU), taps 9 (3x3, zero padding 1) or 1.
 // x: [N][H][W] pixels, channel stride ldx, channels [cx0, cx0 + Cin);
 // y: channel stride ldy, channels [cy0, cy0 + Cout); w: [taps][Cout][Cin] bf16.
-// mask (optional): y is zeroed where the bf16 mask tensor is <= 0 (the ReLU of
-// a forward activation, for input gradients); accumulate: y += result.
+// FP32 output (input gradients): mask (optional): y is zeroed where the bf16
+// mask tensor is <= 0 (the ReLU of a forward activation).
 template <typename TX, typename TY>
 struct ConvArgs {
   const TX* x;
@@ -21,7 +21,7 @@ struct ConvArgs {
   const uint16_t* mask;
   int ldm, cm0;
   int N, H, W, Cin, Cout, taps;
-  int relu, accumulate;
+  int relu;
   // optional: input channels [0, Cup) read from `up` (H/2 x W/2 pixels,
   // nearest-neighbour 2x upsampling) instead of x
   const uint16_t* up;
@@ -49,6 +49,18 @@ struct ConvArgs {
   int w1_cin;
   const float* b1;
   uint16_t* a1_out;
+  // optional (FP32 output): output channels [0, Cus) as sums of 2x2 pixels to
+  // usum (H/2 x W/2 pixels; the gradient of a nearest 2x upsample), the others
+  // at channel c - Cus of y
+  float* usum;
+  int ldus, Cus;
+  // optional (FP32 output): y is not stored; a quarter of it is added to the
+  // 2H x 2W gradient pgrad (the gradient of a 2x2 average pool), which is
+  // zeroed where the bf16 tensor pmask is <= 0
+  float* pgrad;
+  int ldpg;
+  const uint16_t* pmask;
+  int ldpm, cpm0;
 };
 
 // dw[tap][co][ci] = sum over pixels of dy[p][co] * x[p + offset(tap)][ci] and
@@ -84,24 +96,13 @@ struct ReduceGroup {
   int n, blocks;
 };
 
-// 2x2 average pool (fwd: in H x W -> out H/2 x W/2) or nearest 2x upsample
-// (fwd: in H x W -> out 2H x 2W); bf16 with channel sub-ranges.
+// Nearest 2x upsample (in H x W -> out 2H x 2W); bf16 with channel sub-ranges.
 struct PoolArgs {
   const uint16_t* in;
   int ldi, ci0;
   uint16_t* out;
   int ldo, co0;
   int N, H, W, C;   // input dims
-};
-
-// Gradients of pool / upsample (fp32).  H, W are the dims of din.
-struct PoolGradArgs {
-  const float* dout;
-  int ldo, co0;
-  float* din;
-  int ldi, ci0;
-  int N, H, W, C;
-  int accumulate;
 };
 
 template <typename TX, typename TY>
@@ -115,11 +116,7 @@ hipError_t launch_wgrad(WgradGroup& g, int blocks, float* part, ReduceGroup& r, 
 void add_reduce(ReduceGroup& r, const float* part, int nparts, long n, float* out, bool wide);
 hipError_t launch_grad_reduce(const ReduceGroup& r, hipStream_t st);
 constexpr int kHeadGradParts = 512;   // blocks of launch_head_bwd (its part: [512][33])
-hipError_t launch_pool_bwd(const PoolGradArgs& a, hipStream_t st);
 hipError_t launch_up_fwd(const PoolArgs& a, hipStream_t st);
-hipError_t launch_up_bwd(const PoolGradArgs& a, hipStream_t st);
-hipError_t launch_relu_mask(float* g, int ldg, int cg0, const uint16_t* act, int lda, int ca0, long P, int C,
-                            hipStream_t st);
 hipError_t launch_head_fwd(const uint16_t* x, int ldx, const float* w, const float* b, int C, long P, float* out,
                            hipStream_t st);
 hipError_t launch_head_bwd(const uint16_t* x, int ldx, const float* w, long P, const float* dout, float* dx, int lddx,

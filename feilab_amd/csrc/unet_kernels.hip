@@ -52,10 +52,6 @@ __device__ __forceinline__ float head_group(const V8& v, const float* w, float s
 }
 
 
-__device__ __forceinline__ void store1(uint16_t* p, float v) { *p = f2bf(v); }
-__device__ __forceinline__ float load1(const uint16_t* p) { return bf2f(*p); }
-__device__ __forceinline__ float load1(const float* p) { return *p; }
-__device__ __forceinline__ void store1(float* p, float v) { *p = v; }
 
 // ----------------------------------------------------------------- conv
 // Block: 256 threads = 4 waves on a 4R x 16 pixel tile of one image and COB
@@ -132,16 +128,14 @@ __device__ __forceinline__ float bf_lo(uint32_t u) { return __uint_as_float(u <<
 __device__ __forceinline__ float bf_hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
 
 template <typename TX, typename TY, int COB, int R, bool FIRST>
-__global__ __launch_bounds__(256, COB == 32 && R == 4 ? 3 : 2) void k_conv(ConvArgs<TX, TY> a) {
+__global__ __launch_bounds__(256, COB == 32 && R <= 4 ? 3 : 2) void k_conv(ConvArgs<TX, TY> a) {
   constexpr int CT = COB / 16;
   constexpr int CL = COB / 4;                        // consecutive output channels per lane
   constexpr int PW = sizeof(TX) / 2;                 // 16-byte loads per input piece
-  // BF16 input: the next chunk's weights are prefetched into registers with
-  // its input; FP32 input (no registers to spare): they are loaded when
-  // stored, all pieces in flight at once
+  // the next chunk's weights are prefetched into registers with its input
   // FIRST: the input is computed from the FP32 images (a single chunk whose
   // weights are staged once, no prefetch)
-  constexpr bool kWPrefetch = PW == 1 && !FIRST;
+  constexpr bool kWPrefetch = !FIRST;
   constexpr int kTH = 4 * R;       // tile rows: R per wave
   constexpr int kHY = kTH + 2;     // halo rows
   // FIRST: the BF16 image over the halo's own halo (kRY x kRX pixels), per
@@ -568,22 +562,82 @@ __global__ __launch_bounds__(256, COB == 32 && R == 4 ? 3 : 2) void k_conv(ConvA
           }
         }
       } else {
-        // FP32 output (masked, accumulating), one element at a time
+        // FP32 output (an input gradient), in whole 16-byte accesses, with
+        // what the backward pass does next to it: the ReLU mask, and instead
+        // of a pass of its own each
+        //   usum: channels below Cus go to the half-size gradient of the
+        //         upsampled tensor, as 2x2 sums
+        //   pgrad: a pooled gradient goes to the four full-size pixels
+        const bool up2 = co0 < a.Cus;
 #pragma unroll
-        for (int i = 0; i < R; i++) {
-          const int y = y0 + R * wave + i;
-          if (y >= a.H || x >= a.W) continue;
-          const long p = ((long)n * a.H + y) * a.W + x;
+        for (int i0 = 0; i0 < R; i0 += 2) {
+          float v[2][CL];
+          const bool inx = x < a.W;
 #pragma unroll
-          for (int k = 0; k < CL; k++) {
-            const int co = cl0 + k;
-            if (co >= a.Cout) continue;
-            float v = acc[i][k >> 2][k & 3] + bl[k];
-            if (a.relu) v = relu(v);
-            if (a.mask && !(bf2f(a.mask[p * a.ldm + a.cm0 + co]) > 0.f)) v = 0.f;
-            TY* dst = a.y + p * a.ldy + a.cy0 + co;
-            if (a.accumulate) v += load1(dst);
-            store1(dst, v);
+          for (int h = 0; h < 2; h++) {
+            const int i = i0 + h, y = y0 + R * wave + i;
+            const bool in = inx && y < a.H;
+            const long p = ((long)n * a.H + y) * a.W + x;
+#pragma unroll
+            for (int k = 0; k < CL; k++) v[h][k] = acc[i][k >> 2][k & 3];
+            if (a.mask && in) {
+#pragma unroll
+              for (int h8 = 0; h8 < CL / 8; h8++) {
+                if (cl0 + 8 * h8 >= a.Cout) continue;
+                V8 m;
+                m.u = *reinterpret_cast<const uint4*>(a.mask + p * a.ldm + a.cm0 + cl0 + 8 * h8);
+#pragma unroll
+                for (int k = 0; k < 8; k++)
+                  if (!(bf2f(m.h[k]) > 0.f)) v[h][8 * h8 + k] = 0.f;
+              }
+            }
+            if (!in || up2 || a.pgrad) continue;
+            f4* dst = reinterpret_cast<f4*>(a.y + p * a.ldy + a.cy0 + cl0 - a.Cus);
+#pragma unroll
+            for (int k = 0; k < CL; k += 4)
+              if (cl0 + k < a.Cout) dst[k / 4] = f4{v[h][k], v[h][k + 1], v[h][k + 2], v[h][k + 3]};
+          }
+          const int y = y0 + R * wave + i0;
+          if (up2) {
+            // (y, x) + (y, x+1) + (y+1, x) + (y+1, x+1); pixel x + 1 is the
+            // next lane's (DPP row_shl:1)
+            f4 o[CL / 4];
+#pragma unroll
+            for (int k = 0; k < CL; k++) {
+              const float r0 = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[0][k]), 0x101, 0xf, 0xf, true));
+              const float r1 = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[1][k]), 0x101, 0xf, 0xf, true));
+              o[k >> 2][k & 3] = ((v[0][k] + r0) + v[1][k]) + r1;
+            }
+            if (!(r16 & 1) && y + 1 < a.H && x + 1 < a.W) {
+              f4* dst = reinterpret_cast<f4*>(
+                  a.usum + (((long)n * (a.H >> 1) + (y >> 1)) * (a.W >> 1) + (x >> 1)) * a.ldus + cl0);
+#pragma unroll
+              for (int k = 0; k < CL / 4; k++) dst[k] = o[k];
+            }
+          } else if (a.pgrad) {
+            // pgrad = (pgrad + v / 4) where its forward value (pmask) is positive
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+              if (!inx || y + h >= a.H) continue;
+#pragma unroll
+              for (int q = 0; q < 4; q++) {
+                const long p = ((long)n * (2 * a.H) + 2 * (y + h) + (q >> 1)) * (2 * a.W) + 2 * x + (q & 1);
+#pragma unroll
+                for (int h8 = 0; h8 < CL / 8; h8++) {
+                  const int c = cl0 + 8 * h8;
+                  if (c >= a.Cout) continue;
+                  f4* d = reinterpret_cast<f4*>(a.pgrad + p * a.ldpg + c);
+                  V8 m;
+                  m.u = *reinterpret_cast<const uint4*>(a.pmask + p * a.ldpm + a.cpm0 + c);
+                  f4 g[2] = {d[0], d[1]};
+#pragma unroll
+                  for (int k = 0; k < 8; k++)
+                    g[k >> 2][k & 3] = bf2f(m.h[k]) > 0.f ? g[k >> 2][k & 3] + 0.25f * v[h][8 * h8 + k] : 0.f;
+                  d[0] = g[0];
+                  d[1] = g[1];
+                }
+              }
+            }
           }
         }
       }
@@ -851,21 +905,6 @@ __global__ __launch_bounds__(256) void k_grad_reduce(ReduceGroup a) {
 
 // ------------------------------------------------------------ small ops
 
-// 2x2 average pool (bf16 NHWC, channel sub-ranges); 8 channels per thread
-// (C, strides and channel offsets are multiples of 8).
-__global__ void k_pool_bwd(PoolGradArgs a) {
-  const long n = (long)a.N * a.H * a.W * a.C;   // H, W of the input
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int c = (int)(i % a.C);
-    const long q = i / a.C;
-    const int x = (int)(q % a.W), y = (int)((q / a.W) % a.H);
-    const long nn = q / ((long)a.W * a.H);
-    const float v = 0.25f * a.dout[((nn * (a.H / 2) + y / 2) * (a.W / 2) + x / 2) * a.ldo + a.co0 + c];
-    float* d = a.din + q * a.ldi + a.ci0 + c;
-    *d = a.accumulate ? *d + v : v;
-  }
-}
-
 // nearest 2x upsample (bf16): out[2y+u][2x+v] = in[y][x]; 8 channels per thread
 __global__ void k_up_fwd(PoolArgs a) {
   const int C8 = a.C / 8;
@@ -877,31 +916,6 @@ __global__ void k_up_fwd(PoolArgs a) {
     const long nn = q / ((long)(2 * a.W) * (2 * a.H));
     *reinterpret_cast<uint4*>(a.out + q * a.ldo + a.co0 + c) =
         *reinterpret_cast<const uint4*>(a.in + ((nn * a.H + y / 2) * a.W + x / 2) * a.ldi + a.ci0 + c);
-  }
-}
-
-// gradient of the upsample: dIn[y][x] = sum of the 2x2 dOut block (fp32)
-__global__ void k_up_bwd(PoolGradArgs a) {
-  const long n = (long)a.N * a.H * a.W * a.C;   // H, W of the (small) input
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int c = (int)(i % a.C);
-    const long q = i / a.C;
-    const int x = (int)(q % a.W), y = (int)((q / a.W) % a.H);
-    const long nn = q / ((long)a.W * a.H);
-    const long b = ((nn * 2 * a.H + 2 * y) * 2 * a.W + 2 * x) * a.ldo + a.co0 + c;
-    const float v = a.dout[b] + a.dout[b + a.ldo] + a.dout[b + 2L * a.W * a.ldo] + a.dout[b + 2L * a.W * a.ldo + a.ldo];
-    float* d = a.din + q * a.ldi + a.ci0 + c;
-    *d = a.accumulate ? *d + v : v;
-  }
-}
-
-// dIn *= (act > 0) in place (fp32 gradient, bf16 activation)
-__global__ void k_relu_mask(float* g, int ldg, int cg0, const uint16_t* act, int lda, int ca0, long P, int C) {
-  const long n = P * C;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const long p = i / C;
-    const int c = (int)(i % C);
-    if (!(bf2f(act[p * lda + ca0 + c]) > 0.f)) g[p * ldg + cg0 + c] = 0.f;
   }
 }
 
@@ -1063,15 +1077,16 @@ __global__ void k_residual_add(const float* m, const float* y, const float* scal
 
 static int blocks_for(long n, int per = 256) { return (int)std::min<long>((n + per - 1) / per, 65536); }
 
-// Rows per wave of the 32-channel convolutions with BF16 input (tiles of
-// 4 kRows32 x 16 pixels); the others use 4 (their registers are full).
-constexpr int kRows32 = 8;
+// Blocks of a convolution's tiles of 4 R x 16 pixels and COB output channels.
+static long conv_blocks(int N, int H, int W, int Cout, int COB, int R) {
+  return (long)N * ((H + 4 * R - 1) / (4 * R)) * ((W + kTile - 1) / kTile) * ((Cout + COB - 1) / COB);
+}
 
 template <typename TX, typename TY, int COB, int R, bool FIRST = false>
 void launch_conv_tiles(const ConvArgs<TX, TY>& a, int cus, hipStream_t st) {
   // LDS per block: the staged halo tile and one chunk's weights
   constexpr long lds = ((4L * R + 2) * kPitch + 9L * COB) * kLdsRow * 2 + (FIRST ? ((4L * R + 4) * (kHalo + 2) + 1) * 8 : 0);
-  constexpr long per_cu = std::min<long>(COB == 32 && R == 4 ? 3 : 2, (160L * 1024) / lds);
+  constexpr long per_cu = std::min<long>(COB == 32 && R <= 4 ? 3 : 2, (160L * 1024) / lds);
   const long tiles = (long)a.N * ((a.H + 4 * R - 1) / (4 * R)) * ((a.W + kTile - 1) / kTile);
   const int cb = (a.Cout + COB - 1) / COB;
   const long gx = std::max<long>(1, std::min<long>(tiles, per_cu * cus / cb));
@@ -1082,12 +1097,17 @@ template <typename TX, typename TY>
 hipError_t launch_conv(const ConvArgs<TX, TY>& a, hipStream_t st) {
   if (a.taps != 9 && a.taps != 1) return hipErrorInvalidValue;
   // the fused head needs all 32 output channels in one block's BF16 epilogue
-  if (a.head_out && (sizeof(TY) != 2 || a.Cout != 32 || a.mask || a.accumulate || a.pool || a.ldy % 8 ||
+  if (a.head_out && (sizeof(TY) != 2 || a.Cout != 32 || a.mask || a.pool || a.ldy % 8 ||
                      a.cy0 % 8 || !a.head_w || !a.head_b))
     return hipErrorInvalidValue;
-  // BF16 output is plain (no mask, no accumulation) and stored 8 channels at
-  // a time, as is its optional pool; FP32 output has no pool
-  if (sizeof(TY) == 2 && (a.mask || a.accumulate || a.Cout % 8 || a.ldy % 8 || a.cy0 % 8)) return hipErrorInvalidValue;
+  // BF16 output is plain (no mask) and stored 8 channels at a time, as is its
+  // optional pool; FP32 output has no bias, ReLU or pool
+  if (sizeof(TY) == 2 && (a.mask || a.usum || a.pgrad || a.Cout % 8 || a.ldy % 8 || a.cy0 % 8)) return hipErrorInvalidValue;
+  if (sizeof(TY) == 4 &&
+      (a.bias || a.relu || a.Cout % 8 || a.ldy % 4 || a.cy0 % 4 || (a.mask && (a.ldm % 8 || a.cm0 % 8)) ||
+       (a.usum ? a.Cus % 64 || a.Cus < 1 || a.ldus % 4 || a.H % 2 || a.W % 2 || a.pgrad : a.Cus) ||
+       (a.pgrad && (!a.pmask || a.ldpg % 4 || a.ldpm % 8 || a.cpm0 % 8))))
+    return hipErrorInvalidValue;
   if (a.pool && (sizeof(TY) != 2 || a.ldp % 8 || a.cp0 % 8)) return hipErrorInvalidValue;
   // the input is staged in whole 32-channel chunks, each from x or from up;
   // one image's bytes are addressed by 32-bit buffer offsets
@@ -1108,13 +1128,29 @@ hipError_t launch_conv(const ConvArgs<TX, TY>& a, hipStream_t st) {
     if (sizeof(TX) != 2 || sizeof(TY) != 2 || a.Cin != 32 || a.Cout != 32 || a.taps != 9 || a.up || !a.w1 ||
         !a.b1 || a.w1_cin < 1 || (long)a.N * a.H * a.W * 4 >= (1L << 31))
       return hipErrorInvalidValue;
-    if constexpr (sizeof(TX) == 2 && sizeof(TY) == 2) launch_conv_tiles<TX, TY, 32, kRows32, true>(a, cus, st);
-  } else if (a.Cout <= 32 || (sizeof(TX) == 2 && a.Cin >= 128)) {
-    // (BF16 layers with 4 or more input chunks: measured faster on 32-channel
-    // 32 x 16 tiles than on 64-channel 16 x 16 ones)
-    launch_conv_tiles<TX, TY, 32, sizeof(TX) == 2 ? kRows32 : 4>(a, cus, st);
-  } else {
+    if constexpr (sizeof(TX) == 2 && sizeof(TY) == 2) launch_conv_tiles<TX, TY, 32, 8, true>(a, cus, st);
+    return hipGetLastError();
+  }
+  // Tile shape.  Large problems: 64 channels x 16 x 16 pixels, or 32 channels x
+  // 32 x 16 (BF16 input) for 32 output channels and from 4 input chunks on
+  // (measured faster).  Where those blocks leave CUs idle, smaller ones: the
+  // shape with the smallest blocks per CU x (MFMA cycles of a chunk + its
+  // staging, in the same unit).  16 images of 128^2: the forward pass's
+  // convolutions 250 -> 215 us, the input gradients' 670 -> 320 us (with the
+  // weights' prefetch and without the passes that their epilogue took over,
+  // 153 us).
+  const bool wide = a.Cout > 32 && !(sizeof(TX) == 2 && a.Cin >= 128);
+  auto cost = [&](int COB, int R, long chunk) { return (conv_blocks(a.N, a.H, a.W, a.Cout, COB, R) + cus - 1) / cus * chunk; };
+  const long big = wide ? cost(64, 4, 3000) : sizeof(TX) == 2 ? cost(32, 8, 3000) : cost(32, 4, 1650);
+  const long mid = cost(32, 4, 1650), small = cost(32, 2, 1000);
+  if (small < mid && small < big) {
+    launch_conv_tiles<TX, TY, 32, 2>(a, cus, st);
+  } else if (mid < big || (!wide && sizeof(TX) != 2)) {
+    launch_conv_tiles<TX, TY, 32, 4>(a, cus, st);
+  } else if (wide) {
     launch_conv_tiles<TX, TY, 64, 4>(a, cus, st);
+  } else {
+    if constexpr (sizeof(TX) == 2) launch_conv_tiles<TX, TY, 32, 8>(a, cus, st);
   }
   return hipGetLastError();
 }
@@ -1200,21 +1236,8 @@ hipError_t launch_grad_reduce(const ReduceGroup& r, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_pool_bwd(const PoolGradArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL(k_pool_bwd, dim3(blocks_for((long)a.N * a.H * a.W * a.C)), dim3(256), 0, st, a);
-  return hipGetLastError();
-}
 hipError_t launch_up_fwd(const PoolArgs& a, hipStream_t st) {
   hipLaunchKernelGGL(k_up_fwd, dim3(blocks_for((long)a.N * a.H * a.W * a.C / 2)), dim3(256), 0, st, a);
-  return hipGetLastError();
-}
-hipError_t launch_up_bwd(const PoolGradArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL(k_up_bwd, dim3(blocks_for((long)a.N * a.H * a.W * a.C)), dim3(256), 0, st, a);
-  return hipGetLastError();
-}
-hipError_t launch_relu_mask(float* g, int ldg, int cg0, const uint16_t* act, int lda, int ca0, long P, int C,
-                            hipStream_t st) {
-  hipLaunchKernelGGL(k_relu_mask, dim3(blocks_for(P * C)), dim3(256), 0, st, g, ldg, cg0, act, lda, ca0, P, C);
   return hipGetLastError();
 }
 hipError_t launch_head_fwd(const uint16_t* x, int ldx, const float* w, const float* b, int C, long P, float* out,
