@@ -45,18 +45,19 @@ __host__ __device__ constexpr int col_lds() {
 }
 
 // Buffer over the N0 grid rows of slice s, and the byte offset in it of grid
-// row x (x FFT order; image row X = x + N0/2 mod NC) and column y: past the
-// buffer where the row is padding, so that its load gives 0 and its store is
-// dropped.  32-bit offsets from one scalar base (the rows of a slice are at
-// most 16 MiB) keep the kernels' addresses in few registers.
+// row x = t + c (x FFT order, thread t < NC/16, slot constant c outside [NC/4,
+// 3NC/4); image row X = x + N0/2 mod NC) and column y: past the buffer where the
+// row is padding, so that its load gives 0 and its store is dropped.  32-bit
+// offsets from one scalar base (the rows of a slice are at most 16 MiB) keep
+// the kernels' addresses in few registers; the slots' offsets differ by scalars.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t slice_rows(const float2* p, const ColArgs& a, int s) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float2*>(p + (size_t)s * a.N0 * a.n1), (short)0,
                                            a.N0 * a.n1 * (int)sizeof(float2), 0x00020000);
 }
 template <int NC>
-__device__ __forceinline__ unsigned row_offset(const ColArgs& a, int x, int y) {
-  const int X = (x + (a.N0 >> 1)) & (NC - 1);
-  return X < a.N0 ? (unsigned)(X * a.n1 + y) * 8u : 0x80000000u;
+__device__ __forceinline__ unsigned row_offset(const ColArgs& a, int t, int c, int y) {
+  const int X0 = t + (a.N0 >> 1), d = c < NC / 2 ? c : c - NC;
+  return (unsigned)(X0 + d) < (unsigned)a.N0 ? (unsigned)((X0 * a.n1 + y) * 8 + d * a.n1 * 8) : 0x80000000u;
 }
 
 // x FFT of column c = tid % C of slice s: the first pass takes its 16 inputs
@@ -75,7 +76,7 @@ __device__ __forceinline__ void col_fft_fwd(float2 (&v)[16], const ColArgs& a, f
 #pragma unroll
   for (int j = 0; j < 8; j++)
     g[j] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
-                                          rs, row_offset<NC>(a, in_index<NC>(t, j < 4 ? j : j + 8), y0 + c), 0, 0));
+                                          rs, row_offset<NC>(a, t, (j < 4 ? j : j + 8) * (NC / 16), y0 + c), 0, 0));
   // the twiddles (first used after the first pass) are requested after
   // the grid rows, so that the first pass waits for the rows only
   FftTwiddles T;

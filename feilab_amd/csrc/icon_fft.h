@@ -124,19 +124,47 @@ template <int ES, int PSH = 0, int PN = 0>
 struct Lay {
   static constexpr int kES = ES;
   __host__ __device__ static constexpr int at(int i) { return i * ES + (PN ? (i >> PSH) * PN : 0); }
+  // at(base + c) for a constant c: one address and constant offsets, where the
+  // two low parts do not carry into a further padding (holds for every access
+  // of the passes, split_ok below).  The compiler cannot know that and computed
+  // each padded address by itself: 300 of 1800 vector instructions of the
+  // solve's column kernel at 1024 points, which they bound.
+  __host__ __device__ static constexpr int at(int base, int c) { return at(base) + at(c); }
   // float2 needed for a line of n elements
   __host__ __device__ static constexpr int size(int n) { return at(n - 1) + 1; }
 };
+
+// Whether L::at(base, c) is L::at(base + c) for all accesses of the transform
+// of size N: a pass with radix RP loads from base t < N/16 at c = q N/16 + r
+// N/RP; the stores (radix 16) are to base (j - k) 16 + k, k = j mod NS, at c =
+// r NS.
+template <int N, typename L, int NS = 1>
+__host__ __device__ constexpr bool split_ok() {
+  constexpr int T = N / 16, RP = (N / NS) >= 16 ? 16 : N / NS, B = 16 / RP;
+  for (int t = 0; t < T; t++) {
+    for (int q = 0; q < B; q++)
+      for (int r = 0; r < RP; r++)
+        if (L::at(t, q * T + r * (N / RP)) != L::at(t + q * T + r * (N / RP))) return false;
+    if (NS * RP < N) {
+      const int k = t & (NS - 1), base = (t - k) * RP + k;
+      for (int r = 0; r < RP; r++)
+        if (B != 1 || L::at(base, r * NS) != L::at(base + r * NS)) return false;
+    }
+  }
+  if constexpr (NS * RP < N) return split_ok<N, L, NS * RP>();
+  else return true;
+}
 
 // Loads a pass's inputs from LDS (layout L).
 template <int N, int RP, typename L>
 __device__ __forceinline__ void pass_load(float2 (&v)[16], const float2* lds, int t) {
   constexpr int T = N / 16;
   constexpr int B = 16 / RP;
+  static_assert(split_ok<N, L>(), "constant offsets");
 #pragma unroll
   for (int q = 0; q < B; q++)
 #pragma unroll
-    for (int r = 0; r < RP; r++) v[q * RP + r] = lds[L::at(t + q * T + r * (N / RP))];
+    for (int r = 0; r < RP; r++) v[q * RP + r] = lds[L::at(t, q * T + r * (N / RP))];
 }
 
 // Twiddles of the passes after the first (at most two for N <= 4096), per
@@ -205,7 +233,7 @@ __device__ __forceinline__ void pass_store(const float2 (&v)[16], float2* lds, i
     const int k = j & (NS - 1);
     const int base = (j - k) * RP + k;
 #pragma unroll
-    for (int r = 0; r < RP; r++) lds[L::at(base + r * NS)] = v[q * RP + r];
+    for (int r = 0; r < RP; r++) lds[L::at(base, r * NS)] = v[q * RP + r];
   }
 }
 
@@ -351,6 +379,13 @@ __host__ __device__ constexpr bool out_slot_cropped(int i) {
   return lo >= N / 4 && lo + T <= 3 * N / 4;
 }
 
+// out_index less the thread index.
+template <int N>
+__host__ __device__ constexpr int out_offset(int i) {
+  constexpr int RL = last_radix<N>();
+  return (i / RL) * (N / 16) + (i % RL) * (N / RL);
+}
+
 // Element index held in input slot r of thread t.
 template <int N>
 __device__ __forceinline__ int in_index(int t, int r) {
@@ -371,7 +406,7 @@ __device__ __forceinline__ void fft_lds(float2* lds, int t, const float2* __rest
   // the last pass_load is followed by a barrier inside fft_from, so the
   // line can be overwritten now
 #pragma unroll
-  for (int i = 0; i < 16; i++) lds[L::at(out_index<N>(t, i))] = v[i];
+  for (int i = 0; i < 16; i++) lds[L::at(t, out_offset<N>(i))] = v[i];
 }
 
 // FP64 transform of a line, registers (input order) -> registers (output
@@ -404,7 +439,7 @@ __device__ __forceinline__ void fft64(double2 (&v)[16], double* lds, int t, cons
       for (int q = 0; q < B; q++) {
         const int j = t + q * T, k = j & (NS - 1), base = (j - k) * RP + k;
 #pragma unroll
-        for (int r = 0; r < RP; r++) lds[L::at(base + r * NS)] = c ? im[q * RP + r] : v[q * RP + r].x;
+        for (int r = 0; r < RP; r++) lds[L::at(base, r * NS)] = c ? im[q * RP + r] : v[q * RP + r].x;
       }
       if (c == 0) {
 #pragma unroll
@@ -415,7 +450,7 @@ __device__ __forceinline__ void fft64(double2 (&v)[16], double* lds, int t, cons
       for (int q = 0; q < BN; q++)
 #pragma unroll
         for (int r = 0; r < RN; r++) {
-          const double x = lds[L::at(t + q * T + r * (N / RN))];
+          const double x = lds[L::at(t, q * T + r * (N / RN))];
           if (c) v[q * RN + r].y = x;
           else v[q * RN + r].x = x;
         }

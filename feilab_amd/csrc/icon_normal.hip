@@ -86,7 +86,7 @@ __device__ __forceinline__ void col_normal_body(const ColArgs& a, int bid) {
   for (int i = 0; i < 16; i++) {
     if (out_slot_cropped<NC>(i)) continue;   // padding rows, as N0 <= NC/2
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, u[i]), rs,
-                                          row_offset<NC>(a, out_index<NC>(t, i), y0 + c), 0, 0);
+                                          row_offset<NC>(a, t, out_offset<NC>(i), y0 + c), 0, 0);
   }
 }
 
@@ -178,13 +178,21 @@ __global__ __launch_bounds__(C * (NC / 16), 4) void k_col_energy_multi(const Col
 // in v (FFT output order): Z(y) and Z(NR - y) give row 0 as (Z + conj Z')/2 and
 // row 1 as (Z - conj Z')/2i.  A thread's lower-half elements are its own; their
 // mirrors come from the team through LDS.  Columns 0..NR/2 + 7, the last 7 zero.
+// LDS address of the mirror NR - y of element y = t + k T.
+template <int NR>
+__device__ __forceinline__ int mirror_at(int t, int k) {
+  constexpr int T = NR / 16;
+  if constexpr (T % 32 == 0) return RowLay::at(NR - t) - RowLay::at(k * T);   // whole paddings apart
+  else return RowLay::at(NR - t - k * T);
+}
+
 template <int NR>
 __device__ __forceinline__ void half_store(const float2 (&v)[16], float2* L, int t, float2* o0, float2* o1,
                                            bool valid) {
   constexpr int T = NR / 16, RL = last_radix<NR>();
 #pragma unroll
   for (int i = 0; i < 16; i++)
-    if (i / RL + (i % RL) * (16 / RL) >= 8) L[RowLay::at(out_index<NR>(t, i))] = v[i];
+    if (i / RL + (i % RL) * (16 / RL) >= 8) L[RowLay::at(t, out_offset<NR>(i))] = v[i];
   __syncthreads();
   if (!valid) return;
 #pragma unroll
@@ -193,7 +201,7 @@ __device__ __forceinline__ void half_store(const float2 (&v)[16], float2* L, int
     if (k < 8) {
       const int y = t + k * T;
       float2 z = v[i];
-      if (y != 0) z = L[RowLay::at(NR - y)];
+      if (y != 0) z = L[mirror_at<NR>(t, k)];
       o0[y] = make_float2(0.5f * (v[i].x + z.x), 0.5f * (v[i].y - z.y));
       o1[y] = make_float2(0.5f * (v[i].y + z.y), 0.5f * (z.x - v[i].x));
     } else if (k == 8) {
@@ -316,13 +324,13 @@ __device__ __forceinline__ void row_grad_half_body(const RowAdjArgs& a, int bid)
 #pragma unroll
     for (int r = 0; r < 8; r++) {
       v[r] = make_float2(p[r].x - q[r].y, p[r].y + q[r].x);
-      L[RowLay::at(t + r * T)] = make_float2(p[r].x + q[r].y, q[r].x - p[r].y);
+      L[RowLay::at(t, r * T)] = make_float2(p[r].x + q[r].y, q[r].x - p[r].y);
     }
     __syncthreads();
 #pragma unroll
     for (int r = 8; r < 16; r++) {
       const int y = (16 - r) * T - t;   // NR - (t + r T), in (0, NR/2]
-      v[r] = y == NR / 2 ? make_float2(ph.x - qh.y, ph.y + qh.x) : L[RowLay::at(y)];
+      v[r] = y == NR / 2 ? make_float2(ph.x - qh.y, ph.y + qh.x) : L[mirror_at<NR>(t, r)];
     }
     __syncthreads();
   }
@@ -440,13 +448,13 @@ __device__ __forceinline__ void row_fwd64_body(const RefArgs& a, int bid) {
     for (int c = 0; c < 2; c++) {
 #pragma unroll
       for (int i = 0; i < 16; i++)
-        if (i / RL + (i % RL) * (16 / RL) >= 8) lds[RowLay::at(out_index<NR>(t, i))] = c ? v[i].y : v[i].x;
+        if (i / RL + (i % RL) * (16 / RL) >= 8) lds[RowLay::at(t, out_offset<NR>(i))] = c ? v[i].y : v[i].x;
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         const int k = i / RL + (i % RL) * (16 / RL), y = t + k * T;
         if (k >= 8) continue;
-        const double z = y ? lds[RowLay::at(NR - y)] : (c ? v[i].y : v[i].x);
+        const double z = y ? lds[mirror_at<NR>(t, k)] : (c ? v[i].y : v[i].x);
         if (c == 0) {
           zx[i] = z;
         } else {
