@@ -329,6 +329,7 @@ int enqueue_solve(icon_plan* p, int S, const float* sino, float* m, const float*
   ColArgs ca = normal_args(p, S, resid != nullptr);
   const ColArgs ce = energy_args(p, S), c64 = normal64_args(p, S, resid != nullptr);
   RowAdjArgs ra = grad_args(p, S);
+  split_dense(p, S, ca, ra);
   RefArgs rr = ref_args(p, S, m);
   rr.data_type = o.data_type; rr.thr = o.threshold;
   FinishArgs fa = finish_args(p, S);
@@ -420,6 +421,16 @@ int build_normal(icon_plan* p) {
   double chol[kInterpTaps * kInterpTaps];
   interp_factor(chol);
   int rc;
+  // a round of a tile's entries: its block's threads
+  const int round = kNormalC * (g.n0 / 16);
+  std::vector<int> parts;
+  std::vector<int2> xt;
+  for (size_t t = 0; t + 1 < nb.off.size(); t++) {
+    parts.push_back(std::max(1, std::min(8, (nb.off[t + 1] - nb.off[t] + round - 1) / round)));
+    for (int k = 1; k < parts.back(); k++) xt.push_back(make_int2((int)t, k));
+  }
+  p->nd_nx = (int)xt.size();
+  if (p->nd_nx && ((rc = upload(p, &p->d_nd_parts, parts)) || (rc = upload(p, &p->d_nd_xt, xt)))) return rc;
   if ((rc = upload(p, &p->d_nd_off, nb.off)) || (rc = upload(p, &p->d_nd_ent, nb.ent)) ||
       (rc = upload(p, &p->d_nd_nslot, nb.nslot)) || (rc = dalloc(p, &p->d_nd_px, E * kInterpTaps)) ||
       (rc = dalloc(p, &p->d_nd_py, E * kNormalC)) || (rc = dalloc(p, &p->d_spec, (size_t)g.n0 * p->ncol)) ||
@@ -575,6 +586,25 @@ RowAdjArgs icon::grad_args(const icon_plan* p, int S) {
   a.ahwb_re = reinterpret_cast<const float*>(p->d_ahwb); a.grad = p->d_grad; a.rowpart = p->d_rowpart;
   a.fwd_out = p->d_tmp;
   return a;
+}
+
+// Few slices leave CUs idle while the tiles around ky = 0, which all tilt lines
+// cross, interpolate 6 and more rounds of entries (one 256^2 slice, 61 tilts:
+// 22 us instead of 10 for a tile without): their entries are shared among
+// further blocks, which transform the tile again.  The grid goes to the other
+// half of d_tmp, as those read the rows that the tile's own block would
+// overwrite.  Where all blocks are not resident at once they would cost more
+// than the wait.
+void icon::split_dense(const icon_plan* p, int S, ColArgs& ca, RowAdjArgs& ra) {
+  const Geometry& g = p->g;
+  const long resident = (long)p->cus * std::max(1, 2048 / g.n0);
+  if (ca.ent_off != p->d_nd_off || !p->nd_nx || !p->refreshes() || (long)S * (p->ncol / kNormalC + p->nd_nx) > resident)
+    return;
+  ca.parts = p->d_nd_parts;
+  ca.xt = p->d_nd_xt;
+  ca.nx = p->nd_nx;
+  ca.out = p->d_tmp + (size_t)p->S_max * g.N0 * g.n1;
+  ra.in = ca.out;
 }
 
 FinishArgs icon::finish_args(const icon_plan* p, int S) {
@@ -758,6 +788,7 @@ int plan_create(icon_plan** out, int device, int nx, int thickness, int nz, cons
   HIPCHK(hipSetDevice(device));
   auto* p = new icon_plan();
   p->device = device;
+  (void)hipDeviceGetAttribute(&p->cus, hipDeviceAttributeMultiprocessorCount, device);
   std::string err;
   if (!build_geometry(p->g, nx, thickness > 0 ? thickness : nx, nz, tilt_deg, &err, cv, window, false)) {
     delete p;
@@ -837,7 +868,7 @@ int icon_plan_destroy(icon_plan* p) {
   drop_graph(p);
   void* ptrs[] = {p->d_nodes, p->d_ck1, p->d_w, p->d_phi1, p->d_i10, p->d_fw,
                   p->d_b, p->d_part, p->d_ahwb, p->d_grad, p->d_tmp, p->d_frep, p->d_rowpart,
-                  p->d_bnorm, p->d_alpha, p->d_spec, p->d_nd_off, p->d_nd_ent, p->d_nd_nslot, p->d_nd_px, p->d_nd_py,
+                  p->d_bnorm, p->d_alpha, p->d_spec, p->d_nd_off, p->d_nd_ent, p->d_nd_parts, p->d_nd_xt, p->d_nd_nslot, p->d_nd_px, p->d_nd_py,
                   p->d_epart, p->d_nq_off, p->d_nq_ent, p->d_nq_entr, p->d_nq_px, p->d_nq_py, p->d_nq_nslot,
                   p->d_rpart, p->d_gram, p->d_base, p->d_mref, p->d_beff};
   for (void* q : ptrs)
@@ -1047,8 +1078,10 @@ int icon_time_kernel(icon_plan* p, int kernel, int S, int reps, double* avg_ms) 
   rf.rows = S * g.N0; rf.N0 = g.N0; rf.N1 = g.N1; rf.cplx = 0; rf.update = 2; rf.data_type = 1;
   rf.m = reinterpret_cast<float*>(p->d_ahwb); rf.grad = p->d_grad; rf.alpha = p->d_alpha;
   rf.tw = p->d_tw1; rf.out = p->d_tmp;
-  const ColArgs cn = normal_args(p, S, true), ce = energy_args(p, S);
-  const RowAdjArgs ra = grad_args(p, S);
+  ColArgs cn = normal_args(p, S, true);
+  const ColArgs ce = energy_args(p, S);
+  RowAdjArgs ra = grad_args(p, S);
+  split_dense(p, S, cn, ra);
   // (the residuals of these stale values go to the bnorm buffer, rewritten by the next solve's set-up)
   FinishArgs fr = finish_args(p, S);
   fr.resid = p->d_bnorm; fr.resid_stride = 1; fr.alpha = p->d_alpha;

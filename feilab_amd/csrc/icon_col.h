@@ -88,9 +88,11 @@ __device__ __forceinline__ void col_fft_fwd(float2 (&v)[16], const ColArgs& a, f
 }
 
 // Interpolation partials of tile blk of slice s, whose x-transformed grid
-// columns lie in the LDS tile (row stride col_stride<NC, C>()).
+// columns lie in the LDS tile (row stride col_stride<NC, C>()); of its entries
+// those of share `part` of `parts`.
 template <int NC, int C, int K>
-__device__ __forceinline__ void interp_tile(const ColArgs& a, const float2* tile, int blk, int s) {
+__device__ __forceinline__ void interp_tile(const ColArgs& a, const float2* tile, int blk, int s, int part = 0,
+                                            int parts = 1) {
   constexpr int NT = C * (NC / 16);
   constexpr int LS = col_stride<NC, C>();
   const int tid = threadIdx.x;
@@ -98,7 +100,7 @@ __device__ __forceinline__ void interp_tile(const ColArgs& a, const float2* tile
   // the entry's record (first x-tap, 14 x-taps, C y-taps) comes in with
   // vector loads and the thread sums its 14 x C cells from the LDS tile
   const int e0 = a.ent_off[blk], e1 = a.ent_off[blk + 1], ne = e1 - e0;
-  for (int e = e0 + tid; e < e1; e += NT) {
+  for (int e = e0 + part * NT + tid; e < e1; e += parts * NT) {
     const int4 en = a.fent[e];
     float px[K];
     const float2* pxv = reinterpret_cast<const float2*>(a.fent_px + (size_t)e0 * K) + (e - e0);
@@ -158,19 +160,31 @@ __device__ __forceinline__ void interp_tile(const ColArgs& a, const float2* tile
   }
 }
 
-// FP64 sum over a block of 1024 threads, in a fixed order.
-__device__ __forceinline__ double block_sum_1024(double v, double* red) {
+// FP64 sums of N values over a block of 1024 threads, in a fixed order: by lane
+// halves within each wavefront, then the wavefronts in order.  red: 16 N doubles.
+template <int N>
+__device__ __forceinline__ void block_sums_1024(double (&v)[N], double* red) {
   const int tid = threadIdx.x;
-  red[tid] = v;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+#pragma unroll
+    for (int h = 32; h > 0; h >>= 1) v[k] += __shfl_down(v[k], h);
+    if ((tid & 63) == 0) red[16 * k + (tid >> 6)] = v[k];
+  }
   __syncthreads();
 #pragma unroll
-  for (int h = 512; h > 0; h >>= 1) {
-    if (tid < h) red[tid] += red[tid + h];
-    __syncthreads();
+  for (int k = 0; k < N; k++) {
+    double r = red[16 * k];
+#pragma unroll
+    for (int w = 1; w < 16; w++) r += red[16 * k + w];
+    v[k] = r;
   }
-  const double r = red[0];
   __syncthreads();
-  return r;
+}
+__device__ __forceinline__ double block_sum_1024(double v, double* red) {
+  double x[1] = {v};
+  block_sums_1024(x, red);
+  return x[0];
 }
 
 // Value of node j: its partials of up to `slots` column tiles, in slot order.

@@ -69,6 +69,12 @@ struct ColArgs {
   const double2* w64;      // col_normal64: exp(-2 pi i q / n0)
   int slots;               // partials per node in part
   int nyq;                 // half grid: its column n1/2; otherwise 0
+  // col_normal, few slices: shares of the dense tiles' entries in blocks of
+  // their own (out then is not in): shares per tile, and (tile, share > 0) of
+  // the nx further blocks per slice
+  const int* parts;
+  const int2* xt;
+  int nx;
 };
 
 struct CombineArgs {

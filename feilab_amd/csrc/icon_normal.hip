@@ -47,8 +47,17 @@ __device__ __forceinline__ void col_normal_body(const ColArgs& a, int bid) {
   extern __shared__ __align__(16) float2 tile[];   // col_lds<NC, C>()
   // tile-major order, as the transforms' column kernels: blocks in flight
   // together share the tile's spectrum and interpolation records in L2
-  const int blk = bid / a.S;
+  int blk = bid / a.S, part = 0, parts = 1;
   const int s = bid % a.S;
+  if (a.parts) {
+    // blocks past the tiles: a further share of a dense tile's entries
+    if (blk >= a.n1 / C) {
+      const int2 x = a.xt[blk - a.n1 / C];
+      blk = x.x;
+      part = x.y;
+    }
+    parts = a.parts[blk];
+  }
   const int y0 = blk * C;
   const int c = threadIdx.x % C, t = threadIdx.x / C;
   float2 v[16];
@@ -61,7 +70,8 @@ __device__ __forceinline__ void col_normal_body(const ColArgs& a, int bid) {
 #pragma unroll
     for (int i = 0; i < 16; i++) tile[out_index<NC>(t, i) * LS + c] = v[i];
     __syncthreads();
-    interp_tile<NC, C, K>(a, tile, blk, s);
+    interp_tile<NC, C, K>(a, tile, blk, s, part, parts);
+    if (part) return;
     // the column back from the tile rather than held through the interpolation
 #pragma unroll
     for (int r = 0; r < 16; r++) u[r] = tile[in_index<NC>(t, r) * LS + c];
@@ -630,21 +640,23 @@ __device__ __forceinline__ int node_of(const FinishArgs& a, int r, int* jm) {
 // R = sqrt(sum w |A m - b|^2 / sum w |b|^2) and the values at the omit tilt.
 // One block per (slice, role); FP64 sums in a fixed order.
 __device__ __forceinline__ void finish_body(const FinishArgs& a, int s, int role) {
-  __shared__ double red[1024];
+  __shared__ double red[32];
   __shared__ double z[4 * kMaxUnpaired];
   const int tid = threadIdx.x;
   double acc = 0.0;
   const float2* P = a.part + (size_t)s * a.M * a.slots;
+  // One block per slice waits on its loads: each round issues those of several
+  // elements together (one 256^2 slice, 61 tilts: 12.5 -> 9.5 us;
+  // 256 slices of 512^2, 41 tilts: 48 -> 36 us)
   if (role == 0) {
-    for (int X = tid; X < a.nrow; X += 1024) acc += a.rowpart[(size_t)s * a.nrow + X];
-    double rtr = block_sum_1024(acc, red);
-    double tot = block_sum_1024(tid < a.nblk ? a.epart[(size_t)s * a.nblk + tid] : 0.0, red);
+    double sums[2] = {0.0, tid < a.nblk ? a.epart[(size_t)s * a.nblk + tid] : 0.0};
+    for (int X = tid; X < a.nrow; X += 1024) sums[0] += a.rowpart[(size_t)s * a.nrow + X];
     if (a.nq) {
       // the gradient's imaginary part I = sum_a zd_a e_a over the waves e =
       // (cos, sin)(2 pi v_t x): |I|^2 = zd G zd, <I, A^H W A I> = zd H zd and
       // 2 <I, Im(A^H W A) Re rhat> = 2 zd G zr, with the coefficients z of the
       // residual d_t (zd) and of (A Re rhat)_t (zr)
-      const int nf = 2 * a.nq;
+      const int nf = 2 * a.nq, nn = nf * nf;
       double *zd = z, *zr = z + nf;
       for (int t = tid; t < a.nq; t += 1024) {
         const int j = t * a.N0;
@@ -660,44 +672,80 @@ __device__ __forceinline__ void finish_body(const FinishArgs& a, int s, int role
         zr[a.nq + t] = w * (double)r.x;
       }
       __syncthreads();
-      double ii = 0.0, q = 0.0;
-      for (int e = tid; e < nf * nf; e += 1024) {
-        const int p = e / nf, c = e - p * nf;
-        const double g = a.gram[e], h = a.gram[nf * nf + e];
-        ii += zd[p] * g * zd[c];
-        q += zd[p] * (h * zd[c] + 2.0 * g * zr[c]);
+      constexpr int U = 8;
+      for (int e0 = tid; e0 < nn; e0 += U * 1024) {
+        float g[U], h[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int e = e0 + u * 1024;
+          g[u] = e < nn ? a.gram[e] : 0.f;
+          h[u] = e < nn ? a.gram[nn + e] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int e = min(e0 + u * 1024, nn - 1), p = e / nf, c = e - p * nf;
+          sums[0] += zd[p] * (double)g[u] * zd[c];
+          sums[1] += zd[p] * ((double)h[u] * zd[c] + 2.0 * (double)g[u] * zr[c]);
+        }
       }
-      rtr += block_sum_1024(ii, red);
-      tot += block_sum_1024(q, red);
     }
+    block_sums_1024(sums, red);
     if (tid == 0) {
-      const double al = tot != 0.0 ? rtr / tot : 0.0;
+      const double al = sums[1] != 0.0 ? sums[0] / sums[1] : 0.0;
       a.alpha[s] = al;
       if (a.alpha_trace) a.alpha_trace[(size_t)s * a.alpha_stride + a.alpha_index] = al;
     }
     return;
   }
-  for (int r = tid; r < a.M; r += 1024) {
-    int jm;
-    const int j = node_of(a, r, &jm);
-    const float2 f = node_value(P, a.nslot, r, a.slots);
-    if (a.resid) {
-      const float2 bj = a.b[(size_t)s * a.Mb + j];
-      const double dx = (double)f.x - (double)bj.x, dy = (double)f.y - (double)bj.y;
-      acc += (double)a.w[j] * (dx * dx + dy * dy);
-      if (a.beff) a.beff[(size_t)s * a.Mb + j] = make_float2((float)-dx, (float)-dy);
-      if (jm >= 0) {
-        const float2 bm = a.b[(size_t)s * a.Mb + jm];
-        const double ex = (double)f.x - (double)bm.x, ey = (double)f.y + (double)bm.y;
-        acc += (double)a.w[jm] * (ex * ex + ey * ey);
-        if (a.beff) a.beff[(size_t)s * a.Mb + jm] = make_float2((float)-ex, (float)ey);
+  constexpr int U = 4, SL = 4;   // rows a round; partials loaded together (a.slots of them at most)
+  for (int r0 = tid; r0 < a.M; r0 += U * 1024) {
+    float2 p[U][SL], b0[U], b1[U];
+    float w0[U], w1[U];
+    int j[U], jm[U], ns[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const bool in = r0 + u * 1024 < a.M;
+      const int r = in ? r0 + u * 1024 : r0;
+      j[u] = node_of(a, r, &jm[u]);
+      if (!in) j[u] = jm[u] = -1;
+      ns[u] = a.nslot[r];
+#pragma unroll
+      for (int q = 0; q < SL; q++) p[u][q] = P[(size_t)r * a.slots + min(q, a.slots - 1)];
+      const int k0 = max(j[u], 0), k1 = max(jm[u], 0);
+      w0[u] = a.w[k0];
+      w1[u] = a.w[k1];
+      if (a.resid) {
+        b0[u] = a.b[(size_t)s * a.Mb + k0];
+        b1[u] = a.b[(size_t)s * a.Mb + k1];
       }
     }
-    if (a.frep) {
-      const int i = j / a.N0;
-      if (i == a.iomit) {
-        a.frep[(size_t)s * a.N0 + (j - i * a.N0)] = f;
-        if (jm >= 0) a.frep[(size_t)s * a.N0 + (jm - i * a.N0)] = make_float2(f.x, -f.y);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (j[u] < 0) continue;
+      // as node_value: the partials in slot order
+      float2 f = p[u][0];
+#pragma unroll
+      for (int q = 1; q < SL; q++)
+        if (q < ns[u]) {
+          f.x += p[u][q].x;
+          f.y += p[u][q].y;
+        }
+      if (a.resid) {
+        const double dx = (double)f.x - (double)b0[u].x, dy = (double)f.y - (double)b0[u].y;
+        acc += (double)w0[u] * (dx * dx + dy * dy);
+        if (a.beff) a.beff[(size_t)s * a.Mb + j[u]] = make_float2((float)-dx, (float)-dy);
+        if (jm[u] >= 0) {
+          const double ex = (double)f.x - (double)b1[u].x, ey = (double)f.y + (double)b1[u].y;
+          acc += (double)w1[u] * (ex * ex + ey * ey);
+          if (a.beff) a.beff[(size_t)s * a.Mb + jm[u]] = make_float2((float)-ex, (float)ey);
+        }
+      }
+      if (a.frep) {
+        const int i = j[u] / a.N0;
+        if (i == a.iomit) {
+          a.frep[(size_t)s * a.N0 + (j[u] - i * a.N0)] = f;
+          if (jm[u] >= 0) a.frep[(size_t)s * a.N0 + (jm[u] - i * a.N0)] = make_float2(f.x, -f.y);
+        }
       }
     }
   }
@@ -1071,7 +1119,7 @@ hipError_t set_normal_attrs(int NC) {
   return hipGetLastError()
 
 hipError_t launch_col_normal(int NC, const ColArgs& a, hipStream_t st) {
-  LAUNCH_COL(k_col_normal, a.S * (a.n1 / kNormalC), a);
+  LAUNCH_COL(k_col_normal, a.S * (a.n1 / kNormalC + a.nx), a);
 }
 hipError_t launch_col_energy(int NC, const ColArgs& a, hipStream_t st) {
   LAUNCH_COL(k_col_energy, a.S * (a.n1 / kNormalC), a);

@@ -217,6 +217,10 @@ struct icon_plan {
   float* d_spec = nullptr;          // [ncol/8][n0][8] spectrum of A^H W A's kernel
   int* d_nd_off = nullptr;          // NodeBins and their records
   int4* d_nd_ent = nullptr;
+  int* d_nd_parts = nullptr;        // shares of a tile's entries, and the further ones (split_dense)
+  int2* d_nd_xt = nullptr;
+  int nd_nx = 0;
+  int cus = 256;                    // compute units of the device
   int8_t* d_nd_nslot = nullptr;
   float* d_nd_px = nullptr;
   float* d_nd_py = nullptr;
@@ -258,6 +262,7 @@ namespace icon {
 ColArgs normal_args(const icon_plan* p, int S, bool with_nodes);
 ColArgs energy_args(const icon_plan* p, int S);
 RowAdjArgs grad_args(const icon_plan* p, int S);
+void split_dense(const icon_plan* p, int S, ColArgs& ca, RowAdjArgs& ra);
 ColArgs normal64_args(const icon_plan* p, int S, bool with_nodes);
 RefArgs ref_args(const icon_plan* p, int S, float* m);
 RowFwdArgs rhat_row_args(const icon_plan* p, int S);
