@@ -135,10 +135,23 @@ int upload(icon_plan* p, T** ptr, const std::vector<T>& h) {
 
 void free_bins(DevBins& b) {
   for (void* q : {(void*)b.ck, (void*)b.off, (void*)b.order, (void*)b.xoff, (void*)b.of_node, (void*)b.ent,
-                  (void*)b.fent, (void*)b.px, (void*)b.py, (void*)b.fpx, (void*)b.fpy, (void*)b.nslot})
+                  (void*)b.fent, (void*)b.parts, (void*)b.xt, (void*)b.px, (void*)b.py, (void*)b.fpx, (void*)b.fpy, (void*)b.nslot})
     if (q) (void)hipFree(q);
   b = DevBins{};
 }
+
+// Shares of the tiles' entries, a round of the block's threads each (8 at most):
+// shares per tile, and (tile, share) of those past the first.
+void dense_shares(const std::vector<int>& off, int round, std::vector<int>& parts, std::vector<int2>& xt) {
+  for (size_t t = 0; t + 1 < off.size(); t++) {
+    parts.push_back(std::max(1, std::min(8, (off[t + 1] - off[t] + round - 1) / round)));
+    for (int k = 1; k < parts.back(); k++) xt.push_back(make_int2((int)t, k));
+  }
+}
+
+// Blocks of a column tile of C columns resident on the device at once: 1024
+// threads of up to 128 registers per CU.
+long resident_tiles(const icon_plan* p, int C) { return (long)p->cus * std::max(1, 16384 / (C * p->g.n0)); }
 
 // Bins of a Kaiser-Bessel window of K taps in tiles of C columns; records and
 // deapodisation are computed on the device.
@@ -152,6 +165,11 @@ int make_bins(icon_plan* p, DevBins& b, int C, int K) {
   kb_deapod(g.N0, g.sig0, b.beta0, K, c.data());
   kb_deapod(g.N1, g.sig1, b.beta1, K, c.data() + g.N0);
   int rc;
+  std::vector<int> parts;
+  std::vector<int2> xt;
+  dense_shares(b.h.off, C * (g.n0 / 16), parts, xt);
+  b.nx = (int)xt.size();
+  if (b.nx && ((rc = upload(p, &b.parts, parts)) || (rc = upload(p, &b.xt, xt)))) return rc;
   if ((rc = upload(p, &b.off, b.h.off)) || (rc = upload(p, &b.order, b.h.order)) || (rc = upload(p, &b.ent, b.h.ent)) ||
       (rc = upload(p, &b.fent, b.h.fent)) || (rc = upload(p, &b.nslot, b.h.nslot)) ||
       (rc = upload(p, &b.xoff, b.h.xoff)) || (rc = upload(p, &b.of_node, b.h.of_node)) ||
@@ -195,6 +213,13 @@ ColArgs window_args(icon_plan* p, const DevBins& b, int S) {
   a.split_min = split_min_entries(b.h); a.ent = b.ent; a.xoff = b.xoff; a.ent_px = b.px; a.ent_py = b.py;
   a.fent = b.fent; a.fent_px = b.fpx; a.fent_py = b.fpy; a.part = p->d_part; a.slots = kMaxSlot; a.fw = p->d_fw;
   zero_band(b.h, &a.zlo, &a.zhi);
+  // few slices: the dense tiles' entries shared among further blocks, as in
+  // split_dense (one 64^2 image, 21 tilts: 10.7 -> 4.7 us)
+  if (b.nx && (long)S * (g.n1 / b.h.C + b.nx) <= resident_tiles(p, b.h.C)) {
+    a.parts = b.parts;
+    a.xt = b.xt;
+    a.nx = b.nx;
+  }
   return a;
 }
 
@@ -421,20 +446,16 @@ int build_normal(icon_plan* p) {
   double chol[kInterpTaps * kInterpTaps];
   interp_factor(chol);
   int rc;
-  // a round of a tile's entries: its block's threads
-  const int round = kNormalC * (g.n0 / 16);
   std::vector<int> parts;
   std::vector<int2> xt;
-  for (size_t t = 0; t + 1 < nb.off.size(); t++) {
-    parts.push_back(std::max(1, std::min(8, (nb.off[t + 1] - nb.off[t] + round - 1) / round)));
-    for (int k = 1; k < parts.back(); k++) xt.push_back(make_int2((int)t, k));
-  }
+  dense_shares(nb.off, kNormalC * (g.n0 / 16), parts, xt);
   p->nd_nx = (int)xt.size();
   if (p->nd_nx && ((rc = upload(p, &p->d_nd_parts, parts)) || (rc = upload(p, &p->d_nd_xt, xt)))) return rc;
   if ((rc = upload(p, &p->d_nd_off, nb.off)) || (rc = upload(p, &p->d_nd_ent, nb.ent)) ||
       (rc = upload(p, &p->d_nd_nslot, nb.nslot)) || (rc = dalloc(p, &p->d_nd_px, E * kInterpTaps)) ||
       (rc = dalloc(p, &p->d_nd_py, E * kNormalC)) || (rc = dalloc(p, &p->d_spec, (size_t)g.n0 * p->ncol)) ||
-      (rc = dalloc(p, &p->d_epart, S * (p->ncol / kNormalC))) || (rc = upload(p, &p->d_nq_off, ub.off)))
+      (rc = dalloc(p, &p->d_epart, S * (p->ncol / kNormalC))) ||
+      (rc = dalloc(p, &p->d_rsum, S * kFinishGroups)) || (rc = dalloc(p, &p->d_rcnt, S)) || (rc = upload(p, &p->d_nq_off, ub.off)))
     return rc;
   if (p->half &&
       ((rc = upload(p, &p->d_nq_ent, ub.ent)) || (rc = upload(p, &p->d_nq_entr, entr)) ||
@@ -457,6 +478,7 @@ int build_normal(icon_plan* p) {
   hipStream_t st = p->stream;
   const int half = p->half ? g.N0 / 2 : 0;
   hipError_t e = hipMemcpy(d_chol, chol, sizeof(chol), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = launch_zero(reinterpret_cast<float*>(p->d_rcnt), S, st);
   if (e == hipSuccess)
     e = launch_interp_records(p->d_nd_ent, p->d_nd_off, nodes, (int)E, g.n0, g.n1, half, d_chol, p->d_nd_px,
                               p->d_nd_py, st);
@@ -597,8 +619,8 @@ RowAdjArgs icon::grad_args(const icon_plan* p, int S) {
 // than the wait.
 void icon::split_dense(const icon_plan* p, int S, ColArgs& ca, RowAdjArgs& ra) {
   const Geometry& g = p->g;
-  const long resident = (long)p->cus * std::max(1, 2048 / g.n0);
-  if (ca.ent_off != p->d_nd_off || !p->nd_nx || !p->refreshes() || (long)S * (p->ncol / kNormalC + p->nd_nx) > resident)
+  if (ca.ent_off != p->d_nd_off || !p->nd_nx || !p->refreshes() ||
+      (long)S * (p->ncol / kNormalC + p->nd_nx) > resident_tiles(p, kNormalC))
     return;
   ca.parts = p->d_nd_parts;
   ca.xt = p->d_nd_xt;
@@ -614,6 +636,11 @@ FinishArgs icon::finish_args(const icon_plan* p, int S) {
   a.slots = kNodeSlots; a.part = p->d_part; a.nslot = p->d_nd_nslot;
   a.w = p->d_w; a.b = p->d_b; a.bnorm = p->d_bnorm; a.iomit = g.iomit;
   a.rowpart = p->d_rowpart; a.epart = p->d_epart;
+  // one round of 4 rows per thread while blocks are fewer than CUs (16 slices of
+  // 1007^2, 61400 nodes: 73 -> 17 us with 15 blocks per slice; 256 slices of
+  // 512^2: 36 us with one, 41 with three)
+  a.rsum = p->d_rsum; a.rcnt = p->d_rcnt;
+  a.groups = std::max(1, std::min({kFinishGroups, (a.M + 4095) / 4096, p->cus / S}));
   a.nq = p->nq; a.rpart = p->d_rpart; a.rslot = p->d_nq_nslot; a.gram = p->d_gram;
   return a;
 }
@@ -868,7 +895,7 @@ int icon_plan_destroy(icon_plan* p) {
   drop_graph(p);
   void* ptrs[] = {p->d_nodes, p->d_ck1, p->d_w, p->d_phi1, p->d_i10, p->d_fw,
                   p->d_b, p->d_part, p->d_ahwb, p->d_grad, p->d_tmp, p->d_frep, p->d_rowpart,
-                  p->d_bnorm, p->d_alpha, p->d_spec, p->d_nd_off, p->d_nd_ent, p->d_nd_parts, p->d_nd_xt, p->d_nd_nslot, p->d_nd_px, p->d_nd_py,
+                  p->d_bnorm, p->d_alpha, p->d_spec, p->d_nd_off, p->d_nd_ent, p->d_nd_parts, p->d_nd_xt, p->d_rsum, p->d_rcnt, p->d_nd_nslot, p->d_nd_px, p->d_nd_py,
                   p->d_epart, p->d_nq_off, p->d_nq_ent, p->d_nq_entr, p->d_nq_px, p->d_nq_py, p->d_nq_nslot,
                   p->d_rpart, p->d_gram, p->d_base, p->d_mref, p->d_beff};
   for (void* q : ptrs)

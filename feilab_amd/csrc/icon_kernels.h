@@ -69,8 +69,8 @@ struct ColArgs {
   const double2* w64;      // col_normal64: exp(-2 pi i q / n0)
   int slots;               // partials per node in part
   int nyq;                 // half grid: its column n1/2; otherwise 0
-  // col_normal, few slices: shares of the dense tiles' entries in blocks of
-  // their own (out then is not in): shares per tile, and (tile, share > 0) of
+  // col_normal, col_fwd, few slices: shares of the dense tiles' entries in blocks of
+  // their own (col_normal: out then is not in): shares per tile, and (tile, share > 0) of
   // the nx further blocks per slice
   const int* parts;
   const int2* xt;
@@ -114,6 +114,7 @@ constexpr int kMaxUnpaired = 256;
 
 // End of an iteration: the data residual of the image (from the node partials
 // of A m) and the step size of the gradient.
+constexpr int kFinishGroups = 16;
 struct FinishArgs {
   int S, M, N0, nblk, nrow;   // M: rows of part per slice
   int Mb;                // nodes per slice in b
@@ -123,6 +124,9 @@ struct FinishArgs {
   const float* w;
   const float2* b;       // [S][Mb]
   const double* bnorm;   // [S]
+  unsigned long long* rsum;   // [S][kFinishGroups] sums of the residual's row groups (double bits)
+  unsigned* rcnt;             // [S] groups done, zero between launches
+  int groups;                 // blocks per slice over the residual's rows, at most kFinishGroups
   double* resid;         // trace base or null
   int resid_stride, resid_index;
   float2* frep;          // [S][N0] values of A m at the omit tilt, or null
@@ -176,6 +180,7 @@ struct FinishLaunch {
   int resid_index, alpha_index;   // < 0: no residual / no step size
   int with_frep;                  // 0: the series' frep pointers are ignored
   int beff;                       // 0: not used; 1: written; 2: read in place of b
+  int groups;                     // the largest of the series' groups
 };
 
 // While set (non-null) on the calling thread, the next launches of the

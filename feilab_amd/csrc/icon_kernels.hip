@@ -332,8 +332,17 @@ __device__ __forceinline__ void col_fwd_body(const ColArgs& a, int bid) {
   // the memory-side cache).  (The spread's order by entry count measured no
   // faster here: an interpolation block's time varies far less with its
   // tile's entries.)
-  const int blk = bid / a.S;
+  int blk = bid / a.S, part = 0, parts = 1;
   const int s = bid % a.S;
+  if (a.parts) {
+    // blocks past the tiles: a further share of a dense tile's entries
+    if (blk >= a.n1 / C) {
+      const int2 x = a.xt[blk - a.n1 / C];
+      blk = x.x;
+      part = x.y;
+    }
+    parts = a.parts[blk];
+  }
   const int y0 = blk * C;
   const int tid = threadIdx.x;
   // a tile no node reaches (beyond the largest |ky| of the tilt range) has
@@ -348,7 +357,7 @@ __device__ __forceinline__ void col_fwd_body(const ColArgs& a, int bid) {
     for (int i = 0; i < 16; i++) tile[out_index<NC>(t, i) * LS + c] = v[i];
   }
   __syncthreads();
-  interp_tile<NC, C, K>(a, tile, blk, s);
+  interp_tile<NC, C, K>(a, tile, blk, s, part, parts);
 }
 
 template <int NC, int C, int K>
@@ -360,7 +369,8 @@ template <int NC, int C, int K>
 __global__ __launch_bounds__(C * (NC / 16), 4) void k_col_fwd_multi(const ColArgs* __restrict__ descs,
                                                                    const int2* __restrict__ items) {
   const int2 it = items[blockIdx.x];
-  const ColArgs a = descs[it.x];
+  ColArgs a = descs[it.x];
+  a.parts = nullptr;   // the items are the tiles
   col_fwd_body<NC, C, K>(a, it.y);
 }
 
@@ -1109,7 +1119,7 @@ hipError_t launch_col(int NC, int C, bool adjoint, const ColArgs& a, hipStream_t
       LAUNCH_TIMED((k_col_adj<N, CC, KK>), dim3(h.S * nblk), dim3(CC * (N / 16)),                  \
                          (col_lds<N, CC>()) * sizeof(float2), st, a);                                    \
     else                                                                                                 \
-      LAUNCH_TIMED((k_col_fwd<N, CC, KK>), dim3(h.S * nblk), dim3(CC * (N / 16)),                  \
+      LAUNCH_TIMED((k_col_fwd<N, CC, KK>), dim3(h.S * (nblk + h.nx)), dim3(CC * (N / 16)),                  \
                          (col_lds<N, CC>()) * sizeof(float2), st, a);                                    \
     return hipGetLastError();                                                                            \
   }
@@ -1191,7 +1201,7 @@ hipError_t launch_col_fwd_nodes(int NC, const ColArgs& a, hipStream_t st) {
 #define CASE(N, CC, KK)                                                                                  \
   if (NC == N) {                                                                                         \
     static_assert(CC == kNormalC && KK == kInterpTaps, "the solve's interpolation");                     \
-    LAUNCH_TIMED((k_col_fwd<N, CC, KK>), dim3(a.S * (a.n1 / CC)), dim3(CC * (N / 16)),                   \
+    LAUNCH_TIMED((k_col_fwd<N, CC, KK>), dim3(a.S * (a.n1 / CC + a.nx)), dim3(CC * (N / 16)),            \
                  (col_lds<N, CC>()) * sizeof(float2), st, a);                                            \
     return hipGetLastError();                                                                            \
   }

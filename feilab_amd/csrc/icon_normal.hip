@@ -639,7 +639,11 @@ __device__ __forceinline__ int node_of(const FinishArgs& a, int r, int* jm) {
 // role 0: alpha = |rhat|^2 / <rhat, A^H W A rhat>; role 1: the data residual
 // R = sqrt(sum w |A m - b|^2 / sum w |b|^2) and the values at the omit tilt.
 // One block per (slice, role); FP64 sums in a fixed order.
-__device__ __forceinline__ void finish_body(const FinishArgs& a, int s, int role) {
+// Role 1 is shared among a.groups blocks per slice: the last to finish adds
+// their sums in order (rsum) and leaves their counter (rcnt) at zero again.  The
+// blocks exchange nothing but device-scope read-modify-writes, the store of a
+// sum waited for before the count.
+__device__ __forceinline__ void finish_body(const FinishArgs& a, int s, int role, int grp) {
   __shared__ double red[32];
   __shared__ double z[4 * kMaxUnpaired];
   const int tid = threadIdx.x;
@@ -698,7 +702,7 @@ __device__ __forceinline__ void finish_body(const FinishArgs& a, int s, int role
     return;
   }
   constexpr int U = 4, SL = 4;   // rows a round; partials loaded together (a.slots of them at most)
-  for (int r0 = tid; r0 < a.M; r0 += U * 1024) {
+  for (int r0 = grp * U * 1024 + tid; r0 < a.M; r0 += a.groups * U * 1024) {
     float2 p[U][SL], b0[U], b1[U];
     float w0[U], w1[U];
     int j[U], jm[U], ns[U];
@@ -750,18 +754,29 @@ __device__ __forceinline__ void finish_body(const FinishArgs& a, int s, int role
     }
   }
   if (!a.resid) return;
-  const double tot = block_sum_1024(acc, red);
+  double tot = block_sum_1024(acc, red);
   if (tid == 0) {
+    if (a.groups > 1) {
+      unsigned long long* q = a.rsum + (size_t)s * kFinishGroups;
+      const unsigned long long old = atomicExch(q + grp, (unsigned long long)__double_as_longlong(tot));
+      asm volatile("" ::"v"((unsigned)old) : "memory");
+      if (atomicAdd(a.rcnt + s, 1u) != (unsigned)a.groups - 1) return;
+      unsigned long long v[kFinishGroups];
+      for (int k = 0; k < a.groups; k++) v[k] = atomicAdd(q + k, 0ull);
+      tot = 0.0;
+      for (int k = 0; k < a.groups; k++) tot += __longlong_as_double((long long)v[k]);
+      atomicExch(a.rcnt + s, 0u);
+    }
     const double bn = a.bnorm[s];
     a.resid[(size_t)s * a.resid_stride + a.resid_index] = bn > 0 ? sqrt(tot / bn) : 0.0;
   }
 }
 
-// blocks [0, S): the step size where asked for (alpha non-null), else the
-// residual; blocks [S, 2S): the residual
+// blocks [0, S): the step size where asked for (alpha non-null); then S blocks
+// per group of the residual's rows
 __global__ __launch_bounds__(1024) void k_finish(FinishArgs a) {
-  const int role = a.alpha ? (int)blockIdx.x / a.S : 1;
-  finish_body(a, blockIdx.x % a.S, role);
+  const int k = (int)blockIdx.x / a.S - (a.alpha ? 1 : 0);
+  finish_body(a, blockIdx.x % a.S, k < 0 ? 0 : 1, k);
 }
 
 __global__ __launch_bounds__(1024) void k_finish_multi(const FinishArgs* __restrict__ descs,
@@ -774,9 +789,9 @@ __global__ __launch_bounds__(1024) void k_finish_multi(const FinishArgs* __restr
   if (!L.with_frep) a.frep = nullptr;
   if (L.beff == 2 && a.beff) a.b = a.beff;
   if (L.beff != 1) a.beff = nullptr;
-  const int role = L.alpha_index >= 0 ? (int)blockIdx.x / n : 1;
-  if (role == 1 && !a.resid && !a.frep) return;
-  finish_body(a, it.y, role);
+  const int k = (int)blockIdx.x / n - (L.alpha_index >= 0 ? 1 : 0);
+  if (k >= 0 && ((!a.resid && !a.frep) || k >= a.groups)) return;
+  finish_body(a, it.y, k < 0 ? 0 : 1, k);
 }
 
 // ------------------------------------------------------- plan-time kernels
@@ -1221,7 +1236,7 @@ hipError_t launch_row_grad64_multi(int NR, bool half, const RefArgs* descs, cons
 }
 
 hipError_t launch_finish(const FinishArgs& a, hipStream_t st) {
-  const int roles = (a.alpha ? 1 : 0) + (a.resid || a.frep ? 1 : 0);
+  const int roles = (a.alpha ? 1 : 0) + (a.resid || a.frep ? a.groups : 0);
   if (!roles) return hipSuccess;
   LAUNCH_TIMED(k_finish, dim3(roles * a.S), dim3(1024), 0, st, a);
   return hipGetLastError();
@@ -1229,7 +1244,7 @@ hipError_t launch_finish(const FinishArgs& a, hipStream_t st) {
 
 hipError_t launch_finish_multi(const FinishArgs* descs, const int2* items, int n, const FinishLaunch& L,
                                hipStream_t st) {
-  const int roles = (L.alpha_index >= 0 ? 1 : 0) + (L.resid_index >= 0 || L.with_frep ? 1 : 0);
+  const int roles = (L.alpha_index >= 0 ? 1 : 0) + (L.resid_index >= 0 || L.with_frep ? L.groups : 0);
   if (n <= 0 || !roles) return hipSuccess;
   LAUNCH_TIMED(k_finish_multi, dim3(roles * n), dim3(1024), 0, st, descs, items, n, L);
   return hipGetLastError();

@@ -79,6 +79,9 @@ struct DevBins {
   int4* fent = nullptr;
   float *px = nullptr, *py = nullptr, *fpx = nullptr, *fpy = nullptr;
   int8_t* nslot = nullptr;
+  int* parts = nullptr;           // shares of a tile's entries, and the further ones
+  int2* xt = nullptr;
+  int nx = 0;
 };
 
 // Entries of the solve's interpolation (16 taps, tiles of 8 columns): per tile
@@ -220,6 +223,8 @@ struct icon_plan {
   int* d_nd_parts = nullptr;        // shares of a tile's entries, and the further ones (split_dense)
   int2* d_nd_xt = nullptr;
   int nd_nx = 0;
+  unsigned long long* d_rsum = nullptr;   // FinishArgs
+  unsigned* d_rcnt = nullptr;
   int cus = 256;                    // compute units of the device
   int8_t* d_nd_nslot = nullptr;
   float* d_nd_px = nullptr;
