@@ -21,6 +21,7 @@
 #include <cstdio>
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -68,6 +69,8 @@ struct T32 {
 
 }  // namespace
 
+constexpr int kCopyPieces = 8;
+
 struct icon_unet {
   int device = 0;
   int maxB = 0, H = 0, W = 0;
@@ -92,6 +95,10 @@ struct icon_unet {
   // gradients (fp32)
   T32 g_d1b, g_d1a, g_cat1, g_d2b, g_d2a, g_cat2, g_d3b, g_d3a, g_cat3, g_bb, g_ab, g_a3, g_a2, g_a1, g_out;
   std::vector<void*> allocs;
+  // training: the gradients' way to the host (icon_unet_get_gradients)
+  float* pinned = nullptr;
+  hipEvent_t copied[kCopyPieces] = {};
+  mutable std::mutex copy_mutex;
 };
 
 namespace {
@@ -380,6 +387,10 @@ int icon_unet_create(icon_unet** out, int device, int max_batch, int H, int W, i
     if ((rc = alloc_bytes(n, (void**)&n->gpart,
                           sizeof(float) * (kHeadGradParts * 33 + (long)n->wgrad_blocks * (9 * 64 * 64 + 64)))))
       return bail(rc);
+    if (hipHostMalloc((void**)&n->pinned, sizeof(float) * off, hipHostMallocDefault) != hipSuccess)
+      return bail(ufail(2, "icon_unet_create: %ld bytes of pinned memory", (long)sizeof(float) * off));
+    for (hipEvent_t& e : n->copied)
+      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return bail(ufail(2, "icon_unet_create: event"));
     if ((rc = alloc_bytes(n, (void**)&n->grads, sizeof(float) * off)) ||
         (rc = alloc_bytes(n, (void**)&n->adam_m, sizeof(float) * off)) ||
         (rc = alloc_bytes(n, (void**)&n->adam_v, sizeof(float) * off)))
@@ -399,6 +410,9 @@ int icon_unet_destroy(icon_unet* n) {
   if (!n) return 0;
   (void)hipDeviceSynchronize();
   for (void* p : n->allocs) (void)hipFree(p);
+  if (n->pinned) (void)hipHostFree(n->pinned);
+  for (hipEvent_t e : n->copied)
+    if (e) (void)hipEventDestroy(e);
   delete n;
   return 0;
 }
@@ -490,9 +504,31 @@ int icon_unet_gradients(icon_unet* n, int B, const float* d_in, const float* d_t
   return 0;
 }
 
+// Through a pinned buffer in pieces, the host's copy of one while the next are
+// on their way: 7.8 MB into pageable memory in 455 us with hipMemcpy, 290 us
+// so (the transfer alone 146).
 int icon_unet_get_gradients(const icon_unet* n, float* host, int64_t count) {
   if (!n || !n->train || !host || count != n->nparam) return ufail(1, "icon_unet_get_gradients: bad argument");
-  UCHK(hipMemcpy(host, n->grads, sizeof(float) * count, hipMemcpyDeviceToHost));
+  const int64_t piece = (count + kCopyPieces - 1) / kCopyPieces;
+  std::lock_guard<std::mutex> lock(n->copy_mutex);
+  // (the events are the net's device's)
+  struct OnDevice {
+    int before = -1;
+    explicit OnDevice(int d) {
+      if (hipGetDevice(&before) != hipSuccess || before == d || hipSetDevice(d) != hipSuccess) before = -1;
+    }
+    ~OnDevice() { if (before >= 0) (void)hipSetDevice(before); }
+  } on(n->device);
+  for (int k = 0; k < kCopyPieces; k++) {
+    const int64_t at = k * piece, len = std::min(piece, count - at);
+    if (len > 0) UCHK(hipMemcpyAsync(n->pinned + at, n->grads + at, sizeof(float) * len, hipMemcpyDeviceToHost, nullptr));
+    UCHK(hipEventRecord(n->copied[k], nullptr));
+  }
+  for (int k = 0; k < kCopyPieces; k++) {
+    const int64_t at = k * piece, len = std::min(piece, count - at);
+    UCHK(hipEventSynchronize(n->copied[k]));
+    if (len > 0) std::memcpy(host + at, n->pinned + at, sizeof(float) * len);
+  }
   return 0;
 }
 
