@@ -678,17 +678,18 @@ __global__ __launch_bounds__(256, COB == 32 && R <= 4 ? 3 : 2) void k_conv(ConvA
 //
 // One launch for all layers: each needs only as many pixel splits as its share
 // of the device, so the partial sums are 2 blocks per CU x 64 x 64 x 9 floats
-// at most.  Measured, 14 layers of 16 images of 128^2: 177 us and 16 us for
+// at most.  Measured, 14 layers of 16 images of 128^2: 131 us and 16 us for
 // their reduction (one launch per layer, 64 x 64 x 1 tap tiles, gradients and
 // inputs re-read for every tap, the sums and the bias gradients by kernels of
 // their own: 3056 us).
 typedef __attribute__((ext_vector_type(16))) float f16v;
-constexpr int kWgR = 8;                  // gradient rows per wavefront and pixel tile
-constexpr int kWgLds = 32 * 1024 + 34 * 1024 + 34 * 256;   // 32 x 32 channels, 4 segments: the largest
+// gradient rows per wavefront and pixel tile
+__host__ __device__ constexpr int wgrad_rows(int co, int ci) { return ci == 2 ? 4 : 2; }
+constexpr int kWgLds = 2 * 9 * 16 * 64 * 4;   // the segments' sums of two tiles; the staged rows take less
 
 template <int CO, int CI>
 __device__ __forceinline__ void wgrad_block(const WgradLayer& L, int bt, int split, char* lds) {
-  constexpr int KS = 4 / (CO * CI), TR = kWgR * KS;
+  constexpr int kWgR = wgrad_rows(CO, CI), KS = 4 / (CO * CI), TR = kWgR * KS;
   constexpr int DYB = CO * 1024, XB = CI * 1024;        // bytes of a pixel row
   char* const s_dy = lds;
   char* const s_x = s_dy + TR * DYB;
@@ -718,70 +719,86 @@ __device__ __forceinline__ void wgrad_block(const WgradLayer& L, int bt, int spl
   auto rot = [](int g, int row, int G) { return G == 8 ? g : (g | (row & 1) << 2); };
   const int h = lane >> 5, c32 = lane & 31;
   const int t_end = min(L.tiles, (split + 1) * L.per);
-  for (int tile = split * L.per; tile < t_end; tile++) {
+  // the next tile's loads are in flight during this one's MFMAs: a tile's rows
+  // are few enough that they fit the registers beside the accumulators (8 rows
+  // per wavefront, loaded when staged: 172 us instead of 131)
+  constexpr int ND = TR / RO, NX = (TR + 2 + RI - 1) / RI;
+  static_assert(TR % RO == 0 && (TR + 2) * 2 * GI <= 256, "one halo piece per thread");
+  f4 da[ND][2], db[ND][2];
+  V8 xa[NX], xb[NX], xh;
+  const int gh = tid % GI, sh = tid / GI & 1, rh = tid / (2 * GI);   // halo piece: group, side, row
+  auto fetch = [&](int tile) {
     const int tx = tile % L.tiles_x, rest = tile / L.tiles_x;
     const int x0 = 16 * tx, y0 = TR * (rest % L.tiles_y), n = rest / L.tiles_y;
     const auto rdy = image_rsrc(L.dy + (long)n * H * W * L.lddy + L.cdy0 + co0, 0x7fffffffu);
     const auto rx = image_rsrc(L.x + (long)n * H * W * L.ldx + L.cx0 + ci0, 0x7fffffffu);
-    // gradient rows, FP32 to BF16 (nearest even) with the transposition
-    {
-      const int x = x0 + 2 * po;
-      const bool ok0 = x < W, ok1 = x + 1 < W;
-#pragma unroll 2
-      for (int k = 0; k < TR / RO; k++) {
-        const int row = ro + RO * k, y = y0 + row;
-        const unsigned o = (unsigned)(((y * W + x) * L.lddy + 8 * go) * 4);
-        const unsigned o0 = ok0 && y < H ? o : kOutside, o1 = ok1 && y < H ? o + 4u * L.lddy : kOutside;
-        f4 a[2], b[2];
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-          a[q] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rdy, o0 + 16 * q, 0, 0));
-          b[q] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rdy, o1 + 16 * q, 0, 0));
-        }
-        char* d = s_dy + row * DYB + go * 256 + po * 4;
-        const int ro8 = rot(go, row, GO);
+    for (int k = 0; k < ND; k++) {
+      const int x = x0 + 2 * po, y = y0 + ro + RO * k;
+      const unsigned o = (unsigned)(((y * W + x) * L.lddy + 8 * go) * 4);
+      const unsigned o0 = x < W && y < H ? o : kOutside, o1 = x + 1 < W && y < H ? o + 4u * L.lddy : kOutside;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-          bs[i] += a[i >> 2][i & 3] + b[i >> 2][i & 3];
-          *reinterpret_cast<uint32_t*>(d + ((i ^ ro8) & 7) * 32) = pack_bf16(a[i >> 2][i & 3], b[i >> 2][i & 3]);
-        }
+      for (int q = 0; q < 2; q++) {
+        da[k][q] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rdy, o0 + 16 * q, 0, 0));
+        db[k][q] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rdy, o1 + 16 * q, 0, 0));
       }
     }
     // input rows y0 - 1 .. y0 + TR
-    auto pair = [](const V8& a, const V8& b, int i) { return (uint32_t)a.h[i] | (uint32_t)b.h[i] << 16; };
-    const bool okc = ci0 + 8 * gi < L.Cin;
+#pragma unroll
+    for (int k = 0; k < NX; k++) {
+      const int x = x0 + 2 * pi, row = ri + RI * k, y = y0 - 1 + row;
+      const bool ok = ci0 + 8 * gi < L.Cin && row < TR + 2 && (unsigned)y < (unsigned)H;
+      const unsigned o = (unsigned)(((y * W + x) * L.ldx + 8 * gi) * 2);
+      xa[k].u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, ok && x < W ? o : kOutside, 0, 0));
+      xb[k].u = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, ok && x + 1 < W ? o + 2u * L.ldx : kOutside, 0, 0));
+    }
+    // their neighbours: pixels x0 - 1 and x0 + 16
     {
-      const int x = x0 + 2 * pi;
-      const bool ok0 = okc && x < W, ok1 = okc && x + 1 < W;
+      const int x = sh ? x0 + 16 : x0 - 1, y = y0 - 1 + rh;
+      const bool ok = rh < TR + 2 && ci0 + 8 * gh < L.Cin && (unsigned)x < (unsigned)W && (unsigned)y < (unsigned)H;
+      xh.u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                           rx, ok ? (unsigned)(((y * W + x) * L.ldx + 8 * gh) * 2) : kOutside, 0, 0));
+    }
+  };
+  auto put = [&]() {
+    // gradient rows, FP32 to BF16 (nearest even) with the transposition
 #pragma unroll
-      for (int k = 0; k < (TR + 2 + RI - 1) / RI; k++) {
-        const int row = ri + RI * k, y = y0 - 1 + row;
-        if (row >= TR + 2) break;
-        const bool oky = (unsigned)y < (unsigned)H;
-        const unsigned o = (unsigned)(((y * W + x) * L.ldx + 8 * gi) * 2);
-        V8 a, b;
-        a.u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, ok0 && oky ? o : kOutside, 0, 0));
-        b.u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, ok1 && oky ? o + 2u * L.ldx : kOutside, 0, 0));
-        char* d = s_x + row * XB + gi * 256 + pi * 4;
-        const int ro8 = rot(gi, row, GI);
+    for (int k = 0; k < ND; k++) {
+      const int row = ro + RO * k, ro8 = rot(go, row, GO);
+      char* d = s_dy + row * DYB + go * 256 + po * 4;
 #pragma unroll
-        for (int i = 0; i < 8; i++) *reinterpret_cast<uint32_t*>(d + ((i ^ ro8) & 7) * 32) = pair(a, b, i);
+      for (int i = 0; i < 8; i++) {
+        const float u = da[k][i >> 2][i & 3], v = db[k][i >> 2][i & 3];
+        bs[i] += u + v;
+        *reinterpret_cast<uint32_t*>(d + ((i ^ ro8) & 7) * 32) = pack_bf16(u, v);
       }
     }
-    // their neighbours: pixel x0 - 1 in the high half of side 0, x0 + 16 in the
-    // low half of side 1 (the other halves are not used)
-    for (int u = tid; u < (TR + 2) * 2 * GI; u += 256) {
-      const int g = u % GI, side = u / GI & 1, row = u / (2 * GI);
-      const int x = side ? x0 + 16 : x0 - 1, y = y0 - 1 + row;
-      const bool ok = ci0 + 8 * g < L.Cin && (unsigned)x < (unsigned)W && (unsigned)y < (unsigned)H;
-      V8 a;
-      a.u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                          rx, ok ? (unsigned)(((y * W + x) * L.ldx + 8 * g) * 2) : kOutside, 0, 0));
-      uint32_t* d = reinterpret_cast<uint32_t*>(s_h) + (row * 2 + side) * 32 * CI + 8 * g;
 #pragma unroll
-      for (int i = 0; i < 8; i++) d[i] = side ? (uint32_t)a.h[i] : (uint32_t)a.h[i] << 16;
+    for (int k = 0; k < NX; k++) {
+      const int row = ri + RI * k, ro8 = rot(gi, row, GI);
+      char* d = s_x + row * XB + gi * 256 + pi * 4;
+      if (row < TR + 2) {
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          *reinterpret_cast<uint32_t*>(d + ((i ^ ro8) & 7) * 32) = (uint32_t)xa[k].h[i] | (uint32_t)xb[k].h[i] << 16;
+      }
     }
+    // pixel x0 - 1 in the high half of side 0, x0 + 16 in the low half of side
+    // 1 (the other halves are not used)
+    if (rh < TR + 2) {
+      uint32_t* d = reinterpret_cast<uint32_t*>(s_h) + (rh * 2 + sh) * 32 * CI + 8 * gh;
+#pragma unroll
+      for (int i = 0; i < 8; i++) d[i] = sh ? (uint32_t)xh.h[i] : (uint32_t)xh.h[i] << 16;
+    }
+    // (as in k_conv: the loads are waited for on every path)
+    vm_wait_all();
+  };
+  if (split * L.per < t_end) fetch(split * L.per);
+  for (int tile = split * L.per; tile < t_end; tile++) {
+    put();
     __syncthreads();
+    if (tile + 1 < t_end) fetch(tile + 1);
     {
       bf8 D[kWgR];
       const int co = 32 * co_t + c32, ci = 32 * ci_t + c32;
@@ -842,13 +859,11 @@ __device__ __forceinline__ void wgrad_block(const WgradLayer& L, int bt, int spl
   // result row 8 (r / 4) + 4 h + r % 4, column lane % 32
   const int ci = ci0 + 32 * ci_t + c32;
   if (ks == 0 && ci < L.Cin) {
+    float* dst = L.part + (long)split * 9 * L.Cout * L.Cin + (co0 + 32 * co_t + 4 * h) * L.Cin + ci;
 #pragma unroll
     for (int t = 0; t < 9; t++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int co = co0 + 32 * co_t + 8 * (r >> 2) + 4 * h + (r & 3);
-        L.part[(((long)split * 9 + t) * L.Cout + co) * L.Cin + ci] = acc[t][r];
-      }
+      for (int r = 0; r < 16; r++) dst[(t * L.Cout + 8 * (r >> 2) + (r & 3)) * L.Cin] = acc[t][r];
   }
   if (bias) {
     // [thread][8] in LDS, then channel c adds its group's threads in order
@@ -1161,15 +1176,15 @@ template hipError_t launch_conv<float, float>(const ConvArgs<float, float>&, hip
 static void wgrad_shape(WgradLayer& L) {
   L.co = L.Cout % 64 == 0 ? 2 : 1;
   L.ci = L.Cin % 64 == 0 ? 2 : 1;
-  const int tr = kWgR * 4 / (L.co * L.ci);
+  const int rows = wgrad_rows(L.co, L.ci), tr = rows * 4 / (L.co * L.ci);
   L.nco = L.Cout / (32 * L.co);
   L.nci = (L.Cin + 32 * L.ci - 1) / (32 * L.ci);
   L.tiles_x = (L.W + 15) / 16;
   L.tiles_y = (L.H + tr - 1) / tr;
   L.tiles = L.N * L.tiles_x * L.tiles_y;
-  // cost of a pixel tile: 8 rows of MFMAs, and the staging of the rows of 4 KB
+  // cost of a pixel tile: the rows' MFMAs, and the staging of the rows of 4 KB
   // of gradient and 2 KB of input per 64 channels
-  L.cost = 8 * 4 + (tr * L.co * 2 + (tr + 2) * L.ci) / 2;
+  L.cost = rows * 4 + (tr * L.co * 2 + (tr + 2) * L.ci) / 2;
 }
 
 // Splits of every layer's pixels: the smallest largest cost per block such that
