@@ -81,7 +81,9 @@ void sampling_mask(int N, const float* thita, int ang_num, std::vector<float>& o
 // rows), a column pass (forward transform, mask, inverse transform) and a row
 // pass back.  The spectrum of a real row of N samples is N floats: F_0, for even
 // N F_{N/2}, and the pairs F_k, 0 < k < N/2, so it replaces the row in the stack
-// and no other buffer is needed.  Two real rows share one complex transform.
+// and no other buffer is needed.  Two real rows of a slice share one complex
+// transform (an odd slice's last row has one alone: rows of two slices in one
+// would mix their rounding, and spread a NaN from one to the next).
 //
 // Lengths that are not powers of two (or below 128) use Bluestein's chirp-z
 // transform on a power-of-two transform of length M >= 2N - 1.  With
@@ -153,10 +155,12 @@ __global__ __launch_bounds__(RPB * (M / 16)) void k_filt_rows(FiltArgs a) {
   constexpr int T = M / 16;
   __shared__ float2 lds[RPB * RowLay::size(M)];
   const int team = threadIdx.x / T, t = threadIdx.x % T;
-  const long row = 2 * ((long)blockIdx.x * RPB + team);
-  const int N = a.N;
+  const int N = a.N, pairs = (N + 1) / 2;   // row pairs of a slice
+  const long p = (long)blockIdx.x * RPB + team, slice = p / pairs;
+  const int y = 2 * (int)(p - slice * pairs);
+  const long row = slice * N + y;
   float2* L = lds + team * RowLay::size(M);
-  const bool v0 = row < a.rows, v1 = row + 1 < a.rows;
+  const bool v0 = row < a.rows, v1 = v0 && y + 1 < N;
   float *p0 = a.data + (v0 ? row : 0) * N, *p1 = a.data + (v1 ? row + 1 : 0) * N;
   float2 v[16];
 #pragma unroll
@@ -327,7 +331,7 @@ hipError_t launch_filter(const FiltArgs& a, int count, hipStream_t st) {
   const hipError_t e = hipFuncSetAttribute((const void*)k_filt_cols<M, C, CHIRP>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return e;
-  const long pairs = (a.rows + 1) / 2;
+  const long pairs = (long)count * ((a.N + 1) / 2);
   const unsigned blocks = (unsigned)((pairs + RPB - 1) / RPB);
   const int ntiles = ((a.N + 1) / 2 + C - 1) / C;
   hipLaunchKernelGGL((k_filt_rows<M, RPB, CHIRP, false>), dim3(blocks), dim3(RPB * (M / 16)), 0, st, a);
