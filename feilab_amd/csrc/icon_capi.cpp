@@ -193,13 +193,31 @@ int make_bins(icon_plan* p, DevBins& b, int C, int K) {
 
 int op_taps(const Geometry& g) { return g.window == ICON_WINDOW_KB6 ? kTapsKB : kTapsWide; }
 
-// The transforms' bins at tile width C, and the weighted values' buffer.
+// The transforms' bins at tile width C, and the weighted values' buffer.  The
+// solve keeps the bins that it was made with (accurate window, tiles of
+// kSolveTile columns): its data set-up has an FP64 kernel for those alone, and
+// its results do not depend on a choice made by timing the transforms.
 int make_op_bins(icon_plan* p, int C) {
+  const int K = op_taps(p->g);
+  DevBins t;
+  int rc = ICON_OK;
+  if (K == kTapsWide && C == kSolveTile && p->own_data) {
+    free_bins(p->op);
+    p->op = std::exchange(p->data, DevBins{});
+    p->own_data = false;
+  } else if ((rc = make_bins(p, t, C, K))) {
+    free_bins(t);
+    return rc;
+  } else {
+    if (p->op.ck && !p->own_data) {
+      p->data = std::exchange(p->op, DevBins{});
+      p->own_data = true;
+    }
+    free_bins(p->op);
+    p->op = std::move(t);
+  }
   if (p->d_fw) (void)hipFree(p->d_fw);
   p->d_fw = nullptr;
-  free_bins(p->op);
-  int rc = make_bins(p, p->op, C, op_taps(p->g));
-  if (rc) return rc;
   const size_t E = std::max(p->op.h.ent.size(), p->data.h.ent.size());
   return dalloc(p, &p->d_fw, (size_t)p->S_max * E);
 }
@@ -848,8 +866,9 @@ int plan_create(icon_plan** out, int device, int nx, int thickness, int nz, cons
   // iterations: it needs the accurate window also where the transforms use the
   // 6-tap one (with it, and with the 14-tap Gaussian, a 100-iteration solve was
   // 4 to 5 times as far from the exact one as now).
+  static_assert(kSolveTile == 8, "the tile of the FP64 data adjoint (COL64_CASES)");
   p->own_data = op_taps(g) != kTapsWide;
-  if (p->own_data && (rc = make_bins(p, p->data, 8, kTapsWide))) return bail(rc);
+  if (p->own_data && (rc = make_bins(p, p->data, kSolveTile, kTapsWide))) return bail(rc);
   if ((rc = make_op_bins(p, default_col_block(g.n0)))) return bail(rc);
   if ((rc = twiddles(g.n0, &p->d_tw0))) return bail(rc);
   if ((rc = twiddles(g.n1, &p->d_tw1))) return bail(rc);

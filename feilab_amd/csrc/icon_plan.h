@@ -17,6 +17,7 @@ constexpr int kTapsKB = 6;     // Kaiser-Bessel window of width 6
 // 10.  Its transforms are within 1e-9 of the exact ones before rounding (the
 // 14-tap Gaussian: 7e-7 rms, 3.5e-6 at most) from fewer taps and column tiles.
 constexpr int kTapsWide = 10;
+constexpr int kSolveTile = 8;  // grid columns per tile of the solve's data set-up
 constexpr int kMaxSlot = 3;    // node y-taps split over at most 3 column tiles (tile >= 8)
 
 // Host-side geometry of one tilt series, computed exactly as the reference's
@@ -190,7 +191,7 @@ struct icon_plan {
   hipStream_t stream = nullptr;     // plan-owned stream (capturable)
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
   // the transforms' window: bins and tables; data: those of the solve's data
-  // set-up where the plan's own window is not accurate enough (else op's)
+  // set-up (kTapsWide, kSolveTile) where the transforms' are others (else op's)
   icon::DevBins op, data;
   bool own_data = false;
   icon::DevBins& spread() { return own_data ? data : op; }
