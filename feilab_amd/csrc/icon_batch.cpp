@@ -70,7 +70,6 @@ struct icon_batch {
   int device = 0;
   std::vector<icon_plan*> plans;
   std::vector<int> S;
-  std::vector<int> C_built;   // column tile of each plan's spread when the items were built
   hipStream_t stream = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
   // item tables per size class
@@ -142,8 +141,6 @@ int build_items(icon_batch* b) {
   if (b->combine.d) (void)hipFree(b->combine.d);
   b->combine = Items{};
   const int ns = (int)b->plans.size();
-  b->C_built.assign(ns, 0);
-  for (int i = 0; i < ns; i++) b->C_built[i] = b->plans[i]->spread().h.C;
   auto group = [](std::vector<Items>& v, int k0, int k1, int k2) -> Items& {
     for (auto& it : v)
       if (it.key0 == k0 && it.key1 == k1 && it.key2 == k2) return it;
@@ -513,15 +510,7 @@ int icon_batch_reconstruct(icon_batch* b, const void* const* d_sino, void* const
     p->data_sino = nullptr;
     p->data_S = 0;
   }
-  // a plan whose column tile changed since the items were built (its bins
-  // have another tile count): rebuild the items before any launch
-  for (int i = 0; i < ns && rc == ICON_OK; i++)
-    if (b->plans[i]->spread().h.C != b->C_built[i]) {
-      drop_batch_graph(b);
-      rc = build_items(b);
-    }
   do {
-    if (rc) break;
     hipError_t e = hipEventRecord(b->ev_in, user);
     if (e == hipSuccess) e = hipStreamWaitEvent(b->stream, b->ev_in, 0);
     if (e != hipSuccess) { rc = bfail(ICON_ERR_DEVICE, "icon_batch_reconstruct: %s", hipGetErrorString(e)); break; }

@@ -193,10 +193,11 @@ int make_bins(icon_plan* p, DevBins& b, int C, int K) {
 
 int op_taps(const Geometry& g) { return g.window == ICON_WINDOW_KB6 ? kTapsKB : kTapsWide; }
 
-// The transforms' bins at tile width C, and the weighted values' buffer.  The
-// solve keeps the bins that it was made with (accurate window, tiles of
-// kSolveTile columns): its data set-up has an FP64 kernel for those alone, and
-// its results do not depend on a choice made by timing the transforms.
+// The transforms' bins at tile width C.  The solve keeps the bins that it was
+// made with (accurate window, tiles of kSolveTile columns): its data set-up has
+// an FP64 kernel for those alone, its results do not depend on a choice made by
+// timing the transforms, and captured solves, of the plan and of batches that
+// hold it, keep tables and buffers that live as long as the plan.
 int make_op_bins(icon_plan* p, int C) {
   const int K = op_taps(p->g);
   DevBins t;
@@ -216,10 +217,7 @@ int make_op_bins(icon_plan* p, int C) {
     free_bins(p->op);
     p->op = std::move(t);
   }
-  if (p->d_fw) (void)hipFree(p->d_fw);
-  p->d_fw = nullptr;
-  const size_t E = std::max(p->op.h.ent.size(), p->data.h.ent.size());
-  return dalloc(p, &p->d_fw, (size_t)p->S_max * E);
+  return ICON_OK;
 }
 
 // Column-kernel arguments of a window's bins over S slices.
@@ -870,6 +868,9 @@ int plan_create(icon_plan** out, int device, int nx, int thickness, int nz, cons
   p->own_data = op_taps(g) != kTapsWide;
   if (p->own_data && (rc = make_bins(p, p->data, kSolveTile, kTapsWide))) return bail(rc);
   if ((rc = make_op_bins(p, default_col_block(g.n0)))) return bail(rc);
+  // (a tile of 16 columns has no more entries than the two of 8 that it covers)
+  const size_t E = std::max(p->op.h.ent.size(), p->data.h.ent.size());
+  if ((rc = dalloc(p, &p->d_fw, (size_t)p->S_max * E))) return bail(rc);
   if ((rc = twiddles(g.n0, &p->d_tw0))) return bail(rc);
   if ((rc = twiddles(g.n1, &p->d_tw1))) return bail(rc);
   if ((rc = twiddles64(g.n0, &p->d_w640))) return bail(rc);
@@ -942,12 +943,12 @@ int icon_plan_set_col_block(icon_plan* p, int C) {
   if (!p) return fail(ICON_ERR_ARG, "icon_plan_set_col_block: null plan");
   if (!col_tile_ok(p->g.n0, p->g.n1, C, op_taps(p->g)))
     return fail(ICON_ERR_ARG, "column tile %d unsupported for grid %d x %d", C, p->g.n0, p->g.n1);
+  if (C == p->op.h.C) return ICON_OK;
   DevGuard dg(p->device);
   HIPCHK(hipStreamSynchronize(p->stream));
   drop_graph(p);
-  int rc = make_op_bins(p, C);
-  if (rc) return rc;
-  return prepare_col(p->g.n0, p->g.n1, C, op_taps(p->g));
+  const int rc = prepare_col(p->g.n0, p->g.n1, C, op_taps(p->g));
+  return rc ? rc : make_op_bins(p, C);
 }
 
 int icon_nufft_forward_real(icon_plan* p, int S, const void* d_img, void* d_f, void* stream) {
