@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -254,24 +255,30 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace {
 
-// Device address of `scratch` on each device, resolved once per device with
-// that device current (the array's name in host code is only a stand-in).
+// `scratch` of each device: its address, resolved once with that device current
+// (the array's name in host code is only a stand-in), and a lock held by the
+// call that uses it until its last kernel has ended, so that calls that overlap
+// on one device take turns.
+struct DeviceScratch {
+  unsigned char* p = nullptr;
+  std::mutex busy;
+};
 std::mutex g_scratch_mu;
-std::vector<unsigned char*> g_scratch_ptr;
+std::map<int, DeviceScratch> g_scratch;
 
-hipError_t scratch_on_current_device(unsigned char** out) {
+hipError_t scratch_on_current_device(DeviceScratch** out) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if ((int)g_scratch_ptr.size() <= dev) g_scratch_ptr.resize(dev + 1, nullptr);
-  if (!g_scratch_ptr[dev]) {
+  DeviceScratch& d = g_scratch[dev];
+  if (!d.p) {
     void* p = nullptr;
     e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
     if (e != hipSuccess) return e;
-    g_scratch_ptr[dev] = static_cast<unsigned char*>(p);
+    d.p = static_cast<unsigned char*>(p);
   }
-  *out = g_scratch_ptr[dev];
+  *out = &d;
   return hipSuccess;
 }
 
@@ -314,10 +321,11 @@ int icon_preprocess_noalloc(int device, float* d_stack, int nx, int ny, int nz, 
     return perr(ICON_ERR_CAPACITY, "icon_preprocess_noalloc: " + std::to_string(nz) + " images exceed the " +
                                        std::to_string(kNoAllocMaxImages) + " its device scratch holds per call");
   if (hipSetDevice(device) != hipSuccess) return perr(ICON_ERR_ARG, "icon_preprocess_noalloc: no such device");
-  unsigned char* base = nullptr;
-  hipError_t e = scratch_on_current_device(&base);
+  DeviceScratch* d = nullptr;
+  hipError_t e = scratch_on_current_device(&d);
   if (e != hipSuccess)
     return perr(ICON_ERR_DEVICE, std::string("icon_preprocess_noalloc: hipGetSymbolAddress: ") + hipGetErrorString(e));
+  std::lock_guard<std::mutex> busy(d->busy);
   hipStream_t st = (hipStream_t)stream;
   const bool norm = tilt_deg && thickness > 0;
   // every call writes what it reads of the scratch, so nothing left in it by
@@ -325,14 +333,15 @@ int icon_preprocess_noalloc(int device, float* d_stack, int nx, int ny, int nz, 
   PreArgs a{};
   a.stack = d_stack; a.nx = nx; a.ny = ny; a.thickness = thickness;
   a.nb = blocks_per_image(nz, (long)nx * ny);
-  a.w = carve(base, nz, (long)nz * a.nb);
+  a.w = carve(d->p, nz, (long)nz * a.nb);
   if (norm) {
     a.tilt = a.w.tilt;
     e = hipMemcpyAsync(a.w.tilt, tilt_deg, sizeof(float) * nz, hipMemcpyHostToDevice, st);
   }
   if (e == hipSuccess) e = run_passes(a, nz, st);
   if (e == hipSuccess && modes) e = hipMemcpyAsync(modes, a.w.modes, sizeof(double) * nz, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  const hipError_t es = hipStreamSynchronize(st);   // (also after an error: nothing uses the scratch past the lock)
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return perr(ICON_ERR_DEVICE, std::string("icon_preprocess_noalloc: ") + hipGetErrorString(e));
   return ICON_OK;
 }

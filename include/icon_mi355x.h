@@ -312,11 +312,12 @@ int icon_preprocess(int device, float* d_stack, int nx, int ny, int nz, const fl
 /* icon_preprocess without any device allocation, for callers that cannot
  * allocate device memory (serving loops, harnesses that forbid hipMalloc).
  * No counterpart in the reference.  Same arguments, results and
- * synchronisation as icon_preprocess; the tilt angles and modes are staged in
- * a fixed device array of the library (48 KiB per device, held until the
- * process ends) instead of buffers allocated per call, so nz is limited to
- * 4096 images per call (ICON_ERR_CAPACITY beyond).  Calls that overlap on one
- * device share that array and race; calls on different devices do not. */
+ * synchronisation as icon_preprocess; the passes' partial sums and histograms,
+ * the tilt angles and the modes lie in a fixed device array of the library (4.2
+ * MiB per device, held until the process ends) instead of a buffer allocated
+ * per call, so nz is limited to 4096 images per call (ICON_ERR_CAPACITY
+ * beyond).  Calls of several threads on one device take turns with that array;
+ * calls on different devices do not wait for each other. */
 int icon_preprocess_noalloc(int device, float* d_stack, int nx, int ny, int nz, const float* tilt_deg, int thickness,
                             double* modes, void* stream);
 /* The same on MRC files: in_path -> out_path (float, header copied from the
