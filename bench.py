@@ -580,7 +580,7 @@ def main():
         plan.set_col_block(args.col_block)
     else:
         c, ms = plan.autotune(S)
-        autotune = dict(col_block=c, ms_column_kernels_per_iteration={str(k): round(v, 4) for k, v in ms.items()})
+        autotune = dict(col_block=c, ms_column_kernels_forward_adjoint={str(k): round(v, 4) for k, v in ms.items()})
         log("autotuned column tile:", json.dumps(autotune))
     iomit = plan.info.iomit
     band = (1, plan.N0 // 4)

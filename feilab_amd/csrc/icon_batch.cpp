@@ -17,7 +17,6 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
-#include <map>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -73,9 +72,9 @@ struct icon_batch {
   hipStream_t stream = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
   // item tables per size class
-  std::vector<Items> row_fwd, row_adj, col, sino, reproj;
-  // the spread's items: those of col, by their tile's entry count, largest
-  // first across the class's series (each tile's blocks stay together)
+  std::vector<Items> row_fwd, row_adj, sino, reproj;
+  // the data adjoint's spread: items by their tile's entry count, largest first
+  // across the class's series (each tile's blocks stay together)
   std::vector<Items> col_adj;
   std::vector<Items> normal;   // the normal operator's column kernels, by n0
   std::vector<Items> row_grad, row64;   // the iteration's gradient; rows (or pairs) of the FP64 one
@@ -126,20 +125,9 @@ int upload_items(Items& it) {
   return ICON_OK;
 }
 
-// (series, block) items of every size class; called at creation and after the
-// column tiles change.
+// (series, block) items of every size class, built once: they depend on the
+// tables that a plan keeps for its life.
 int build_items(icon_batch* b) {
-  free_items(b->row_fwd);
-  free_items(b->row_adj);
-  free_items(b->col);
-  free_items(b->col_adj);
-  free_items(b->normal);
-  free_items(b->row_grad);
-  free_items(b->row64);
-  free_items(b->sino);
-  free_items(b->reproj);
-  if (b->combine.d) (void)hipFree(b->combine.d);
-  b->combine = Items{};
   const int ns = (int)b->plans.size();
   auto group = [](std::vector<Items>& v, int k0, int k1, int k2) -> Items& {
     for (auto& it : v)
@@ -175,7 +163,7 @@ int build_items(icon_batch* b) {
     for (int k = 0; k < (rows + rpg - 1) / rpg; k++) rg.h.push_back(make_int2(i, k));
     if (!col_tile_ok(g.n0, g.n1, sb.C, sb.K))
       return bfail(ICON_ERR_ARG, "series %d: column tile %d unsupported for grid %d x %d", i, sb.C, g.n0, g.n1);
-    Items& cl = group(b->col, g.n0, sb.C, sb.K);
+    Items& cl = group(b->col_adj, g.n0, sb.C, sb.K);
     for (int k = 0; k < S * (g.n1 / sb.C); k++) cl.h.push_back(make_int2(i, k));
     Items& nm = group(b->normal, g.n0, 0, 0);
     for (int k = 0; k < S * (p->ncol / kNormalC); k++) nm.h.push_back(make_int2(i, k));
@@ -189,26 +177,21 @@ int build_items(icon_batch* b) {
   // the spread's order: a stable sort of each class's items by the entry
   // count of the tile the block runs (the plan's own largest-first tile order
   // maps a series' block k to tile bins.order[k / S])
-  for (const Items& c : b->col) {
-    Items a = c;
-    a.d = nullptr;
+  for (Items& a : b->col_adj) {
     auto cnt = [&](const int2& q) {
       const Bins& sb = b->plans[q.x]->spread().h;
       const int t = sb.order[q.y / b->S[q.x]];
       return sb.off[t + 1] - sb.off[t];
     };
     std::stable_sort(a.h.begin(), a.h.end(), [&](const int2& u, const int2& v) { return cnt(u) > cnt(v); });
-    b->col_adj.push_back(std::move(a));
   }
   int rc;
-  for (auto* v : {&b->row_fwd, &b->row_adj, &b->col, &b->col_adj, &b->normal, &b->row_grad, &b->row64, &b->sino, &b->reproj})
+  for (auto* v : {&b->row_fwd, &b->row_adj, &b->col_adj, &b->normal, &b->row_grad, &b->row64, &b->sino, &b->reproj})
     for (auto& it : *v)
       if ((rc = upload_items(it))) return rc;
   if ((rc = upload_items(b->combine))) return rc;
-  for (auto& it : b->col) {
-    hipError_t e = set_col_multi_attrs(it.key0, it.key1, it.key2);
-    if (e != hipSuccess) return bfail(ICON_ERR_DEVICE, "column kernel attributes: %s", hipGetErrorString(e));
-  }
+  const hipError_t e = set_col_adj_multi_attrs();
+  if (e != hipSuccess) return bfail(ICON_ERR_DEVICE, "column kernel attributes: %s", hipGetErrorString(e));
   return ICON_OK;
 }
 
@@ -345,7 +328,7 @@ int enqueue_batch(icon_batch* b, float* const* m, const float* const* m_init, bo
   for (auto& it : b->col_adj)
     if ((rc = ck(adj64_ok(it.key0, it.key1, it.key2)
                      ? launch_col_adj64_multi(it.key0, it.key1, b->d_ca, it.d, it.n(), st)
-                     : launch_col_multi(it.key0, it.key1, it.key2, true, b->d_ca, it.d, it.n(), st), "col_adj")))
+                     : launch_col_adj_multi(it.key0, b->d_ca, it.d, it.n(), st), "col_adj")))
       return rc;
   for (auto& it : b->row_adj)
     if ((rc = ck(it.key1 ? launch_row_adj64_multi(it.key0, b->d_ra, it.d, it.n(), st)
@@ -395,7 +378,6 @@ int icon_batch_destroy(icon_batch* b) {
   drop_batch_graph(b);
   free_items(b->row_fwd);
   free_items(b->row_adj);
-  free_items(b->col);
   free_items(b->col_adj);
   free_items(b->normal);
   free_items(b->row_grad);
@@ -560,75 +542,17 @@ int icon_batch_launches_per_iteration(const icon_batch* b, int* launches) {
   return ICON_OK;
 }
 
-// Column-tile autotuner of a batch: for every column size class (n0, window)
-// each tile width the class supports is timed on the class's packed
-// interpolation and spread launches (2 + 1, as in an iteration) over the
-// plans' current buffers, and the fastest is kept for all plans of the class.
+// The column tile is the transforms' alone: a packed solve does not depend on it.
 int icon_batch_autotune(icon_batch* b, int* col_blocks) {
   if (!b) return bfail(ICON_ERR_ARG, "icon_batch_autotune: null batch");
-  int prev = -1;
-  (void)hipGetDevice(&prev);
-  if (prev != b->device) BCHK(hipSetDevice(b->device));
-  drop_batch_graph(b);
-  const int ns = (int)b->plans.size();
-  // classes by (n0, K)
-  std::map<std::pair<int, int>, std::vector<int>> cls;
-  for (int i = 0; i < ns; i++) cls[{b->plans[i]->g.n0, b->plans[i]->op.h.K}].push_back(i);
-  int rc = ICON_OK;
-  hipEvent_t e0 = nullptr, e1 = nullptr;
-  (void)hipEventCreate(&e0);
-  (void)hipEventCreate(&e1);
-  std::vector<const float*> sino(ns, nullptr);
-  std::vector<float*> m(ns, nullptr), rp(ns, nullptr);
-  std::vector<double*> rs(ns, nullptr), al(ns, nullptr);
-  for (auto& kv : cls) {
-    const int n0 = kv.first.first, K = kv.first.second;
-    double best = -1.0;
-    int best_c = 0;
-    for (int C : {8, 16}) {
-      bool ok = true;
-      for (int i : kv.second) ok = ok && col_tile_ok(n0, b->plans[i]->g.n1, C, K);
-      if (!ok) continue;
-      for (int i : kv.second)
-        if (b->plans[i]->op.h.C != C && (rc = icon_plan_set_col_block(b->plans[i], C)))
-          return bfail(rc, "icon_batch_autotune: %s", icon_last_error());
-      if ((rc = build_items(b))) return rc;
-      fill_args(b, sino.data(), m.data(), rp.data(), rs.data(), al.data(), 0, false);
-      if ((rc = upload_args(b->d_ca, b->h_ca, b->stream))) return rc;
-      const Items *it = nullptr, *ia = nullptr;
-      for (auto& c : b->col)
-        if (c.key0 == n0 && c.key1 == C && c.key2 == K) it = &c;
-      for (auto& c : b->col_adj)
-        if (c.key0 == n0 && c.key1 == C && c.key2 == K) ia = &c;
-      if (!it || !ia) continue;
-      double t = 0.0;
-      for (int rep = 0; rep < 4 && rc == ICON_OK; rep++) {
-        hipError_t e = hipEventRecord(e0, b->stream);
-        for (int k = 0; k < 3 && e == hipSuccess; k++)
-          e = k == 1 ? launch_col_multi(n0, C, K, true, b->d_ca, ia->d, ia->n(), b->stream)
-                     : launch_col_multi(n0, C, K, false, b->d_ca, it->d, it->n(), b->stream);
-        if (e == hipSuccess) e = hipEventRecord(e1, b->stream);
-        if (e == hipSuccess) e = hipEventSynchronize(e1);
-        float ms = 0.f;
-        if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-        if (e != hipSuccess) rc = bfail(ICON_ERR_DEVICE, "icon_batch_autotune: %s", hipGetErrorString(e));
-        if (rep > 0) t += ms;   // the first pass is a warm-up
-      }
-      if (rc) break;
-      if (best < 0 || t < best) { best = t; best_c = C; }
-    }
-    if (rc) break;
-    for (int i : kv.second)
-      if (best_c && b->plans[i]->op.h.C != best_c && (rc = icon_plan_set_col_block(b->plans[i], best_c)))
-        return bfail(rc, "icon_batch_autotune: %s", icon_last_error());
+  BCHK(hipStreamSynchronize(b->stream));   // the plans' buffers are overwritten
+  for (size_t i = 0; i < b->plans.size(); i++) {
+    int c = 0;
+    if (const int rc = icon_plan_autotune(b->plans[i], b->S[i], &c, nullptr))
+      return bfail(rc, "icon_batch_autotune: series %d: %s", (int)i, icon_last_error());
+    if (col_blocks) col_blocks[i] = c;
   }
-  if (e0) (void)hipEventDestroy(e0);
-  if (e1) (void)hipEventDestroy(e1);
-  if (!rc) rc = build_items(b);
-  if (!rc && col_blocks)
-    for (int i = 0; i < ns; i++) col_blocks[i] = b->plans[i]->op.h.C;
-  if (prev >= 0 && prev != b->device) (void)hipSetDevice(prev);
-  return rc;
+  return ICON_OK;
 }
 
 }  // extern "C"

@@ -1214,7 +1214,7 @@ int icon_plan_autotune(icon_plan* p, int S, int* col_block, double* ms_per_width
     if (!rc) rc = icon_time_kernel(p, ICON_K_COL_FWD, S, 3, &tf);
     if (!rc) rc = icon_time_kernel(p, ICON_K_COL_ADJ, S, 3, &ta);
     if (rc) return rc;
-    const double t = 2.0 * tf + ta;
+    const double t = tf + ta;
     if (ms_per_width) ms_per_width[i] = t;
     if (best_c == 0 || t < best) { best = t; best_c = C; }
   }

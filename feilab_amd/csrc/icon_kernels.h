@@ -223,8 +223,7 @@ hipError_t launch_row_fwd_multi(int NR, const RowFwdArgs* descs, const int2* ite
                                 hipStream_t st);
 hipError_t launch_row_adj_multi(int NR, const RowAdjArgs* descs, const int2* items, int n, bool grad,
                                 hipStream_t st);
-hipError_t launch_col_multi(int NC, int C, int K, bool adjoint, const ColArgs* descs, const int2* items, int n,
-                            hipStream_t st);
+hipError_t launch_col_adj_multi(int NC, const ColArgs* descs, const int2* items, int n, hipStream_t st);
 hipError_t launch_combine_multi(const CombineArgs* descs, const int2* items, int n, hipStream_t st);
 hipError_t launch_sino_multi(int NR, const SinoArgs* descs, const int2* items, int n, hipStream_t st);
 hipError_t launch_reproj_multi(int NR, const ReprojArgs* descs, const int2* items, int n, hipStream_t st);
@@ -294,6 +293,6 @@ bool col_config_ok(int NC, int C, int K);
 // A column tile of C grid columns usable on an n0 x n1 grid with K taps.
 bool col_tile_ok(int NC, int n1, int C, int K);
 hipError_t set_col_attrs(int NC, int C, int K);
-hipError_t set_col_multi_attrs(int NC, int C, int K);
+hipError_t set_col_adj_multi_attrs();
 
 }  // namespace icon

@@ -1352,48 +1352,19 @@ hipError_t launch_reproj_multi(int NR, const ReprojArgs* descs, const int2* item
   return hipGetLastError();
 }
 
-template <int NC, int C, int K>
-static hipError_t col_multi_attr() {
-  static bool done = false;
-  if (!done) {
-    hipError_t e = hipFuncSetAttribute((const void*)k_col_fwd_multi<NC, C, K>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, col_lds<NC, C>() * (int)sizeof(float2));
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)k_col_adj_multi<NC, C, K>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            col_lds<NC, C>() * (int)sizeof(float2));
-    if (e != hipSuccess) return e;
-    done = true;
-  }
-  return hipSuccess;
+// The packed data adjoint in single precision: at n0 = 2048, where there is none
+// in FP64.
+hipError_t set_col_adj_multi_attrs() {
+  return hipFuncSetAttribute((const void*)k_col_adj_multi<2048, 8, 10>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             col_lds<2048, 8>() * (int)sizeof(float2));
 }
 
-hipError_t set_col_multi_attrs(int NC, int C, int K) {
-#define CASE(N, CC, KK) \
-  if (NC == N && C == CC && K == KK) return col_multi_attr<N, CC, KK>();
-  COL_CASES(CASE)
-#undef CASE
-  return hipErrorInvalidValue;
-}
-
-hipError_t launch_col_multi(int NC, int C, int K, bool adjoint, const ColArgs* descs, const int2* items, int n,
-                            hipStream_t st) {
+hipError_t launch_col_adj_multi(int NC, const ColArgs* descs, const int2* items, int n, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  hipError_t e = hipErrorInvalidValue;
-#define CASE(N, CC, KK)                                                                                   \
-  if (NC == N && C == CC && K == KK) {                                                                    \
-    e = col_multi_attr<N, CC, KK>();                                                                      \
-    if (e != hipSuccess) return e;                                                                        \
-    if (adjoint)                                                                                          \
-      LAUNCH_TIMED((k_col_adj_multi<N, CC, KK>), dim3(n), dim3(CC * (N / 16)),                            \
-                   (col_lds<N, CC>()) * sizeof(float2), st, descs, items);                                \
-    else                                                                                                  \
-      LAUNCH_TIMED((k_col_fwd_multi<N, CC, KK>), dim3(n), dim3(CC * (N / 16)),                            \
-                   (col_lds<N, CC>()) * sizeof(float2), st, descs, items);                                \
-    return hipGetLastError();                                                                             \
-  }
-  COL_CASES(CASE)
-#undef CASE
-  return e;
+  if (NC != 2048) return hipErrorInvalidValue;
+  LAUNCH_TIMED((k_col_adj_multi<2048, 8, 10>), dim3(n), dim3(8 * (2048 / 16)), (col_lds<2048, 8>()) * sizeof(float2),
+               st, descs, items);
+  return hipGetLastError();
 }
 
 hipError_t launch_combine_multi(const CombineArgs* descs, const int2* items, int n, hipStream_t st) {

@@ -319,7 +319,8 @@ class Plan:
         self.info.col_block = int(c)
 
     def autotune(self, S):
-        """Picks the fastest column tile for S slices; returns (C, {C: ms per iteration's column kernels})."""
+        """Picks the transforms' fastest column tile for S slices; returns (C, {C: ms of a forward and an
+        adjoint transform's column kernels})."""
         c = ctypes.c_int(0)
         ms = (ctypes.c_double * 2)()
         _check(lib().icon_plan_autotune(self.h, int(S), ctypes.byref(c), ms), "icon_plan_autotune")
@@ -477,7 +478,7 @@ class Batch:
         return v.value
 
     def autotune(self):
-        """Column tile per size class; returns the tile chosen for each series."""
+        """Column tile of every plan's transforms (Plan.autotune); returns the tile chosen for each series."""
         out = (ctypes.c_int * len(self.plans))()
         _check(lib().icon_batch_autotune(self.h, out), "icon_batch_autotune")
         for p, c in zip(self.plans, out):

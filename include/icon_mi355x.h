@@ -132,15 +132,15 @@ int icon_plan_create_window(icon_plan** plan, int device, int nx, int thickness,
                             const float* tilt_deg, int max_slices, int cross_validation, int window);
 int icon_plan_destroy(icon_plan* plan);
 int icon_plan_get_info(const icon_plan* plan, icon_plan_info* info);
-/* Tune the spread/interp column tile (8 or 16 grid columns); rebuilds the
- * bin lists.  Optional. */
+/* Column tile of the plan's transforms (icon_nufft_*): 8 or 16 grid columns per
+ * spread/interpolation tile; rebuilds their bin lists.  Solves do not depend on
+ * it.  Optional. */
 int icon_plan_set_col_block(icon_plan* plan, int col_block);
-/* Autotuner of the column tile (the spread/interpolation tile and bin width):
- * times one iteration's column kernels (2 interpolations + 1 spread, each
- * after its predecessor) over S slices for every tile width the plan's grid
- * and window support, keeps the fastest and reports it in *col_block and, if
- * ms_per_width is not NULL, the measured ms in ms_per_width[0] (C = 8) and
- * [1] (C = 16, or 0 when unsupported).  Overwrites the solve buffers, like
+/* Autotuner of that tile: times the column kernels of a forward and an adjoint
+ * transform of S slices for every tile width the plan's grid and window
+ * support, keeps the fastest and reports it in *col_block and, if ms_per_width
+ * is not NULL, the measured ms (forward + adjoint) in ms_per_width[0] (C = 8)
+ * and [1] (C = 16, or 0 when unsupported).  Overwrites the solve buffers, like
  * icon_time_kernel.  No counterpart in the reference. */
 int icon_plan_autotune(icon_plan* plan, int S, int* col_block, double* ms_per_width);
 
@@ -216,12 +216,10 @@ int icon_batch_reconstruct(icon_batch* batch, const void* const* d_sino, void* c
                            void* const* d_alpha, const icon_solve_opts* opts, void* stream);
 /* Kernel launches of one iteration of the packed solve. */
 int icon_batch_launches_per_iteration(const icon_batch* batch, int* launches);
-/* Autotuner of the column tile (the spread/interpolation tile and bin width)
- * per column size class: times the class's packed interpolation and spread
- * launches for every tile width it supports and keeps the fastest for all
- * its plans; col_blocks (nseries entries, or NULL) receives the choice per
- * series.  Overwrites the plans' solve buffers.  No counterpart in the
- * reference. */
+/* icon_plan_autotune of every series' plan over its slices (the packed solve
+ * itself does not depend on the tile); col_blocks (nseries entries, or NULL)
+ * receives the choice per series.  Waits for the batch's solves and overwrites
+ * the plans' solve buffers.  No counterpart in the reference. */
 int icon_batch_autotune(icon_batch* batch, int* col_blocks);
 
 /* ---- host-only helpers (no device needed) -------------------------------- */

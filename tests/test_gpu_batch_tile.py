@@ -1,7 +1,9 @@
 """A packed solve's captured graph outlives changes of its plans' column tile:
 the tile is set to another width and back, with other allocations in between
 that take freed memory, and to the width that it has; the next solves, with
-the plans' tables at either width, must give the first one's bits.
+the plans' tables at either width, must give the first one's bits.  The batch
+autotuner tunes every plan's transforms, 6-tap ones too, and leaves the packed
+solve's bits.
 """
 import numpy as np
 import pytest
@@ -39,4 +41,23 @@ def test_packed_solve_after_tile_changes(icon):
         print("  tiles %s: same bits" % (tiles,), flush=True)
     with pytest.raises(icon.IconError):
         plans[2].set_col_block(16)
+    batch.close()
+
+
+def test_batch_autotune_keeps_bits(icon):
+    print("packed solve before and after the batch autotuner", flush=True)
+    cfg = [(200, "gauss"), (512, "gauss"), (900, "gauss"), (256, "kb6"), (256, "gauss")]
+    tilt, rng, S = phantom.tilt_series(60, 4), np.random.default_rng(78), 2
+    plans = [icon.Plan(N, tilt, max_slices=S, window=w) for N, w in cfg]
+    sinos = [rng.standard_normal((S, len(tilt), N)).astype(np.float32) for N, _ in cfg]
+    batch = icon.Batch(plans, [S] * len(plans))
+    before = batch.solve(sinos, 2, 4, 2, trace=True)
+    tiles = batch.autotune()
+    print("  tiles", tiles, flush=True)
+    assert all(t in ((8, 16) if N <= 512 and w == "gauss" else (8,)) for t, (N, w) in zip(tiles, cfg))
+    assert [p.info.col_block for p in plans] == tiles
+    after = batch.solve(sinos, 2, 4, 2, trace=True)
+    for k in (0, 1):
+        for a, b in zip(after[k], before[k]):
+            np.testing.assert_array_equal(a, b)
     batch.close()
