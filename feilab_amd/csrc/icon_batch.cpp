@@ -318,7 +318,7 @@ int enqueue_batch(icon_batch* b, float* const* m, const float* const* m_init, bo
   };
   auto finish = [&](int ri, int ai, bool with_frep, int beff) -> int {
     FinishLaunch L{any_resid ? ri : -1, ai, with_frep ? 1 : 0, beff, 1};
-    for (const FinishArgs& f : b->h_fa) L.groups = std::max(L.groups, f.groups);
+    for (const FinishArgs& f : b->h_fa) L.blocks = std::max(L.blocks, f.blocks);
     return ck(launch_finish_multi(b->d_fa, b->combine.d, b->combine.n(), L, st), "finish");
   };
   // data set-up: b, w b, bnorm, A^H W b

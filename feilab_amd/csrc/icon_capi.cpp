@@ -652,11 +652,12 @@ FinishArgs icon::finish_args(const icon_plan* p, int S) {
   a.slots = kNodeSlots; a.part = p->d_part; a.nslot = p->d_nd_nslot;
   a.w = p->d_w; a.b = p->d_b; a.bnorm = p->d_bnorm; a.iomit = g.iomit;
   a.rowpart = p->d_rowpart; a.epart = p->d_epart;
-  // one round of 4 rows per thread while blocks are fewer than CUs (16 slices of
-  // 1007^2, 61400 nodes: 73 -> 17 us with 15 blocks per slice; 256 slices of
-  // 512^2: 36 us with one, 41 with three)
+  // one round of 4 rows per thread, and a block for each while blocks are fewer
+  // than CUs (16 slices of 1007^2, 61400 nodes: 73 -> 17 us with 15 blocks per
+  // slice; 256 slices of 512^2: 36 us with one, 41 with three)
   a.rsum = p->d_rsum; a.rcnt = p->d_rcnt;
-  a.groups = std::max(1, std::min({kFinishGroups, (a.M + 4095) / 4096, p->cus / S}));
+  a.groups = std::max(1, std::min(kFinishGroups, (a.M + kFinishRows - 1) / kFinishRows));
+  a.blocks = std::max(1, std::min(a.groups, p->cus / S));
   a.nq = p->nq; a.rpart = p->d_rpart; a.rslot = p->d_nq_nslot; a.gram = p->d_gram;
   return a;
 }

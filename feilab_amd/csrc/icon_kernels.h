@@ -115,6 +115,7 @@ constexpr int kMaxUnpaired = 256;
 // End of an iteration: the data residual of the image (from the node partials
 // of A m) and the step size of the gradient.
 constexpr int kFinishGroups = 16;
+constexpr int kFinishRows = 4096;   // rows of a group's round
 struct FinishArgs {
   int S, M, N0, nblk, nrow;   // M: rows of part per slice
   int Mb;                // nodes per slice in b
@@ -125,8 +126,9 @@ struct FinishArgs {
   const float2* b;       // [S][Mb]
   const double* bnorm;   // [S]
   unsigned long long* rsum;   // [S][kFinishGroups] sums of the residual's row groups (double bits)
-  unsigned* rcnt;             // [S] groups done, zero between launches
-  int groups;                 // blocks per slice over the residual's rows, at most kFinishGroups
+  unsigned* rcnt;             // [S] blocks done, zero between launches
+  int groups;                 // groups of the residual's rows, at most kFinishGroups
+  int blocks;                 // blocks per slice that share them, at most groups
   double* resid;         // trace base or null
   int resid_stride, resid_index;
   float2* frep;          // [S][N0] values of A m at the omit tilt, or null
@@ -180,7 +182,7 @@ struct FinishLaunch {
   int resid_index, alpha_index;   // < 0: no residual / no step size
   int with_frep;                  // 0: the series' frep pointers are ignored
   int beff;                       // 0: not used; 1: written; 2: read in place of b
-  int groups;                     // the largest of the series' groups
+  int blocks;                     // the largest of the series' blocks
 };
 
 // While set (non-null) on the calling thread, the next launches of the

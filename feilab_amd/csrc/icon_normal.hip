@@ -639,15 +639,17 @@ __device__ __forceinline__ int node_of(const FinishArgs& a, int r, int* jm) {
 // role 0: alpha = |rhat|^2 / <rhat, A^H W A rhat>; role 1: the data residual
 // R = sqrt(sum w |A m - b|^2 / sum w |b|^2) and the values at the omit tilt.
 // One block per (slice, role); FP64 sums in a fixed order.
-// Role 1 is shared among a.groups blocks per slice: the last to finish adds
-// their sums in order (rsum) and leaves their counter (rcnt) at zero again.  The
-// blocks exchange nothing but device-scope read-modify-writes, the store of a
-// sum waited for before the count.
-__device__ __forceinline__ void finish_body(const FinishArgs& a, int s, int role, int grp) {
+// Role 1 sums a.groups groups of rows, as many as the geometry asks for, and adds
+// the groups' sums in order, whether one block takes all of them or a.blocks
+// blocks per slice share them: the residual's bits do not depend on the number
+// of slices.  Of several blocks the last to finish adds the sums (rsum) and
+// leaves their counter (rcnt) at zero again.  The blocks exchange nothing but
+// device-scope read-modify-writes, the store of a sum waited for before the
+// count.
+__device__ __forceinline__ void finish_body(const FinishArgs& a, int s, int role, int blk) {
   __shared__ double red[32];
   __shared__ double z[4 * kMaxUnpaired];
   const int tid = threadIdx.x;
-  double acc = 0.0;
   const float2* P = a.part + (size_t)s * a.M * a.slots;
   // One block per slice waits on its loads: each round issues those of several
   // elements together (one 256^2 slice, 61 tilts: 12.5 -> 8.2 us;
@@ -711,78 +713,102 @@ __device__ __forceinline__ void finish_body(const FinishArgs& a, int s, int role
     return;
   }
   constexpr int U = 4, SL = 4;   // rows a round; partials loaded together (a.slots of them at most)
-  for (int r0 = grp * U * 1024 + tid; r0 < a.M; r0 += a.groups * U * 1024) {
-    float2 p[U][SL], b0[U], b1[U];
-    float w0[U], w1[U];
-    int j[U], jm[U], ns[U];
+  double* gsum = z;              // [group][wavefront], then the groups' sums
+  static_assert(kFinishRows == U * 1024 && 17 * kFinishGroups <= 4 * kMaxUnpaired, "a group's round; the sums fit z");
+  for (int g = blk; g < a.groups; g += a.blocks) {
+    double acc = 0.0;
+    for (int r0 = g * U * 1024 + tid; r0 < a.M; r0 += a.groups * U * 1024) {
+      float2 p[U][SL], b0[U], b1[U];
+      float w0[U], w1[U];
+      int j[U], jm[U], ns[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const bool in = r0 + u * 1024 < a.M;
-      const int r = in ? r0 + u * 1024 : r0;
-      j[u] = node_of(a, r, &jm[u]);
-      if (!in) j[u] = jm[u] = -1;
-      ns[u] = a.nslot[r];
+      for (int u = 0; u < U; u++) {
+        const bool in = r0 + u * 1024 < a.M;
+        const int r = in ? r0 + u * 1024 : r0;
+        j[u] = node_of(a, r, &jm[u]);
+        if (!in) j[u] = jm[u] = -1;
+        ns[u] = a.nslot[r];
 #pragma unroll
-      for (int q = 0; q < SL; q++) p[u][q] = P[(size_t)r * a.slots + min(q, a.slots - 1)];
-      const int k0 = max(j[u], 0), k1 = max(jm[u], 0);
-      w0[u] = a.w[k0];
-      w1[u] = a.w[k1];
-      if (a.resid) {
-        b0[u] = a.b[(size_t)s * a.Mb + k0];
-        b1[u] = a.b[(size_t)s * a.Mb + k1];
+        for (int q = 0; q < SL; q++) p[u][q] = P[(size_t)r * a.slots + min(q, a.slots - 1)];
+        const int k0 = max(j[u], 0), k1 = max(jm[u], 0);
+        w0[u] = a.w[k0];
+        w1[u] = a.w[k1];
+        if (a.resid) {
+          b0[u] = a.b[(size_t)s * a.Mb + k0];
+          b1[u] = a.b[(size_t)s * a.Mb + k1];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (j[u] < 0) continue;
+        // as node_value: the partials in slot order
+        float2 f = p[u][0];
+#pragma unroll
+        for (int q = 1; q < SL; q++)
+          if (q < ns[u]) {
+            f.x += p[u][q].x;
+            f.y += p[u][q].y;
+          }
+        if (a.resid) {
+          const double dx = (double)f.x - (double)b0[u].x, dy = (double)f.y - (double)b0[u].y;
+          acc += (double)w0[u] * (dx * dx + dy * dy);
+          if (a.beff) a.beff[(size_t)s * a.Mb + j[u]] = make_float2((float)-dx, (float)-dy);
+          if (jm[u] >= 0) {
+            const double ex = (double)f.x - (double)b1[u].x, ey = (double)f.y + (double)b1[u].y;
+            acc += (double)w1[u] * (ex * ex + ey * ey);
+            if (a.beff) a.beff[(size_t)s * a.Mb + jm[u]] = make_float2((float)-ex, (float)ey);
+          }
+        }
+        if (a.frep) {
+          const int i = j[u] / a.N0;
+          if (i == a.iomit) {
+            a.frep[(size_t)s * a.N0 + (j[u] - i * a.N0)] = f;
+            if (jm[u] >= 0) a.frep[(size_t)s * a.N0 + (jm[u] - i * a.N0)] = make_float2(f.x, -f.y);
+          }
+        }
       }
     }
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (j[u] < 0) continue;
-      // as node_value: the partials in slot order
-      float2 f = p[u][0];
-#pragma unroll
-      for (int q = 1; q < SL; q++)
-        if (q < ns[u]) {
-          f.x += p[u][q].x;
-          f.y += p[u][q].y;
-        }
-      if (a.resid) {
-        const double dx = (double)f.x - (double)b0[u].x, dy = (double)f.y - (double)b0[u].y;
-        acc += (double)w0[u] * (dx * dx + dy * dy);
-        if (a.beff) a.beff[(size_t)s * a.Mb + j[u]] = make_float2((float)-dx, (float)-dy);
-        if (jm[u] >= 0) {
-          const double ex = (double)f.x - (double)b1[u].x, ey = (double)f.y + (double)b1[u].y;
-          acc += (double)w1[u] * (ex * ex + ey * ey);
-          if (a.beff) a.beff[(size_t)s * a.Mb + jm[u]] = make_float2((float)-ex, (float)ey);
-        }
-      }
-      if (a.frep) {
-        const int i = j[u] / a.N0;
-        if (i == a.iomit) {
-          a.frep[(size_t)s * a.N0 + (j[u] - i * a.N0)] = f;
-          if (jm[u] >= 0) a.frep[(size_t)s * a.N0 + (jm[u] - i * a.N0)] = make_float2(f.x, -f.y);
-        }
-      }
-    }
+    for (int h = 32; h > 0; h >>= 1) acc += __shfl_down(acc, h);
+    if ((tid & 63) == 0) gsum[16 * g + (tid >> 6)] = acc;
   }
   if (!a.resid) return;
-  double tot = block_sum_1024(acc, red);
-  if (tid == 0) {
-    if (a.groups > 1) {
-      unsigned long long* q = a.rsum + (size_t)s * kFinishGroups;
-      const unsigned long long old = atomicExch(q + grp, (unsigned long long)__double_as_longlong(tot));
+  __syncthreads();
+  if (tid >= 64) return;
+  // the first wavefront: thread g the sum of group g, thread 0 their sum
+  double* sums = gsum + 16 * kFinishGroups;
+  if (tid < a.groups && tid % a.blocks == blk) {
+    double t = gsum[16 * tid];
+#pragma unroll
+    for (int w = 1; w < 16; w++) t += gsum[16 * tid + w];
+    if (a.blocks > 1) {
+      const unsigned long long old =
+          atomicExch(a.rsum + (size_t)s * kFinishGroups + tid, (unsigned long long)__double_as_longlong(t));
       asm volatile("" ::"v"((unsigned)old) : "memory");
-      if (atomicAdd(a.rcnt + s, 1u) != (unsigned)a.groups - 1) return;
+    } else {
+      sums[tid] = t;
+    }
+  }
+  line_sync<1>();
+  if (tid == 0) {
+    double tot = 0.0;
+    if (a.blocks > 1) {
+      unsigned long long* q = a.rsum + (size_t)s * kFinishGroups;
+      if (atomicAdd(a.rcnt + s, 1u) != (unsigned)a.blocks - 1) return;
       unsigned long long v[kFinishGroups];
       for (int k = 0; k < a.groups; k++) v[k] = atomicAdd(q + k, 0ull);
-      tot = 0.0;
       for (int k = 0; k < a.groups; k++) tot += __longlong_as_double((long long)v[k]);
       atomicExch(a.rcnt + s, 0u);
+    } else {
+      for (int k = 0; k < a.groups; k++) tot += sums[k];
     }
     const double bn = a.bnorm[s];
     a.resid[(size_t)s * a.resid_stride + a.resid_index] = bn > 0 ? sqrt(tot / bn) : 0.0;
   }
 }
 
-// blocks [0, S): the step size where asked for (alpha non-null); then S blocks
-// per group of the residual's rows
+// blocks [0, S): the step size where asked for (alpha non-null); then a.blocks
+// times S blocks for the residual's rows
 __global__ __launch_bounds__(1024) void k_finish(FinishArgs a) {
   const int k = (int)blockIdx.x / a.S - (a.alpha ? 1 : 0);
   finish_body(a, blockIdx.x % a.S, k < 0 ? 0 : 1, k);
@@ -799,7 +825,7 @@ __global__ __launch_bounds__(1024) void k_finish_multi(const FinishArgs* __restr
   if (L.beff == 2 && a.beff) a.b = a.beff;
   if (L.beff != 1) a.beff = nullptr;
   const int k = (int)blockIdx.x / n - (L.alpha_index >= 0 ? 1 : 0);
-  if (k >= 0 && ((!a.resid && !a.frep) || k >= a.groups)) return;
+  if (k >= 0 && ((!a.resid && !a.frep) || k >= a.blocks)) return;
   finish_body(a, it.y, k < 0 ? 0 : 1, k);
 }
 
@@ -1245,7 +1271,7 @@ hipError_t launch_row_grad64_multi(int NR, bool half, const RefArgs* descs, cons
 }
 
 hipError_t launch_finish(const FinishArgs& a, hipStream_t st) {
-  const int roles = (a.alpha ? 1 : 0) + (a.resid || a.frep ? a.groups : 0);
+  const int roles = (a.alpha ? 1 : 0) + (a.resid || a.frep ? a.blocks : 0);
   if (!roles) return hipSuccess;
   LAUNCH_TIMED(k_finish, dim3(roles * a.S), dim3(1024), 0, st, a);
   return hipGetLastError();
@@ -1253,7 +1279,7 @@ hipError_t launch_finish(const FinishArgs& a, hipStream_t st) {
 
 hipError_t launch_finish_multi(const FinishArgs* descs, const int2* items, int n, const FinishLaunch& L,
                                hipStream_t st) {
-  const int roles = (L.alpha_index >= 0 ? 1 : 0) + (L.resid_index >= 0 || L.with_frep ? L.groups : 0);
+  const int roles = (L.alpha_index >= 0 ? 1 : 0) + (L.resid_index >= 0 || L.with_frep ? L.blocks : 0);
   if (n <= 0 || !roles) return hipSuccess;
   LAUNCH_TIMED(k_finish_multi, dim3(roles * n), dim3(1024), 0, st, descs, items, n, L);
   return hipGetLastError();
