@@ -893,9 +893,9 @@ int plan_create(icon_plan** out, int device, int nx, int thickness, int nz, cons
   if ((rc = build_normal(p))) return bail(rc);
   if ((rc = dalloc(p, &p->d_part, S * std::max(M * kMaxSlot, (size_t)p->rows * kNodeSlots)))) return bail(rc);
   if ((rc = dalloc(p, &p->d_ahwb, p->half ? (S * NN + 1) / 2 : S * NN))) return bail(rc);
-  if ((rc = dalloc(p, &p->d_base, p->half ? (S * NN + 1) / 2 : S * NN))) return bail(rc);
-  if ((rc = dalloc(p, &p->d_mref, S * NN))) return bail(rc);
-  if ((rc = dalloc(p, &p->d_beff, S * M))) return bail(rc);
+  if (p->refreshes() && ((rc = dalloc(p, &p->d_base, p->half ? (S * NN + 1) / 2 : S * NN)) ||
+                         (rc = dalloc(p, &p->d_mref, S * NN)) || (rc = dalloc(p, &p->d_beff, S * M))))
+    return bail(rc);
   // the grid rows, in single precision or (the FP64 gradients) in double
   if ((rc = dalloc(p, &p->d_tmp, S * g.N0 * (size_t)g.n1 * (p->refreshes() ? 2 : 1)))) return bail(rc);
   {
