@@ -77,7 +77,10 @@ struct icon_batch {
   // across the class's series (each tile's blocks stay together)
   std::vector<Items> col_adj;
   std::vector<Items> normal;   // the normal operator's column kernels, by n0
-  std::vector<Items> row_grad, row64;   // the iteration's gradient; rows (or pairs) of the FP64 one
+  std::vector<Items> row_grad;
+  // FP64 passes over up to S64 slices of a series (key2: which): rows (or pairs) and
+  // columns; argument block pass * nseries + series
+  std::vector<Items> row64, normal64;
   Items combine;
   // argument blocks, one per series (device copies written before each solve)
   std::vector<RowFwdArgs> h_rf;
@@ -125,6 +128,11 @@ int upload_items(Items& it) {
   return ICON_OK;
 }
 
+// Slices that a series of S takes in one pass of its data adjoint and FP64
+// gradient; kPasses passes at most.
+constexpr int kPasses = 2;
+int pass_slices(const icon_plan* p, int S) { return p->refreshes() ? p->S64 : S; }
+
 // (series, block) items of every size class, built once: they depend on the
 // tables that a plan keeps for its life.
 int build_items(icon_batch* b) {
@@ -149,23 +157,27 @@ int build_items(icon_batch* b) {
     Items& rf = group(b->row_fwd, g.n1, half, r64ok);
     const int rpf = half ? 2 * half_row_pairs_per_block(g.n1) : row_fwd_rows_per_block(g.n1);
     for (int k = 0; k < (rows + rpf - 1) / rpf; k++) rf.h.push_back(make_int2(i, k));
-    // the data adjoint's rows: key1 1 in FP64 (one row per block)
-    const int a64 = adj64_ok(g.n0, sb.C, sb.K) ? 1 : 0;
-    Items& ra = group(b->row_adj, g.n1, a64, 0);
-    const int rpa = row_adj_rows_per_block(g.n1), rpd = a64 ? 1 : rpa;
-    for (int k = 0; k < (rows + rpd - 1) / rpd; k++) ra.h.push_back(make_int2(i, k));
-    if (r64ok) {
-      Items& r64 = group(b->row64, g.n1, half, 0);
-      for (int k = 0; k < (half ? rows / 2 : rows); k++) r64.h.push_back(make_int2(i, k));
+    const int rpa = row_adj_rows_per_block(g.n1);
+    if (!col_tile_ok(g.n0, g.n1, sb.C, sb.K))
+      return bfail(ICON_ERR_ARG, "series %d: column tile %d unsupported for grid %d x %d", i, sb.C, g.n0, g.n1);
+    // the data adjoint (key1 1: in FP64, one row per block) and the FP64 gradient
+    for (int c = 0, s0 = 0; s0 < S; c++, s0 += pass_slices(p, S)) {
+      const int n = std::min(pass_slices(p, S), S - s0), q = c * ns + i;
+      Items& ra = group(b->row_adj, g.n1, r64ok, c);
+      const int rpd = r64ok ? 1 : rpa;
+      for (int k = 0; k < (n * g.N0 + rpd - 1) / rpd; k++) ra.h.push_back(make_int2(q, k));
+      Items& cl = group(b->col_adj, g.n0, r64ok, c);
+      for (int k = 0; k < n * (g.n1 / sb.C); k++) cl.h.push_back(make_int2(q, k));
+      if (!r64ok) continue;
+      Items& r64 = group(b->row64, g.n1, half, c);
+      for (int k = 0; k < (half ? n * g.N0 / 2 : n * g.N0); k++) r64.h.push_back(make_int2(q, k));
+      Items& n64 = group(b->normal64, g.n0, 0, c);
+      for (int k = 0; k < n * (p->ncol / kNormalC); k++) n64.h.push_back(make_int2(q, k));
     }
     Items& rg = group(b->row_grad, g.n1, half, r64ok);
     const int rpg = half ? 2 * half_row_pairs_per_block(g.n1) : rpa;
     for (int k = 0; k < (rows + rpg - 1) / rpg; k++) rg.h.push_back(make_int2(i, k));
-    if (!col_tile_ok(g.n0, g.n1, sb.C, sb.K))
-      return bfail(ICON_ERR_ARG, "series %d: column tile %d unsupported for grid %d x %d", i, sb.C, g.n0, g.n1);
-    Items& cl = group(b->col_adj, g.n0, sb.C, sb.K);
-    for (int k = 0; k < S * (g.n1 / sb.C); k++) cl.h.push_back(make_int2(i, k));
-    Items& nm = group(b->normal, g.n0, 0, 0);
+    Items& nm = group(b->normal, g.n0, r64ok, 0);
     for (int k = 0; k < S * (p->ncol / kNormalC); k++) nm.h.push_back(make_int2(i, k));
     Items& sn = group(b->sino, g.n0, 0, 0);
     const int rps = sino_rows_per_block(g.n0);
@@ -176,17 +188,20 @@ int build_items(icon_batch* b) {
   }
   // the spread's order: a stable sort of each class's items by the entry
   // count of the tile the block runs (the plan's own largest-first tile order
-  // maps a series' block k to tile bins.order[k / S])
+  // maps a pass's block k to tile bins.order[k / its slices])
   for (Items& a : b->col_adj) {
     auto cnt = [&](const int2& q) {
-      const Bins& sb = b->plans[q.x]->spread().h;
-      const int t = sb.order[q.y / b->S[q.x]];
+      icon_plan* p = b->plans[q.x % ns];
+      const Bins& sb = p->spread().h;
+      const int S = b->S[q.x % ns], per = pass_slices(p, S), n = std::min(per, S - a.key2 * per);
+      const int t = sb.order[q.y / n];
       return sb.off[t + 1] - sb.off[t];
     };
     std::stable_sort(a.h.begin(), a.h.end(), [&](const int2& u, const int2& v) { return cnt(u) > cnt(v); });
   }
   int rc;
-  for (auto* v : {&b->row_fwd, &b->row_adj, &b->col_adj, &b->normal, &b->row_grad, &b->row64, &b->sino, &b->reproj})
+  for (auto* v : {&b->row_fwd, &b->row_adj, &b->col_adj, &b->normal, &b->row_grad, &b->row64, &b->normal64, &b->sino,
+                  &b->reproj})
     for (auto& it : *v)
       if ((rc = upload_items(it))) return rc;
   if ((rc = upload_items(b->combine))) return rc;
@@ -206,15 +221,15 @@ void fill_args(icon_batch* b, const float* const* sino, float* const* m, float* 
                double* const* alpha, int iters, bool any_resid) {
   const int ns = (int)b->plans.size();
   b->h_rf.assign(ns, RowFwdArgs{});
-  b->h_ra.assign(ns, RowAdjArgs{});
-  b->h_ca.assign(ns, ColArgs{});
   b->h_cm.assign(ns, CombineArgs{});
   b->h_sa.assign(ns, SinoArgs{});
   b->h_rp.assign(ns, ReprojArgs{});
   for (auto* v : {&b->h_rg, &b->h_rg2}) v->assign(ns, RowAdjArgs{});
   for (auto* v : {&b->h_rf2, &b->h_rr}) v->assign(ns, RowFwdArgs{});
-  b->h_re.assign(ns, RefArgs{});
-  for (auto* v : {&b->h_cn, &b->h_ce, &b->h_cl, &b->h_c64}) v->assign(ns, ColArgs{});
+  b->h_ra.assign(kPasses * ns, RowAdjArgs{});
+  b->h_re.assign(kPasses * ns, RefArgs{});
+  for (auto* v : {&b->h_ca, &b->h_c64}) v->assign(kPasses * ns, ColArgs{});
+  for (auto* v : {&b->h_cn, &b->h_ce, &b->h_cl}) v->assign(ns, ColArgs{});
   b->h_fa.assign(ns, FinishArgs{});
   for (int i = 0; i < ns; i++) {
     icon_plan* p = b->plans[i];
@@ -223,9 +238,6 @@ void fill_args(icon_batch* b, const float* const* sino, float* const* m, float* 
     RowFwdArgs& rf = b->h_rf[i];
     rf.rows = S * g.N0; rf.N0 = g.N0; rf.N1 = g.N1; rf.m = m[i]; rf.grad = p->d_grad; rf.alpha = p->d_alpha;
     rf.tw = p->d_tw1; rf.out = p->d_tmp;
-    // the adjoint of the data set-up, then the gradient
-    RowAdjArgs& ra = b->h_ra[i];
-    ra = data_row_args(p, S);
     b->h_rg[i] = grad_args(p, S);
     b->h_rg2[i] = b->h_rg[i];
     b->h_rf2[i] = rf;
@@ -235,9 +247,15 @@ void fill_args(icon_batch* b, const float* const* sino, float* const* m, float* 
       b->h_rf2[i].mref = p->d_mref;
     }
     b->h_rr[i] = rhat_row_args(p, S);
-    b->h_re[i] = ref_args(p, S, m[i]);
-    b->h_c64[i] = normal64_args(p, S, any_resid);
-    b->h_ca[i] = spread_args(p, S);
+    // the adjoint of the data set-up and the FP64 gradient, by passes
+    for (int s0 = 0, q = i; s0 < S; s0 += pass_slices(p, S), q += ns) {
+      const int n = std::min(pass_slices(p, S), S - s0);
+      b->h_ra[q] = data_row_args(p, s0, n);
+      b->h_ca[q] = spread_args(p, s0, n);
+      if (!p->refreshes()) continue;
+      b->h_re[q] = ref_args(p, s0, n, m[i]);
+      b->h_c64[q] = normal64_args(p, s0, n, any_resid);
+    }
     CombineArgs& cm = b->h_cm[i];
     cm.S = S; cm.M = g.M; cm.N0 = g.N0; cm.nz = g.nz; cm.mode = 2; cm.E = b->h_ca[i].E;
     cm.w = p->d_w; cm.b = p->d_b; cm.fw = p->d_fw; cm.ent_of_node = p->spread().of_node; cm.bnorm = p->d_bnorm;
@@ -291,7 +309,7 @@ int enqueue_batch(icon_batch* b, float* const* m, const float* const* m_init, bo
   auto gradient = [&](bool against_ref, int update, int which) -> int {
     if ((rc = row_fwd_all(against_ref ? b->d_rf2 : b->d_rf, update, which))) return rc;
     for (auto& nm : b->normal)
-      if (which < 0 || (nm.key0 <= 1024) == (which == 1))
+      if (which < 0 || nm.key1 == which)
         if ((rc = ck(launch_col_normal_multi(nm.key0, b->d_cn, nm.d, nm.n(), st), "col_normal"))) return rc;
     for (auto& it : b->row_grad) {
       if (which >= 0 && it.key2 != which) continue;
@@ -306,13 +324,17 @@ int enqueue_batch(icon_batch* b, float* const* m, const float* const* m_init, bo
   // series takes it
   auto reference = [&](int update) -> int {
     RowFwdLaunch L{0, update, o.data_type, o.threshold};
-    for (auto& it : b->row64)
-      if ((rc = ck(launch_row_fwd64_multi(it.key0, it.key1, b->d_re, it.d, it.n(), L, st), "row_fwd64"))) return rc;
-    for (auto& nm : b->normal)
-      if (nm.key0 <= 1024)
-        if ((rc = ck(launch_col_normal64_multi(nm.key0, b->d_c64, nm.d, nm.n(), st), "col_normal64"))) return rc;
-    for (auto& it : b->row64)
-      if ((rc = ck(launch_row_grad64_multi(it.key0, it.key1, b->d_re, it.d, it.n(), st), "row_grad64"))) return rc;
+    for (int c = 0; c < kPasses; c++) {
+      for (auto& it : b->row64)
+        if (it.key2 == c && (rc = ck(launch_row_fwd64_multi(it.key0, it.key1, b->d_re, it.d, it.n(), L, st), "row_fwd64")))
+          return rc;
+      for (auto& nm : b->normal64)
+        if (nm.key2 == c && (rc = ck(launch_col_normal64_multi(nm.key0, b->d_c64, nm.d, nm.n(), st), "col_normal64")))
+          return rc;
+      for (auto& it : b->row64)
+        if (it.key2 == c && (rc = ck(launch_row_grad64_multi(it.key0, it.key1, b->d_re, it.d, it.n(), st), "row_grad64")))
+          return rc;
+    }
     if ((rc = row_fwd_all(b->d_rr, 0, 1))) return rc;
     return gradient(false, update, 0);
   };
@@ -325,15 +347,17 @@ int enqueue_batch(icon_batch* b, float* const* m, const float* const* m_init, bo
   for (auto& it : b->sino)
     if ((rc = ck(launch_sino_multi(it.key0, b->d_sa, it.d, it.n(), st), "sino"))) return rc;
   if ((rc = ck(launch_combine_multi(b->d_cm, b->combine.d, b->combine.n(), st), "combine"))) return rc;
-  for (auto& it : b->col_adj)
-    if ((rc = ck(adj64_ok(it.key0, it.key1, it.key2)
-                     ? launch_col_adj64_multi(it.key0, it.key1, b->d_ca, it.d, it.n(), st)
-                     : launch_col_adj_multi(it.key0, b->d_ca, it.d, it.n(), st), "col_adj")))
-      return rc;
-  for (auto& it : b->row_adj)
-    if ((rc = ck(it.key1 ? launch_row_adj64_multi(it.key0, b->d_ra, it.d, it.n(), st)
-                         : launch_row_adj_multi(it.key0, b->d_ra, it.d, it.n(), false, st), "row_adj")))
-      return rc;
+  for (int c = 0; c < kPasses; c++) {
+    for (auto& it : b->col_adj)
+      if (it.key2 == c &&
+          (rc = ck(it.key1 ? launch_col_adj64_multi(it.key0, kSolveTile, b->d_ca, it.d, it.n(), st)
+                           : launch_col_adj_multi(it.key0, b->d_ca, it.d, it.n(), st), "col_adj")))
+        return rc;
+    for (auto& it : b->row_adj)
+      if (it.key2 == c && (rc = ck(it.key1 ? launch_row_adj64_multi(it.key0, b->d_ra, it.d, it.n(), st)
+                                           : launch_row_adj_multi(it.key0, b->d_ra, it.d, it.n(), false, st), "row_adj")))
+        return rc;
+  }
   // m = 0 or the warm start
   for (int i = 0; i < ns; i++) {
     const size_t n = (size_t)b->S[i] * b->plans[i]->g.N0 * b->plans[i]->g.N1;
@@ -382,6 +406,7 @@ int icon_batch_destroy(icon_batch* b) {
   free_items(b->normal);
   free_items(b->row_grad);
   free_items(b->row64);
+  free_items(b->normal64);
   free_items(b->sino);
   free_items(b->reproj);
   if (b->combine.d) (void)hipFree(b->combine.d);
@@ -428,8 +453,8 @@ int icon_batch_create(icon_batch** out, int nseries, icon_plan* const* plans, co
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev_in, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ev_out, hipEventDisableTiming);
   if (e == hipSuccess) e = hipMalloc(&b->d_rf, sizeof(RowFwdArgs) * nseries);
-  if (e == hipSuccess) e = hipMalloc(&b->d_ra, sizeof(RowAdjArgs) * nseries);
-  if (e == hipSuccess) e = hipMalloc(&b->d_ca, sizeof(ColArgs) * nseries);
+  if (e == hipSuccess) e = hipMalloc(&b->d_ra, sizeof(RowAdjArgs) * kPasses * nseries);
+  if (e == hipSuccess) e = hipMalloc(&b->d_ca, sizeof(ColArgs) * kPasses * nseries);
   if (e == hipSuccess) e = hipMalloc(&b->d_cm, sizeof(CombineArgs) * nseries);
   if (e == hipSuccess) e = hipMalloc(&b->d_sa, sizeof(SinoArgs) * nseries);
   if (e == hipSuccess) e = hipMalloc(&b->d_rp, sizeof(ReprojArgs) * nseries);
@@ -437,8 +462,9 @@ int icon_batch_create(icon_batch** out, int nseries, icon_plan* const* plans, co
   if (e == hipSuccess) e = hipMalloc(&b->d_rg2, sizeof(RowAdjArgs) * nseries);
   if (e == hipSuccess) e = hipMalloc(&b->d_rf2, sizeof(RowFwdArgs) * nseries);
   if (e == hipSuccess) e = hipMalloc(&b->d_rr, sizeof(RowFwdArgs) * nseries);
-  if (e == hipSuccess) e = hipMalloc(&b->d_re, sizeof(RefArgs) * nseries);
-  for (ColArgs** q : {&b->d_cn, &b->d_ce, &b->d_cl, &b->d_c64})
+  if (e == hipSuccess) e = hipMalloc(&b->d_re, sizeof(RefArgs) * kPasses * nseries);
+  if (e == hipSuccess) e = hipMalloc(&b->d_c64, sizeof(ColArgs) * kPasses * nseries);
+  for (ColArgs** q : {&b->d_cn, &b->d_ce, &b->d_cl})
     if (e == hipSuccess) e = hipMalloc(q, sizeof(ColArgs) * nseries);
   if (e == hipSuccess) e = hipMalloc(&b->d_fa, sizeof(FinishArgs) * nseries);
   if (e != hipSuccess) return done(bfail(ICON_ERR_DEVICE, "icon_batch_create: %s", hipGetErrorString(e)));

@@ -153,6 +153,12 @@ void dense_shares(const std::vector<int>& off, int round, std::vector<int>& part
 // threads of up to 128 registers per CU.
 long resident_tiles(const icon_plan* p, int C) { return (long)p->cus * std::max(1, 16384 / (C * p->g.n0)); }
 
+// Slices up to which split_dense shares the dense tiles' entries.
+int split_slices(const icon_plan* p) {
+  if (!p->nd_nx || !p->refreshes()) return 0;
+  return (int)std::min<long>(p->S_max, resident_tiles(p, kNormalC) / (p->ncol / kNormalC + p->nd_nx));
+}
+
 // Bins of a Kaiser-Bessel window of K taps in tiles of C columns; records and
 // deapodisation are computed on the device.
 int make_bins(icon_plan* p, DevBins& b, int C, int K) {
@@ -325,10 +331,14 @@ int op_sino(icon_plan* p, int S, const float* sino, float2* b, hipStream_t st) {
 int op_adjoint_data(icon_plan* p, int S, hipStream_t st) {
   const DevBins& b = p->spread();
   float* re = p->half ? reinterpret_cast<float*>(p->d_ahwb) : nullptr;
-  if (!adj64_ok(p->g.n0, b.h.C, b.h.K)) return op_adjoint_ent(p, b, S, re ? nullptr : p->d_ahwb, st, re);
-  int rc = check_launch(launch_col_adj64(p->g.n0, b.h.C, spread_args(p, S), st), "col_adj64");
-  if (rc) return rc;
-  return check_launch(launch_row_adj64(p->g.n1, data_row_args(p, S), st), "row_adj64");
+  if (!p->refreshes()) return op_adjoint_ent(p, b, S, re ? nullptr : p->d_ahwb, st, re);
+  for (int s0 = 0; s0 < S; s0 += p->S64) {
+    const int n = std::min(p->S64, S - s0);
+    int rc = check_launch(launch_col_adj64(p->g.n0, b.h.C, spread_args(p, s0, n), st), "col_adj64");
+    if (!rc) rc = check_launch(launch_row_adj64(p->g.n1, data_row_args(p, s0, n), st), "row_adj64");
+    if (rc) return rc;
+  }
+  return ICON_OK;
 }
 
 // An iteration's launches over S slices: with paired nodes the real-row
@@ -368,11 +378,9 @@ int enqueue_solve(icon_plan* p, int S, const float* sino, float* m, const float*
   rf.rows = S * g.N0; rf.N0 = g.N0; rf.N1 = g.N1; rf.data_type = o.data_type; rf.thr = o.threshold;
   rf.m = m; rf.grad = p->d_grad; rf.alpha = p->d_alpha; rf.tw = p->d_tw1; rf.out = p->d_tmp;
   ColArgs ca = normal_args(p, S, resid != nullptr);
-  const ColArgs ce = energy_args(p, S), c64 = normal64_args(p, S, resid != nullptr);
+  const ColArgs ce = energy_args(p, S);
   RowAdjArgs ra = grad_args(p, S);
   split_dense(p, S, ca, ra);
-  RefArgs rr = ref_args(p, S, m);
-  rr.data_type = o.data_type; rr.thr = o.threshold;
   FinishArgs fa = finish_args(p, S);
   fa.resid = resid; fa.resid_stride = iters + 1; fa.alpha = p->d_alpha; fa.alpha_trace = alpha_tr;
   fa.alpha_stride = iters;
@@ -384,10 +392,15 @@ int enqueue_solve(icon_plan* p, int S, const float* sino, float* m, const float*
     if (ref) {
       // the iterate's gradient in FP64, from the whole image; from here on the
       // transforms take the difference from it
-      rr.update = update;
-      if ((rc = check_launch(launch_row_fwd64(g.n1, p->half, rr, st), "row_fwd64"))) return rc;
-      if ((rc = check_launch(launch_col_normal64(g.n0, c64, st), "col_normal64"))) return rc;
-      if ((rc = check_launch(launch_row_grad64(g.n1, p->half, rr, st), "row_grad64"))) return rc;
+      for (int s0 = 0; s0 < S; s0 += p->S64) {
+        const int n = std::min(p->S64, S - s0);
+        RefArgs rr = ref_args(p, s0, n, m);
+        rr.update = update; rr.data_type = o.data_type; rr.thr = o.threshold;
+        const ColArgs c64 = normal64_args(p, s0, n, resid != nullptr);
+        if ((rc = check_launch(launch_row_fwd64(g.n1, p->half, rr, st), "row_fwd64"))) return rc;
+        if ((rc = check_launch(launch_col_normal64(g.n0, c64, st), "col_normal64"))) return rc;
+        if ((rc = check_launch(launch_row_grad64(g.n1, p->half, rr, st), "row_grad64"))) return rc;
+      }
       if ((rc = check_launch(iter_row_fwd(p, rhat_row_args(p, S), st), "row_fwd_rhat"))) return rc;
       rf.mref = p->d_mref;
       ra.ahwb = p->d_base;
@@ -556,20 +569,28 @@ ColArgs icon::energy_args(const icon_plan* p, int S) {
   return a;
 }
 
-ColArgs icon::normal64_args(const icon_plan* p, int S, bool with_nodes) {
+ColArgs icon::normal64_args(const icon_plan* p, int s0, int S, bool with_nodes) {
   ColArgs a = normal_args(p, S, with_nodes);
+  a.part += (size_t)s0 * a.M * a.slots;
   a.io64 = reinterpret_cast<double2*>(p->d_tmp);
   a.w64 = p->d_w640;
   return a;
 }
 
-RefArgs icon::ref_args(const icon_plan* p, int S, float* m) {
+RefArgs icon::ref_args(const icon_plan* p, int s0, int S, float* m) {
   const Geometry& g = p->g;
+  const size_t o = (size_t)s0 * g.N0 * g.N1;
   RefArgs a{};
-  a.rows = S * g.N0; a.N0 = g.N0; a.N1 = g.N1; a.ncol = p->ncol; a.m = m; a.mref = p->d_mref; a.alpha = p->d_alpha;
-  a.w64 = p->d_w641; a.io = reinterpret_cast<double2*>(p->d_tmp); a.ahwb = p->d_ahwb;
-  a.ahwb_re = reinterpret_cast<const float*>(p->d_ahwb); a.grad = p->d_grad; a.base = p->d_base;
-  a.base_re = reinterpret_cast<float*>(p->d_base); a.rowpart = p->d_rowpart;
+  a.rows = S * g.N0; a.N0 = g.N0; a.N1 = g.N1; a.ncol = p->ncol; a.m = m + o; a.mref = p->d_mref + o;
+  a.alpha = p->d_alpha + s0; a.w64 = p->d_w641; a.io = reinterpret_cast<double2*>(p->d_tmp); a.grad = p->d_grad + o;
+  a.rowpart = p->d_rowpart + (size_t)s0 * (p->half ? g.N0 / 2 : g.N0);
+  if (p->half) {
+    a.ahwb_re = reinterpret_cast<const float*>(p->d_ahwb) + o;
+    a.base_re = reinterpret_cast<float*>(p->d_base) + o;
+  } else {
+    a.ahwb = p->d_ahwb + o;
+    a.base = p->d_base + o;
+  }
   return a;
 }
 
@@ -599,20 +620,22 @@ RowFwdArgs icon::rhat_row_args(const icon_plan* p, int S) {
   return a;
 }
 
-ColArgs icon::spread_args(icon_plan* p, int S) {
+ColArgs icon::spread_args(icon_plan* p, int s0, int S) {
   ColArgs a = window_args(p, p->spread(), S);
+  a.fw += (size_t)s0 * a.E;
   a.io64 = reinterpret_cast<double2*>(p->d_tmp);
   a.w64 = p->d_w640;
   return a;
 }
 
-RowAdjArgs icon::data_row_args(icon_plan* p, int S) {
+RowAdjArgs icon::data_row_args(icon_plan* p, int s0, int S) {
   const Geometry& g = p->g;
+  const size_t o = (size_t)s0 * g.N0 * g.N1;
   RowAdjArgs a{};
   a.rows = S * g.N0; a.N0 = g.N0; a.N1 = g.N1; a.in = p->d_tmp; a.ck = p->spread().ck; a.tw = p->d_tw1;
   a.in64 = reinterpret_cast<const double2*>(p->d_tmp); a.w64 = p->d_w641;
-  if (p->half) a.img_re = reinterpret_cast<float*>(p->d_ahwb);
-  else a.img = p->d_ahwb;
+  if (p->half) a.img_re = reinterpret_cast<float*>(p->d_ahwb) + o;
+  else a.img = p->d_ahwb + o;
   zero_band(p->spread().h, &a.zlo, &a.zhi);
   return a;
 }
@@ -629,15 +652,12 @@ RowAdjArgs icon::grad_args(const icon_plan* p, int S) {
 // Few slices leave CUs idle while the tiles around ky = 0, which all tilt lines
 // cross, interpolate 6 and more rounds of entries (one 256^2 slice, 61 tilts:
 // 22 us instead of 10 for a tile without): their entries are shared among
-// further blocks, which transform the tile again.  The grid goes to the other
-// half of d_tmp, as those read the rows that the tile's own block would
-// overwrite.  Where all blocks are not resident at once they would cost more
-// than the wait.
+// further blocks, which transform the tile again.  The grid goes behind the rows
+// in d_tmp, as those blocks read the rows that the tile's own would overwrite.
+// Where all blocks are not resident at once they would cost more than the wait.
 void icon::split_dense(const icon_plan* p, int S, ColArgs& ca, RowAdjArgs& ra) {
   const Geometry& g = p->g;
-  if (ca.ent_off != p->d_nd_off || !p->nd_nx || !p->refreshes() ||
-      (long)S * (p->ncol / kNormalC + p->nd_nx) > resident_tiles(p, kNormalC))
-    return;
+  if (ca.ent_off != p->d_nd_off || S > split_slices(p)) return;
   ca.parts = p->d_nd_parts;
   ca.xt = p->d_nd_xt;
   ca.nx = p->nd_nx;
@@ -869,9 +889,6 @@ int plan_create(icon_plan** out, int device, int nx, int thickness, int nz, cons
   p->own_data = op_taps(g) != kTapsWide;
   if (p->own_data && (rc = make_bins(p, p->data, kSolveTile, kTapsWide))) return bail(rc);
   if ((rc = make_op_bins(p, default_col_block(g.n0)))) return bail(rc);
-  // (a tile of 16 columns has no more entries than the two of 8 that it covers)
-  const size_t E = std::max(p->op.h.ent.size(), p->data.h.ent.size());
-  if ((rc = dalloc(p, &p->d_fw, (size_t)p->S_max * E))) return bail(rc);
   if ((rc = twiddles(g.n0, &p->d_tw0))) return bail(rc);
   if ((rc = twiddles(g.n1, &p->d_tw1))) return bail(rc);
   if ((rc = twiddles64(g.n0, &p->d_w640))) return bail(rc);
@@ -892,12 +909,21 @@ int plan_create(icon_plan** out, int device, int nx, int thickness, int nz, cons
   if (p->own_data && (rc = prepare_col(g.n0, g.n1, p->data.h.C, p->data.h.K))) return bail(rc);
   if ((rc = build_normal(p))) return bail(rc);
   if ((rc = dalloc(p, &p->d_part, S * std::max(M * kMaxSlot, (size_t)p->rows * kNodeSlots)))) return bail(rc);
+  // weighted values are spread before, and in other calls than, any interpolation;
+  // a node has kMaxSlot entries at most, whatever the tile
+  p->d_fw = p->d_part;
   if ((rc = dalloc(p, &p->d_ahwb, p->half ? (S * NN + 1) / 2 : S * NN))) return bail(rc);
   if (p->refreshes() && ((rc = dalloc(p, &p->d_base, p->half ? (S * NN + 1) / 2 : S * NN)) ||
                          (rc = dalloc(p, &p->d_mref, S * NN)) || (rc = dalloc(p, &p->d_beff, S * M))))
     return bail(rc);
-  // the grid rows, in single precision or (the FP64 gradients) in double
-  if ((rc = dalloc(p, &p->d_tmp, S * g.N0 * (size_t)g.n1 * (p->refreshes() ? 2 : 1)))) return bail(rc);
+  // the grid rows, in single precision or, for FP64 passes, in double: in two
+  // passes where each still has slices for the whole device (64), so that a plan
+  // for many takes no more for them
+  p->S64 = max_slices < 128 ? max_slices : (max_slices + 1) / 2;
+  const size_t grid = (size_t)g.N0 * g.n1;
+  size_t tmp = S * grid + (size_t)split_slices(p) * g.N0 * p->ncol;
+  if (p->refreshes()) tmp = std::max(tmp, 2 * p->S64 * grid);
+  if ((rc = dalloc(p, &p->d_tmp, tmp))) return bail(rc);
   {
     const hipError_t e = set_adj64_attrs();
     if (e != hipSuccess) return bail(fail(ICON_ERR_DEVICE, "hipFuncSetAttribute: %s", hipGetErrorString(e)));
@@ -914,7 +940,7 @@ int icon_plan_destroy(icon_plan* p) {
   DevGuard dg(p->device);
   if (p->stream) (void)hipStreamSynchronize(p->stream);
   drop_graph(p);
-  void* ptrs[] = {p->d_nodes, p->d_ck1, p->d_w, p->d_phi1, p->d_i10, p->d_fw,
+  void* ptrs[] = {p->d_nodes, p->d_ck1, p->d_w, p->d_phi1, p->d_i10,
                   p->d_b, p->d_part, p->d_ahwb, p->d_grad, p->d_tmp, p->d_frep, p->d_rowpart,
                   p->d_bnorm, p->d_alpha, p->d_spec, p->d_nd_off, p->d_nd_ent, p->d_nd_parts, p->d_nd_xt, p->d_rsum, p->d_rcnt, p->d_nd_nslot, p->d_nd_px, p->d_nd_py,
                   p->d_epart, p->d_nq_off, p->d_nq_ent, p->d_nq_entr, p->d_nq_px, p->d_nq_py, p->d_nq_nslot,

@@ -261,7 +261,6 @@ hipError_t launch_col_fwd_nodes_multi(int NC, const ColArgs* descs, const int2* 
 hipError_t launch_col_fwd_nodes(int NC, const ColArgs& a, hipStream_t st);
 // A^H of the weighted data in FP64 (rows [S][N0][n1] in io64 / in64)
 hipError_t set_adj64_attrs();
-bool adj64_ok(int NC, int C, int K);
 hipError_t launch_col_adj64(int NC, int C, const ColArgs& a, hipStream_t st);
 hipError_t launch_row_adj64(int NR, const RowAdjArgs& a, hipStream_t st);
 hipError_t launch_col_adj64_multi(int NC, int C, const ColArgs* descs, const int2* items, int n, hipStream_t st);

@@ -1153,13 +1153,6 @@ hipError_t set_adj64_attrs() {
   return hipSuccess;
 }
 
-bool adj64_ok(int NC, int C, int K) {
-#define CASE(N, CC) if (NC == N && C == CC) return K == 10;
-  COL64_CASES(CASE)
-#undef CASE
-  return false;
-}
-
 hipError_t launch_col_adj64(int NC, int C, const ColArgs& a, hipStream_t st) {
 #define CASE(N, CC)                                                                                    \
   if (NC == N && C == CC) {                                                                            \

@@ -210,6 +210,9 @@ struct icon_plan {
   // registers, 424 bytes of scratch per lane) ended in a memory aperture
   // violation inside a packed graph; its indexes are in bounds on the CPU
   bool refreshes() const { return g.n0 <= 1024; }
+  // slices that an FP64 pass takes at once: the grid rows in double of half the
+  // slices fit the room of all in single precision
+  int S64 = 0;
   int* d_nq_off = nullptr;          // unpaired nodes: entries (rows of d_part / of d_rpart), records
   int4* d_nq_ent = nullptr;
   int4* d_nq_entr = nullptr;
@@ -235,11 +238,13 @@ struct icon_plan {
   const float2* d_tw1 = nullptr;    // twiddles for n1
   // per-slice work buffers (capacity S_max)
   float2* d_b = nullptr;            // [S][M] Fourier-slice data
-  float2* d_fw = nullptr;           // [S][E] weighted node value of every bin entry (of op or spread())
   float2* d_part = nullptr;         // [S][M][kMaxSlot] interpolation partials
+  float2* d_fw = nullptr;           // the same room, [S][E]: weighted node value of every bin entry (op's or spread()'s)
   float2* d_ahwb = nullptr;         // [S][N0][N1]
   float* d_grad = nullptr;          // [S][N0][N1] Re(rhat), the gradient the update takes
-  float2* d_tmp = nullptr;          // [S][N0][n1] row-transform intermediate, in single or double precision
+  // [S][N0][n1] row-transform intermediate, or [S64][N0][n1] in double; then room
+  // for the grid rows of few slices in split_dense
+  float2* d_tmp = nullptr;
   // the reference iterate of the solve's differences: image, -rhat (half: real), b - A m
   float* d_mref = nullptr;
   float2* d_base = nullptr;
@@ -269,11 +274,12 @@ ColArgs normal_args(const icon_plan* p, int S, bool with_nodes);
 ColArgs energy_args(const icon_plan* p, int S);
 RowAdjArgs grad_args(const icon_plan* p, int S);
 void split_dense(const icon_plan* p, int S, ColArgs& ca, RowAdjArgs& ra);
-ColArgs normal64_args(const icon_plan* p, int S, bool with_nodes);
-RefArgs ref_args(const icon_plan* p, int S, float* m);
+// (of S slices from s0 on, at most S64: an FP64 pass)
+ColArgs normal64_args(const icon_plan* p, int s0, int S, bool with_nodes);
+RefArgs ref_args(const icon_plan* p, int s0, int S, float* m);
 RowFwdArgs rhat_row_args(const icon_plan* p, int S);
 bool refresh(const icon_plan* p, const icon_solve_opts& o, int it);
 FinishArgs finish_args(const icon_plan* p, int S);
-ColArgs spread_args(icon_plan* p, int S);   // of the data set-up
-RowAdjArgs data_row_args(icon_plan* p, int S);
+ColArgs spread_args(icon_plan* p, int s0, int S);   // of the data set-up
+RowAdjArgs data_row_args(icon_plan* p, int s0, int S);
 }  // namespace icon
