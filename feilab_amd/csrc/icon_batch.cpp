@@ -270,9 +270,7 @@ void fill_args(icon_batch* b, const float* const* sino, float* const* m, float* 
     SinoArgs& sa = b->h_sa[i];
     sa.rows = S * g.nz; sa.N0 = g.N0; sa.K = g.K; sa.nz = g.nz; sa.skip = g.cv_skip; sa.sino = sino[i];
     sa.ck1 = p->d_ck1; sa.phi1 = p->d_phi1; sa.i10 = p->d_i10; sa.tw = p->d_tw0; sa.b = p->d_b;
-    ReprojArgs& rp = b->h_rp[i];
-    rp.S = S; rp.N0 = g.N0; rp.K = g.K; rp.sigma = g.sig0; rp.frep = p->d_frep; rp.ck1 = p->d_ck1;
-    rp.phi1 = p->d_phi1; rp.i10 = p->d_i10; rp.tw = p->d_tw0; rp.out = reproj ? reproj[i] : nullptr;
+    b->h_rp[i] = reproj_args(p, S, reproj ? reproj[i] : nullptr);
   }
 }
 

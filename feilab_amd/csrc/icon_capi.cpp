@@ -441,11 +441,7 @@ int enqueue_solve(icon_plan* p, int S, const float* sino, float* m, const float*
     fa.frep = reproj ? p->d_frep : nullptr;
     if ((rc = check_launch(launch_finish(fa, st), "finish_final"))) return rc;
     if (reproj) {
-      ReprojArgs rp{};
-      rp.K = p->g.K;
-      rp.S = S; rp.N0 = g.N0; rp.sigma = g.sig0; rp.frep = p->d_frep; rp.ck1 = p->d_ck1;
-      rp.phi1 = p->d_phi1; rp.i10 = p->d_i10; rp.tw = p->d_tw0; rp.out = reproj;
-      if ((rc = check_launch(launch_reproj(g.n0, rp, st), "reproj"))) return rc;
+      if ((rc = check_launch(launch_reproj(g.n0, reproj_args(p, S, reproj), st), "reproj"))) return rc;
     }
   }
   return ICON_OK;
@@ -637,6 +633,13 @@ RowAdjArgs icon::data_row_args(icon_plan* p, int s0, int S) {
   if (p->half) a.img_re = reinterpret_cast<float*>(p->d_ahwb) + o;
   else a.img = p->d_ahwb + o;
   zero_band(p->spread().h, &a.zlo, &a.zhi);
+  return a;
+}
+
+ReprojArgs icon::reproj_args(const icon_plan* p, int S, float* out) {
+  ReprojArgs a{};
+  a.S = S; a.N0 = p->g.N0; a.K = kTapsWide; a.sigma = p->g.sig0; a.frep = p->d_frep; a.ck = p->d_rck; a.phi = p->d_rphi;
+  a.i0 = p->d_ri0; a.tw = p->d_tw0; a.out = out;
   return a;
 }
 
@@ -880,6 +883,13 @@ int plan_create(icon_plan** out, int device, int nx, int thickness, int nz, cons
   if ((rc = upload(p, &p->d_w, g.w))) return bail(rc);
   if ((rc = upload(p, &p->d_phi1, g.phi1))) return bail(rc);
   if ((rc = upload(p, &p->d_i10, g.i10))) return bail(rc);
+  if (2 * g.N0 != g.n0) {
+    std::vector<float> ck, phi;
+    std::vector<int> first;
+    reproj_tables(g, ck, phi, first);
+    if ((rc = upload(p, &p->d_rck, ck)) || (rc = upload(p, &p->d_rphi, phi)) || (rc = upload(p, &p->d_ri0, first)))
+      return bail(rc);
+  }
   // The solve subtracts A^H W b from the exact A^H W A m in every iteration, so
   // that an error of it in the directions that no tilt covers adds up over the
   // iterations: it needs the accurate window also where the transforms use the
@@ -940,7 +950,7 @@ int icon_plan_destroy(icon_plan* p) {
   DevGuard dg(p->device);
   if (p->stream) (void)hipStreamSynchronize(p->stream);
   drop_graph(p);
-  void* ptrs[] = {p->d_nodes, p->d_ck1, p->d_w, p->d_phi1, p->d_i10,
+  void* ptrs[] = {p->d_nodes, p->d_ck1, p->d_w, p->d_phi1, p->d_i10, p->d_rck, p->d_rphi, p->d_ri0,
                   p->d_b, p->d_part, p->d_ahwb, p->d_grad, p->d_tmp, p->d_frep, p->d_rowpart,
                   p->d_bnorm, p->d_alpha, p->d_spec, p->d_nd_off, p->d_nd_ent, p->d_nd_parts, p->d_nd_xt, p->d_rsum, p->d_rcnt, p->d_nd_nslot, p->d_nd_px, p->d_nd_py,
                   p->d_epart, p->d_nq_off, p->d_nq_ent, p->d_nq_entr, p->d_nq_px, p->d_nq_py, p->d_nq_nslot,

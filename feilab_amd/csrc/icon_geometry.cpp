@@ -65,7 +65,7 @@ void taps(float c, int N, float sigma, float b, float bf, int m, float* phi, int
 // transform W sinh(a) / a, a = sqrt(beta^2 - (pi W k / n)^2), over Z) is 1
 // at k = 0 like the Gaussian's.  Computed in double, stored in float.
 double bessel_i0(double x) {
-  // power series sum_k ((x/2)^k / k!)^2; |x| <= 20 here
+  // power series sum_k ((x/2)^k / k!)^2; |x| <= 50 here
   double term = 1.0, sum = 1.0;
   const double q = 0.25 * x * x;
   for (int k = 1; k < 200 && term > 1e-17 * sum; k++) {
@@ -89,19 +89,22 @@ float deapod_kb(int k, int N, float sigma, float beta, int taps) {
   return (float)(v / kb_norm(bt, taps));
 }
 
-// Kaiser-Bessel taps of one coordinate: grid points floor(n c) - 2 .. + 3.
-void taps_kb(float c, int N, float sigma, float beta, float* phi, int* first) {
+// The K Kaiser-Bessel taps of one coordinate: grid points floor(n c) - (K/2 - 1) .. + K/2.
+void taps_kb(float c, int N, float sigma, float beta, int K, float* phi, int* first) {
   const int n = (int)std::ceil((float)N * sigma);
   const double u = (double)n * (double)c;
-  const int l0 = (int)std::floor(u) - (kTapsKB / 2 - 1);
-  const double Z = kb_norm(beta, kTapsKB);
-  for (int t = 0; t < kTapsKB; t++) {
+  const int l0 = (int)std::floor(u) - (K / 2 - 1);
+  const double Z = kb_norm(beta, K);
+  for (int t = 0; t < K; t++) {
     const double d = u - (double)(l0 + t);
-    const double r = 1.0 - (2.0 * d / kTapsKB) * (2.0 * d / kTapsKB);
+    const double r = 1.0 - (2.0 * d / K) * (2.0 * d / K);
     phi[t] = r > 0 ? (float)(bessel_i0((double)beta * std::sqrt(r)) / Z) : 0.f;
   }
   *first = ((l0 % n) + n) % n;
 }
+
+// The projection rows' node k, in the reference's float.
+float row_node(int k, int N0) { return (float)(((double)(float)k - (double)(float)N0 / 2.0) / (double)(float)N0); }
 }  // namespace
 
 float kb_beta(float sigma, int taps) {
@@ -227,7 +230,7 @@ bool build_geometry(Geometry& g, int N0, int N1, int nz, const float* tilt_deg, 
   // 2D window taps and first indices
   const int K = g.K;
   auto node_taps = [&](float c, int N, float sigma, float b, float bf, float* phi, int* first) {
-    if (kb) taps_kb(c, N, sigma, b, phi, first);
+    if (kb) taps_kb(c, N, sigma, b, kTapsKB, phi, first);
     else taps(c, N, sigma, b, bf, kWindowM, phi, first);
   };
   auto deapod_of = [&](int k, int N, float sigma, float b) {
@@ -260,11 +263,20 @@ bool build_geometry(Geometry& g, int N0, int N1, int nz, const float* tilt_deg, 
   g.phi1.resize((size_t)N0 * K);
   g.i10.resize(N0);
   for (int k = 0; k < N0; k++) {
-    const float x = (float)(((double)(float)k - (double)(float)N0 / 2.0) / (double)(float)N0);
-    node_taps(x, N0, g.sig0, g.b0, g.bf0, &g.phi1[(size_t)k * K], &g.i10[k]);
+    node_taps(row_node(k, N0), N0, g.sig0, g.b0, g.bf0, &g.phi1[(size_t)k * K], &g.i10[k]);
     g.ck1[k] = deapod_of(k - N0 / 2, N0, g.sig0, g.b0);
   }
   return true;
+}
+
+void reproj_tables(const Geometry& g, std::vector<float>& ck, std::vector<float>& phi, std::vector<int>& first) {
+  constexpr int K = kTapsWide;
+  const float beta = kb_beta(g.sig0, K);
+  ck.resize(g.N0);
+  phi.resize((size_t)g.N0 * K);
+  first.resize(g.N0);
+  kb_deapod(g.N0, g.sig0, beta, K, ck.data());
+  for (int k = 0; k < g.N0; k++) taps_kb(row_node(k, g.N0), g.N0, g.sig0, beta, K, &phi[(size_t)k * K], &first[k]);
 }
 
 // The entries of each tile in groups of 16, one of every residue of the first

@@ -161,12 +161,12 @@ struct SinoArgs {
 
 struct ReprojArgs {
   int S, N0;
-  int K;                 // window taps
+  int K;                 // window taps (N0 a power of two: no window, its tables null)
   float sigma;
   const float2* frep;    // [S][N0]
-  const float* ck1;
-  const float* phi1;
-  const int* i10;
+  const float* ck;
+  const float* phi;
+  const int* i0;
   const float2* tw;
   float* out;            // [S][N0]
 };

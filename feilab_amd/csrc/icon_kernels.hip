@@ -842,9 +842,9 @@ __device__ __forceinline__ void reproj_body(const ReprojArgs& a, int s) {
       const int kc = (int)floorf((float)u / a.sigma) + (a.N0 >> 1);
       const int klo = max(max(kc - 10, 0), kprev + 1), khi = min(kc + 10, a.N0 - 1);
       for (int k = klo; k <= khi; k++) {
-        const int d = (x - a.i10[k]) & (NR - 1);
+        const int d = (x - a.i0[k]) & (NR - 1);
         if (d < a.K) {
-          const float ph = a.phi1[(size_t)k * a.K + d];
+          const float ph = a.phi[(size_t)k * a.K + d];
           ax = __fmaf_rn(f[k].x, ph, ax);
           ay = __fmaf_rn(f[k].y, ph, ay);
         }
@@ -860,7 +860,7 @@ __device__ __forceinline__ void reproj_body(const ReprojArgs& a, int s) {
     if (out_slot_cropped<NR>(i)) continue;   // padding, as N0 <= NR/2
     const int y = out_index<NR>(t, i);
     const int X = (y + h) & (NR - 1);
-    if (X < a.N0) a.out[(size_t)s * a.N0 + X] = exact ? v[i].x : v[i].x / a.ck1[X];
+    if (X < a.N0) a.out[(size_t)s * a.N0 + X] = exact ? v[i].x : v[i].x / a.ck[X];
   }
 }
 

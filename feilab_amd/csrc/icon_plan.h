@@ -146,6 +146,9 @@ void build_bins(const Geometry& g, int C, int K, Bins& b);
 // deapodisation over N samples.
 float kb_beta(float sigma, int W);
 void kb_deapod(int N, float sigma, float beta, int W, float* out);
+// The reprojection's 1D window, kTapsWide taps: deapodisation [N0], taps [N0][K]
+// and first taps [N0].
+void reproj_tables(const Geometry& g, std::vector<float>& ck, std::vector<float>& phi, std::vector<int>& first);
 // Every tilt line's nodes but the first in exact pairs (v, -v) of equal weight.
 bool paired_nodes(const Geometry& g);
 void build_node_bins(const Geometry& g, bool half, NodeBins& b);
@@ -201,6 +204,9 @@ struct icon_plan {
   float* d_w = nullptr;
   float* d_phi1 = nullptr;
   int* d_i10 = nullptr;
+  float* d_rck = nullptr;           // the reprojection's window (null where N0 is a power of two: it needs none)
+  float* d_rphi = nullptr;
+  int* d_ri0 = nullptr;
   // the solve's normal operator (icon_normal.hip)
   bool half = false;                // paired nodes: real images on half grids
   int nq = 0;                       // ... and its unpaired nodes
@@ -280,6 +286,7 @@ RefArgs ref_args(const icon_plan* p, int s0, int S, float* m);
 RowFwdArgs rhat_row_args(const icon_plan* p, int S);
 bool refresh(const icon_plan* p, const icon_solve_opts& o, int it);
 FinishArgs finish_args(const icon_plan* p, int S);
+ReprojArgs reproj_args(const icon_plan* p, int S, float* out);
 ColArgs spread_args(icon_plan* p, int s0, int S);   // of the data set-up
 RowAdjArgs data_row_args(icon_plan* p, int s0, int S);
 }  // namespace icon
