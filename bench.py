@@ -77,9 +77,10 @@ def algorithmic_bytes(plan):
     half = N0 & (N0 - 1) == 0
     rows = 8 * N0 * (n1 // 2 + 8 if half else n1)
     nodes, img = (M // 2 if half else M), (4 if half else 8)
+    ref = 4 if n0 <= 1024 else 0   # the reference iterate of the differences
     return {
         # the update: image and Re(rhat) in, image out (f32), the reference iterate in; + the grid rows out
-        "row_fwd": 16 * N0 * N1 + rows,
+        "row_fwd": (12 + ref) * N0 * N1 + rows,
         # A^H W A along x: the grid rows in and out + the node values of the residual out
         "col_normal": 2 * rows + 8 * nodes,
         # grid rows in + A^H W b in + Re(rhat) out (f32, all the update reads) + the grid rows of rhat out

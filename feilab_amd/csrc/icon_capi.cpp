@@ -1162,6 +1162,7 @@ int icon_time_kernel(icon_plan* p, int kernel, int S, int reps, double* avg_ms) 
   rf.rows = S * g.N0; rf.N0 = g.N0; rf.N1 = g.N1; rf.cplx = 0; rf.update = 2; rf.data_type = 1;
   rf.m = reinterpret_cast<float*>(p->d_ahwb); rf.grad = p->d_grad; rf.alpha = p->d_alpha;
   rf.tw = p->d_tw1; rf.out = p->d_tmp;
+  rf.mref = p->d_mref;   // as in the iterations after the first FP64 gradient (n0 = 2048: null)
   ColArgs cn = normal_args(p, S, true);
   const ColArgs ce = energy_args(p, S);
   RowAdjArgs ra = grad_args(p, S);
