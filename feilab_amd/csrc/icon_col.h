@@ -97,8 +97,8 @@ __device__ __forceinline__ void interp_tile(const ColArgs& a, const float2* tile
   constexpr int LS = col_stride<NC, C>();
   const int tid = threadIdx.x;
   // interpolation partials of this tile's nodes: one bin entry per thread;
-  // the entry's record (first x-tap, 14 x-taps, C y-taps) comes in with
-  // vector loads and the thread sums its 14 x C cells from the LDS tile
+  // the entry's record (first x-tap, K x-taps, C y-taps) comes in with
+  // vector loads and the thread sums its K x C cells from the LDS tile
   const int e0 = a.ent_off[blk], e1 = a.ent_off[blk + 1], ne = e1 - e0;
   for (int e = e0 + part * NT + tid; e < e1; e += parts * NT) {
     const int4 en = a.fent[e];

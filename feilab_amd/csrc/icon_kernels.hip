@@ -2,11 +2,11 @@
 //
 // Data layout in HBM (S slices batched, complex = interleaved float2):
 //   m      [S][N0][N1] f32       image, index X*N1 + Y (X = width, Y = depth)
-//   rhat   [S][N0][N1] c64       gradient  A^H W (A m) - A^H W b
-//   ahwb   [S][N0][N1] c64       A^H W b
+//   grad   [S][N0][N1] f32       real part of the gradient A^H W (A m) - A^H W b
+//   ahwb   [S][N0][N1] c64       A^H W b (real images on half grids: f32)
 //   tmp    [S][N0][n1] c64       the N0 non-zero grid rows after the y-pass
 //   part   [S][M][3]   c64       interpolation partials, one per column tile
-//   fw     [S][M]      c64       weighted node values (spread input)
+//   fw     [S][E]      c64       weighted node value per bin entry (spread input)
 //   b      [S][M]      c64       Fourier-slice data
 // The oversampled grid (n0 x n1, x slow) never exists in HBM as a whole: the
 // forward transform writes only the N0 rows that the zero padding leaves
@@ -17,8 +17,8 @@
 //   k_row_fwd      nufft_fhatDivCk_assignGhat(_R2C) :754-809 + y half of cufftExecC2C
 //                  (+ ICONUpdateCU_R / INFRUpdateCU_R :1597-1639 fused in front)
 //   k_col_fwd      x half of cufftExecC2C + nufft_GPhi_p1CU_noPreCompute :669-700
-//   k_combine      nufft_GPhi_p2CU :704-727, complexMulDoubleCU :1539-1549,
-//                  alpha1/matrixAdd/alpha2 :1652-1703 (FP64), data residual
+//   k_combine      nufft_GPhi_p2CU :704-727, complexMulDoubleCU :1539-1549 (the
+//                  step size and the data residual: k_finish, icon_normal.hip)
 //   k_col_adj      cudaMemset + nufft_adjoint_fullpre_FPhi :1078-1102 + x half of
 //                  the inverse cufftExecC2C
 //   k_row_adj      y half of the inverse FFT + nufft_assignF_HAT :1104-1121 +
@@ -301,16 +301,15 @@ __global__ __launch_bounds__(RPB * (NR / 16), 2) void k_row_adj_multi(const RowA
 
 // --------------------------------------------------------------- column pass
 // One block per (slice, tile of C grid columns); the n0 x C tile lives in LDS,
-// row-major with a padded row stride of C+1 float2 so that rows map to
-// different banks.  FFT: thread (c = tid % C, t = tid / C) works on column c.
-// Interpolation: one bin entry (node, run of y-taps inside the tile) per
-// thread, summing its 14 x C cells of the tile.
-// Spread: see k_col_adj (row-owner gather, no atomics).
+// row-major with a padded row stride (col_stride).  FFT: thread (c = tid % C,
+// t = tid / C) works on column c.  Interpolation: one bin entry (node, run of
+// y-taps inside the tile) per thread, summing its K x C cells of the tile (K
+// window taps).  Spread: see col_adj_body (row-owner gather, no atomics).
 
 // A tile's bin records are interleaved by field so that a wavefront reading
 // one field of consecutive entries reads contiguous memory: for the tile's
 // entries [e0, e1), x-tap pair q of entry e is float2 number q*(e1-e0) + e-e0
-// of the block at float e0*14, and y-tap quad c4 is float4 number
+// of the block at float e0*K, and y-tap quad c4 is float4 number
 // c4*(e1-e0) + e-e0 of the block at float e0*C (K = window taps).
 template <int K>
 __device__ __forceinline__ const float2* tile_px(const ColArgs& a, int e0) {
@@ -412,7 +411,7 @@ __device__ __forceinline__ void col_adj_body(const ColArgs& a, int bid) {
     return;
   }
   // Spread as a gather.  Rows [x, x+RL) of the tile are covered by the
-  // entries with first x-tap z in [x-13, x+RL-1] (mod n0): one or two index
+  // entries with first x-tap z in [x-K+1, x+RL-1] (mod n0): one or two index
   // ranges of the tile's z-sorted list (run 0: the entries whose taps wrap
   // from the top rows, for the first K-1 rows only, else empty; run 1: the
   // rest).  The block stages the tile's records in LDS (CAP at a time) and

@@ -38,12 +38,17 @@ typedef enum {
   ICON_ERR_STATE = 5     /* call out of order (e.g. plan not prepared) */
 } icon_status;
 
-/* NUFFT window of a plan.  ICON_WINDOW_GAUSS is the reference's Gaussian,
- * m = 6, 14 taps per dimension (nufft_gpu_v8.cu:221-235); icon_plan_create
- * and icon_plan_create_cv always use it.  ICON_WINDOW_KB6 is a Kaiser-Bessel
- * window of width 6 (6 taps per dimension, beta from the oversampling
- * factor): about 5e-6 relative error per transform against the exact
- * non-uniform DFT, for about a third of the gridding work. */
+/* NUFFT window of a plan.
+ *   ICON_WINDOW_GAUSS (icon_plan_create, icon_plan_create_cv): the reference's
+ *     Gaussian, m = 6, 14 taps (nufft_gpu_v8.cu:221-235), for the projection
+ *     rows; the 2D transforms take a Kaiser-Bessel window of 10 taps per
+ *     dimension, within 1e-9 of the exact non-uniform DFT before rounding.
+ *   ICON_WINDOW_KB6: a Kaiser-Bessel window of 6 taps (beta from the
+ *     oversampling factor) for both: about 5e-6 relative error per transform;
+ *     its column kernels take 10 to 20 % less time.
+ * A solve's iteration uses neither (the normal operator is applied exactly), so
+ * the window enters it through the projection rows alone: with
+ * ICON_WINDOW_KB6 a solve is as fast and less exact. */
 typedef enum {
   ICON_WINDOW_GAUSS = 0,
   ICON_WINDOW_KB6 = 1
@@ -58,13 +63,13 @@ typedef struct {
   int32_t nz;            /* number of tilts */
   int32_t M;             /* nodes = N0 * nz */
   int32_t n0, n1;        /* oversampled grid, n = 2 * nextpow2(N) */
-  int32_t m;             /* window half-width: 6 for the Gaussian (2m+2 = 14 taps),
-                            3 for Kaiser-Bessel (2m = 6 taps) */
+  int32_t m;             /* half-width of the projection rows' window: 6 for the
+                            Gaussian (2m+2 = 14 taps), 3 for Kaiser-Bessel (2m = 6) */
   int32_t iomit;         /* first tilt of minimal |theta| (MainCode.cu:46-49) */
   float sigma0, sigma1;  /* oversampling factors, float as the reference */
-  float b0, b1;          /* window shape: Gaussian b, or Kaiser-Bessel beta */
+  float b0, b1;          /* that window's shape: Gaussian b, or Kaiser-Bessel beta */
   int32_t max_slices;    /* batch capacity */
-  int32_t col_block;     /* grid columns per spread/interp tile */
+  int32_t col_block;     /* grid columns per spread/interp tile of the transforms */
   int32_t window;        /* icon_window */
   int64_t device_bytes;  /* device memory held by the plan */
 } icon_plan_info;
@@ -223,8 +228,9 @@ int icon_batch_launches_per_iteration(const icon_batch* batch, int* launches);
 int icon_batch_autotune(icon_batch* batch, int* col_blocks);
 
 /* ---- host-only helpers (no device needed) -------------------------------- */
-/* The plan geometry computed on the host exactly as icon_plan_create does
- * (MainCode.cu:38-78, weight.cu:8-41, px2D.cu:8-47, nufft_gpu_v8.cu:22-42,
+/* The plan geometry and the reference's window tables, computed on the host
+ * (the plan's 2D transforms have records of their own window instead of phix,
+ * phiy and ck) (MainCode.cu:38-78, weight.cu:8-41, px2D.cu:8-47, nufft_gpu_v8.cu:22-42,
  * 221-235, 1242-1271).  Any output pointer may be NULL.  Sizes: nodes 2*M,
  * weights M, phix/phiy M*14, ix0/iy0 M (first wrapped tap index), ck N0*N1,
  * ck1 N0, phi1 N0*14, i10 N0; info as icon_plan_info (device fields 0). */
