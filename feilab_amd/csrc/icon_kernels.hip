@@ -830,16 +830,17 @@ __device__ __forceinline__ void reproj_body(const ReprojArgs& a, int s) {
       else v[r] = make_float2(0.f, 0.f);
       continue;
     }
-    // Nodes touching cell x sit within a few cells of x (unwrapped as x - NR
-    // for nodes near k = 0, as x otherwise); node spacing is sigma >= 2 cells,
-    // so +-10 nodes around each candidate covers every tap.  The two windows
-    // are visited in ascending k without overlap; membership is the exact
-    // wrapped-tap test.
+    // Nodes touching cell x sit within K/2 cells of x (unwrapped as x - NR for
+    // nodes near k = 0, as x otherwise); node spacing is sigma >= 2 cells, so
+    // K/4 nodes around each candidate, and two for the floor and an odd width's
+    // half node, cover every tap.  The two windows are visited in ascending k
+    // without overlap; membership is the exact wrapped-tap test.
+    const int rad = a.K / 4 + 2;
     int kprev = -1;
     for (int pass = 0; pass < 2; pass++) {
       const int u = pass == 0 ? x - NR : x;
       const int kc = (int)floorf((float)u / a.sigma) + (a.N0 >> 1);
-      const int klo = max(max(kc - 10, 0), kprev + 1), khi = min(kc + 10, a.N0 - 1);
+      const int klo = max(max(kc - rad, 0), kprev + 1), khi = min(kc + rad, a.N0 - 1);
       for (int k = klo; k <= khi; k++) {
         const int d = (x - a.i0[k]) & (NR - 1);
         if (d < a.K) {
