@@ -200,8 +200,8 @@ int icon_reconstruct_host(icon_plan* plan, int S, const float* sino, float* m, c
 /* ---- packed solve of several series ------------------------------------ */
 /* A batch packs tilt series of uneven width, thickness, tilt range and slice
  * count (one plan each, all on one device) into the same launches: every
- * kernel of the iteration runs once per size class (row length, column grid
- * and tile width) over all series of that class, and the whole solve is
+ * kernel of the iteration runs once per size class (row length or column grid,
+ * real or complex images) over all series of that class, and the whole solve is
  * replayed as one HIP graph.  Replaces the reference's per-series set-up and
  * slice loop (MainCode.cu:63-71,113-162) for a whole set of series.
  * slices[i] (<= the plan's max_slices) slices of series i are solved by
